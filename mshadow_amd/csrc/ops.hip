@@ -69,9 +69,9 @@ const size_t kPatchLdsBudget = 24 * 1024;  // per workgroup (col2im: every tap's
 /* input rows staged per workgroup: small bands, many workgroups in different phases per CU
    ((16,64,224,224) 3x3 stride 2: 117 us against 150 us with 40 KB) */
 const size_t kIm2ColLdsBudget = 16 * 1024;
-/* reductions long enough to fill the LDS ring of the direct-to-LDS kernels (which hold
-   a whole CU's LDS); shorter ones run the register-staged kernels, several per CU */
-const int kDmaMinRows = 2048;
+/* reductions long enough to fill the LDS ring of the direct-to-LDS kernels that hold a whole
+   CU's LDS; shorter ones run kernels of which several share a CU */
+const int kDmaMinRows = 8192;
 const long long kDmaMinPerKept = 1ll << 16;
 
 int MakePatchGeom(PatchGeom *g, int n, int c, int h, int w, int ky, int kx, int sy, int sx,
@@ -845,32 +845,40 @@ int mshadow_hip_reduce_keep_lowest_f32(float *dst, const float *src, int sstride
   if (cols == 0) return MSHADOW_HIP_OK;
   ABI_REQUIRE(dst != NULL && src != NULL, "NULL tensor");
   ABI_REQUIRE(sstride >= cols, "pitch smaller than the row");
-  RawPlan1D<float> d = {dst};
-  RawPlan2D<const float> sp = {src, sstride};
-  const unsigned grid = (cols + mshadow::hip::kLowestCols - 1) / mshadow::hip::kLowestCols;
   hipStream_t s = AsStream(stream);
+  const uint32_t cus = mshadow_abi::ComputeUnits();
+  const int strip = mshadow::hip::LowestColumnsPerStrip(cols, cus);
   int st = DispatchReducer(reducer, [&](auto red) {
     return DispatchSaver(saver, [&](auto sv) {
       typedef decltype(red) R;
       typedef decltype(sv) S;
-      if (rows >= kDmaMinRows) {
-        hipLaunchKernelGGL((mshadow::hip::ReduceKeepLowestDmaKernel<S, R>), dim3(grid),
+#define LOWEST_STRIP(STRIP)                                                                     \
+  hipLaunchKernelGGL((mshadow::hip::ReduceKeepLowestStripKernel<S, R, mshadow::hip::STRIP>),    \
+                     dim3((cols + mshadow::hip::STRIP::kCols - 1) / mshadow::hip::STRIP::kCols), \
+                     dim3(mshadow::hip::STRIP::kThreads), 0, s, dst, src,                       \
+                     static_cast<uint32_t>(sstride), static_cast<uint32_t>(rows),               \
+                     static_cast<uint32_t>(cols), scale)
+      if (strip == 16 && rows >= kDmaMinRows) {
+        /* a strip for each CU at most and a long chain: four rows to an LDS read and stages of
+           512 rows make its step 3.5 instead of 4.2 ns (65536 x 1000: 231 against 276 us;
+           16384 x 1000: 64 against 72 us; 4096 x 2000: 22 against 20 us) */
+        hipLaunchKernelGGL((mshadow::hip::ReduceKeepLowestDmaKernel<S, R>),
+                           dim3((cols + mshadow::hip::kLowestCols - 1) / mshadow::hip::kLowestCols),
                            dim3(mshadow::hip::kDmaThreads), 0, s, dst, src,
                            static_cast<uint32_t>(sstride), static_cast<uint32_t>(rows),
                            static_cast<uint32_t>(cols), scale);
-      } else if (rows >= 4096) {
-        hipLaunchKernelGGL(
-            (mshadow::hip::ReduceKeepLowestKernel<S, R, float, mshadow::hip::kRedBlockLarge,
-                                                  RawPlan1D<float>, RawPlan2D<const float> >),
-            dim3(grid), dim3(mshadow::hip::kRedBlockLarge), 0, s, d, sp,
-            static_cast<uint32_t>(rows), static_cast<uint32_t>(cols), scale);
+      } else if (strip == 16 && rows >= 2048) {
+        LOWEST_STRIP(LowestStrip16Long);
+      } else if (strip == 16) {
+        LOWEST_STRIP(LowestStrip16);
+      } else if (strip == 32) {
+        LOWEST_STRIP(LowestStrip32);
+      } else if (rows > 1024 || static_cast<uint32_t>(cols) <= 128 * cus) {
+        LOWEST_STRIP(LowestStrip64);
       } else {
-        hipLaunchKernelGGL(
-            (mshadow::hip::ReduceKeepLowestKernel<S, R, float, mshadow::hip::kRedBlockSmall,
-                                                  RawPlan1D<float>, RawPlan2D<const float> >),
-            dim3(grid), dim3(mshadow::hip::kRedBlockSmall), 0, s, d, sp,
-            static_cast<uint32_t>(rows), static_cast<uint32_t>(cols), scale);
+        LOWEST_STRIP(LowestStrip64Short);
       }
+#undef LOWEST_STRIP
       return MSHADOW_HIP_OK;
     });
   });

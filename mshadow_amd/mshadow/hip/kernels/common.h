@@ -22,6 +22,8 @@ namespace mshadow {
 namespace hip {
 
 const int kWave = 64;
+/*! \brief compute units of the chip, where a dispatch of the headers weighs work against them */
+const uint32_t kChipCus = 256;
 
 __device__ __forceinline__ int LaneId() { return threadIdx.x & (kWave - 1); }
 __device__ __forceinline__ int WaveId() { return threadIdx.x >> 6; }
@@ -258,12 +260,12 @@ struct SaverReadsDst<sv::saveto> {
 
 /*! \brief which piece of the work a workgroup takes. Workgroups are dealt to the 8 XCDs
  *  round-robin, and each XCD has its own L2: handing XCD k the k-th contiguous eighth of
- *  the pieces (when the count divides evenly) keeps neighbouring pieces - which share
- *  cache lines, halos or, for windowed expressions, whole operands - behind one L2. */
+ *  the pieces (the first nblocks % 8 eighths have one more) keeps neighbouring pieces - which
+ *  share cache lines, halos or, for windowed expressions, whole operands - behind one L2. */
 __device__ __forceinline__ uint32_t StripOfBlock(uint32_t block, uint32_t nblocks) {
   const uint32_t kXcd = 8;
-  if (nblocks % kXcd != 0) return block;
-  return (block % kXcd) * (nblocks / kXcd) + block / kXcd;
+  const uint32_t xcd = block % kXcd, longer = nblocks % kXcd;
+  return xcd * (nblocks / kXcd) + (xcd < longer ? xcd : longer) + block / kXcd;
 }
 
 }  // namespace hip

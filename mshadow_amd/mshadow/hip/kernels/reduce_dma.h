@@ -64,6 +64,18 @@ __device__ __forceinline__ void LoadDwordToLds(const void *gsrc_of_lane, void *l
       (const __attribute__((address_space(1))) void *)gsrc_of_lane,
       (__attribute__((address_space(3))) void *)lds_wave_base, 4, 0, kDmaCachePolicy);
 }
+template <int BYTES>
+__device__ __forceinline__ void LoadLaneToLds(const void *gsrc_of_lane, void *lds_wave_base) {
+  const __attribute__((address_space(1))) void *from =
+      (const __attribute__((address_space(1))) void *)gsrc_of_lane;
+  __attribute__((address_space(3))) void *to = (__attribute__((address_space(3))) void *)lds_wave_base;
+  if (BYTES == 16) {
+    __builtin_amdgcn_global_load_lds(from, to, 16, 0, kDmaCachePolicy);
+  } else {
+    __builtin_amdgcn_global_load_lds(from, to, 4, 0, kDmaCachePolicy);
+  }
+}
+
 /*! \brief all but the newest kAhead stages of this wave's loads have landed */
 template <typename Ring>
 __device__ __forceinline__ void WaitStageLanded() {
@@ -137,6 +149,224 @@ __global__ void __launch_bounds__(kDmaThreads)
       }
     }
     if (chain_lane) Saver::template Save<float>(dst[x0 + lane], res * scale);
+  }
+}
+
+/* ------------------------------------------------------------------ KeepLowest in strips
+ * The same roles and ring, a slot holding ROWS rows as they lie in memory. A load instruction
+ * covers one or more whole rows of the strip, so a strip of 64 floats fetches whole cache lines
+ * where the kernel above fetches 64 bytes at a time, and every lane of the chain wave has a
+ * column to add; a chain lane reads its column of one row after the other, neighbouring lanes
+ * neighbouring words. The ring is small (16 to 64 KB), so that several workgroups share a CU and
+ * a short reduction does not fetch rows it does not have.
+ *
+ * What bounds it, and hence the width of the strips: a CU's requests bring about 43 GB/s at most
+ * and a chain step takes 4.2 to 5.9 ns, so as many CUs as possible must have a strip, and as few
+ * as possible more than one round of them (LowestColumnsPerStrip). Measured, sums of floats,
+ * before (16 columns per workgroup, 128 KB ring) and now: 8192 x 32000 299 -> 174 us (6.0 TB/s),
+ * 2048 x 50257 215 -> 77 us (5.3 TB/s), 512 x 50000 78 -> 20 us, 128 x 128000 106 -> 13 us,
+ * 16384 x 8192 149 -> 87 us, 1500 x 1000 12.5 -> 10 us, 128 x 10 3.8 -> 2.8 us; binary16
+ * (register-staged kernel of reduce.h before) 8192 x 32000 260 -> 81 us, 4096 x 9000 52 -> 25 us.
+ * Sixteen bytes a lane instead of four fetch no faster (8192 x 32000: 174 us both). */
+
+/*! \brief columns of a strip by the number of columns and of CUs: narrow strips until every CU
+ *  has one (with 8192 x 6000 floats: 16 columns 52 us, 32 columns 43 us, 64 columns 52 us), wide
+ *  ones - whole cache lines - from there on (8192 x 10000: 78, 71 and 59 us) */
+inline int LowestColumnsPerStrip(uint32_t cols, uint32_t cus) {
+  return cols <= 16 * cus ? 16 : cols <= 32 * cus ? 32 : 64;
+}
+
+/*! \brief PITCH elements of a row in LDS, ROWS rows a slot. SHIFTED (16-bit elements only): rows
+ *  need not start at 4-byte borders. A load then brings the dwords that hold the strip, whose
+ *  elements sit one place further in rows that start at an odd element, and a strip has two
+ *  columns less than the pitch. */
+template <typename DType, int PITCH, int ROWS, int SLOTS, int LOADERS, int PER_LANE, bool SHIFTED>
+struct LowestStrip {
+  typedef DType Type;
+  static const bool kShifted = SHIFTED;
+  static const int kPitch = PITCH;
+  static const int kCols = SHIFTED ? PITCH - 2 : PITCH;
+  static const int kRows = ROWS;
+  static const int kSlots = SLOTS;
+  static const int kAhead = SLOTS - 2;
+  static const int kLoaders = LOADERS;
+  static const int kThreads = (LOADERS + 1) * kWave;
+  static const int kElemsPerDword = 4 / sizeof(DType);
+  static const int kLanesPerRow = PITCH / kElemsPerDword;
+  static const int kRowsPerLoad = kWave / kLanesPerRow;
+  static const int kPerWave = ROWS / kRowsPerLoad / LOADERS;
+  /*! \brief columns of a chain lane */
+  static const int kPerLane = PER_LANE;
+  static const int kChainLanes = kCols / PER_LANE;
+  static_assert(kWave % kLanesPerRow == 0 && ROWS % (kRowsPerLoad * LOADERS) == 0, "whole loads");
+  static_assert(kChainLanes <= kWave && kAhead >= 1 && kAhead * kPerWave < 64, "ring");
+  static_assert(!SHIFTED || (sizeof(DType) == 2 && PER_LANE == 1 && LOADERS % 2 == 0), "shifted rows");
+};
+typedef LowestStrip<float, 16, 64, 4, 4, 1, false> LowestStrip16;
+/*! \brief 2048 to 8191 rows: longer stages, whose first LDS reads are waited for less often
+ *  (4096 x 2000: 20.4 us, with 64 rows a stage 22.9 us, the kernel above 22.1 us) */
+typedef LowestStrip<float, 16, 256, 4, 8, 1, false> LowestStrip16Long;
+typedef LowestStrip<float, 32, 64, 4, 4, 1, false> LowestStrip32;
+typedef LowestStrip<float, 64, 64, 4, 8, 1, false> LowestStrip64;
+/*! \brief up to 1024 rows and more than two strips per CU: half the ring, twice the workgroups on
+ *  a CU (128 x 128000: 13 against 18 us; 4096 x 9000: 38 against 32 us) */
+typedef LowestStrip<float, 64, 32, 4, 4, 1, false> LowestStrip64Short;
+typedef LowestStrip<half::half_t, 32, 128, 4, 4, 1, false> LowestHalfStrip32;
+typedef LowestStrip<half::half_t, 64, 64, 4, 4, 1, false> LowestHalfStrip64;
+/*! \brief a packed add of two columns has a longer latency (5.7 ns against 4.9 ns a row) but makes
+ *  strips of whole cache lines possible: 8192 x 32000 81 against 87 us */
+typedef LowestStrip<half::half_t, 128, 32, 4, 4, 2, false> LowestHalfStrip128;
+typedef LowestStrip<half::half_t, 32, 128, 4, 4, 1, true> LowestHalfStrip30;
+typedef LowestStrip<half::half_t, 64, 64, 4, 4, 1, true> LowestHalfStrip62;
+
+/*! \brief one step of the chains of a lane: N columns side by side */
+template <typename Reducer, typename DType, int N>
+struct ChainStep {
+  static __device__ __forceinline__ void Run(expr::Pack<DType, N> &res, const expr::Pack<DType, N> &v) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) Reducer::Reduce(res.v[i], v.v[i]);
+  }
+};
+/*! \brief two binary16 sums: one packed add, which rounds each half as half_t's += does */
+template <>
+struct ChainStep<red::sum, half::half_t, 2> {
+  typedef _Float16 Pair __attribute__((ext_vector_type(2)));
+  static __device__ __forceinline__ void Run(expr::Pack<half::half_t, 2> &res,
+                                             const expr::Pack<half::half_t, 2> &v) {
+    Pair a, b;
+    __builtin_memcpy(&a, &res, sizeof(a));
+    __builtin_memcpy(&b, &v, sizeof(b));
+    a += b;
+    __builtin_memcpy(static_cast<void *>(&res), &a, sizeof(a));
+  }
+};
+
+/*! \brief fold a lane's column(s) of a slot, `count` rows (FULL: the whole slot), in order; even
+ *  rows from `even`, odd ones from `odd`. The slot is read block by block, one block ahead of the
+ *  folds; everything is unrolled, so that the waits are for exactly the block in front. `first`:
+ *  the chain starts from row 0's values, as the reference's does, not from an initial value. */
+template <typename Reducer, typename Strip, bool FULL, typename P>
+__device__ __forceinline__ void StripFold(P &res, const typename Strip::Type *even,
+                                          const typename Strip::Type *odd, int count, bool first) {
+  typedef typename Strip::Type DType;
+  const int kBlk = 16, kBlocks = Strip::kRows / kBlk;
+  static_assert(Strip::kRows % kBlk == 0, "whole blocks");
+  P v[2][kBlk];
+#pragma unroll
+  for (int k = 0; k < kBlk; ++k) {
+    v[0][k] = *reinterpret_cast<const P *>((k & 1 ? odd : even) + k * Strip::kPitch);
+  }
+#pragma unroll
+  for (int b = 0; b < kBlocks; ++b) {
+    if (b + 1 < kBlocks) {
+#pragma unroll
+      for (int k = 0; k < kBlk; ++k) {
+        v[(b + 1) & 1][k] = *reinterpret_cast<const P *>((k & 1 ? odd : even) +
+                                                         ((b + 1) * kBlk + k) * Strip::kPitch);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (!FULL && b * kBlk >= count) break;
+#pragma unroll
+    for (int k = 0; k < kBlk; ++k) {
+      if (b == 0 && k == 0 && first) {
+        res = v[0][0];
+      } else if (FULL || b * kBlk + k < count) {
+        ChainStep<Reducer, DType, Strip::kPerLane>::Run(res, v[b & 1][k]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+template <typename Saver, typename Reducer, typename Strip>
+__global__ void __launch_bounds__(Strip::kThreads)
+    ReduceKeepLowestStripKernel(typename Strip::Type *dst, const typename Strip::Type *src, uint32_t stride,
+                                uint32_t rows, uint32_t cols, typename Strip::Type scale) {
+  typedef typename Strip::Type DType;
+  const int ROWS = Strip::kRows, kSlots = Strip::kSlots, kAhead = Strip::kAhead;
+  const int kPerWave = Strip::kPerWave, N = Strip::kPerLane;
+  typedef expr::Pack<DType, Strip::kPerLane> P;
+  __shared__ MSHADOW_ALIGNED(16) DType ring[kSlots][ROWS * Strip::kPitch];
+
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  const uint32_t x0 = StripOfBlock(blockIdx.x, gridDim.x) * Strip::kCols;
+  const uint32_t nstage = (rows + ROWS - 1) / ROWS;
+  const uint32_t nstep = nstage + kAhead;
+  /* workgroups that share a CU run their chains on different SIMDs (see the split kernel below) */
+  const uint32_t chain_wave = (blockIdx.x ^ (blockIdx.x >> 8)) & 1u;
+  if (wave != chain_wave) {
+    const uint32_t lw = wave < chain_wave ? wave : wave - 1;
+    /* This lane's place in a row of the strip. Out-of-range columns and rows re-read the last valid
+       ones: never consumed. The rows of a lane's loads lie an even number of rows apart and so are
+       shifted alike: one address, moved on by a constant. */
+    const uint32_t at = lane % Strip::kLanesPerRow;
+    auto place = [&](uint32_t row) -> const char * {
+      const DType *from = src + static_cast<size_t>(row) * stride;
+      if (Strip::kShifted) {
+        const uintptr_t whole = ~static_cast<uintptr_t>(3);
+        const uintptr_t mine = (reinterpret_cast<uintptr_t>(from + x0) & whole) + at * 4u;
+        const uintptr_t last = reinterpret_cast<uintptr_t>(from + (cols - 1)) & whole;
+        return reinterpret_cast<const char *>(mine < last ? mine : last);
+      }
+      const uint32_t x = x0 + at * Strip::kElemsPerDword;
+      return reinterpret_cast<const char *>(from + (x < cols ? x : cols - Strip::kElemsPerDword));
+    };
+    const uint32_t row0 = lw * Strip::kRowsPerLoad + lane / Strip::kLanesPerRow;
+    const uint32_t step_rows = Strip::kLoaders * Strip::kRowsPerLoad;
+    const char *from = place(row0 < rows ? row0 : rows - 1);
+    const size_t step = static_cast<size_t>(step_rows) * stride * sizeof(DType);
+    for (uint32_t i = 0; i < nstep; ++i) {
+      if (i < nstage) {
+        DType *slot = ring[i % kSlots] + lw * Strip::kRowsPerLoad * Strip::kPitch;
+        const bool whole_stage = (i + 1) * ROWS <= rows;
+#pragma unroll
+        for (int q = 0; q < kPerWave; ++q) {
+          const char *p = from + q * step;
+          if (!whole_stage) {
+            const uint32_t row = i * ROWS + q * step_rows + row0;
+            p = place(row < rows ? row : rows - 1);
+          }
+          LoadLaneToLds<4>(p, slot + q * step_rows * Strip::kPitch);
+        }
+        from += kPerWave * step;
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAhead * kPerWave) : "memory");
+      } else {
+        WaitAllLanded();
+      }
+      BareBarrier();
+    }
+    return;
+  }
+  P res;
+#pragma unroll
+  for (int k = 0; k < N; ++k) res.v[k] = DType(0);
+  const uint32_t chain_lane = lane < static_cast<uint32_t>(Strip::kChainLanes) ? lane : 0;
+  uint32_t even = chain_lane * N, odd = even;
+  if (Strip::kShifted) {  // a slot has an even number of rows: the same places in every slot
+    const uint32_t first = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(src) / sizeof(DType)) + x0;
+    even += first & 1u;
+    odd += (first + stride) & 1u;
+  }
+  for (uint32_t i = 0; i < nstep; ++i) {
+    BareBarrier();
+    if (i < static_cast<uint32_t>(kAhead)) continue;
+    const uint32_t st = i - kAhead;
+    const DType *slot = ring[st % kSlots];
+    const uint32_t left = rows - st * ROWS;
+    if (left >= static_cast<uint32_t>(ROWS)) {
+      StripFold<Reducer, Strip, true>(res, slot + even, slot + odd, ROWS, st == 0);
+    } else {
+      StripFold<Reducer, Strip, false>(res, slot + even, slot + odd, static_cast<int>(left), st == 0);
+    }
+  }
+  const uint32_t x = x0 + lane * N;
+  if (lane < static_cast<uint32_t>(Strip::kChainLanes)) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      if (x + k < cols) Saver::template Save<DType>(dst[x + k], res.v[k] * scale);
+    }
   }
 }
 
@@ -269,18 +499,6 @@ typedef SplitRing<16, 8, 4, 16> HighDimSplitRingPacks;
  *  took 105 us) */
 typedef SplitRing<32, 8, 4, 16> HighDimSplitRingPacksWide;
 typedef SplitRing<32, 8, 8, 4> HighDimSplitRing;
-
-template <int BYTES>
-__device__ __forceinline__ void LoadLaneToLds(const void *gsrc_of_lane, void *lds_wave_base) {
-  const __attribute__((address_space(1))) void *from =
-      (const __attribute__((address_space(1))) void *)gsrc_of_lane;
-  __attribute__((address_space(3))) void *to = (__attribute__((address_space(3))) void *)lds_wave_base;
-  if (BYTES == 16) {
-    __builtin_amdgcn_global_load_lds(from, to, 16, 0, kDmaCachePolicy);
-  } else {
-    __builtin_amdgcn_global_load_lds(from, to, 4, 0, kDmaCachePolicy);
-  }
-}
 
 /*! \brief the counters of the split reduction: a root and kSplitLeaves leaves, each in a cache
  *  line of its own (kSplitCounterStride words apart), all zero between launches */

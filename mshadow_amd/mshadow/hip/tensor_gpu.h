@@ -1115,16 +1115,47 @@ struct ReduceRoute<Saver, Reducer, Tensor<gpu, 1, float>, Tensor<gpu, dim, float
   }
 };
 #if defined(__HIPCC__)
-/*! \brief sumall_except_dim of a half_t tensor in memory: the LDS-ring kernel of the float path
+/*! \brief reductions of a half_t tensor in memory: the LDS-ring kernels of the float path
  *  (kernels/reduce_dma.h) instantiated for 16-bit elements, a load bringing two neighbouring
- *  elements of a row. Run() returns false when the shape does not allow that (odd row length or
- *  pitch, unaligned base, little work per kept index) and the generic kernel has to do it. */
+ *  elements of a row. HighDim() returns false when the shape does not allow that (odd row length or
+ *  pitch, unaligned base, little work per kept index), Lowest() where the generic kernel is the
+ *  faster one; the generic kernel then has to do it. */
 template <typename Saver, typename Reducer, typename R, typename E>
 struct HalfRingRoute {
   template <typename... Args> static bool HighDim(Args...) { return false; }
+  template <typename... Args> static bool Lowest(Args...) { return false; }
 };
 template <typename Saver, typename Reducer, int dim>
 struct HalfRingRoute<Saver, Reducer, Tensor<gpu, 1, half::half_t>, Tensor<gpu, dim, half::half_t> > {
+  template <typename Strip>
+  static void LaunchStrip(half::half_t *d, const half::half_t *s, uint32_t stride, uint32_t rows, uint32_t cols,
+                          half::half_t scale, void *stream) {
+    void *args[] = {&d, &s, &stride, &rows, &cols, &scale};
+    Launch(hip::ReduceKeepLowestStripKernel<Saver, Reducer, Strip>, (cols + Strip::kCols - 1) / Strip::kCols,
+           Strip::kThreads, args, stream);
+  }
+  static bool Lowest(const Tensor<gpu, 1, half::half_t> &dst, const Tensor<gpu, dim, half::half_t> &src,
+                     uint32_t rows, uint32_t cols, half::half_t scale) {
+    half::half_t *d = dst.dptr_;
+    const half::half_t *s = src.dptr_;
+    const uint32_t stride = src.stride_;
+    void *stream = Stream<gpu>::GetStream(dst.stream_);
+    const int strip = hip::LowestColumnsPerStrip(cols, hip::kChipCus);
+    /* long chains, a strip of 16 columns for each CU: the generic kernel reads four rows at a time
+       from LDS (16384 x 4096: 73 us, strips 80 us) */
+    if (strip == 16 && rows >= 4096) return false;
+    if (cols % 2 != 0 || stride % 2 != 0 || reinterpret_cast<uintptr_t>(s) % 4 != 0) {
+      if (strip < 64) LaunchStrip<hip::LowestHalfStrip30>(d, s, stride, rows, cols, scale, stream);
+      else LaunchStrip<hip::LowestHalfStrip62>(d, s, stride, rows, cols, scale, stream);
+    } else if (strip < 64) {
+      LaunchStrip<hip::LowestHalfStrip32>(d, s, stride, rows, cols, scale, stream);
+    } else if (cols <= 64 * hip::kChipCus) {
+      LaunchStrip<hip::LowestHalfStrip64>(d, s, stride, rows, cols, scale, stream);
+    } else {
+      LaunchStrip<hip::LowestHalfStrip128>(d, s, stride, rows, cols, scale, stream);
+    }
+    return true;
+  }
   static bool HighDim(const Tensor<gpu, 1, half::half_t> &dst, const Tensor<gpu, dim, half::half_t> &src,
                       uint32_t n_out, uint32_t n_keep, uint32_t n_y, uint32_t n_x,
                       half::half_t scale) {
@@ -1208,10 +1239,15 @@ inline void MapReduceKeepLowest(TRValue<R, gpu, 1, DType> *dst,
   SPlan splan = expr::MakePlan(exp.self());
   uint32_t rows = eshape[0], cols = eshape[1];
   if (cols == 0) return;
+  if (gpu_detail::HalfRingRoute<Saver, Reducer, R, E>::Lowest(dst->self(), exp.self(), rows, cols, scale)) {
+    return;
+  }
   void *args[] = {&dplan, &splan, &rows, &cols, &scale};
   void *stream = Stream<gpu>::GetStream(expr::StreamInfo<gpu, R>::Get(dst->self()));
   const uint32_t strips = (cols + hip::kLowestCols - 1) / hip::kLowestCols;
-  if (rows >= 4096) {
+  /* the large workgroup has a CU to itself: only where every CU gets at most one (binary16
+     16384 x 4096: 73 against 86 us; 8192 x 32000: 260 against 180 us) */
+  if (rows >= 4096 && strips <= hip::kChipCus) {
     gpu_detail::Launch(hip::ReduceKeepLowestKernel<Saver, Reducer, DType, hip::RedBlockLargeFor<DType>::value,
                                                    DPlan, SPlan>,
                        strips, hip::RedBlockLargeFor<DType>::value, args, stream);
