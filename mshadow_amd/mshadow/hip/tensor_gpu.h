@@ -28,6 +28,7 @@
 #include "./kernels/reduce_dma.h"
 #include "./kernels/rows_by_index.h"
 #include "./kernels/softmax_any.h"
+#include "./kernels/softmax_half.h"
 #include "./kernels/sort_any.h"
 #endif
 
@@ -177,24 +178,64 @@ inline bool AnyPackable(const DType *a, uint32_t astride, const DType *b, uint32
 }  // namespace gpu_detail
 namespace gpu_detail {
 #if defined(__HIPCC__)
-/*! \brief long half_t rows: one workgroup per row, the row kept in registers; false = not
- *  this shape or element type */
+template <typename K>
+inline void Launch(K kernel, uint32_t grid_x, uint32_t block_x, void **args, void *stream) {
+  const uint32_t grid[3] = {grid_x, 1, 1};
+  const uint32_t block[3] = {block_x, 1, 1};
+  MSHADOW_HIP_CALL(mshadow_hip_launch(reinterpret_cast<const void *>(kernel), grid, block, args, 0,
+                                      stream));
+}
+
+/*! \brief half_t rows that are kept in registers, a workgroup of as many waves as hold one; false =
+ *  not this shape or element type */
 template <typename DType>
-inline bool SoftmaxLongRows(DType *, uint32_t, const DType *, uint32_t, uint32_t, uint32_t, bool, void *) {
+inline bool SoftmaxRowsOnChip(DType *, uint32_t, const DType *, uint32_t, uint32_t, uint32_t, void *) {
   return false;
 }
-inline bool SoftmaxLongRows(half::half_t *d, uint32_t dstride, const half::half_t *s, uint32_t sstride,
-                            uint32_t rows, uint32_t cols, bool vec, void *stream) {
-  if (cols < static_cast<uint32_t>(hip::kHalfRowMinCols) ||
-      cols > static_cast<uint32_t>(hip::kHalfRowMaxCols)) {
+template <int WAVES, int PACKS>
+inline void LaunchHalfRows(uint32_t rows, void **args, void *stream) {
+  Launch(hip::SoftmaxHalfRowKernel<WAVES, PACKS>, rows, WAVES * hip::kWave, args, stream);
+}
+inline bool SoftmaxRowsOnChip(half::half_t *d, uint32_t dstride, const half::half_t *s, uint32_t sstride,
+                              uint32_t rows, uint32_t cols, void *stream) {
+  /* a row costs a wave its walk however short it is, so the shortest rows stay with the kernel that
+     adds eight rows side by side (131072 rows of 256: 96 against 112 us; of 512: 160 against 133 us),
+     unless it would fetch them element by element (of 101: 112 against 113 us; of 129: 117 against 105 us) */
+  const bool packs = AnyPackable(s, sstride, const_cast<const half::half_t *>(d), dstride, cols, hip::kAnyTile);
+  if (cols <= (packs ? 256u : 128u)) return false;
+  /* what a wave has to hold where rows start at any column of an aligned pack */
+  const bool aligned = (reinterpret_cast<uintptr_t>(s) | sstride * sizeof(half::half_t)) % 16 == 0;
+  const uint32_t reach = aligned ? cols : cols + hip::kHalfPack - 1;
+  const uint32_t runs = (reach + hip::kHalfRun - 1) / hip::kHalfRun;
+  void *args[] = {&d, &dstride, &s, &sstride, &cols};
+  /* As few waves as hold the row: a wave more is a link more in the walk. Waves of 8 runs (72
+     registers, 20 to a CU) as long as four of them do: 16384 x 12000 162 us with three, 176 with
+     four, 184 with two of 16 runs (114 registers, 16 to a CU); 8192 x 16000 109 us with four of 8,
+     119 with two of 16; from there on four of 16 and eight of 8 are level (8192 x 32000: 230 and
+     235 us). Few packs for short rows: 65536 x 1000 97 us with two, 105 with four, 140 with 16. */
+  if (runs <= 2) {
+    LaunchHalfRows<1, 2>(rows, args, stream);
+  } else if (runs <= 4) {
+    LaunchHalfRows<1, 4>(rows, args, stream);
+  } else if (runs <= 8) {
+    LaunchHalfRows<1, 8>(rows, args, stream);
+  } else if (runs <= 16) {
+    LaunchHalfRows<2, 8>(rows, args, stream);
+  } else if (runs <= 24) {
+    LaunchHalfRows<3, 8>(rows, args, stream);
+  } else if (runs <= 32) {
+    LaunchHalfRows<4, 8>(rows, args, stream);
+  } else if (runs <= 48) {
+    LaunchHalfRows<3, 16>(rows, args, stream);
+  } else if (runs <= 64) {
+    LaunchHalfRows<4, 16>(rows, args, stream);
+  } else if (runs <= 128) {
+    LaunchHalfRows<8, 16>(rows, args, stream);
+  } else if (runs <= 256) {
+    LaunchHalfRows<16, 16>(rows, args, stream);
+  } else {
     return false;
   }
-  void *args[] = {&d, &dstride, &s, &sstride, &cols};
-  const uint32_t grid[3] = {rows, 1, 1};
-  const uint32_t block[3] = {static_cast<uint32_t>(hip::kHalfRowBlock), 1, 1};
-  const void *kernel = vec ? reinterpret_cast<const void *>(hip::SoftmaxHalfRowKernel<true>)
-                           : reinterpret_cast<const void *>(hip::SoftmaxHalfRowKernel<false>);
-  MSHADOW_HIP_CALL(mshadow_hip_launch(kernel, grid, block, args, 0, stream));
   return true;
 }
 #endif
@@ -208,10 +249,7 @@ inline void Softmax(Tensor<gpu, 2, DType> dst, const Tensor<gpu, 2, DType> &src)
   DType *d = dst.dptr_;
   const DType *s = src.dptr_;
   uint32_t dstride = dst.stride_, sstride = src.stride_;
-  if (gpu_detail::SoftmaxLongRows(d, dstride, s, sstride, rows, cols,
-                                  gpu_detail::AnyPackable(s, sstride, const_cast<const DType *>(d),
-                                                          dstride, cols, hip::kAnyTile),
-                                  Stream<gpu>::GetStream(dst.stream_))) {
+  if (gpu_detail::SoftmaxRowsOnChip(d, dstride, s, sstride, rows, cols, Stream<gpu>::GetStream(dst.stream_))) {
     return;
   }
   void *args[] = {&d, &dstride, &s, &sstride, &rows, &cols};
@@ -931,14 +969,6 @@ inline uint32_t RowsPerLaunch(uint32_t units) {
 }
 
 #if defined(__HIPCC__)
-template <typename K>
-inline void Launch(K kernel, uint32_t grid_x, uint32_t block_x, void **args, void *stream) {
-  const uint32_t grid[3] = {grid_x, 1, 1};
-  const uint32_t block[3] = {block_x, 1, 1};
-  MSHADOW_HIP_CALL(mshadow_hip_launch(reinterpret_cast<const void *>(kernel), grid, block, args, 0,
-                                      stream));
-}
-
 /*! \brief generic elementwise evaluation: pack kernel when the plan allows, else scalar */
 template <typename Saver, typename DType, typename DPlan, typename SPlan, bool kPackable>
 struct MapLauncher {

@@ -1,0 +1,105 @@
+"""Softmax on half_t rows kept on chip: every width of workgroup the dispatch takes, at its first and
+last column and at rows that start at any column of an aligned pack, for rows of every kind the sum
+in 16 bits can meet. Bit-exact against the oracle."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from checkers import Checker
+from gpu_util import f32
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def G():
+    import mshadow_amd
+    g = mshadow_amd.load_cases()
+    g.set_device(0)
+    return g
+
+
+@pytest.fixture(scope="module")
+def O():
+    return Checker("orc")
+
+
+def part(buf, cols, shift):
+    """the `cols` columns of a device buffer from column `shift` on"""
+    return SimpleNamespace(ptr=buf.ptr + shift * buf.dtype.itemsize, stride=buf.stride, rows=buf.rows, cols=cols,
+                           dtype=buf.dtype, shape=(buf.rows, cols))
+
+
+def logits(kind, rows, cols):
+    rng = np.random.default_rng(cols)
+    x = rng.standard_normal((rows, cols), dtype=f32) * f32({"flat": 0.1, "wide": 6.0}.get(kind, 3.0))
+    if kind == "equal":
+        x[:] = f32(-0.5)
+    elif kind == "rising":
+        x = np.sort(x, axis=1)
+    elif kind == "ties":      # terms 1, 1/2, 3/8, ... of few bits: half-way cases all along
+        x = np.log(rng.choice(np.array([1, 0.75, 0.5, 0.375, 0.0625], f32), (rows, cols))).astype(f32)
+    elif kind == "late":      # nothing but zero terms in front of the largest
+        x[:, : cols // 2] = -np.inf
+    return x
+
+
+def check(G, O, x, shift, dst_shift):
+    rows, cols = x.shape
+    x = O.float2half(x)
+    want = np.empty_like(x)
+    O.softmax(want, x)
+    wide = np.full((rows, cols + 9), 0x3c00, np.uint16)
+    wide[:, shift:shift + cols] = x
+    src, dst = G.to_device(wide), G.to_device(np.full((rows, cols + 9), 0x1234, np.uint16))
+    G.case_softmax(part(dst, cols, dst_shift), part(src, cols, shift))
+    got = dst.download()
+    inside = got[:, dst_shift:dst_shift + cols]
+    nan = np.isnan(O.half2float(want))
+    assert np.array_equal(np.isnan(O.half2float(inside)), nan)
+    assert np.array_equal(inside[~nan], want[~nan]), f"{np.count_nonzero(inside != want)} of {want.size} differ"
+    assert np.all(got[:, :dst_shift] == 0x1234) and np.all(got[:, dst_shift + cols:] == 0x1234), "written outside"
+    G.case_softmax(part(src, cols, shift), part(src, cols, shift))  # in place
+    assert np.array_equal(src.download()[:, shift:shift + cols], inside)
+
+
+# 129: the shortest; runs of 512 columns in one, two, three, four waves of eight, three, four, eight and
+# sixteen of sixteen; one column more than the longest goes to the kernel of other lengths
+COLS = [129, 264, 505, 512, 1024, 1025, 2049, 4090, 4097, 8192, 8193, 12288, 12290, 16384, 16385, 24577, 32761, 32769,
+        65529, 65537, 131065, 131066, 131072]
+
+
+@pytest.mark.parametrize("cols", COLS)
+def test_half_rows_widths(G, O, cols):
+    rows = 2 if cols > 20000 else 5
+    for shift, dst_shift in ((0, 0), (1, 1), (5, 2), (8, 0)):
+        check(G, O, logits("normal", rows, cols), shift, dst_shift)
+
+
+@pytest.mark.parametrize("kind", ["flat", "wide", "equal", "rising", "ties", "late"])
+@pytest.mark.parametrize("cols", [300, 1500, 5000, 15000, 31000, 50257])
+def test_half_rows_kinds(G, O, cols, kind):
+    check(G, O, logits(kind, 3, cols), 0, 0)
+
+
+def test_half_rows_special_values(G, O):
+    """a NaN anywhere, an infinite maximum and rows of -infinity make every result of the row NaN"""
+    x = logits("normal", 7, 3000)
+    x[0, 0], x[1, 2999], x[2, 1234], x[3, 77], x[4, 5] = np.nan, np.nan, np.nan, np.inf, -np.inf
+    x[5] = -np.inf
+    check(G, O, x, 3, 3)
+
+
+def test_half_rows_every_exponential(G, O):
+    """x - max takes every binary16 value from -0 down to -infinity: one wrong exponential shows in its
+    quotient. Rows of 4096 of them, the largest first, so that the sum keeps its bits."""
+    every = np.arange(0x8000, 0x7c01 + 0x8000, dtype=np.uint32).astype(np.uint16)
+    d = O.half2float(every).astype(f32)
+    rows = -(-d.size // 4095)
+    x = np.full((rows, 4096), -np.inf, f32)
+    x[:, 0] = 0.0
+    for r in range(rows):
+        piece = d[r * 4095:(r + 1) * 4095]
+        x[r, 1:1 + piece.size] = piece
+    check(G, O, x, 0, 0)
