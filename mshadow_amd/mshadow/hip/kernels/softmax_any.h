@@ -29,6 +29,7 @@
 #ifndef MSHADOW_HIP_KERNELS_SOFTMAX_ANY_H_
 #define MSHADOW_HIP_KERNELS_SOFTMAX_ANY_H_
 
+#include "../../core/fastdiv.h"
 #include "../../half.h"
 #include "./common.h"
 
@@ -87,12 +88,25 @@ __device__ __forceinline__ void ChainAdd(half::half_t &sum, const half::half_t &
   sum.half_ = __builtin_bit_cast(uint16_t, static_cast<_Float16>(a + b));
 }
 
-/*! \brief elements [x, x + kAnyTile) of a row; VEC: whole aligned packs only */
+/*! \brief sixteen bytes at an address aligned only to a 16-bit element, which costs no more than the
+ *  cache lines it touches */
+typedef uint32_t AnyWords __attribute__((ext_vector_type(4)));
+typedef AnyWords AnyLooseWords __attribute__((aligned(2)));
+/*! \brief elements [x, x + kAnyTile) of a row, the last of a row that is not whole packs element by
+ *  element (VEC: whole aligned packs only). Of 131072 x 101 half_t the Softmax took 112 us with every
+ *  pack of such rows taken apart, 4096 x 50257 the gradient 408 us. */
 template <typename DType, bool VEC>
 __device__ __forceinline__ void LoadAnyPack(AnyPack<DType> *p, const DType *row, uint32_t x,
                                             uint32_t cols, DType absent) {
   if (VEC) {
     *p = *reinterpret_cast<const AnyPack<DType> *>(row + x);
+  } else if (x + kAnyTile <= cols) {
+    AnyWords w[sizeof(AnyPack<DType>) / sizeof(AnyWords)];
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(w) / sizeof(w[0]); ++i) {
+      w[i] = reinterpret_cast<const AnyLooseWords *>(row + x)[i];
+    }
+    __builtin_memcpy(static_cast<void *>(p), w, sizeof(w));
   } else {
 #pragma unroll
     for (int i = 0; i < kAnyTile; ++i) p->v[i] = (x + i < cols) ? row[x + i] : absent;
@@ -103,6 +117,13 @@ __device__ __forceinline__ void StoreAnyPack(DType *row, uint32_t x, uint32_t co
                                              const AnyPack<DType> &p) {
   if (VEC) {
     *reinterpret_cast<AnyPack<DType> *>(row + x) = p;
+  } else if (x + kAnyTile <= cols) {
+    AnyWords w[sizeof(AnyPack<DType>) / sizeof(AnyWords)];
+    __builtin_memcpy(w, &p, sizeof(w));
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(w) / sizeof(w[0]); ++i) {
+      reinterpret_cast<AnyLooseWords *>(row + x)[i] = w[i];
+    }
   } else {
 #pragma unroll
     for (int i = 0; i < kAnyTile; ++i) {
@@ -295,34 +316,55 @@ __device__ __forceinline__ DType GradElement(const DType &p, bool at_label, bool
   return p;
 }
 
-/*! \brief dst = the gradient FLAGS selects for probabilities src and labels label; a label
- *  outside the row marks no column. blockIdx.x = row, blockIdx.y = stretch of columns; a
- *  thread moves packs of kAnyTile elements. VEC as for SoftmaxAnyKernel. */
-template <typename DType, bool VEC, int FLAGS>
+/*! \brief a pack of the gradient FLAGS selects for probabilities src and the row's label k; a label
+ *  outside the row marks no column */
+template <typename DType, int FLAGS>
+__device__ __forceinline__ void GradPack(DType *o, const DType *s, uint32_t x, uint32_t cols, int k,
+                                         int ignore_k, float alpha, float smooth) {
+  AnyPack<DType> v;
+  LoadAnyPack<DType, false>(&v, s, x, cols, DType(0.0f));
+  const bool ignored = (FLAGS & kAnyGradIgnore) && k == ignore_k;
+  const uint32_t off = static_cast<uint32_t>(k) - x;  // wraps for k < x
+  const bool label_here = k >= 0 && off < static_cast<uint32_t>(kAnyTile);
+  if (FLAGS != 0 || label_here) {
+#pragma unroll
+    for (int i = 0; i < kAnyTile; ++i) {
+      v.v[i] = GradElement<DType, FLAGS>(v.v[i], label_here && static_cast<uint32_t>(i) == off,
+                                         ignored, alpha, smooth);
+    }
+  }
+  StoreAnyPack<DType, false>(o, x, cols, v);
+}
+/*! \brief blockIdx.x = row, blockIdx.y = stretch of columns; a thread moves packs of kAnyTile */
+template <typename DType, int FLAGS>
 __global__ void __launch_bounds__(kAnyBlock)
     SoftmaxGradAnyKernel(DType *dst, uint32_t dstride, const DType *src, uint32_t sstride,
                          const DType *label, uint32_t cols, int ignore_k, float alpha,
                          float smooth) {
   const uint32_t row = blockIdx.x;
   const int k = LabelIndex(label[row]);
-  const bool ignored = (FLAGS & kAnyGradIgnore) && k == ignore_k;
   const DType *s = src + static_cast<size_t>(row) * sstride;
   DType *o = dst + static_cast<size_t>(row) * dstride;
   const uint32_t step = gridDim.y * kAnyBlock * kAnyTile;
   for (uint32_t x = (blockIdx.y * kAnyBlock + threadIdx.x) * kAnyTile; x < cols; x += step) {
-    AnyPack<DType> v;
-    LoadAnyPack<DType, VEC>(&v, s, x, cols, DType(0.0f));
-    const uint32_t off = static_cast<uint32_t>(k) - x;  // wraps for k < x
-    const bool label_here = k >= 0 && off < static_cast<uint32_t>(kAnyTile);
-    if (FLAGS != 0 || label_here) {
-#pragma unroll
-      for (int i = 0; i < kAnyTile; ++i) {
-        v.v[i] = GradElement<DType, FLAGS>(v.v[i], label_here && static_cast<uint32_t>(i) == off,
-                                           ignored, alpha, smooth);
-      }
-    }
-    StoreAnyPack<DType, VEC>(o, x, cols, v);
+    GradPack<DType, FLAGS>(o, s, x, cols, k, ignore_k, alpha, smooth);
   }
+}
+/*! \brief the same for rows of up to kAnyGradShort columns, where a workgroup per row leaves most of
+ *  its threads idle: a workgroup takes kAnyBlock / packs consecutive rows of `packs` = ceil(cols /
+ *  kAnyTile) packs each (`div_packs` divides by it), a thread one pack */
+const uint32_t kAnyGradShort = 1024;
+template <typename DType, int FLAGS>
+__global__ void __launch_bounds__(kAnyBlock)
+    SoftmaxGradAnyShortKernel(DType *dst, uint32_t dstride, const DType *src, uint32_t sstride,
+                              const DType *label, uint32_t cols, int ignore_k, float alpha, float smooth,
+                              uint32_t rows, uint32_t rows_per_block, FastDivU32 div_packs) {
+  const uint32_t r = div_packs.Div(threadIdx.x);
+  const uint32_t row = blockIdx.x * rows_per_block + r;
+  if (r >= rows_per_block || row >= rows) return;
+  const uint32_t x = (threadIdx.x - r * div_packs.div) * kAnyTile;
+  GradPack<DType, FLAGS>(dst + static_cast<size_t>(row) * dstride, src + static_cast<size_t>(row) * sstride,
+                         x, cols, LabelIndex(label[row]), ignore_k, alpha, smooth);
 }
 
 /* ---- tensors of three dimensions (d0, d1, d2): the softmax runs over the middle one

@@ -290,19 +290,21 @@ inline void AnyGrad2D(const Tensor<gpu, 2, DType> &dst, const Tensor<gpu, 2, DTy
   const DType *l = label.dptr_;
   uint32_t dstride = dst.stride_, sstride = src.stride_;
   float smooth = SmoothShare(alpha, dst.size(1));
-  void *args[] = {&d, &dstride, &s, &sstride, &l, &cols, &ignore_k, &alpha, &smooth};
-  /* rows on the grid's x axis (up to 2^31 - 1), a row's packs over a few workgroups */
-  const uint32_t per_block = hip::kAnyBlock * hip::kAnyTile;
-  uint32_t per_row = (cols + per_block - 1) / per_block;
+  /* several short rows to a workgroup, a long one over a few workgroups (65536 x 300 half_t: 39 us a
+     workgroup per row, 15 us) */
+  const bool several = cols <= hip::kAnyGradShort;
+  const uint32_t packs = (cols + hip::kAnyTile - 1) / hip::kAnyTile;
+  uint32_t rows_per_block = several ? hip::kAnyBlock / packs : 1u;
+  FastDivU32 div_packs(packs);
+  void *args[] = {&d, &dstride, &s, &sstride, &l, &cols, &ignore_k, &alpha, &smooth, &rows, &rows_per_block, &div_packs};
+  uint32_t per_row = several ? 1u : (packs + hip::kAnyBlock - 1) / hip::kAnyBlock;
   if (per_row > 64) per_row = 64;
-  const uint32_t grid[3] = {rows, per_row, 1};
+  const uint32_t grid[3] = {(rows - 1) / rows_per_block + 1, per_row, 1};  // rows up to 2^31 - 1 on the x axis
   const uint32_t block[3] = {static_cast<uint32_t>(hip::kAnyBlock), 1, 1};
-  const bool vec = AnyPackable(s, sstride, const_cast<const DType *>(d), dstride, cols,
-                               hip::kAnyTile);
   const void *kernel = NULL;
-#define MSHADOW_ANY_GRAD(FLAGS)                                                              \
-  kernel = vec ? reinterpret_cast<const void *>(hip::SoftmaxGradAnyKernel<DType, true, FLAGS>) \
-               : reinterpret_cast<const void *>(hip::SoftmaxGradAnyKernel<DType, false, FLAGS>)
+#define MSHADOW_ANY_GRAD(FLAGS)                                                                      \
+  kernel = several ? reinterpret_cast<const void *>(hip::SoftmaxGradAnyShortKernel<DType, FLAGS>)    \
+                   : reinterpret_cast<const void *>(hip::SoftmaxGradAnyKernel<DType, FLAGS>)
   switch (flags) {
     case 0: MSHADOW_ANY_GRAD(0); break;
     case 1: MSHADOW_ANY_GRAD(1); break;

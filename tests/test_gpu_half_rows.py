@@ -1,6 +1,6 @@
 """Softmax on half_t rows kept on chip: every width of workgroup the dispatch takes, at its first and
 last column and at rows that start at any column of an aligned pack, for rows of every kind the sum
-in 16 bits can meet. Bit-exact against the oracle."""
+in 16 bits can meet; its gradient on rows of any length and start. Bit-exact against the oracle."""
 from types import SimpleNamespace
 
 import numpy as np
@@ -103,3 +103,21 @@ def test_half_rows_every_exponential(G, O):
         piece = d[r * 4095:(r + 1) * 4095]
         x[r, 1:1 + piece.size] = piece
     check(G, O, x, 0, 0)
+
+
+@pytest.mark.parametrize("rows,cols", [(300, 1), (300, 7), (300, 8), (513, 9), (129, 33), (65, 511), (33, 1000), (9, 1024),
+                                       (9, 1025), (5, 2047), (3, 4097), (2, 50257)])
+def test_half_gradient_rows(G, O, rows, cols):
+    rng = np.random.default_rng(rows)
+    prob = O.float2half(rng.random((rows, cols), dtype=f32))
+    lab = rng.integers(-1, min(cols, 2048) + 1, rows).astype(f32)   # a few outside the row
+    want = np.empty_like(prob)
+    O.softmax_grad(want, prob, O.float2half(lab))
+    for shift in (0, 1, 6):
+        wide = np.zeros((rows, cols + 7), np.uint16)
+        wide[:, shift:shift + cols] = prob
+        src, dst = G.to_device(wide), G.to_device(np.full_like(wide, 0x1234))
+        G.case_softmax_grad(part(dst, cols, 7 - shift), part(src, cols, shift), G.to_device(O.float2half(lab)))
+        got = dst.download()
+        assert np.array_equal(got[:, 7 - shift:7 - shift + cols], want)
+        assert np.all(got[:, :7 - shift] == 0x1234) and np.all(got[:, 7 - shift + cols:] == 0x1234)
