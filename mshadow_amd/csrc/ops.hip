@@ -987,9 +987,11 @@ static SlideGeom MakeSlideGeom(int planes, int rows, int w) {
   SlideGeom sg;
   sg.groups = static_cast<uint32_t>((w + 3) / 4);
   sg.strips_per_wave = 64u / sg.groups;
-  uint32_t r = 16;
+  /* equal strips of up to 16 rows (65 rows as 5 x 13, not 4 x 16 and one: 63 against 70 us) */
+  const uint32_t least = static_cast<uint32_t>((rows + 15) / 16);
+  uint32_t r = (static_cast<uint32_t>(rows) + least - 1) / least;
   const long long want = 16ll * mshadow_abi::ComputeUnits();  // waves
-  while (r > 2 && static_cast<long long>(planes) * ((rows + r - 1) / r) / sg.strips_per_wave < want) r /= 2;
+  while (r > 2 && static_cast<long long>(planes) * ((rows + r - 1) / r) / sg.strips_per_wave < want) r = (r + 1) / 2;
   sg.strip_rows = r;
   sg.strips_per_plane = static_cast<uint32_t>((rows + r - 1) / r);
   sg.total_strips = static_cast<uint32_t>(planes) * sg.strips_per_plane;
@@ -1040,9 +1042,15 @@ int mshadow_hip_pool_f32(float *dst, int dstride, const float *src, int sstride,
     case MSHADOW_HIP_MAX: hipLaunchKernelGGL((KERNEL<MSHADOW_HIP_MAX>), __VA_ARGS__); break;    \
     default: hipLaunchKernelGGL((KERNEL<MSHADOW_HIP_MIN>), __VA_ARGS__); break;                 \
   }
-  /* small planes: several whole planes per workgroup, about 24 KB of them */
+  /* windows that move by one element, all of them whole: PoolColumnsS1Kernel below has a variant */
+  const bool columns = sy == 1 && sx == 1 && ky == kx && (ky == 2 || ky == 3 || ky == 5) &&
+                       ph <= h - ky + 1 && pw <= w - kx + 1;
+  /* small planes: several whole planes per workgroup, about 24 KB of them. Planes of 1024 pixels and
+     more keep the threads of the columns kernel busy (12 M pixels, 5x5: 50x50 24 against 35 us, 3x3:
+     100x30 21 against 28 us; level at 32x32, and 7x7 is 16 us here against 312 us there), but for the
+     small windows on very narrow ones (3x3: 224x7 21 us here, 24 us there). */
   const long long plane_bytes = static_cast<long long>(h) * row_bytes;
-  if (plane_bytes * 2 <= 24 * 1024 && planes >= 2) {
+  if (plane_bytes * 2 <= 24 * 1024 && planes >= 2 && !(columns && band >= 1 && h * w >= 1024 && (ky == 5 || w >= 16))) {
     long long per_block = (24 * 1024) / plane_bytes;
     /* ... but no fewer workgroups than keep every CU busy four times over */
     while (per_block > 1 && (planes + per_block - 1) / per_block < 4ll * mshadow_abi::ComputeUnits()) {
@@ -1069,6 +1077,7 @@ int mshadow_hip_pool_f32(float *dst, int dstride, const float *src, int sstride,
   }
       if (ky == 3 && kx == 3) { POOL_PLANES(3, 3) }
       else if (ky == 2 && kx == 2) { POOL_PLANES(2, 2) }
+      else if (ky == 5 && kx == 5) { POOL_PLANES(5, 5) }
       else { POOL_PLANES(0, 0) }
 #undef POOL_PLANES
       return AfterLaunch("pool");
@@ -1083,8 +1092,7 @@ int mshadow_hip_pool_f32(float *dst, int dstride, const float *src, int sstride,
     /* windows that move by one element: a thread walks down an output column, KX reads of LDS an
        output. The band's rows are cut into `nruns` runs so that the columns of all runs fill the
        workgroup's threads in as few, as short rounds as can be. */
-    if (sy == 1 && sx == 1 && ky == kx && (ky == 2 || ky == 3 || ky == 5) && ph <= h - ky + 1 &&
-        pw <= w - kx + 1) {
+    if (columns) {
       int nruns = 1, run_len = g.band;
       long long best = -1;
       for (int n = 1; n <= g.band; ++n) {
@@ -1196,10 +1204,17 @@ int mshadow_hip_unpool_f32(float *dst, int dstride, const float *src, int sstrid
 #undef UNPOOL_ROWS
     return AfterLaunch("unpool");
   }
-  /* 2 x 2 and 3 x 3 windows with stride 1 on planes of 64 to 256 pixels a side: no staging, the
-     pooled rows over the current source row in registers ((128,64,112,112): 368 us against 513 us
-     for the kernels below; on planes of 57 x 57 the two are level, below that the staged ones win) */
-  if (ky == kx && (ky == 2 || ky == 3 || ky == 5) && sy == 1 && sx == 1 && w >= 64 && w <= 256 && h >= 64 && ph >= 1 && pw >= 1 &&
+  /* 2 x 2, 3 x 3 and 5 x 5 windows with stride 1 on rows of up to 256 pixels: no staging, the pooled
+     rows over the current source row in registers ((128,64,112,112) 3 x 3: 368 us against 513 us for
+     the kernels below). A lane has four pixels of a row, so narrow planes make its accesses short
+     and scattered, which the staged kernels do not mind; what those mind is many windows a pixel.
+     12 M pixels: 3 x 3 56x56 54 us against 51, 63x70 58 against 52, 20x200 46 against 56; 2 x 2 28x28 74 against 64,
+     56x56 50 against 65; 5 x 5 13x13 145 against 127, 16x16 76 against 103, 8x40 72 against 123,
+     28x28 83 against 106, and beyond 4 KB a plane - one plane per workgroup there - 100x14 119 against
+     317, 224x7 251 against 472. */
+  const bool slides = ky == 5 ? static_cast<long long>(h) * w > 1024 || w >= 24 || (w >= 16 && w % 4 == 0)
+                      : ky == 2 ? w >= 32 : w >= 64 && (h >= 64 || (w >= 96 && h >= 16));
+  if (ky == kx && (ky == 2 || ky == 3 || ky == 5) && sy == 1 && sx == 1 && w <= 256 && slides && ph >= 1 && pw >= 1 &&
       static_cast<long long>(planes) * ph * pw >= 4 && static_cast<long long>(planes) * ((h + 1) / 2) < (1ll << 31)) {
     SlideGeom sg = MakeSlideGeom(planes, h, w);
     sg.src_floats = (static_cast<size_t>(planes) * h - 1) * sstride + w;
