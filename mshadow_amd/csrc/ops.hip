@@ -442,24 +442,45 @@ static int LaunchRowsByIndex(float *dst, int dstride, int k_rows, const void *ro
 }
 
 namespace {
-/*! \brief rows of at most 256 columns: one thread per row up to 32 columns, one wave per row
- *  above (1, 2 or 4 columns per lane) */
+/*! \brief rows that a thread, a part of a wave or a wave takes; false: longer ones, which take a
+ *  workgroup */
 template <bool TERMS_GIVEN>
-void LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, int rows, int cols,
+bool LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, int rows, int cols,
                         hipStream_t s) {
-  if (cols <= 32) {
-    hipLaunchKernelGGL((SoftmaxThreadRowKernel<32, TERMS_GIVEN>), dim3((rows + 255) / 256), dim3(256),
-                       0, s, dst, dstride, src, sstride, rows, cols);
-  } else if (cols <= 64) {   // four rows to a wave
-    hipLaunchKernelGGL((SoftmaxPartWaveKernel<16, 4, TERMS_GIVEN>), dim3((rows + 15) / 16), dim3(256), 0, s,
-                       dst, dstride, src, sstride, rows, cols);
-  } else if (cols <= 128) {
-    hipLaunchKernelGGL((SoftmaxPartWaveKernel<16, 8, TERMS_GIVEN>), dim3((rows + 15) / 16), dim3(256), 0, s,
-                       dst, dstride, src, sstride, rows, cols);
-  } else {                   // two rows to a wave
-    hipLaunchKernelGGL((SoftmaxPartWaveKernel<32, 8, TERMS_GIVEN>), dim3((rows + 7) / 8), dim3(256), 0, s,
-                       dst, dstride, src, sstride, rows, cols);
-  }
+#define SHORT_THREAD(CMAX) \
+  hipLaunchKernelGGL((SoftmaxThreadRowKernel<CMAX, TERMS_GIVEN>), dim3((rows + 255) / 256), dim3(256), 0, s, \
+                     dst, dstride, src, sstride, rows, cols)
+#define SHORT_PART(LANES, N) \
+  hipLaunchKernelGGL((SoftmaxPartWaveKernel<LANES, N, TERMS_GIVEN>), dim3((rows + 256 / LANES - 1) / (256 / LANES)), \
+                     dim3(256), 0, s, dst, dstride, src, sstride, rows, cols)
+#define WAVE_SLABS(SLABS) \
+  hipLaunchKernelGGL((SoftmaxWaveSlabsKernel<SLABS, TERMS_GIVEN>), dim3((rows + 3) / 4), dim3(256), 0, s, dst, \
+                     dstride, src, sstride, rows, cols)
+  const int cus = mshadow_abi::ComputeUnits();
+  /* Four or two rows side by side in a wave are fewer instructions, a wave to itself brings a row to
+     its end sooner: 4000 rows of 64 columns 3.8 us a wave each, 4.9 us in quarters, of 200 5.5 and
+     6.8 us, 16000 of 200 11.2 and 12.3 us; 131072 rows of 128 56 and 35 us, of 193 69 and 63 us */
+  const bool few = rows <= (cols <= 128 ? 16 : 64) * cus;
+  if (cols <= 16) SHORT_THREAD(16);
+  else if (cols <= 32) SHORT_THREAD(32);
+  else if (cols <= 256 && few) WAVE_SLABS(1);
+  else if (cols <= 64) SHORT_PART(16, 4);
+  else if (cols <= 128) SHORT_PART(16, 8);
+  else if (cols <= 256) SHORT_PART(32, 8);
+  /* a wave per row for any number of rows of up to 512 columns, and for many of up to 3072 (65536
+     rows of 300 / 1000 columns: 47 / 94 us against 163 / 193 us with a workgroup per row, 16384 of
+     2304 73 against 120 us; at 4096 columns, 64 of them a lane, 151 against 127 us). 100 rows of
+     500: 5.0 against 5.6 us; 1000 rows of 1000 / 2000: 7.8 / 10.9 against 7.3 / 9.3 us, 2000 rows
+     8.4 / 12.5 against 10.1 / 15.3 us. */
+  else if (cols <= 512) WAVE_SLABS(2);
+  else if (cols > 3072 || rows < 6 * cus) return false;
+  else if (cols <= 1024) WAVE_SLABS(4);
+  else if (cols <= 2048) WAVE_SLABS(8);
+  else WAVE_SLABS(12);
+#undef SHORT_THREAD
+#undef SHORT_PART
+#undef WAVE_SLABS
+  return true;
 }
 }  // namespace
 
@@ -567,29 +588,12 @@ int mshadow_hip_softmax_f32(float *dst, int dstride, const float *src, int sstri
   ABI_REQUIRE(dst != NULL && src != NULL, "NULL tensor");
   ABI_REQUIRE(dstride >= cols && sstride >= cols, "pitch smaller than the row");
   hipStream_t s = AsStream(stream);
-  if (cols <= 256) {  // short rows: a thread or a wave per row instead of a workgroup
-    LaunchShortSoftmax<false>(dst, dstride, src, sstride, rows, cols, s);
-    return AfterLaunch("softmax");
-  }
+  if (LaunchShortSoftmax<false>(dst, dstride, src, sstride, rows, cols, s)) return AfterLaunch("softmax");
   /* 16-byte packs wherever the rows start and whatever their length (the accesses need no
      alignment; a row's last, partial pack goes element by element) */
 #define SOFTMAX_LAUNCH(T, S, V) \
   hipLaunchKernelGGL((SoftmaxRowKernel<T, S, V, false>), dim3(rows), dim3(T), 0, s, dst, dstride, \
                      src, sstride, cols)
-#define SOFTMAX_WAVE(SLABS) \
-  hipLaunchKernelGGL((SoftmaxWaveSlabsKernel<SLABS, false>), dim3((rows + 3) / 4), dim3(256), 0, s, dst, \
-                     dstride, src, sstride, rows, cols)
-  /* many rows of up to 3072 columns: a wave per row (65536 rows of 300 / 1000 / 2000 columns:
-     71 / 109 / 122 us against 163 / 193 / 139 us with a workgroup per row; 16384 rows of 2304 /
-     3000 columns: 80 / 98 us against 120 / 133 us; at 4096 columns, 64 of them a lane, the wave
-     takes 176 us against 127 us, and with few rows the workgroup per row is faster) */
-  if (cols <= 3072 && rows >= 8 * mshadow_abi::ComputeUnits()) {
-    if (cols <= 512) SOFTMAX_WAVE(2);
-    else if (cols <= 1024) SOFTMAX_WAVE(4);
-    else if (cols <= 2048) SOFTMAX_WAVE(8);
-    else SOFTMAX_WAVE(12);
-    return AfterLaunch("softmax");
-  }
   /* many rows of 8193 to 16384 columns: four waves a row with 64 columns a thread, eight rows to a
      CU instead of four ((4096,10000): 82 against 104 us, (8192,12288): 153 against 196 us; with
      2048 rows the eight waves a row below finish them sooner, 57 against 70 us) */
@@ -597,7 +601,6 @@ int mshadow_hip_softmax_f32(float *dst, int dstride, const float *src, int sstri
     SOFTMAX_LAUNCH(256, 16, 4);
     return AfterLaunch("softmax");
   }
-#undef SOFTMAX_WAVE
   if (cols <= 1024) SOFTMAX_LAUNCH(256, 1, 4);
   else if (cols <= 2048) SOFTMAX_LAUNCH(256, 2, 4);
   else if (cols <= 4096) SOFTMAX_LAUNCH(256, 4, 4);
@@ -628,21 +631,7 @@ int mshadow_hip_softmax_rowsum_f32(float *sums, const float *terms, int tstride,
   ABI_REQUIRE(sums != NULL && (terms != NULL || cols == 0), "NULL tensor");
   ABI_REQUIRE(tstride >= cols, "pitch smaller than the row");
   hipStream_t s = AsStream(stream);
-  if (cols <= 256) {
-    LaunchShortSoftmax<true>(sums, 0, terms, tstride, rows, cols, s);
-    return AfterLaunch("softmax_rowsum");
-  }
-  if (cols <= 3072 && rows >= 8 * mshadow_abi::ComputeUnits()) {  // as in mshadow_hip_softmax_f32
-#define ROWSUM_WAVE(SLABS) \
-  hipLaunchKernelGGL((SoftmaxWaveSlabsKernel<SLABS, true>), dim3((rows + 3) / 4), dim3(256), 0, s, sums, 0, \
-                     terms, tstride, rows, cols)
-    if (cols <= 512) ROWSUM_WAVE(2);
-    else if (cols <= 1024) ROWSUM_WAVE(4);
-    else if (cols <= 2048) ROWSUM_WAVE(8);
-    else ROWSUM_WAVE(12);
-#undef ROWSUM_WAVE
-    return AfterLaunch("softmax_rowsum");
-  }
+  if (LaunchShortSoftmax<true>(sums, 0, terms, tstride, rows, cols, s)) return AfterLaunch("softmax_rowsum");
   const bool vec = Aligned16(terms) && tstride % 4 == 0 && cols % 4 == 0;
   /* rows longer than a workgroup's registers hold: stretch by stretch, at any alignment */
   if (cols > 65536 || (!vec && cols > 32768)) {

@@ -226,6 +226,26 @@ OSUM_HD LaneQuantum LaneDualQuant(const float (&t)[N], uint32_t e) {
   return r;
 }
 
+/*! \brief how many ulps of a sum in the binade that begins at bit pattern `base` (sign and
+ *  fraction zero) one lane's N terms add to it: at least 2^23, which leaves any binade, where
+ *  that cannot be said - a tie, a NaN, an infinite or (SIGNED) a negative term, no finite binade.
+ *  The two sums never come together or part by rounding in the next binade unnoticed: one ulp
+ *  apart at the end and the lower one inside the binade, they were so all along. */
+template <bool SIGNED, int N>
+OSUM_HD uint32_t LaneUlps(const float (&t)[N], uint32_t base) {
+  const uint32_t kNone = 1u << 24;
+  float lo = FloatOf(base), hi = FloatOf(base + 1u);
+  uint32_t signs = 0u;
+  for (int i = 0; i < N; ++i) {
+    lo = lo + t[i];
+    hi = hi + t[i];
+    if (SIGNED) signs |= BitsOf(t[i]);
+  }
+  const uint32_t q = BitsOf(lo) - base;
+  const bool ok = BitsOf(hi) - BitsOf(lo) == 1u && q < kNone && (!SIGNED || (signs >> 31) == 0u);
+  return ok && base < 0x7f800000u ? q : kNone;
+}
+
 /*! \brief bounds on the sequential sum from an accurate sum `approx` of the same terms:
  *  every addition rounds by at most half an ulp, so after n terms the sequential sum sits
  *  within n * 2^-24 of it (relative); sums of softmax terms stay well inside a quarter of
