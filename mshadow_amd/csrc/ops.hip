@@ -71,7 +71,7 @@ const size_t kPatchLdsBudget = 24 * 1024;  // per workgroup (col2im: every tap's
 const size_t kIm2ColLdsBudget = 16 * 1024;
 /* reductions long enough to fill the LDS ring of the direct-to-LDS kernels that hold a whole
    CU's LDS; shorter ones run kernels of which several share a CU */
-const int kDmaMinRows = 8192;
+const int kDmaMinRows = 6144;
 const long long kDmaMinPerKept = 1ll << 16;
 
 int MakePatchGeom(PatchGeom *g, int n, int c, int h, int w, int ky, int kx, int sy, int sx,
@@ -850,7 +850,7 @@ int mshadow_hip_reduce_keep_lowest_f32(float *dst, const float *src, int sstride
       if (strip == 16 && rows >= kDmaMinRows) {
         /* a strip for each CU at most and a long chain: four rows to an LDS read and stages of
            512 rows make its step 3.5 instead of 4.2 ns (65536 x 1000: 231 against 276 us;
-           16384 x 1000: 64 against 72 us; 4096 x 2000: 22 against 20 us) */
+           8191 x 1000: 36.7 against 38.2 us; level at 6000; 4096 x 2000: 22 against 20 us) */
         hipLaunchKernelGGL((mshadow::hip::ReduceKeepLowestDmaKernel<S, R>),
                            dim3((cols + mshadow::hip::kLowestCols - 1) / mshadow::hip::kLowestCols),
                            dim3(mshadow::hip::kDmaThreads), 0, s, dst, src,
