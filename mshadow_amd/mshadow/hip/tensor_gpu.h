@@ -24,6 +24,7 @@
 
 #if defined(__HIPCC__)
 #include "./kernels/map.h"
+#include "./kernels/pool_half.h"
 #include "./kernels/reduce.h"
 #include "./kernels/reduce_dma.h"
 #include "./kernels/rows_by_index.h"
@@ -763,6 +764,65 @@ struct FastPath<sv::saveto, dim, float,
     return true;
   }
 };
+#if defined(__HIPCC__)
+/* dst = pool<Reducer>(half_t tensor, ...): the windows that kernels/pool_half.h knows */
+template <typename Reducer, int dim>
+struct FastPath<sv::saveto, dim, half::half_t,
+                expr::PoolingExp<Reducer, Tensor<gpu, dim, half::half_t>, half::half_t, dim> > {
+  typedef expr::PoolingExp<Reducer, Tensor<gpu, dim, half::half_t>, half::half_t, dim> E;
+  template <typename R, int K, int S>
+  static bool Launch(Tensor<gpu, dim, half::half_t> *dst, const E &e) {
+    const Tensor<gpu, dim, half::half_t> &src = e.src_;
+    hip::PoolHalfGeom g;
+    g.h = e.src_height_, g.w = e.src_width_, g.ph = e.shape_[dim - 2], g.pw = e.shape_[dim - 1];
+    const uint64_t planes = src.shape_.ProdShape(0, dim - 2);
+    const uint32_t rows = hip::kPoolHalfRows / S;
+    g.groups = (g.pw + 3) / 4;
+    g.strips = (g.ph + rows - 1) / rows;
+    const uint64_t total = planes * g.strips * g.groups;
+    /* rows of four outputs at least, whole windows only, 31-bit thread numbers */
+    if (planes == 0 || g.ph == 0 || g.pw < 4 || total >= (1ull << 31) - hip::kPoolHalfBlock ||
+        (static_cast<uint64_t>(g.ph) - 1) * S + K > g.h || (static_cast<uint64_t>(g.pw) - 1) * S + K > g.w) {
+      return false;
+    }
+    g.total = static_cast<uint32_t>(total);
+    g.div_groups = FastDivU32(g.groups);
+    g.div_strips = FastDivU32(g.strips);
+    half::half_t *d = dst->dptr_;
+    const half::half_t *s = src.dptr_;
+    uint32_t dstride = dst->stride_, sstride = src.stride_;
+    void *args[] = {&d, &dstride, &s, &sstride, &g};
+    gpu_detail::Launch(hip::PoolHalfKernel<R, K, S>, (g.total + hip::kPoolHalfBlock - 1) / hip::kPoolHalfBlock,
+                       hip::kPoolHalfBlock, args, Stream<gpu>::GetStream(dst->stream_));
+    return true;
+  }
+  template <typename R>
+  static bool ByWindow(Tensor<gpu, dim, half::half_t> *dst, const E &e) {
+    if (e.ksize_y_ != e.ksize_x_ || e.kstride_y_ != e.kstride_x_) return false;
+    if (e.kstride_y_ == 1) {
+      if (e.ksize_y_ == 2) return Launch<R, 2, 1>(dst, e);
+      if (e.ksize_y_ == 3) return Launch<R, 3, 1>(dst, e);
+      if (e.ksize_y_ == 5) return Launch<R, 5, 1>(dst, e);
+    } else if (e.kstride_y_ == 2) {
+      if (e.ksize_y_ == 2) return Launch<R, 2, 2>(dst, e);
+      if (e.ksize_y_ == 3) return Launch<R, 3, 2>(dst, e);
+      if (e.ksize_y_ == 5) return Launch<R, 5, 2>(dst, e);
+    }
+    return false;
+  }
+  template <bool KNOWN, typename R>
+  struct Choice {
+    static bool Run(Tensor<gpu, dim, half::half_t> *, const E &) { return false; }
+  };
+  template <typename R>
+  struct Choice<true, R> {
+    static bool Run(Tensor<gpu, dim, half::half_t> *dst, const E &e) { return ByWindow<R>(dst, e); }
+  };
+  inline static bool Run(Tensor<gpu, dim, half::half_t> *dst, const E &e) {
+    return Choice<(ReducerCode<Reducer>::value >= 0), Reducer>::Run(dst, e);
+  }
+};
+#endif
 /* dst = unpool<Reducer>(float tensors, ...) */
 template <typename Reducer, int dim>
 struct FastPath<sv::saveto, dim, float,
