@@ -1252,35 +1252,39 @@ struct HalfRingRoute<Saver, Reducer, Tensor<gpu, 1, half::half_t>, Tensor<gpu, d
                       uint32_t n_out, uint32_t n_keep, uint32_t n_y, uint32_t n_x,
                       half::half_t scale) {
     const uint64_t per_kept = static_cast<uint64_t>(n_out) * n_y * n_x;
-    if (n_x % 2 != 0 || src.stride_ % 2 != 0 || reinterpret_cast<uintptr_t>(src.dptr_) % 4 != 0 ||
-        per_kept < (1u << 16) || static_cast<uint64_t>(n_y) * n_x >= (1ull << 31)) {
-      return false;
-    }
+    if (per_kept < (1u << 16) || static_cast<uint64_t>(n_y) * n_x >= (1ull << 31)) return false;
     half::half_t *d = dst.dptr_;
     const half::half_t *s = src.dptr_;
     uint32_t stride = src.stride_;
+    /* Dense rows are walked as one row per segment, whose length then is what has to be even. Rows of
+       odd length where that was measured to be the faster way: (64,256,56,55) 21 us, 50 us with the
+       generic kernel, (128,16,100,75) 45 and 120 us, (32,64,112,111) 53 and 84 us, (256,192,32,17) 21
+       and 42 us; but (16,512,66,63) 43 and 33 us - the ring holds a whole CU - and (1,195,512,129),
+       one chain a CU, 267 and 247 us. */
+    const bool odd_rows = n_x % 2 != 0;
+    if (odd_rows && (n_keep > 256u || n_out < 16u || static_cast<uint64_t>(n_y) * n_x < 512u)) return false;
+    if (stride == n_x) {
+      n_x = stride = n_y * n_x;
+      n_y = 1;
+    }
+    if (n_x % 2 != 0 || stride % 2 != 0 || reinterpret_cast<uintptr_t>(s) % 4 != 0) return false;
     void *stream = Stream<gpu>::GetStream(dst.stream_);
     /* the inner chains spread over as many workgroups as there are groups of segments, where
-       rows are whole 16-byte packs (dense rows are walked as one row per segment) and the
-       library has scratch memory for the inner results of this stream */
+       rows are whole 16-byte packs and the library has scratch memory for the inner results of
+       this stream */
     {
-      uint32_t v_y = n_y, v_x = n_x, v_stride = stride;
-      if (stride == n_x) {
-        v_x = v_stride = n_y * n_x;
-        v_y = 1;
-      }
       uint32_t *partial = NULL, *counter = NULL;
       /* fewer kept indices than CUs (the chip's 256: the one-workgroup-per-kept-index kernel
          below would leave some idle): the inner chains are dealt out by segments */
       const bool few_kept = n_keep < 192u;
-      const bool packs = v_x % 8 == 0 && v_stride % 8 == 0 && reinterpret_cast<uintptr_t>(s) % 16 == 0;
+      const bool packs = n_x % 8 == 0 && stride % 8 == 0 && reinterpret_cast<uintptr_t>(s) % 16 == 0;
       if (few_kept && static_cast<uint64_t>(n_out) * n_keep < (1ull << 31)) {
         MSHADOW_HIP_CALL(mshadow_hip_reduce_scratch(stream, static_cast<size_t>(n_out) * n_keep,
                                                     &partial, &counter));
       }
       if (partial != NULL) {
-        FastDivU32 v_div_x(v_x);
-        void *sargs[] = {&d, &s, &v_stride, &n_out, &n_keep, &v_y, &v_x, &v_div_x, &scale, &partial,
+        FastDivU32 div_x(n_x);
+        void *sargs[] = {&d, &s, &stride, &n_out, &n_keep, &n_y, &n_x, &div_x, &scale, &partial,
                          &counter};
         if (packs) {
           typedef hip::HighDimSplitRingPacks Ring;
