@@ -187,6 +187,13 @@ inline void Launch(K kernel, uint32_t grid_x, uint32_t block_x, void **args, voi
                                       stream));
 }
 
+/*! \brief rows that a launch of workgroups of `threads`, `rows_per_block` rows each, takes at most: with
+ *  2^32 threads or more along an axis workgroups are dropped, and no error says so */
+inline uint32_t RowsOfLaunch(uint32_t threads, uint32_t rows_per_block) {
+  const uint64_t most = 0xffffffffull / threads * rows_per_block;
+  return most < 0xffffffffull ? static_cast<uint32_t>(most) : 0xffffffffu;
+}
+
 /*! \brief half_t rows that are kept in registers, a workgroup of as many waves as hold one; false =
  *  not this shape or element type */
 template <typename DType>
@@ -194,8 +201,16 @@ inline bool SoftmaxRowsOnChip(DType *, uint32_t, const DType *, uint32_t, uint32
   return false;
 }
 template <int WAVES, int PACKS>
-inline void LaunchHalfRows(uint32_t rows, void **args, void *stream) {
-  Launch(hip::SoftmaxHalfRowKernel<WAVES, PACKS>, rows, WAVES * hip::kWave, args, stream);
+inline void LaunchHalfRows(half::half_t *dst, uint32_t dstride, const half::half_t *src, uint32_t sstride,
+                           uint32_t rows, uint32_t cols, void *stream) {
+  const uint32_t threads = WAVES * hip::kWave, most = RowsOfLaunch(threads, 1);
+  for (uint64_t row = 0; row < rows; row += most) {
+    half::half_t *d = dst + row * dstride;
+    const half::half_t *s = src + row * sstride;
+    void *args[] = {&d, &dstride, &s, &sstride, &cols};
+    Launch(hip::SoftmaxHalfRowKernel<WAVES, PACKS>, rows - row < most ? static_cast<uint32_t>(rows - row) : most,
+           threads, args, stream);
+  }
 }
 inline bool SoftmaxRowsOnChip(half::half_t *d, uint32_t dstride, const half::half_t *s, uint32_t sstride,
                               uint32_t rows, uint32_t cols, void *stream) {
@@ -208,32 +223,31 @@ inline bool SoftmaxRowsOnChip(half::half_t *d, uint32_t dstride, const half::hal
   const bool aligned = (reinterpret_cast<uintptr_t>(s) | sstride * sizeof(half::half_t)) % 16 == 0;
   const uint32_t reach = aligned ? cols : cols + hip::kHalfPack - 1;
   const uint32_t runs = (reach + hip::kHalfRun - 1) / hip::kHalfRun;
-  void *args[] = {&d, &dstride, &s, &sstride, &cols};
   /* As few waves as hold the row: a wave more is a link more in the walk. Waves of 8 runs (72
      registers, 20 to a CU) as long as four of them do: 16384 x 12000 162 us with three, 176 with
      four, 184 with two of 16 runs (114 registers, 16 to a CU); 8192 x 16000 109 us with four of 8,
      119 with two of 16; from there on four of 16 and eight of 8 are level (8192 x 32000: 230 and
      235 us). Few packs for short rows: 65536 x 1000 97 us with two, 105 with four, 140 with 16. */
   if (runs <= 2) {
-    LaunchHalfRows<1, 2>(rows, args, stream);
+    LaunchHalfRows<1, 2>(d, dstride, s, sstride, rows, cols, stream);
   } else if (runs <= 4) {
-    LaunchHalfRows<1, 4>(rows, args, stream);
+    LaunchHalfRows<1, 4>(d, dstride, s, sstride, rows, cols, stream);
   } else if (runs <= 8) {
-    LaunchHalfRows<1, 8>(rows, args, stream);
+    LaunchHalfRows<1, 8>(d, dstride, s, sstride, rows, cols, stream);
   } else if (runs <= 16) {
-    LaunchHalfRows<2, 8>(rows, args, stream);
+    LaunchHalfRows<2, 8>(d, dstride, s, sstride, rows, cols, stream);
   } else if (runs <= 24) {
-    LaunchHalfRows<3, 8>(rows, args, stream);
+    LaunchHalfRows<3, 8>(d, dstride, s, sstride, rows, cols, stream);
   } else if (runs <= 32) {
-    LaunchHalfRows<4, 8>(rows, args, stream);
+    LaunchHalfRows<4, 8>(d, dstride, s, sstride, rows, cols, stream);
   } else if (runs <= 48) {
-    LaunchHalfRows<3, 16>(rows, args, stream);
+    LaunchHalfRows<3, 16>(d, dstride, s, sstride, rows, cols, stream);
   } else if (runs <= 64) {
-    LaunchHalfRows<4, 16>(rows, args, stream);
+    LaunchHalfRows<4, 16>(d, dstride, s, sstride, rows, cols, stream);
   } else if (runs <= 128) {
-    LaunchHalfRows<8, 16>(rows, args, stream);
+    LaunchHalfRows<8, 16>(d, dstride, s, sstride, rows, cols, stream);
   } else if (runs <= 256) {
-    LaunchHalfRows<16, 16>(rows, args, stream);
+    LaunchHalfRows<16, 16>(d, dstride, s, sstride, rows, cols, stream);
   } else {
     return false;
   }

@@ -8,6 +8,7 @@ import pytest
 
 from checkers import Checker
 from gpu_util import f32
+from mshadow_amd.capi import DeviceBuffer
 
 pytestmark = pytest.mark.gpu
 
@@ -103,6 +104,23 @@ def test_half_rows_every_exponential(G, O):
         piece = d[r * 4095:(r + 1) * 4095]
         x[r, 1:1 + piece.size] = piece
     check(G, O, x, 0, 0)
+
+
+def test_half_rows_more_than_a_launch_takes(G, O):
+    """a wave per row of these is more threads than one launch may have (fewer than 2^32). In place; rows at
+    both ends and in between are looked at, the others hold whatever the memory held."""
+    rows, cols, some = (1 << 26) + 1024, 129, 100
+    x = O.float2half(logits("normal", some, cols))
+    want = np.empty_like(x)
+    O.softmax(want, x)
+    m = G.buffer((rows, cols), np.uint16)
+    at = [SimpleNamespace(lib=G, ptr=m.ptr + r * cols * 2, stride=cols, rows=some, cols=cols, dtype=m.dtype, shape=x.shape)
+          for r in (0, 1000, rows // 2 - 7, (1 << 26) - 50, rows - some)]
+    for piece in at:
+        DeviceBuffer.upload(piece, x)
+    G.case_softmax(m, m)
+    for piece in at:
+        assert np.array_equal(DeviceBuffer.download(piece), want)
 
 
 @pytest.mark.parametrize("rows,cols", [(300, 1), (300, 7), (300, 8), (513, 9), (129, 33), (65, 511), (33, 1000), (9, 1024),
