@@ -442,6 +442,15 @@ static int LaunchRowsByIndex(float *dst, int dstride, int k_rows, const void *ro
 }
 
 namespace {
+/*! \brief rows (or kept indices) of one launch that gives each `threads` threads at most: with 2^32
+ *  threads or more along an axis workgroups are dropped, and no error says so */
+int RowsOfLaunch(unsigned threads) {
+  const unsigned long long most = (0xffffffffull - 1024u) / threads;  // the last workgroup may not be full
+  return most < static_cast<unsigned long long>(INT_MAX) ? static_cast<int>(most) : INT_MAX;
+}
+/*! \brief threads a row of the kernels below takes, where there are many rows */
+unsigned SoftmaxThreadsPerRow(int cols) { return cols <= 32 ? 1u : cols <= 256 ? 32u : cols <= 3072 ? 64u : 1024u; }
+
 /*! \brief rows that a thread, a part of a wave or a wave takes; false: longer ones, which take a
  *  workgroup */
 template <bool TERMS_GIVEN>
@@ -587,6 +596,15 @@ int mshadow_hip_softmax_f32(float *dst, int dstride, const float *src, int sstri
   if (rows == 0 || cols == 0) return MSHADOW_HIP_OK;
   ABI_REQUIRE(dst != NULL && src != NULL, "NULL tensor");
   ABI_REQUIRE(dstride >= cols && sstride >= cols, "pitch smaller than the row");
+  const int most = RowsOfLaunch(SoftmaxThreadsPerRow(cols));
+  if (rows > most) {
+    for (long long row = 0; row < rows; row += most) {
+      const int st = mshadow_hip_softmax_f32(dst + row * dstride, dstride, src + row * sstride, sstride,
+                                             rows - row < most ? static_cast<int>(rows - row) : most, cols, stream);
+      if (st != MSHADOW_HIP_OK) return st;
+    }
+    return MSHADOW_HIP_OK;
+  }
   hipStream_t s = AsStream(stream);
   if (LaunchShortSoftmax<false>(dst, dstride, src, sstride, rows, cols, s)) return AfterLaunch("softmax");
   /* 16-byte packs wherever the rows start and whatever their length (the accesses need no
@@ -630,6 +648,15 @@ int mshadow_hip_softmax_rowsum_f32(float *sums, const float *terms, int tstride,
   if (rows == 0) return MSHADOW_HIP_OK;
   ABI_REQUIRE(sums != NULL && (terms != NULL || cols == 0), "NULL tensor");
   ABI_REQUIRE(tstride >= cols, "pitch smaller than the row");
+  const int most = RowsOfLaunch(SoftmaxThreadsPerRow(cols));
+  if (rows > most) {
+    for (long long row = 0; row < rows; row += most) {
+      const int st = mshadow_hip_softmax_rowsum_f32(sums + row, terms + row * tstride, tstride,
+                                                    rows - row < most ? static_cast<int>(rows - row) : most, cols, stream);
+      if (st != MSHADOW_HIP_OK) return st;
+    }
+    return MSHADOW_HIP_OK;
+  }
   hipStream_t s = AsStream(stream);
   if (LaunchShortSoftmax<true>(sums, 0, terms, tstride, rows, cols, s)) return AfterLaunch("softmax_rowsum");
   const bool vec = Aligned16(terms) && tstride % 4 == 0 && cols % 4 == 0;
@@ -674,12 +701,22 @@ int mshadow_hip_softmax_grad_ex_f32(float *dst, int dstride, const float *src, i
   const unsigned chunks = (cols + per_block - 1) / per_block;
   const unsigned long long blocks = static_cast<unsigned long long>(rows) * chunks;
   ABI_REQUIRE(blocks < (1ull << 31), "too many workgroups");
+  /* short rows go several to a workgroup, a pack a thread */
+  const int ppr = (cols + 3) / 4, rows_per_block = cols <= 512 ? kGradBlock / ppr : 1;
+  const int most = RowsOfLaunch((static_cast<unsigned>(kGradBlock) * chunks - 1) / rows_per_block + 1);
+  if (rows > most) {
+    for (long long row = 0; row < rows; row += most) {
+      const int st = mshadow_hip_softmax_grad_ex_f32(dst + row * dstride, dstride, src + row * sstride, sstride, label + row,
+                                                     rows - row < most ? static_cast<int>(rows - row) : most, cols, flags,
+                                                     ignore_label, alpha, stream);
+      if (st != MSHADOW_HIP_OK) return st;
+    }
+    return MSHADOW_HIP_OK;
+  }
   /* alpha / (classes - 1) with the count converted from unsigned, as the reference writes it */
   const GradParams gp = {static_cast<int>(ignore_label), alpha,
                          alpha / static_cast<float>(static_cast<unsigned>(cols - 1))};
-  if (cols <= 512) {  // short rows: several to a workgroup, a pack a thread
-    const int ppr = (cols + 3) / 4;
-    const int rows_per_block = kGradBlock / ppr;
+  if (cols <= 512) {
     const unsigned grid = static_cast<unsigned>((rows + rows_per_block - 1) / rows_per_block);
     const mshadow::FastDivU32 div_ppr(static_cast<uint32_t>(ppr));
 #define GRAD_SHORT(FLAGS)                                                                            \
@@ -890,8 +927,6 @@ int mshadow_hip_reduce_keep_highdim_f32(float *dst, const float *src, int sstrid
                   static_cast<long long>(n) * y * x >= kDmaMinPerKept,
               "too many rows for 32-bit indices");
   ABI_REQUIRE(static_cast<long long>(y) * x < (1ll << 31), "inner extent too large for 32-bit indices");
-  RawPlan1D<float> d = {dst};
-  RawPlan2D<const float> sp = {src, sstride};
   const mshadow::FastDivU32 div_x(static_cast<uint32_t>(x > 0 ? x : 1));
   hipStream_t s = AsStream(stream);
   /* The split kernel walks dense rows as one row per segment. It needs scratch memory for
@@ -920,11 +955,15 @@ int mshadow_hip_reduce_keep_highdim_f32(float *dst, const float *src, int sstrid
       typedef decltype(red) R;
       typedef decltype(sv) S;
 #define HIGHDIM_LAUNCH_T(T, SEGS)                                                              \
-  hipLaunchKernelGGL((mshadow::hip::ReduceKeepHighDimKernel<S, R, float, T, SEGS, RawPlan1D<float>, \
-                                                            RawPlan2D<const float> >),         \
-                     dim3(c), dim3(T), 0, s, d, sp, static_cast<uint32_t>(n),                  \
-                     static_cast<uint32_t>(c), static_cast<uint32_t>(y),                       \
-                     static_cast<uint32_t>(x), div_x, scale)
+  for (long long c0 = 0, most = RowsOfLaunch(T); c0 < c; c0 += most) {                         \
+    RawPlan1D<float> d = {dst + c0};                                                           \
+    RawPlan2D<const float> sp = {src + c0 * y * sstride, sstride};                             \
+    hipLaunchKernelGGL((mshadow::hip::ReduceKeepHighDimKernel<S, R, float, T, SEGS, RawPlan1D<float>, \
+                                                              RawPlan2D<const float> >),       \
+                       dim3(static_cast<unsigned>(c - c0 < most ? c - c0 : most)), dim3(T), 0, s, d, sp, \
+                       static_cast<uint32_t>(n), static_cast<uint32_t>(c), static_cast<uint32_t>(y), \
+                       static_cast<uint32_t>(x), div_x, scale);                                \
+  }
 #define HIGHDIM_LAUNCH(SEGS)                                                                   \
   if (large)                                                                                   \
     hipLaunchKernelGGL((mshadow::hip::ReduceKeepHighDimDmaKernel<S, R, float, SEGS>), dim3(c),        \

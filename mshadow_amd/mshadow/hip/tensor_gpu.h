@@ -267,15 +267,21 @@ inline void Softmax(Tensor<gpu, 2, DType> dst, const Tensor<gpu, 2, DType> &src)
   if (gpu_detail::SoftmaxRowsOnChip(d, dstride, s, sstride, rows, cols, Stream<gpu>::GetStream(dst.stream_))) {
     return;
   }
-  void *args[] = {&d, &dstride, &s, &sstride, &rows, &cols};
-  const uint32_t grid[3] = {(rows + hip::kAnyRows - 1) / hip::kAnyRows, 1, 1};
   const uint32_t block[3] = {static_cast<uint32_t>(hip::kAnyBlock), 1, 1};
   const bool vec = gpu_detail::AnyPackable(s, sstride, const_cast<const DType *>(d), dstride, cols,
                                            hip::kAnyTile);
   const void *kernel = vec ? reinterpret_cast<const void *>(hip::SoftmaxAnyKernel<DType, true>)
                            : reinterpret_cast<const void *>(hip::SoftmaxAnyKernel<DType, false>);
-  MSHADOW_HIP_CALL(mshadow_hip_launch(kernel, grid, block, args, 0,
-                                      Stream<gpu>::GetStream(dst.stream_)));
+  const uint32_t most = gpu_detail::RowsOfLaunch(hip::kAnyBlock, hip::kAnyRows);
+  for (uint64_t row = 0; row < rows; row += most) {
+    uint32_t some = rows - row < most ? static_cast<uint32_t>(rows - row) : most;
+    DType *dr = d + row * dstride;
+    const DType *sr = s + row * sstride;
+    void *args[] = {&dr, &dstride, &sr, &sstride, &some, &cols};
+    const uint32_t grid[3] = {(some - 1) / hip::kAnyRows + 1, 1, 1};
+    MSHADOW_HIP_CALL(mshadow_hip_launch(kernel, grid, block, args, 0,
+                                        Stream<gpu>::GetStream(dst.stream_)));
+  }
 #else
   LOG(FATAL) << "Softmax<gpu> of this element type: compile the calling translation unit with hipcc";
 #endif
@@ -311,10 +317,8 @@ inline void AnyGrad2D(const Tensor<gpu, 2, DType> &dst, const Tensor<gpu, 2, DTy
   const uint32_t packs = (cols + hip::kAnyTile - 1) / hip::kAnyTile;
   uint32_t rows_per_block = several ? hip::kAnyBlock / packs : 1u;
   FastDivU32 div_packs(packs);
-  void *args[] = {&d, &dstride, &s, &sstride, &l, &cols, &ignore_k, &alpha, &smooth, &rows, &rows_per_block, &div_packs};
   uint32_t per_row = several ? 1u : (packs + hip::kAnyBlock - 1) / hip::kAnyBlock;
   if (per_row > 64) per_row = 64;
-  const uint32_t grid[3] = {(rows - 1) / rows_per_block + 1, per_row, 1};  // rows up to 2^31 - 1 on the x axis
   const uint32_t block[3] = {static_cast<uint32_t>(hip::kAnyBlock), 1, 1};
   const void *kernel = NULL;
 #define MSHADOW_ANY_GRAD(FLAGS)                                                                      \
@@ -327,8 +331,16 @@ inline void AnyGrad2D(const Tensor<gpu, 2, DType> &dst, const Tensor<gpu, 2, DTy
     default: MSHADOW_ANY_GRAD(3); break;
   }
 #undef MSHADOW_ANY_GRAD
-  MSHADOW_HIP_CALL(mshadow_hip_launch(kernel, grid, block, args, 0,
-                                      Stream<gpu>::GetStream(dst.stream_)));
+  const uint32_t most = RowsOfLaunch(hip::kAnyBlock, rows_per_block);
+  for (uint64_t row = 0; row < rows; row += most) {
+    uint32_t some = rows - row < most ? static_cast<uint32_t>(rows - row) : most;
+    DType *dr = d + row * dstride;
+    const DType *sr = s + row * sstride, *lr = l + row;
+    void *args[] = {&dr, &dstride, &sr, &sstride, &lr, &cols, &ignore_k, &alpha, &smooth, &some, &rows_per_block, &div_packs};
+    const uint32_t grid[3] = {(some - 1) / rows_per_block + 1, per_row, 1};
+    MSHADOW_HIP_CALL(mshadow_hip_launch(kernel, grid, block, args, 0,
+                                        Stream<gpu>::GetStream(dst.stream_)));
+  }
 #else
   LOG(FATAL) << "SoftmaxGrad<gpu> of this element type: compile the calling translation unit with hipcc";
 #endif
