@@ -29,9 +29,26 @@ inline int FromHip(hipError_t e, const char *what) {
 
 inline hipStream_t AsStream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
+/* With 2^32 threads or more along an axis HIP launches the number modulo 2^32 and reports
+   nothing. Such a launch is not made (LaunchKernelIfFits), and AfterLaunch says so. */
+inline bool LaunchFits(const dim3 &grid, const dim3 &block) {
+  const unsigned long long limit = 1ull << 32;
+  return static_cast<unsigned long long>(grid.x) * block.x < limit &&
+         static_cast<unsigned long long>(grid.y) * block.y < limit &&
+         static_cast<unsigned long long>(grid.z) * block.z < limit;
+}
+/* the calling thread has a launch that was not made since AfterLaunch last looked */
+bool &LaunchRefused();
+
 /* queued-launch check: the reference calls cudaPeekAtLastError after every launch
    (mshadow/cuda/tensor_gpu-inl.cuh:16-21); hipGetLastError also clears the sticky code */
-inline int AfterLaunch(const char *what) { return FromHip(hipGetLastError(), what); }
+inline int AfterLaunch(const char *what) {
+  if (LaunchRefused()) {
+    LaunchRefused() = false;
+    return Fail(MSHADOW_HIP_ERR_ARGUMENT, std::string(what) + ": too large for one launch (2^32 threads or more)");
+  }
+  return FromHip(hipGetLastError(), what);
+}
 
 /* looks up, once per device, where the scratch array of the sort that allocates nothing lives
    on the current device (csrc/sort.hip) */
@@ -51,6 +68,15 @@ void ReleaseReduceScratch(void *stream);
 void ResolveReduceScratch();
 
 }  // namespace mshadow_abi
+
+#define LaunchKernelIfFits(kernel, grid, block, ...)               \
+  do {                                                             \
+    if (mshadow_abi::LaunchFits(grid, block)) {                    \
+      hipLaunchKernelGGL(kernel, grid, block, __VA_ARGS__);        \
+    } else {                                                       \
+      mshadow_abi::LaunchRefused() = true;                         \
+    }                                                              \
+  } while (0)
 
 #define ABI_HIP(call)                                              \
   do {                                                             \

@@ -121,7 +121,7 @@ int Im2Col(T *col, int cstride, const T *img, int istride, const PatchGeom &g, v
     const long long pieces = (static_cast<long long>(g.c) * chunks + 7) / 8 * 8;
     const long long direct_blocks = pieces * g.ky;
     if (direct_blocks < (1ll << 31)) {
-      hipLaunchKernelGGL((Im2ColRow3DirectKernel<T, kIm2ColDirectPer>),
+      LaunchKernelIfFits((Im2ColRow3DirectKernel<T, kIm2ColDirectPer>),
                          dim3(static_cast<unsigned>(direct_blocks)), dim3(kPatchBlock), 0,
                          AsStream(stream), col, cstride, img, g,
                          mshadow::FastDivU32(static_cast<uint32_t>(g.ow / EPT)),
@@ -144,7 +144,7 @@ int Im2Col(T *col, int cstride, const T *img, int istride, const PatchGeom &g, v
     const long long blocks = pieces * g.ky;
     if (places + kPatchBlock < (1ll << 31) && blocks < (1ll << 31)) {
 #define IM2COL_ROW_TAPS(KX, SX)                                                                       \
-  hipLaunchKernelGGL((Im2ColRowTapsKernel<T, KX, SX>), dim3(static_cast<unsigned>(blocks)),           \
+  LaunchKernelIfFits((Im2ColRowTapsKernel<T, KX, SX>), dim3(static_cast<unsigned>(blocks)),           \
                      dim3(kPatchBlock), 0, AsStream(stream), col, cstride, img, istride, g,           \
                      mshadow::FastDivU32(static_cast<uint32_t>(ppr)),                                 \
                      mshadow::FastDivU32(static_cast<uint32_t>(g.oh)), chunks,                        \
@@ -170,7 +170,7 @@ int Im2Col(T *col, int cstride, const T *img, int istride, const PatchGeom &g, v
     const long long pieces = (static_cast<long long>(g.c) * chunks + 7) / 8 * 8;
     const long long blocks = pieces * g.ky * g.kx;
     if (places + kPatchBlock < (1ll << 31) && blocks < (1ll << 31)) {
-      hipLaunchKernelGGL((Im2ColDirectS1Kernel<T>), dim3(static_cast<unsigned>(blocks)),
+      LaunchKernelIfFits((Im2ColDirectS1Kernel<T>), dim3(static_cast<unsigned>(blocks)),
                          dim3(kPatchBlock), 0, AsStream(stream), col, cstride, img, istride, g,
                          mshadow::FastDivU32(static_cast<uint32_t>(ppr)),
                          mshadow::FastDivU32(static_cast<uint32_t>(g.oh)), chunks,
@@ -188,7 +188,7 @@ int Im2Col(T *col, int cstride, const T *img, int istride, const PatchGeom &g, v
     const long long pieces = (static_cast<long long>(g.c) * chunks + 7) / 8 * 8;
     const long long blocks = pieces * g.ky * g.kx;
     if (places + kPatchBlock < (1ll << 31) && blocks < (1ll << 31)) {
-      hipLaunchKernelGGL((Im2ColDirectS2Kernel<T>), dim3(static_cast<unsigned>(blocks)),
+      LaunchKernelIfFits((Im2ColDirectS2Kernel<T>), dim3(static_cast<unsigned>(blocks)),
                          dim3(kPatchBlock), 0, AsStream(stream), col, cstride, img, istride, g,
                          mshadow::FastDivU32(static_cast<uint32_t>(ppr)),
                          mshadow::FastDivU32(static_cast<uint32_t>(g.oh)), chunks,
@@ -215,14 +215,14 @@ int Im2Col(T *col, int cstride, const T *img, int istride, const PatchGeom &g, v
     const long long blocks = planes * nb;
     if (blocks >= (1ll << 31)) return Fail(MSHADOW_HIP_ERR_ARGUMENT, "im2col: too many workgroups");
     const size_t lds = static_cast<size_t>(t.rows_max) * row_bytes;
-    hipLaunchKernelGGL((Im2ColTiledKernel<T, EPT>), dim3(static_cast<unsigned>(blocks)),
+    LaunchKernelIfFits((Im2ColTiledKernel<T, EPT>), dim3(static_cast<unsigned>(blocks)),
                        dim3(kPatchBlock), lds, AsStream(stream), col, cstride, img, istride, g, t);
   } else {
     const unsigned chunks =
         static_cast<unsigned>((cols + kPatchBlock * EPT - 1) / (kPatchBlock * EPT));
     const long long blocks = rows * chunks;
     if (blocks >= (1ll << 31)) return Fail(MSHADOW_HIP_ERR_ARGUMENT, "im2col: too many workgroups");
-    hipLaunchKernelGGL((Im2ColKernel<T, EPT>), dim3(static_cast<unsigned>(blocks)),
+    LaunchKernelIfFits((Im2ColKernel<T, EPT>), dim3(static_cast<unsigned>(blocks)),
                        dim3(kPatchBlock), 0, AsStream(stream), col, cstride, img, istride, g,
                        chunks);
   }
@@ -253,7 +253,7 @@ int Col2Im(T *img, int istride, const T *col, int cstride, const PatchGeom &g, v
     rg.div_c = mshadow::FastDivU32(static_cast<uint32_t>(g.c));
     const uint32_t waves = (rg.total_rows + rg.rows_per_wave - 1) / rg.rows_per_wave;
     const uint32_t blocks = (waves + kPatchBlock / 64 - 1) / (kPatchBlock / 64);
-    hipLaunchKernelGGL(Col2ImHalfRows3x3Kernel, dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream),
+    LaunchKernelIfFits(Col2ImHalfRows3x3Kernel, dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream),
                        reinterpret_cast<uint16_t *>(img), istride,
                        reinterpret_cast<const uint16_t *>(col), cstride, g, rg);
     return AfterLaunch("col2im");
@@ -264,7 +264,7 @@ int Col2Im(T *img, int istride, const T *col, int cstride, const PatchGeom &g, v
     const long long packs = static_cast<long long>(g.n) * g.c * g.h * wpk;
     if (packs + kPatchBlock < (1ll << 31) && cols < (1ll << 31)) {
       const unsigned blocks = static_cast<unsigned>((packs + kPatchBlock - 1) / kPatchBlock);
-      hipLaunchKernelGGL((Col2ImDirectS1Kernel<T>), dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream),
+      LaunchKernelIfFits((Col2ImDirectS1Kernel<T>), dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream),
                          img, istride, col, cstride, g, mshadow::FastDivU32(static_cast<uint32_t>(wpk)),
                          mshadow::FastDivU32(static_cast<uint32_t>(g.h)),
                          mshadow::FastDivU32(static_cast<uint32_t>(g.c)), static_cast<uint32_t>(packs));
@@ -286,14 +286,14 @@ int Col2Im(T *img, int istride, const T *col, int cstride, const PatchGeom &g, v
       const int over = over_y > over_x ? over_y : over_x;
       if (g.dy == 1 && g.dx == 1 && over <= 4) {
 #define COL2IM_FLAT(TY, TX)                                                                                  \
-  hipLaunchKernelGGL((Col2ImGatherFlatKernel<T, TY, TX>), dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream), \
+  LaunchKernelIfFits((Col2ImGatherFlatKernel<T, TY, TX>), dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream), \
                      img, istride, col, cstride, g, dv, mshadow::FastDivU32(static_cast<uint32_t>(wpk)),       \
                      mshadow::FastDivU32(static_cast<uint32_t>(g.h)),                                          \
                      mshadow::FastDivU32(static_cast<uint32_t>(g.c)), static_cast<uint32_t>(packs))
         /* a step of two along x: the patches of every second pixel are neighbours in the matrix */
         if (g.sx == 2 && g.ow >= EPT / 2 && over >= 2) {
 #define COL2IM_S2(TY, TX)                                                                                    \
-  hipLaunchKernelGGL((Col2ImGatherS2Kernel<T, TY, TX>), dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream), \
+  LaunchKernelIfFits((Col2ImGatherS2Kernel<T, TY, TX>), dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream), \
                      img, istride, col, cstride, g, dv, mshadow::FastDivU32(static_cast<uint32_t>(wpk)),       \
                      mshadow::FastDivU32(static_cast<uint32_t>(g.h)),                                          \
                      mshadow::FastDivU32(static_cast<uint32_t>(g.c)), static_cast<uint32_t>(packs))
@@ -310,7 +310,7 @@ int Col2Im(T *img, int istride, const T *col, int cstride, const PatchGeom &g, v
 #undef COL2IM_FLAT
         return AfterLaunch("col2im");
       }
-      hipLaunchKernelGGL((Col2ImGatherKernel<T>), dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream),
+      LaunchKernelIfFits((Col2ImGatherKernel<T>), dim3(blocks), dim3(kPatchBlock), 0, AsStream(stream),
                          img, istride, col, cstride, g, dv, mshadow::FastDivU32(static_cast<uint32_t>(wpk)),
                          mshadow::FastDivU32(static_cast<uint32_t>(g.h)),
                          mshadow::FastDivU32(static_cast<uint32_t>(g.c)), static_cast<uint32_t>(packs));
@@ -339,17 +339,17 @@ int Col2Im(T *img, int istride, const T *col, int cstride, const PatchGeom &g, v
     const long long blocks = planes * nb;
     if (blocks >= (1ll << 31)) return Fail(MSHADOW_HIP_ERR_ARGUMENT, "col2im: too many workgroups");
     if (g.dy == 1 && g.dx == 1 && g.sy == 1 && g.sx == 1) {
-      hipLaunchKernelGGL((Col2ImTiledKernel<T, EPT, true>), dim3(static_cast<unsigned>(blocks)),
+      LaunchKernelIfFits((Col2ImTiledKernel<T, EPT, true>), dim3(static_cast<unsigned>(blocks)),
                          dim3(kPatchBlock), lds, AsStream(stream), img, istride, col, cstride, g, t);
     } else {
-      hipLaunchKernelGGL((Col2ImTiledKernel<T, EPT, false>), dim3(static_cast<unsigned>(blocks)),
+      LaunchKernelIfFits((Col2ImTiledKernel<T, EPT, false>), dim3(static_cast<unsigned>(blocks)),
                          dim3(kPatchBlock), lds, AsStream(stream), img, istride, col, cstride, g, t);
     }
   } else {
     unsigned grid = 0;
     int st = mshadow_hip_suggest_grid(static_cast<size_t>(total), kPatchBlock, 8, &grid);
     if (st != MSHADOW_HIP_OK) return st;
-    hipLaunchKernelGGL((Col2ImKernel<T>), dim3(grid), dim3(kPatchBlock), 0, AsStream(stream), img,
+    LaunchKernelIfFits((Col2ImKernel<T>), dim3(grid), dim3(kPatchBlock), 0, AsStream(stream), img,
                        istride, col, cstride, g, static_cast<unsigned>(total));
   }
   return AfterLaunch("col2im");
@@ -364,15 +364,15 @@ template <int KY, int KX, int SY, int SX, bool VEC>
 void LaunchUnpoolBlock(int reducer, const UnpoolArgs &a, const mshadow::FastDivU32 &div_bw) {
   switch (reducer) {
     case MSHADOW_HIP_SUM:
-      hipLaunchKernelGGL((UnpoolBlockKernel<MSHADOW_HIP_SUM, KY, KX, SY, SX, VEC>), dim3(a.blocks),
+      LaunchKernelIfFits((UnpoolBlockKernel<MSHADOW_HIP_SUM, KY, KX, SY, SX, VEC>), dim3(a.blocks),
                          dim3(kPoolBlock), a.lds, a.s, UNPOOL_ARGS(a), div_bw);
       break;
     case MSHADOW_HIP_MAX:
-      hipLaunchKernelGGL((UnpoolBlockKernel<MSHADOW_HIP_MAX, KY, KX, SY, SX, VEC>), dim3(a.blocks),
+      LaunchKernelIfFits((UnpoolBlockKernel<MSHADOW_HIP_MAX, KY, KX, SY, SX, VEC>), dim3(a.blocks),
                          dim3(kPoolBlock), a.lds, a.s, UNPOOL_ARGS(a), div_bw);
       break;
     default:
-      hipLaunchKernelGGL((UnpoolBlockKernel<MSHADOW_HIP_MIN, KY, KX, SY, SX, VEC>), dim3(a.blocks),
+      LaunchKernelIfFits((UnpoolBlockKernel<MSHADOW_HIP_MIN, KY, KX, SY, SX, VEC>), dim3(a.blocks),
                          dim3(kPoolBlock), a.lds, a.s, UNPOOL_ARGS(a), div_bw);
       break;
   }
@@ -380,15 +380,15 @@ void LaunchUnpoolBlock(int reducer, const UnpoolArgs &a, const mshadow::FastDivU
 void LaunchUnpoolGeneric(int reducer, const UnpoolArgs &a) {
   switch (reducer) {
     case MSHADOW_HIP_SUM:
-      hipLaunchKernelGGL((UnpoolKernel<MSHADOW_HIP_SUM, 0, 0, 0, 0>), dim3(a.blocks), dim3(kPoolBlock),
+      LaunchKernelIfFits((UnpoolKernel<MSHADOW_HIP_SUM, 0, 0, 0, 0>), dim3(a.blocks), dim3(kPoolBlock),
                          a.lds, a.s, UNPOOL_ARGS(a));
       break;
     case MSHADOW_HIP_MAX:
-      hipLaunchKernelGGL((UnpoolKernel<MSHADOW_HIP_MAX, 0, 0, 0, 0>), dim3(a.blocks), dim3(kPoolBlock),
+      LaunchKernelIfFits((UnpoolKernel<MSHADOW_HIP_MAX, 0, 0, 0, 0>), dim3(a.blocks), dim3(kPoolBlock),
                          a.lds, a.s, UNPOOL_ARGS(a));
       break;
     default:
-      hipLaunchKernelGGL((UnpoolKernel<MSHADOW_HIP_MIN, 0, 0, 0, 0>), dim3(a.blocks), dim3(kPoolBlock),
+      LaunchKernelIfFits((UnpoolKernel<MSHADOW_HIP_MIN, 0, 0, 0, 0>), dim3(a.blocks), dim3(kPoolBlock),
                          a.lds, a.s, UNPOOL_ARGS(a));
       break;
   }
@@ -403,7 +403,7 @@ struct GradLaunch {
 template <bool VEC>
 void LaunchGrad(int flags, const GradLaunch &g) {
 #define GRAD2D(FLAGS)                                                                         \
-  hipLaunchKernelGGL((SoftmaxGradKernel<VEC, FLAGS>), dim3(g.blocks), dim3(kGradBlock), 0, g.s, \
+  LaunchKernelIfFits((SoftmaxGradKernel<VEC, FLAGS>), dim3(g.blocks), dim3(kGradBlock), 0, g.s, \
                      g.dst, g.dstride, g.src, g.sstride, g.label, g.cols, g.chunks, g.gp)
   switch (flags) {
     case 0: GRAD2D(0); break;
@@ -429,7 +429,7 @@ static int LaunchRowsByIndex(float *dst, int dstride, int k_rows, const void *ro
                    cols % 4 == 0;
   hipStream_t s = AsStream(stream);
 #define ROWS_LAUNCH(ITYPE, VEC)                                                               \
-  hipLaunchKernelGGL((RowsByIndexKernel<ITYPE, float, OP, VEC>), dim3(grid), dim3(kTakeBlock), 0, \
+  LaunchKernelIfFits((RowsByIndexKernel<ITYPE, float, OP, VEC>), dim3(grid), dim3(kTakeBlock), 0, \
                      s, dst, dstride, k_rows, rows_per_wave, static_cast<const ITYPE *>(rows_of), \
                      static_cast<const ITYPE *>(from_of), n_index, src, sstride, cols)
   if (index_is_int) {
@@ -457,13 +457,13 @@ template <bool TERMS_GIVEN>
 bool LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, int rows, int cols,
                         hipStream_t s) {
 #define SHORT_THREAD(CMAX) \
-  hipLaunchKernelGGL((SoftmaxThreadRowKernel<CMAX, TERMS_GIVEN>), dim3((rows + 255) / 256), dim3(256), 0, s, \
+  LaunchKernelIfFits((SoftmaxThreadRowKernel<CMAX, TERMS_GIVEN>), dim3((rows + 255) / 256), dim3(256), 0, s, \
                      dst, dstride, src, sstride, rows, cols)
 #define SHORT_PART(LANES, N) \
-  hipLaunchKernelGGL((SoftmaxPartWaveKernel<LANES, N, TERMS_GIVEN>), dim3((rows + 256 / LANES - 1) / (256 / LANES)), \
+  LaunchKernelIfFits((SoftmaxPartWaveKernel<LANES, N, TERMS_GIVEN>), dim3((rows + 256 / LANES - 1) / (256 / LANES)), \
                      dim3(256), 0, s, dst, dstride, src, sstride, rows, cols)
 #define WAVE_SLABS(SLABS) \
-  hipLaunchKernelGGL((SoftmaxWaveSlabsKernel<SLABS, TERMS_GIVEN>), dim3((rows + 3) / 4), dim3(256), 0, s, dst, \
+  LaunchKernelIfFits((SoftmaxWaveSlabsKernel<SLABS, TERMS_GIVEN>), dim3((rows + 3) / 4), dim3(256), 0, s, dst, \
                      dstride, src, sstride, rows, cols)
   const int cus = mshadow_abi::ComputeUnits();
   /* Four or two rows side by side in a wave are fewer instructions, a wave to itself brings a row to
@@ -610,7 +610,7 @@ int mshadow_hip_softmax_f32(float *dst, int dstride, const float *src, int sstri
   /* 16-byte packs wherever the rows start and whatever their length (the accesses need no
      alignment; a row's last, partial pack goes element by element) */
 #define SOFTMAX_LAUNCH(T, S, V) \
-  hipLaunchKernelGGL((SoftmaxRowKernel<T, S, V, false>), dim3(rows), dim3(T), 0, s, dst, dstride, \
+  LaunchKernelIfFits((SoftmaxRowKernel<T, S, V, false>), dim3(rows), dim3(T), 0, s, dst, dstride, \
                      src, sstride, cols)
   /* many rows of 8193 to 16384 columns: four waves a row with 64 columns a thread, eight rows to a
      CU instead of four ((4096,10000): 82 against 104 us, (8192,12288): 153 against 196 us; with
@@ -632,10 +632,10 @@ int mshadow_hip_softmax_f32(float *dst, int dstride, const float *src, int sstri
   else if (cols > INT_MAX - 32768) {
     return Fail(MSHADOW_HIP_ERR_ARGUMENT, "softmax: row too long for 32-bit column counts");
   } else if (rows > mshadow_abi::ComputeUnits()) {
-    hipLaunchKernelGGL((SoftmaxStretchRowKernel<512, 16, false, 4>), dim3(rows), dim3(512), 0, s, dst,
+    LaunchKernelIfFits((SoftmaxStretchRowKernel<512, 16, false, 4>), dim3(rows), dim3(512), 0, s, dst,
                        dstride, src, sstride, cols);
   } else {
-    hipLaunchKernelGGL((SoftmaxStretchRowKernel<512, 16, false, 2>), dim3(rows), dim3(512), 0, s, dst,
+    LaunchKernelIfFits((SoftmaxStretchRowKernel<512, 16, false, 2>), dim3(rows), dim3(512), 0, s, dst,
                        dstride, src, sstride, cols);
   }
 #undef SOFTMAX_LAUNCH
@@ -663,12 +663,12 @@ int mshadow_hip_softmax_rowsum_f32(float *sums, const float *terms, int tstride,
   /* rows longer than a workgroup's registers hold: stretch by stretch, at any alignment */
   if (cols > 65536 || (!vec && cols > 32768)) {
     ABI_REQUIRE(cols <= INT_MAX - 32768, "row too long for 32-bit column counts");
-    hipLaunchKernelGGL((SoftmaxStretchRowKernel<512, 16, true, 2>), dim3(rows), dim3(512), 0, s, sums, 0,
+    LaunchKernelIfFits((SoftmaxStretchRowKernel<512, 16, true, 2>), dim3(rows), dim3(512), 0, s, sums, 0,
                        terms, tstride, cols);
     return AfterLaunch("softmax_rowsum");
   }
 #define ROWSUM_LAUNCH(T, S, V) \
-  hipLaunchKernelGGL((SoftmaxRowKernel<T, S, V, true>), dim3(rows), dim3(T), 0, s, sums, 0, terms, \
+  LaunchKernelIfFits((SoftmaxRowKernel<T, S, V, true>), dim3(rows), dim3(T), 0, s, sums, 0, terms, \
                      tstride, cols)
   if (vec) {
     if (cols > 8192 && cols <= 16384 && rows >= 16 * mshadow_abi::ComputeUnits()) ROWSUM_LAUNCH(256, 16, 4);  // as above
@@ -720,7 +720,7 @@ int mshadow_hip_softmax_grad_ex_f32(float *dst, int dstride, const float *src, i
     const unsigned grid = static_cast<unsigned>((rows + rows_per_block - 1) / rows_per_block);
     const mshadow::FastDivU32 div_ppr(static_cast<uint32_t>(ppr));
 #define GRAD_SHORT(FLAGS)                                                                            \
-  hipLaunchKernelGGL((SoftmaxGradShortRowsKernel<FLAGS>), dim3(grid), dim3(kGradBlock), 0, AsStream(stream), \
+  LaunchKernelIfFits((SoftmaxGradShortRowsKernel<FLAGS>), dim3(grid), dim3(kGradBlock), 0, AsStream(stream), \
                      dst, dstride, src, sstride, label, rows, cols, rows_per_block, div_ppr, gp)
     switch (flags) {
       case 0: GRAD_SHORT(0); break;
@@ -756,19 +756,19 @@ int mshadow_hip_softmax3d_f32(float *dst, int dstride, const float *src, int sst
   const unsigned pairs = static_cast<unsigned>(d0) * d2;
   const unsigned one_each = (pairs + kSoftmax3dBlock - 1) / kSoftmax3dBlock;
   if (d1 <= 8) {
-    hipLaunchKernelGGL((Softmax3dSmallKernel<8>), dim3(one_each), dim3(kSoftmax3dBlock), 0,
+    LaunchKernelIfFits((Softmax3dSmallKernel<8>), dim3(one_each), dim3(kSoftmax3dBlock), 0,
                        AsStream(stream), dst, dstride, src, sstride, d0, d1, d2, div_d2s);
     return AfterLaunch("softmax3d");
   }
   if (d1 <= 32) {
-    hipLaunchKernelGGL((Softmax3dSmallKernel<32>), dim3(one_each), dim3(kSoftmax3dBlock), 0,
+    LaunchKernelIfFits((Softmax3dSmallKernel<32>), dim3(one_each), dim3(kSoftmax3dBlock), 0,
                        AsStream(stream), dst, dstride, src, sstride, d0, d1, d2, div_d2s);
     return AfterLaunch("softmax3d");
   }
   unsigned grid = 0;
   int st = mshadow_hip_suggest_grid(static_cast<size_t>(d0) * d2, kSoftmax3dBlock, 8, &grid);
   if (st != MSHADOW_HIP_OK) return st;
-  hipLaunchKernelGGL(Softmax3dKernel, dim3(grid), dim3(kSoftmax3dBlock), 0, AsStream(stream), dst,
+  LaunchKernelIfFits(Softmax3dKernel, dim3(grid), dim3(kSoftmax3dBlock), 0, AsStream(stream), dst,
                      dstride, src, sstride, d0, d1, d2,
                      mshadow::FastDivU32(static_cast<uint32_t>(d2)));
   return AfterLaunch("softmax3d");
@@ -796,7 +796,7 @@ int mshadow_hip_softmax3d_grad_f32(float *dst, int dstride, const float *src, in
     const unsigned vgrid = (packs + kSoftmax3dBlock - 1) / kSoftmax3dBlock;
     const mshadow::FastDivU32 div_q2(static_cast<uint32_t>(d2 / 4));
 #define GRAD3DV(FLAGS)                                                                         \
-  hipLaunchKernelGGL((Softmax3dGradVecKernel<FLAGS>), dim3(vgrid), dim3(kSoftmax3dBlock), 0,   \
+  LaunchKernelIfFits((Softmax3dGradVecKernel<FLAGS>), dim3(vgrid), dim3(kSoftmax3dBlock), 0,   \
                      AsStream(stream), dst, dstride, src, sstride, label, lstride, d0, d1, d2, \
                      div_q2, div_d1, gp)
     switch (flags) {
@@ -809,7 +809,7 @@ int mshadow_hip_softmax3d_grad_f32(float *dst, int dstride, const float *src, in
     return AfterLaunch("softmax3d_grad");
   }
 #define GRAD3D(FLAGS)                                                                          \
-  hipLaunchKernelGGL((Softmax3dGradKernel<FLAGS>), dim3(grid), dim3(kSoftmax3dBlock), 0,       \
+  LaunchKernelIfFits((Softmax3dGradKernel<FLAGS>), dim3(grid), dim3(kSoftmax3dBlock), 0,       \
                      AsStream(stream), dst, dstride, src, sstride, label, lstride, d0, d1, d2, \
                      div_d2, div_d1, gp)
   switch (flags) {
@@ -879,7 +879,7 @@ int mshadow_hip_reduce_keep_lowest_f32(float *dst, const float *src, int sstride
       typedef decltype(red) R;
       typedef decltype(sv) S;
 #define LOWEST_STRIP(STRIP)                                                                     \
-  hipLaunchKernelGGL((mshadow::hip::ReduceKeepLowestStripKernel<S, R, mshadow::hip::STRIP>),    \
+  LaunchKernelIfFits((mshadow::hip::ReduceKeepLowestStripKernel<S, R, mshadow::hip::STRIP>),    \
                      dim3((cols + mshadow::hip::STRIP::kCols - 1) / mshadow::hip::STRIP::kCols), \
                      dim3(mshadow::hip::STRIP::kThreads), 0, s, dst, src,                       \
                      static_cast<uint32_t>(sstride), static_cast<uint32_t>(rows),               \
@@ -888,7 +888,7 @@ int mshadow_hip_reduce_keep_lowest_f32(float *dst, const float *src, int sstride
         /* a strip for each CU at most and a long chain: four rows to an LDS read and stages of
            512 rows make its step 3.5 instead of 4.2 ns (65536 x 1000: 231 against 276 us;
            8191 x 1000: 36.7 against 38.2 us; level at 6000; 4096 x 2000: 22 against 20 us) */
-        hipLaunchKernelGGL((mshadow::hip::ReduceKeepLowestDmaKernel<S, R>),
+        LaunchKernelIfFits((mshadow::hip::ReduceKeepLowestDmaKernel<S, R>),
                            dim3((cols + mshadow::hip::kLowestCols - 1) / mshadow::hip::kLowestCols),
                            dim3(mshadow::hip::kDmaThreads), 0, s, dst, src,
                            static_cast<uint32_t>(sstride), static_cast<uint32_t>(rows),
@@ -958,7 +958,7 @@ int mshadow_hip_reduce_keep_highdim_f32(float *dst, const float *src, int sstrid
   for (long long c0 = 0, most = RowsOfLaunch(T); c0 < c; c0 += most) {                         \
     RawPlan1D<float> d = {dst + c0};                                                           \
     RawPlan2D<const float> sp = {src + c0 * y * sstride, sstride};                             \
-    hipLaunchKernelGGL((mshadow::hip::ReduceKeepHighDimKernel<S, R, float, T, SEGS, RawPlan1D<float>, \
+    LaunchKernelIfFits((mshadow::hip::ReduceKeepHighDimKernel<S, R, float, T, SEGS, RawPlan1D<float>, \
                                                               RawPlan2D<const float> >),       \
                        dim3(static_cast<unsigned>(c - c0 < most ? c - c0 : most)), dim3(T), 0, s, d, sp, \
                        static_cast<uint32_t>(n), static_cast<uint32_t>(c), static_cast<uint32_t>(y), \
@@ -966,7 +966,7 @@ int mshadow_hip_reduce_keep_highdim_f32(float *dst, const float *src, int sstrid
   }
 #define HIGHDIM_LAUNCH(SEGS)                                                                   \
   if (large)                                                                                   \
-    hipLaunchKernelGGL((mshadow::hip::ReduceKeepHighDimDmaKernel<S, R, float, SEGS>), dim3(c),        \
+    LaunchKernelIfFits((mshadow::hip::ReduceKeepHighDimDmaKernel<S, R, float, SEGS>), dim3(c),        \
                        dim3(mshadow::hip::kDmaThreads), 0, s, dst, src,                        \
                        static_cast<uint32_t>(sstride), static_cast<uint32_t>(n),               \
                        static_cast<uint32_t>(c), static_cast<uint32_t>(y),                     \
@@ -975,7 +975,7 @@ int mshadow_hip_reduce_keep_highdim_f32(float *dst, const float *src, int sstrid
       const bool large = static_cast<long long>(n) * y * x >= kDmaMinPerKept;
       if (large && split_partial != NULL) {
 #define HIGHDIM_SPLIT(RING)                                                                    \
-  hipLaunchKernelGGL((mshadow::hip::ReduceKeepHighDimSplitKernel<S, R, float, RING>),          \
+  LaunchKernelIfFits((mshadow::hip::ReduceKeepHighDimSplitKernel<S, R, float, RING>),          \
                      dim3((static_cast<unsigned>(n) * c + RING::kSegs - 1) / RING::kSegs),      \
                      dim3(RING::kThreads), 0, s, dst, src, static_cast<uint32_t>(v_stride),    \
                      static_cast<uint32_t>(n), static_cast<uint32_t>(c),                       \
@@ -1066,9 +1066,9 @@ int mshadow_hip_pool_f32(float *dst, int dstride, const float *src, int sstride,
   }
 #define POOL_SWITCH(KERNEL, ...)                                                               \
   switch (reducer) {                                                                           \
-    case MSHADOW_HIP_SUM: hipLaunchKernelGGL((KERNEL<MSHADOW_HIP_SUM>), __VA_ARGS__); break;    \
-    case MSHADOW_HIP_MAX: hipLaunchKernelGGL((KERNEL<MSHADOW_HIP_MAX>), __VA_ARGS__); break;    \
-    default: hipLaunchKernelGGL((KERNEL<MSHADOW_HIP_MIN>), __VA_ARGS__); break;                 \
+    case MSHADOW_HIP_SUM: LaunchKernelIfFits((KERNEL<MSHADOW_HIP_SUM>), __VA_ARGS__); break;    \
+    case MSHADOW_HIP_MAX: LaunchKernelIfFits((KERNEL<MSHADOW_HIP_MAX>), __VA_ARGS__); break;    \
+    default: LaunchKernelIfFits((KERNEL<MSHADOW_HIP_MIN>), __VA_ARGS__); break;                 \
   }
   /* windows that move by one element, all of them whole: PoolColumnsS1Kernel below has a variant */
   const bool columns = sy == 1 && sx == 1 && ky == kx && (ky == 2 || ky == 3 || ky == 5) &&
@@ -1091,15 +1091,15 @@ int mshadow_hip_pool_f32(float *dst, int dstride, const float *src, int sstride,
 #define POOL_PLANES(KY, KX)                                                                     \
   switch (reducer) {                                                                           \
     case MSHADOW_HIP_SUM:                                                                      \
-      hipLaunchKernelGGL((PoolPlanesKernel<MSHADOW_HIP_SUM, KY, KX>), dim3(blocks), dim3(kPoolBlock), \
+      LaunchKernelIfFits((PoolPlanesKernel<MSHADOW_HIP_SUM, KY, KX>), dim3(blocks), dim3(kPoolBlock), \
                          lds, s, dst, dstride, src, sstride, g, planes, static_cast<int>(per_block), div_ph); \
       break;                                                                                   \
     case MSHADOW_HIP_MAX:                                                                      \
-      hipLaunchKernelGGL((PoolPlanesKernel<MSHADOW_HIP_MAX, KY, KX>), dim3(blocks), dim3(kPoolBlock), \
+      LaunchKernelIfFits((PoolPlanesKernel<MSHADOW_HIP_MAX, KY, KX>), dim3(blocks), dim3(kPoolBlock), \
                          lds, s, dst, dstride, src, sstride, g, planes, static_cast<int>(per_block), div_ph); \
       break;                                                                                   \
     default:                                                                                   \
-      hipLaunchKernelGGL((PoolPlanesKernel<MSHADOW_HIP_MIN, KY, KX>), dim3(blocks), dim3(kPoolBlock), \
+      LaunchKernelIfFits((PoolPlanesKernel<MSHADOW_HIP_MIN, KY, KX>), dim3(blocks), dim3(kPoolBlock), \
                          lds, s, dst, dstride, src, sstride, g, planes, static_cast<int>(per_block), div_ph); \
       break;                                                                                   \
   }
@@ -1133,15 +1133,15 @@ int mshadow_hip_pool_f32(float *dst, int dstride, const float *src, int sstride,
 #define POOL_COLUMNS(K)                                                                        \
   switch (reducer) {                                                                           \
     case MSHADOW_HIP_SUM:                                                                      \
-      hipLaunchKernelGGL((PoolColumnsS1Kernel<MSHADOW_HIP_SUM, K, K>), dim3(static_cast<unsigned>(blocks)), \
+      LaunchKernelIfFits((PoolColumnsS1Kernel<MSHADOW_HIP_SUM, K, K>), dim3(static_cast<unsigned>(blocks)), \
                          dim3(kPoolBlock), lds, s, dst, dstride, src, sstride, g, nruns, run_len, div_pw); \
       break;                                                                                   \
     case MSHADOW_HIP_MAX:                                                                      \
-      hipLaunchKernelGGL((PoolColumnsS1Kernel<MSHADOW_HIP_MAX, K, K>), dim3(static_cast<unsigned>(blocks)), \
+      LaunchKernelIfFits((PoolColumnsS1Kernel<MSHADOW_HIP_MAX, K, K>), dim3(static_cast<unsigned>(blocks)), \
                          dim3(kPoolBlock), lds, s, dst, dstride, src, sstride, g, nruns, run_len, div_pw); \
       break;                                                                                   \
     default:                                                                                   \
-      hipLaunchKernelGGL((PoolColumnsS1Kernel<MSHADOW_HIP_MIN, K, K>), dim3(static_cast<unsigned>(blocks)), \
+      LaunchKernelIfFits((PoolColumnsS1Kernel<MSHADOW_HIP_MIN, K, K>), dim3(static_cast<unsigned>(blocks)), \
                          dim3(kPoolBlock), lds, s, dst, dstride, src, sstride, g, nruns, run_len, div_pw); \
       break;                                                                                   \
   }
@@ -1154,15 +1154,15 @@ int mshadow_hip_pool_f32(float *dst, int dstride, const float *src, int sstride,
 #define POOL_TILED(KY, KX)                                                                     \
   switch (reducer) {                                                                           \
     case MSHADOW_HIP_SUM:                                                                      \
-      hipLaunchKernelGGL((PoolKernel<MSHADOW_HIP_SUM, KY, KX>), dim3(static_cast<unsigned>(blocks)), \
+      LaunchKernelIfFits((PoolKernel<MSHADOW_HIP_SUM, KY, KX>), dim3(static_cast<unsigned>(blocks)), \
                          dim3(kPoolBlock), lds, s, dst, dstride, src, sstride, g);             \
       break;                                                                                   \
     case MSHADOW_HIP_MAX:                                                                      \
-      hipLaunchKernelGGL((PoolKernel<MSHADOW_HIP_MAX, KY, KX>), dim3(static_cast<unsigned>(blocks)), \
+      LaunchKernelIfFits((PoolKernel<MSHADOW_HIP_MAX, KY, KX>), dim3(static_cast<unsigned>(blocks)), \
                          dim3(kPoolBlock), lds, s, dst, dstride, src, sstride, g);             \
       break;                                                                                   \
     default:                                                                                   \
-      hipLaunchKernelGGL((PoolKernel<MSHADOW_HIP_MIN, KY, KX>), dim3(static_cast<unsigned>(blocks)), \
+      LaunchKernelIfFits((PoolKernel<MSHADOW_HIP_MIN, KY, KX>), dim3(static_cast<unsigned>(blocks)), \
                          dim3(kPoolBlock), lds, s, dst, dstride, src, sstride, g);             \
       break;                                                                                   \
   }
@@ -1219,10 +1219,10 @@ int mshadow_hip_unpool_f32(float *dst, int dstride, const float *src, int sstrid
 #define UNPOOL_ROWS(R)                                                                          \
   do {                                                                                          \
     if (whole) {                                                                                \
-      hipLaunchKernelGGL((UnpoolRows3x3s2Kernel<R, false>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, \
+      LaunchKernelIfFits((UnpoolRows3x3s2Kernel<R, false>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, \
                          dstride, src, sstride, pooled, pstride, grad, gstride, g, rg);         \
     } else {                                                                                    \
-      hipLaunchKernelGGL((UnpoolRows3x3s2Kernel<R, true>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, \
+      LaunchKernelIfFits((UnpoolRows3x3s2Kernel<R, true>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, \
                          dstride, src, sstride, pooled, pstride, grad, gstride, g, rg);         \
     }                                                                                           \
   } while (0)
@@ -1253,13 +1253,13 @@ int mshadow_hip_unpool_f32(float *dst, int dstride, const float *src, int sstrid
 #define UNPOOL_SLIDE(R)                                                                        \
   do {                                                                                         \
     if (ky == 2) {                                                                             \
-      hipLaunchKernelGGL((UnpoolSlideS1Kernel<R, 2, 4>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, dstride, \
+      LaunchKernelIfFits((UnpoolSlideS1Kernel<R, 2, 4>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, dstride, \
                          src, sstride, pooled, pstride, grad, gstride, g, sg);                 \
     } else if (ky == 3) {                                                                      \
-      hipLaunchKernelGGL((UnpoolSlideS1Kernel<R, 3, 3>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, dstride, \
+      LaunchKernelIfFits((UnpoolSlideS1Kernel<R, 3, 3>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, dstride, \
                          src, sstride, pooled, pstride, grad, gstride, g, sg);                 \
     } else {                                                                                   \
-      hipLaunchKernelGGL((UnpoolSlideS1Kernel<R, 5, 5>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, dstride, \
+      LaunchKernelIfFits((UnpoolSlideS1Kernel<R, 5, 5>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, dstride, \
                          src, sstride, pooled, pstride, grad, gstride, g, sg);                 \
     }                                                                                          \
   } while (0)
@@ -1314,17 +1314,17 @@ int mshadow_hip_unpool_f32(float *dst, int dstride, const float *src, int sstrid
 #define UNPOOL_PLANES(KY, KX, SY, SX)                                                          \
   switch (reducer) {                                                                           \
     case MSHADOW_HIP_SUM:                                                                      \
-      hipLaunchKernelGGL((UnpoolPlanesKernel<MSHADOW_HIP_SUM, KY, KX, SY, SX>), dim3(blocks),   \
+      LaunchKernelIfFits((UnpoolPlanesKernel<MSHADOW_HIP_SUM, KY, KX, SY, SX>), dim3(blocks),   \
                          dim3(kPoolBlock), lds, s, dst, dstride, src, sstride, pooled, pstride, \
                          grad, gstride, g, planes, static_cast<int>(per_block), div_h);        \
       break;                                                                                   \
     case MSHADOW_HIP_MAX:                                                                      \
-      hipLaunchKernelGGL((UnpoolPlanesKernel<MSHADOW_HIP_MAX, KY, KX, SY, SX>), dim3(blocks),   \
+      LaunchKernelIfFits((UnpoolPlanesKernel<MSHADOW_HIP_MAX, KY, KX, SY, SX>), dim3(blocks),   \
                          dim3(kPoolBlock), lds, s, dst, dstride, src, sstride, pooled, pstride, \
                          grad, gstride, g, planes, static_cast<int>(per_block), div_h);        \
       break;                                                                                   \
     default:                                                                                   \
-      hipLaunchKernelGGL((UnpoolPlanesKernel<MSHADOW_HIP_MIN, KY, KX, SY, SX>), dim3(blocks),   \
+      LaunchKernelIfFits((UnpoolPlanesKernel<MSHADOW_HIP_MIN, KY, KX, SY, SX>), dim3(blocks),   \
                          dim3(kPoolBlock), lds, s, dst, dstride, src, sstride, pooled, pstride, \
                          grad, gstride, g, planes, static_cast<int>(per_block), div_h);        \
       break;                                                                                   \

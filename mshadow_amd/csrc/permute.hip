@@ -486,11 +486,11 @@ extern "C" int mshadow_hip_permute_32(void *dst, const void *src, int ndim, cons
               reinterpret_cast<uintptr_t>(dst) % 16 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0;
   for (int k = 0; k < ba.count; ++k) wide = wide && ba.src_step[k] % 4 == 0 && ba.dst_step[k] % 4 == 0;
   if (wide) {
-    hipLaunchKernelGGL(PermuteTileVecKernel, dim3(static_cast<unsigned>(blocks)), dim3(kPermuteBlock),
+    LaunchKernelIfFits(PermuteTileVecKernel, dim3(static_cast<unsigned>(blocks)), dim3(kPermuteBlock),
                        0, s, d, sp, extent_a, extent_l, sstep[n - 1], dstep[b], FastDivU32(ta),
                        FastDivU32(tl), ba);
   } else {
-    hipLaunchKernelGGL(PermuteTileKernel, dim3(static_cast<unsigned>(blocks)), dim3(kPermuteBlock), 0,
+    LaunchKernelIfFits(PermuteTileKernel, dim3(static_cast<unsigned>(blocks)), dim3(kPermuteBlock), 0,
                        s, d, sp, extent_a, extent_l, sstep[n - 1], dstep[b], FastDivU32(ta),
                        FastDivU32(tl), ba);
   }

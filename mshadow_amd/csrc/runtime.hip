@@ -13,6 +13,10 @@ std::string &LastError() {
   static thread_local std::string msg;
   return msg;
 }
+bool &LaunchRefused() {
+  static thread_local bool refused = false;
+  return refused;
+}
 }  // namespace mshadow_abi
 
 namespace mshadow_abi {
@@ -243,8 +247,9 @@ int mshadow_hip_launch(const void *kernel, const uint32_t grid[3], const uint32_
   ABI_REQUIRE(block[0] * block[1] * block[2] > 0 && block[0] * block[1] * block[2] <= 1024,
               "block size out of range");
   ABI_REQUIRE(lds_bytes <= 160 * 1024, "more than 160 KB of LDS requested");
-  ABI_HIP(hipLaunchKernel(kernel, dim3(grid[0], grid[1], grid[2]),
-                          dim3(block[0], block[1], block[2]), args, lds_bytes, AsStream(stream)));
+  const dim3 blocks(grid[0], grid[1], grid[2]), threads(block[0], block[1], block[2]);
+  ABI_REQUIRE(LaunchFits(blocks, threads), "too large for one launch (2^32 threads or more)");
+  ABI_HIP(hipLaunchKernel(kernel, blocks, threads, args, lds_bytes, AsStream(stream)));
   return AfterLaunch("kernel launch");
 }
 int mshadow_hip_peek_last_error(void) { return FromHip(hipPeekAtLastError(), "pending error"); }

@@ -9,7 +9,7 @@ import pytest
 
 from checkers import Checker
 from gpu_util import assert_bits_equal, f32
-from mshadow_amd.capi import DeviceBuffer
+from mshadow_amd.capi import DeviceBuffer, HipError
 
 pytestmark = pytest.mark.gpu
 SOME = 40
@@ -91,6 +91,13 @@ def test_softmax_gradient(G, O, dtype, cols):
     (G.case_softmax_grad if dtype == np.uint16 else G.softmax_grad)(m, m, labels)
     for p in at:
         assert_bits_equal(DeviceBuffer.download(p), want)
+
+
+def test_columns_of_two_rows(G):
+    """where no call takes less than 2^32 threads the launch is refused, not cut short"""
+    m, dst = G.buffer((2, 870_000_000), f32), G.buffer((870_000_000,), f32)
+    with pytest.raises(HipError, match="2\\^32"):
+        G.reduce_keep_lowest(dst, m)
 
 
 @pytest.mark.parametrize("n", [1, 3])

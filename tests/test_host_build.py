@@ -189,6 +189,16 @@ def test_header_api_on_cpu_matches_oracle(tmp_path, orc):
     assert out.startswith("OK"), out
 
 
+def test_launch_of_too_many_threads_is_refused():
+    """HIP would launch the number of threads modulo 2^32; no device is asked"""
+    lib = _lib("libmshadow_hip.so")
+    lib.mshadow_hip_last_error.restype = ctypes.c_char_p
+    u3 = ctypes.c_uint32 * 3
+    for grid, block in (((1 << 24, 1, 1), (256, 1, 1)), ((1, 1 << 30, 1), (1, 4, 1)), ((2, 2, 1 << 31), (1, 1, 64))):
+        st = lib.mshadow_hip_launch(ctypes.c_void_p(1), u3(*grid), u3(*block), None, ctypes.c_size_t(0), None)
+        assert st == 2 and b"2^32" in lib.mshadow_hip_last_error()   # MSHADOW_HIP_ERR_ARGUMENT
+
+
 def test_half2_on_host_tensors(tmp_path):
     _lib("libmshadow_hip.so")
     out = _compile_and_run(tmp_path, "half2_check.cc",
