@@ -116,7 +116,7 @@ def test_gpu_reductions(G):
     assert_bits_equal(o.download(), GOLD["red_highdim_sum_minusto_scaled"], "minusto")
     o = G.buffer((24,), f32)
     G.reduce_keep_lowest(o, G.to_device(GOLD["red_long"]), SUM, SAVETO, 1.0)
-    assert_bits_equal(o.download(), GOLD["red_long_lowest_sum"], "long columns (direct-to-LDS kernel)")
+    assert_bits_equal(o.download(), GOLD["red_long_lowest_sum"], "long columns (strips of columns)")
 
 
 @pytest.mark.gpu

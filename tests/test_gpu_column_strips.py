@@ -26,9 +26,12 @@ def O():
 
 
 # strips of 16, 32 and 64 columns (up to 4096 and 8192 columns and beyond), the last one not full,
-# and the short ring (up to 1024 rows, more than 32768 columns)
+# and the short ring (up to 1024 rows, more than 32768 columns); 6144 rows and more of up to 4096 float
+# columns, 4000 of up to 64 and 2400 of one take the kernel of long chains, whose stages have 512 rows
 SHAPES = [(1, 16), (15, 17), (16, 1), (64, 15), (65, 4096), (129, 4097), (257, 33), (2047, 40), (2048, 4097),
-          (63, 8192), (64, 8193), (320, 8255), (513, 9000), (1024, 32769), (1025, 32775), (32, 32800), (97, 33000)]
+          (63, 8192), (64, 8193), (320, 8255), (513, 9000), (1024, 32769), (1025, 32775), (32, 32800), (97, 33000),
+          (2399, 1), (2400, 1), (3999, 10), (4000, 64), (4001, 65), (6143, 65), (6144, 70), (6145, 1),
+          (6657, 33), (8191, 1000), (6150, 4095)]
 
 
 def offset_view(buf, cols, shift):

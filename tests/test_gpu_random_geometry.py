@@ -145,7 +145,7 @@ def test_softmax_random_shapes(G, O, stream, seed):
     assert_bits_equal(dg.download(stream), wantg, f"softmax_grad {shape} pad {pad}")
 
 
-@pytest.mark.parametrize("seed", range(80))
+@pytest.mark.parametrize("seed", range(92))
 def test_reductions_random_shapes(G, O, stream, seed):
     """sum_rows and sumall_except_dim<1> bit for bit (the kernels keep the CPU path's order of
     additions) on shapes drawn around the borders between their routes"""
@@ -157,8 +157,11 @@ def test_reductions_random_shapes(G, O, stream, seed):
     if seed % 2 == 0:
         rows = int(rng.choice((1, 2, 63, 64, 65, 255, 256, 257, 1000, 4097)))
         cols = int(rng.choice((1, 3, 4, 15, 16, 17, 31, 32, 33, 64, 100, 255, 256, 1000, 4096, 4100)))
+        if seed >= 80:   # few columns of many rows, where the kernel of long chains begins
+            rows = int(rng.choice((6143, 6144, 6145, 6656, 9001)))
         if rows * cols > 1 << 21:
-            rows = max(1, (1 << 21) // cols)
+            rows = max(1, (1 << 21) // cols) if seed < 80 else rows
+            cols = cols if seed < 80 else (1 << 21) // rows
         m = rng.standard_normal((rows, cols)).astype(f32)
         start = rng.uniform(1, 3, cols).astype(f32)
         want = start.copy()
