@@ -1080,9 +1080,20 @@ int mshadow_hip_pool_f32(float *dst, int dstride, const float *src, int sstride,
   /* small planes: several whole planes per workgroup, about 24 KB of them. Planes of 1024 pixels and
      more keep the threads of the columns kernel busy (12 M pixels, 5x5: 50x50 24 against 35 us, 3x3:
      100x30 21 against 28 us; level at 32x32, and 7x7 is 16 us here against 312 us there), but for the
-     small windows on very narrow ones (3x3: 224x7 21 us here, 24 us there). */
+     small windows on very narrow ones (3x3: 224x7 21 us here, 24 us there). With windows of two and
+     three the two are close: where there are planes for full groups and whole rows fill a wave's
+     lanes here, the columns kernel is the faster one only on larger planes (12 M pixels, 3x3, here
+     and there: 61x17 25 and 32 us, 32x33 24 and 26, 17x63 24 and 30, 8x160 21 and 22, 45x33 26 and 23;
+     31x35, half the lanes idle here, 35 and 28; 3 M pixels, 17x63: 10 and 9). */
   const long long plane_bytes = static_cast<long long>(h) * row_bytes;
-  if (plane_bytes * 2 <= 24 * 1024 && planes >= 2 && !(columns && band >= 1 && h * w >= 1024 && (ky == 5 || w >= 16))) {
+  const auto columns_pay = [&]() {
+    if (ky == 5) return h * w >= 1024;
+    if (w < 16) return false;
+    const bool full_groups = planes / ((24 * 1024) / plane_bytes) >= 4ll * mshadow_abi::ComputeUnits();
+    const int lanes = pw < 64 ? pw * (64 / pw) : pw * 64 / ((pw + 63) / 64 * 64);  // of 64, at work here
+    return h * w >= (w > 100 && h < 13 ? 1300 : !full_groups || lanes < 51 ? 1024 : w % 4 == 0 && w > 16 ? 1100 : 1400);
+  };
+  if (plane_bytes * 2 <= 24 * 1024 && planes >= 2 && !(columns && band >= 1 && columns_pay())) {
     long long per_block = (24 * 1024) / plane_bytes;
     /* ... but no fewer workgroups than keep every CU busy four times over */
     while (per_block > 1 && (planes + per_block - 1) / per_block < 4ll * mshadow_abi::ComputeUnits()) {

@@ -26,14 +26,11 @@ PLANES = [(7, 7), (5, 24), (8, 23), (16, 16), (17, 15), (17, 16), (33, 17), (31,
           (15, 64), (16, 64), (65, 65), (17, 256), (20, 257), (49, 31)]
 
 
-@pytest.mark.parametrize("h,w", PLANES)
-@pytest.mark.parametrize("k", [2, 3, 5])
-def test_stride_one_pooling(G, O, h, w, k):
-    planes = 5
+def check(G, O, planes, h, w, k, reducers):
     # few distinct values: equal maxima inside a window, zeros of both signs
     src = np.round(uniform(80 + k, (planes, h, w)) * f32(4)) / f32(4)
     grad = normal(81, (planes, h - k + 1, w - k + 1))
-    for reducer in (MAX, SUM, MIN):
+    for reducer in reducers:
         want = np.empty(grad.shape, f32)
         O.pool(want, src, k, k, 1, 1, reducer)
         pooled = G.buffer(want.shape, f32)
@@ -44,3 +41,18 @@ def test_stride_one_pooling(G, O, h, w, k):
         dst = G.buffer(src.shape, f32)
         G.unpool(dst, G.to_device(src), pooled, G.to_device(grad), k, k, 1, 1, reducer)
         assert_bits_equal(dst.download(), want_dst, f"unpool {h}x{w} k{k} reducer {reducer}")
+
+
+@pytest.mark.parametrize("h,w", PLANES)
+@pytest.mark.parametrize("k", [2, 3, 5])
+def test_stride_one_pooling(G, O, h, w, k):
+    check(G, O, 5, h, w, k, (MAX, SUM, MIN))
+
+
+# planes enough for full groups of them, on both sides of the pixels from which the columns kernel pays; strips
+# of the 5x5 gradient by the waves there are; more low planes than waves of one turn, and as many
+@pytest.mark.parametrize("planes,h,w,k", [(5200, 61, 17, 2), (5119, 61, 17, 3), (4200, 88, 16, 3), (5200, 34, 33, 2), (3100, 8, 160, 3),
+                                          (300, 11, 130, 2), (2048, 7, 160, 5), (2049, 7, 160, 5), (2100, 40, 20, 5),
+                                          (9000, 16, 20, 5), (700, 33, 16, 5), (40, 130, 64, 5), (2049, 9, 141, 5)])
+def test_stride_one_pooling_of_many_planes(G, O, planes, h, w, k):
+    check(G, O, planes, h, w, k, (MAX,))
