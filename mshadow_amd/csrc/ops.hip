@@ -1015,7 +1015,7 @@ static const size_t kUnpoolLdsBudget = 16 * 1024;  // smaller bands: more workgr
 
 /*! \brief strips of the stride-1 unpool kernel over `rows` rows of `w` columns per plane:
  *  sixteen rows a strip, fewer while that leaves the machine short of waves */
-static SlideGeom MakeSlideGeom(int planes, int rows, int w) {
+static SlideGeom MakeSlideGeom(int planes, int rows, int w, int k) {
   SlideGeom sg;
   sg.groups = static_cast<uint32_t>((w + 3) / 4);
   sg.strips_per_wave = 64u / sg.groups;
@@ -1023,7 +1023,23 @@ static SlideGeom MakeSlideGeom(int planes, int rows, int w) {
   const uint32_t least = static_cast<uint32_t>((rows + 15) / 16);
   uint32_t r = (static_cast<uint32_t>(rows) + least - 1) / least;
   const long long want = 16ll * mshadow_abi::ComputeUnits();  // waves
-  while (r > 2 && static_cast<long long>(planes) * ((rows + r - 1) / r) / sg.strips_per_wave < want) r = (r + 1) / 2;
+  if (k == 5) {
+    /* Two waves of the kernel for 5 x 5 windows fill a SIMD, so strips are cut no further than it takes
+       to deal every SIMD two: a strip costs its rows and about two and a half for the four pooled rows
+       above it, times the turns of eight waves a CU. Against strips cut until there are 16 waves a
+       CU: 1.8 M pixels, 7x160 14.6 and 23.8 us, 9x50 13 and 21, 40x100 15 and 20; 4 M, 24x64 19 and 27,
+       16x32 20 and 29; 12 M, 40x40 66 and 75; 0.6 M level. */
+    long long best = -1;
+    for (uint32_t longest = r; longest >= 2; --longest) {
+      const uint32_t n = (static_cast<uint32_t>(rows) + longest - 1) / longest;
+      const uint32_t each = (static_cast<uint32_t>(rows) + n - 1) / n;
+      const long long waves = (static_cast<long long>(planes) * n + sg.strips_per_wave - 1) / sg.strips_per_wave;
+      const long long turns = (waves + 8ll * mshadow_abi::ComputeUnits() - 1) / (8ll * mshadow_abi::ComputeUnits());
+      const long long cost = turns * (2 * each + 5);
+      if (best < 0 || cost * 10 < best * 9) { best = cost; r = each; }
+    }
+  }
+  while (k != 5 && r > 2 && static_cast<long long>(planes) * ((rows + r - 1) / r) / sg.strips_per_wave < want) r = (r + 1) / 2;
   sg.strip_rows = r;
   sg.strips_per_plane = static_cast<uint32_t>((rows + r - 1) / r);
   sg.total_strips = static_cast<uint32_t>(planes) * sg.strips_per_plane;
@@ -1254,12 +1270,18 @@ int mshadow_hip_unpool_f32(float *dst, int dstride, const float *src, int sstrid
      12 M pixels: 3 x 3 56x56 54 us against 51, 63x70 58 against 52, 20x200 46 against 56; 2 x 2 28x28 74 against 64,
      56x56 50 against 65; 5 x 5 13x13 145 against 127, 16x16 76 against 103, 8x40 72 against 123,
      28x28 83 against 106, and beyond 4 KB a plane - one plane per workgroup there - 100x14 119 against
-     317, 224x7 251 against 472. */
-  const bool slides = ky == 5 ? static_cast<long long>(h) * w > 1024 || w >= 24 || (w >= 16 && w % 4 == 0)
+     317, 224x7 251 against 472. Low planes whose rows leave a third of the lanes idle are made twice
+     over here, most of their windows being cut off: 7x160 80 against 71 us, 8x140 (24 M pixels) 168
+     against 153, 5x128 57 against 46 - unless there are waves for one turn only (1.8 M pixels, 7x160
+     14.6 against 15.5 us). */
+  const int slide_lanes = w <= 256 ? (w + 3) / 4 * (64 / ((w + 3) / 4)) : 0;  // of 64 with pixels: 40 at 140 columns
+  const bool slides = ky == 5 ? (static_cast<long long>(h) * w > 1024 || (h > 5 && (w >= 24 || (w >= 16 && w % 4 == 0)))) &&
+                                    !(slide_lanes < 44 && h <= 9 && static_cast<long long>(h) * w <= 1280 &&
+                                      planes > 8 * mshadow_abi::ComputeUnits())
                       : ky == 2 ? w >= 32 : w >= 64 && (h >= 64 || (w >= 96 && h >= 16));
   if (ky == kx && (ky == 2 || ky == 3 || ky == 5) && sy == 1 && sx == 1 && w <= 256 && slides && ph >= 1 && pw >= 1 &&
       static_cast<long long>(planes) * ph * pw >= 4 && static_cast<long long>(planes) * ((h + 1) / 2) < (1ll << 31)) {
-    SlideGeom sg = MakeSlideGeom(planes, h, w);
+    SlideGeom sg = MakeSlideGeom(planes, h, w, ky);
     sg.src_floats = (static_cast<size_t>(planes) * h - 1) * sstride + w;
     sg.pooled_floats = (static_cast<size_t>(planes) * ph - 1) * pstride + pw;
     sg.grad_floats = (static_cast<size_t>(planes) * ph - 1) * gstride + pw;
