@@ -78,6 +78,14 @@ def test_half_rows_widths(G, O, cols):
         check(G, O, logits("normal", rows, cols), shift, dst_shift)
 
 
+@pytest.mark.parametrize("cols", [1, 7, 8, 9, 12, 15, 17, 31, 63, 101, 127, 128, 132099])
+def test_half_rows_that_end_inside_a_pack(G, O, cols):
+    """rows of the kernel of other lengths, several to a workgroup; the longest ends just behind a tile"""
+    rows = 2 if cols > 20000 else 37
+    for shift, dst_shift in ((0, 0), (1, 1), (5, 2), (8, 3)):
+        check(G, O, logits("normal", rows, cols), shift, dst_shift)
+
+
 @pytest.mark.parametrize("kind", ["flat", "wide", "equal", "rising", "ties", "late"])
 @pytest.mark.parametrize("cols", [300, 1500, 5000, 15000, 31000, 50257])
 def test_half_rows_kinds(G, O, cols, kind):
