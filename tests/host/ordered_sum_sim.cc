@@ -1,12 +1,13 @@
-// Host check of the order-faithful sum used by the softmax kernel.
+// Host check of the order-faithful sum of one wave (WaveResolve and PartWaveResolve of
+// mshadow_amd/csrc/softmax_kernels.h).
 //
-// Emulates one workgroup (W waves x 64 lanes x N terms per lane, slab after slab) with
-// the same decisions the device code takes - per-lane quantisation from
-// mshadow_amd/csrc/ordered_sum.h, wave totals, the block scan for the first rejected
-// wave, the lane scan inside it, real float adds for the rejected lane - and compares the
-// result with a plain serial float loop, bit for bit, on rows built to hit every branch:
-// softmax-like terms, ties, huge dynamic range, leading zeros, subnormals, inf / NaN.
-// Prints "OK <cases>" and exits 0 on success.
+// Takes a row slab after slab - LANES lanes x N terms - with the decisions the device code takes:
+// the first PLAIN lanes added as they are, then every lane's ulps in the binade of the sum
+// (LaneUlps, the very function the device calls), their unsigned prefix sums, the first lane in
+// which the binade ends, real float adds for that one, and on from there. The result must be a
+// plain serial float loop's bit for bit, on rows built to hit every branch: softmax-like terms,
+// ties, sums that double, negative terms, leading zeros, subnormals, infinities and NaN.
+// Prints "OK <cases> cases, <n> lanes added as they are" and exits 0 on success.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -25,84 +26,65 @@ static float Serial(const std::vector<float> &t) {
   return s;
 }
 
-template <int N>
-static float WaveResolveSim(float s, const float (*t)[N]) {  // t[64][N]
+static long lanes_walked = 0;
+
+// SIGNED, PLAIN and N as on the device; LANES = 64, or 16 / 32 for rows side by side in a wave
+template <bool SIGNED, int PLAIN, int LANES, int N>
+static float ResolveSim(float s, const float (*t)[N]) {  // t[LANES][N]
   int start = 0;
+  for (; start < PLAIN; ++start) s = TrueAdd<N>(s, t[start]);
   while (true) {
-    Binade b = BinadeOf(s);
-    float incl[64];
-    float run = 0.0f;
-    for (int l = 0; l < 64; ++l) {
-      run += (l >= start) ? LaneQuant<N>(t[l], b) : 0.0f;  // lane order, like the DPP scan
-      incl[l] = run;
-    }
+    const uint32_t bits = BitsOf(s);
+    uint32_t incl[LANES], run = 0u;
     int first = -1;
-    for (int l = start; l < 64; ++l) {
-      if (!Fits(b, incl[l])) { first = l; break; }
+    for (int l = 0; l < LANES; ++l) {
+      run += l >= start ? LaneUlps<SIGNED, N>(t[l], bits & 0xff800000u) : 0u;
+      incl[l] = run;
+      if (l >= start && first < 0 && (bits & 0x7fffffu) + run >= (1u << 23)) first = l;
     }
-    if (first < 0) return Accept(s, b, incl[63]);
-    s = Accept(s, b, first > 0 ? incl[first - 1] : 0.0f);
+    if (first < 0) return FloatOf(bits + incl[LANES - 1]);
+    if (first > 0) s = FloatOf(bits + incl[first - 1]);
     s = TrueAdd<N>(s, t[first]);
+    ++lanes_walked;
     start = first + 1;
-    if (start == 64) return s;
+    if (start == LANES) return s;
   }
 }
 
-template <int W, int N>
-static float BlockAddSim(float s, const float (*t)[N], long *resolves) {  // t[W*64][N]
-  int pos = 0;
-  while (true) {
-    Binade b = BinadeOf(s);
-    float qw[W];
-    for (int w = pos; w < W; ++w) {
-      float q = 0.0f;
-      for (int l = 0; l < 64; ++l) q += LaneQuant<N>(t[w * 64 + l], b);
-      qw[w] = q;
-    }
-    float acc = 0.0f, prev = 0.0f;
-    int failw = W;
-    for (int w = pos; w < W; ++w) {
-      acc += qw[w];
-      if (!Fits(b, acc)) { failw = w; break; }
-      prev = acc;
-    }
-    s = Accept(s, b, prev);
-    if (failw == W) return s;
-    s = WaveResolveSim<N>(s, t + failw * 64);
-    ++*resolves;
-    pos = failw + 1;
-    if (pos == W) return s;
-  }
-}
-
-template <int W, int N>
-static bool Check(const std::vector<float> &row, const char *name, long *resolves) {
-  const int slab = W * 64 * N;
+// the first slab of a row with its plain lanes, the others without
+template <bool SIGNED, int PLAIN, int LANES, int N>
+static bool Check(const std::vector<float> &row, float want, const char *name) {
   std::vector<float> padded(row);
-  while (padded.size() % slab) padded.push_back(0.0f);
-  float s = 0.0f;
-  for (size_t off = 0; off < padded.size(); off += slab) {
-    s = BlockAddSim<W, N>(s, reinterpret_cast<const float(*)[N]>(padded.data() + off), resolves);
-  }
-  const float want = Serial(row);
+  while (padded.size() % (LANES * N)) padded.push_back(0.0f);
+  const float(*t)[N] = reinterpret_cast<const float(*)[N]>(padded.data());
+  float s = ResolveSim<SIGNED, PLAIN, LANES, N>(0.0f, t);
+  for (size_t l = LANES; l * N < padded.size(); l += LANES) s = ResolveSim<SIGNED, 0, LANES, N>(s, t + l);
   if (BitsOf(s) != BitsOf(want) && !(std::isnan(s) && std::isnan(want))) {
-    fprintf(stderr, "MISMATCH %s W=%d N=%d n=%zu got %a want %a\n", name, W, N, row.size(), s, want);
+    fprintf(stderr, "MISMATCH %s signed=%d plain=%d lanes=%d N=%d n=%zu got %a want %a\n", name, SIGNED, PLAIN, LANES, N,
+            row.size(), s, want);
     return false;
   }
   return true;
 }
 
-static bool CheckAll(const std::vector<float> &row, const char *name, long *resolves) {
-  return Check<8, 4>(row, name, resolves) && Check<4, 4>(row, name, resolves) &&
-         Check<16, 4>(row, name, resolves) && Check<4, 1>(row, name, resolves) &&
-         Check<1, 4>(row, name, resolves);
+template <bool SIGNED>
+static bool CheckShapes(const std::vector<float> &row, float want, const char *name) {
+  return Check<SIGNED, 16, 64, 4>(row, want, name) && Check<SIGNED, 0, 64, 4>(row, want, name) &&
+         Check<SIGNED, 0, 64, 1>(row, want, name) && Check<SIGNED, 2, 16, 4>(row, want, name) &&
+         Check<SIGNED, 2, 16, 8>(row, want, name) && Check<SIGNED, 2, 32, 8>(row, want, name);
+}
+
+// terms that are not negative, by both forms
+static bool CheckAll(const std::vector<float> &row, const char *name) {
+  const float want = Serial(row);
+  return CheckShapes<false>(row, want, name) && CheckShapes<true>(row, want, name);
 }
 
 int main() {
   std::mt19937 rng(1234);
   std::normal_distribution<float> normal(0.0f, 1.0f);
   std::uniform_real_distribution<float> uni(0.0f, 1.0f);
-  long cases = 0, resolves = 0;
+  long cases = 0;
   bool ok = true;
   // 1. softmax-like rows: exp(x - max), x ~ N(0, sigma)
   for (float sigma : {0.1f, 1.0f, 3.0f, 10.0f, 40.0f}) {
@@ -112,7 +94,7 @@ int main() {
         float mx = -INFINITY;
         for (auto &v : x) { v = normal(rng) * sigma; mx = std::fmax(mx, v); }
         for (auto &v : x) v = expf(v - mx);
-        ok = CheckAll(x, "softmax", &resolves) && ok;
+        ok = CheckAll(x, "softmax") && ok;
         ++cases;
       }
     }
@@ -122,13 +104,13 @@ int main() {
     int n = 1 + rng() % 3000;
     std::vector<float> x(n);
     for (auto &v : x) v = std::ldexp(static_cast<float>(rng() % 64), -static_cast<int>(rng() % 30));
-    ok = CheckAll(x, "ties", &resolves) && ok;
+    ok = CheckAll(x, "ties") && ok;
     ++cases;
   }
   // 3. all equal (sum of ones is exact below 2^24, then sticks), and constants
   for (float c : {1.0f, 0.5f, 3.0f, 1e-3f, 0.1f}) {
     std::vector<float> x(40000, c);
-    ok = CheckAll(x, "const", &resolves) && ok;
+    ok = CheckAll(x, "const") && ok;
     ++cases;
   }
   // 4. leading zeros / subnormals / tiny then large; ascending and descending magnitudes
@@ -142,22 +124,22 @@ int main() {
     }
     if (rep % 3 == 1) std::reverse(x.begin(), x.end());
     if (rep % 3 == 2) std::shuffle(x.begin(), x.end(), rng);
-    ok = CheckAll(x, "range", &resolves) && ok;
+    ok = CheckAll(x, "range") && ok;
     ++cases;
   }
   {
     std::vector<float> x(3000, 0.0f);
-    ok = CheckAll(x, "zeros", &resolves) && ok;
+    ok = CheckAll(x, "zeros") && ok;
     x[2999] = 1e-40f;
-    ok = CheckAll(x, "zeros+denorm", &resolves) && ok;
+    ok = CheckAll(x, "zeros+denorm") && ok;
     x[10] = 3e-42f;
-    ok = CheckAll(x, "denorms", &resolves) && ok;
+    ok = CheckAll(x, "denorms") && ok;
     x[1500] = INFINITY;
-    ok = CheckAll(x, "inf", &resolves) && ok;
+    ok = CheckAll(x, "inf") && ok;
     x[100] = NAN;
-    ok = CheckAll(x, "nan", &resolves) && ok;
+    ok = CheckAll(x, "nan") && ok;
     x.assign(5000, 3.0e38f);  // overflow to inf on the way
-    ok = CheckAll(x, "overflow", &resolves) && ok;
+    ok = CheckAll(x, "overflow") && ok;
     cases += 6;
   }
   // 5. uniform magnitudes (binade crossings spread over the whole row)
@@ -165,10 +147,36 @@ int main() {
     int n = 20000 + rng() % 20000;
     std::vector<float> x(n);
     for (auto &v : x) v = uni(rng);
-    ok = CheckAll(x, "uniform", &resolves) && ok;
+    ok = CheckAll(x, "uniform") && ok;
     ++cases;
   }
+  // 6. terms of either sign, by the form that allows them; in every third row sums that end a binade
+  //    exactly, in every third few bits and hence ties
+  for (int rep = 0; rep < 300; ++rep) {
+    int n = 1 + rng() % 4000;
+    std::vector<float> x(n);
+    for (auto &v : x) {
+      v = rep % 3 == 0 ? normal(rng) : std::ldexp(1.0f, -static_cast<int>(rng() % (rep % 3 == 1 ? 4 : 30)));
+      if (rng() % 64 == 0) v = -std::fabs(v);
+      if (rng() % 512 == 0) v = -0.0f;
+    }
+    if (rep % 10 == 9) x[n / 2] = rep % 20 == 9 ? INFINITY : NAN;
+    ok = CheckShapes<true>(x, Serial(x), "signed") && ok;
+    ++cases;
+  }
+  // 7. one lane at the top of a binade: from every sum just below a power of two, terms of half an
+  //    ulp, one ulp and their neighbours, so that the upper of the two sums leaves and the lower stays
+  for (uint32_t top : {1u, 0x00800000u, 0x01000000u, 0x3f800000u, 0x4b800000u, 0x7f000000u, 0x7f800000u}) {
+    for (int rep = 0; rep < 400; ++rep) {
+      const float from = FloatOf(top - 1u - (top > 8u ? rng() % 8 : 0u));
+      const float ulp = FloatOf(top) - FloatOf(top - 1u);  // of the binade below; infinite at the last one
+      std::vector<float> x(1, from);
+      for (int i = 0; i < 300; ++i) x.push_back(std::isinf(ulp) ? 1.0141204801825835e31f : ulp * 0.25f * (rng() % 6));
+      ok = CheckAll(x, "top") && ok;
+      ++cases;
+    }
+  }
   if (!ok) return 1;
-  printf("OK %ld cases, %ld wave resolves\n", cases, resolves);
+  printf("OK %ld cases, %ld lanes added as they are\n", cases, lanes_walked);
   return 0;
 }

@@ -145,8 +145,9 @@ def _compile_and_run(tmp_path, source, extra, args=()):
 
 
 def test_ordered_sum_matches_serial_sum_on_host(tmp_path):
-    """the lane arithmetic of the softmax row sum, driven lane by lane on the host,
-    reproduces a strictly sequential float sum bit for bit"""
+    """the wave's walk of the softmax row sum (whole ulps per lane, unsigned prefix sums, the lane in
+    which a binade ends added as it is), modelled on the host with the device code's own lane
+    function, reproduces a strictly sequential float sum bit for bit"""
     out = _compile_and_run(tmp_path, "ordered_sum_sim.cc", [])
     assert out.startswith("OK"), out[-500:]
 
