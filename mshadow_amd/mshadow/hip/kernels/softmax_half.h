@@ -11,8 +11,9 @@
  * Quotients. t / sum goes through the float reciprocal of the row's sum as two floats, high +
  * low: t * high + t * low is the float quotient bit for bit (a quotient of two 11-bit
  * significands is nowhere near half way between two floats), so rounding it to binary16 gives
- * what the division would. All 185 M pairs of a term in [0, 1] and a sum in [1, 2048] agree.
- * The rounding has to be a step of its own: v_fma_mixlo_f16 rounds once, and 2796 of them differ.
+ * what the division would. All 173,041,665 pairs of a term in [0, 1] and a sum in [1, 2048] agree.
+ * The rounding has to be a step of its own: v_fma_mixlo_f16 rounds once, and 1398 of them differ
+ * (tests/host/half_quotient_check.cc).
  *
  * The sum. `sum += t` on half_t is one 16-bit add, and their order decides the result: the
  * sum stands still once its ulp exceeds twice the terms. While it stays in one binade

@@ -183,6 +183,15 @@ def test_half_sum_pruning_rule_is_exhaustively_sound(tmp_path):
     assert dropped > 10 ** 8 and kept_noops < 10 ** 5   # sound, and nearly tight (ties stay in)
 
 
+def test_half_quotients_are_exhaustively_right(tmp_path):
+    """the binary16 softmax divides by a reciprocal of two floats: for every term in [0, 1] and every
+    sum in [1, 2048] that is the float quotient, bit for bit, rounded to binary16"""
+    out = _compile_and_run(tmp_path, "half_quotient_check.cc", [])
+    assert out.startswith("OK"), out[-500:]
+    pairs, once = (int(v) for v in out.split()[1:3])
+    assert pairs == 15361 * 11265 and once == 1398   # the second rounding is needed
+
+
 def test_header_api_on_cpu_matches_oracle(tmp_path, orc):
     oracle_dir = os.path.join(ROOT, "oracle")
     out = _compile_and_run(tmp_path, "api_cpu_check.cc",
