@@ -162,15 +162,21 @@ def test_planned_row_sum_matches_serial_sum_on_host(tmp_path):
 
 
 def test_signed_column_sums_leave_most_of_the_chain(tmp_path):
-    """sum_rows adds signed terms, and a plan of verified runs (what makes the softmax row sum
-    parallel) leaves too much of its chain: cut with full knowledge of the true running sums,
-    columns of 16384 N(0, 1) terms still keep 14 % of their dependent adds at a granularity of
-    one term, 23 % at four (a lane's pack) and 70 % at 64 (a wave's load). The program rebuilds
-    every column sum from its runs and compares it bit for bit with the serial loop."""
+    """sum_rows adds signed terms, and on N(0, 1) terms a plan of verified runs (what makes the
+    softmax row sum parallel) leaves too much of its chain: cut with full knowledge of the true
+    running sums, columns of 16384 of them still keep 14 % of their dependent adds at a granularity
+    of one term, 23 % at four (a lane's pack) and 70 % at 64 (a wave's load). Of a classifier's
+    gradients it leaves little: the running sums cross a binade or zero in one add of 500, and 88 %
+    of the blocks of 64 rows hold. The program rebuilds every column sum from its runs and compares
+    it bit for bit with the serial loop."""
     out = _compile_and_run(tmp_path, "signed_plan_sim.cc", [], args=["48"])
     assert out.startswith("OK"), out[-500:]
-    shares = {int(g): float(v) for g, v in re.findall(r"grain (\d+): ([0-9.]+)", out)}
+    drawn, gradients = out.splitlines()
+    shares = {int(g): float(v) for g, v in re.findall(r"grain (\d+): ([0-9.]+)", drawn)}
     assert 0.10 < shares[1] < 0.18 and 0.18 < shares[4] < 0.30 and shares[64] > 0.6, shares
+    shares = {int(g): float(v) for g, v in re.findall(r"grain (\d+): ([0-9.]+)", gradients)}
+    hold = {int(g): float(v) for g, v in re.findall(r" of (\d+): ([0-9.]+)", gradients)}
+    assert shares[1] < 0.01 and shares[64] < 0.2 and hold[16] > 0.94 and 0.8 < hold[64] < 0.95, (shares, hold)
 
 
 def test_half_sum_pruning_rule_is_exhaustively_sound(tmp_path):
