@@ -101,16 +101,27 @@ def test_half_rows_special_values(G, O):
 
 
 def test_half_rows_every_exponential(G, O):
-    """x - max takes every binary16 value from -0 down to -infinity: one wrong exponential shows in its
-    quotient. Rows of 4096 of them, the largest first, so that the sum keeps its bits."""
+    """x - max takes every binary16 value from -0 down to -infinity, and one wrong exponential shows in
+    its quotient: a row that begins with 2^k columns of the maximum has a sum of 2^k, and terms of at
+    most half an ulp of that, 2^(k-11), leave it there. Divided by 2^k a term of 2^(k-14) or more keeps
+    all its bits; the smaller ones are in the row whose sum is one."""
     every = np.arange(0x8000, 0x7c01 + 0x8000, dtype=np.uint32).astype(np.uint16)
     d = O.half2float(every).astype(f32)
-    rows = -(-d.size // 4095)
-    x = np.full((rows, 4096), -np.inf, f32)
-    x[:, 0] = 0.0
-    for r in range(rows):
-        piece = d[r * 4095:(r + 1) * 4095]
-        x[r, 1:1 + piece.size] = piece
+    with np.errstate(divide="ignore"):
+        log2 = np.log2(np.exp(d.astype(np.float64)))
+    row_of = np.clip(np.ceil(log2 + 11.5), 0, 11)
+    x = np.full((12, 2048 + d.size), -np.inf, f32)
+    quotients = np.zeros(x.shape, f32)
+    for k in range(12):
+        piece = d[row_of == k]
+        x[k, :1 << k] = 0.0
+        x[k, 1 << k:(1 << k) + piece.size] = piece
+        quotients[k] = O.half2float(O.float2half(np.exp(x[k]))) * f32(2.0 ** -k)
+    used = 2048 + int(max(np.count_nonzero(row_of == k) for k in range(12)))
+    x, quotients = x[:, :used], quotients[:, :used]
+    want = O.float2half(x)
+    O.softmax(want, O.float2half(x))
+    assert np.array_equal(O.half2float(want), quotients)   # nothing of a term is lost
     check(G, O, x, 0, 0)
 
 
