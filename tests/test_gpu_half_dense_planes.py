@@ -1,4 +1,4 @@
-"""sumall_except_dim<1> of half_t planes whose rows are of odd length and whose pixels are even in number:
+"""sumall_except_dim<1> of half_t planes whose pixels are even in number, the rows of even and of odd length:
 dense ones are walked as one row, pitched ones are not. Bit-exact against the oracle."""
 import numpy as np
 import pytest
@@ -22,10 +22,18 @@ def O():
     return Checker("orc")
 
 
-# a segment per lane of one, four, sixteen and 64; fewer and more kept indices than are dealt out by segments;
-# planes of two pixels and of whole 16-byte packs; the least work per kept index that takes the ring, and less
-@pytest.mark.parametrize("n,c,h,w", [(1, 195, 512, 129), (3, 193, 148, 149), (16, 192, 66, 63), (20, 200, 58, 57),
-                                     (65, 7, 34, 31), (33, 5, 40, 55), (32768, 3, 2, 1), (32767, 3, 2, 1), (65, 194, 32, 33)])
+# even rows, which dense planes walk as one row too: a segment per lane of one, four, sixteen and 64
+EVEN = [(1, 195, 512, 130), (3, 193, 148, 150), (16, 192, 66, 64), (20, 200, 58, 58), (65, 7, 34, 32)]
+# odd rows on the ring, dealt out by kept index (192 and more) and by segments (fewer), and where they stay
+# with the kernel of expressions: fewer than 16 images, more than 256 kept indices, planes of fewer than 512
+# pixels, less than 65536 elements per kept index
+ODD = [(16, 192, 66, 63), (20, 200, 58, 57), (33, 5, 40, 55), (65, 194, 32, 33), (65, 7, 34, 31),
+       (15, 200, 60, 75), (16, 200, 60, 75), (20, 256, 58, 57), (20, 257, 58, 57), (129, 194, 34, 15), (128, 194, 2, 257),
+       (16, 194, 2, 2049), (16, 194, 2, 2047), (128, 3, 512, 1), (127, 3, 512, 1), (1, 195, 512, 129), (3, 193, 148, 149),
+       (32768, 3, 2, 1), (32767, 3, 2, 1)]
+
+
+@pytest.mark.parametrize("n,c,h,w", EVEN + ODD)
 @pytest.mark.parametrize("extra", [0, 1])
 def test_half_planes_of_odd_rows(G, O, n, c, h, w, extra):
     x = O.float2half(normal(80, (n, c, h, w)))
