@@ -615,7 +615,7 @@ class Library:
         h, w = src.shape[-2:]
         ph, pw = dst.shape[-2:]
         planes = int(np.prod(src.shape[:-2]))
-        if src.dtype == np.uint16:   # half_t tensors: the generic expression kernel
+        if src.dtype == np.uint16:   # half_t tensors: the expression API
             self.check_case(self.cases.mshadow_case_pool_f16(
                 dst.ptr, dst.stride, src.ptr, src.stride, planes, h, w, ph, pw, ky, kx, sy, sx,
                 reducer, stream))

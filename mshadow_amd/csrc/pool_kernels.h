@@ -957,7 +957,7 @@ __device__ __forceinline__ float FromLaneBelow(float v) {
       __builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(v)), 0x138, 0xf, 0xf, false)));
 }
 
-/*! \brief unpool for K x K windows with stride 1 (K = 2, 3) on rows of up to 256 pixels, with no
+/*! \brief unpool for K x K windows with stride 1 (K = 2, 3, 5) on rows of up to 256 pixels, with no
  *  staging. A pixel lies under up to K * K windows, so a thread that took its pooled values from
  *  memory pixel by pixel would fetch every one of them K * K times. Here a thread owns four
  *  adjacent pixels and walks down a strip of rows with the K pooled rows that cover the current

@@ -22,7 +22,9 @@ namespace mshadow {
 namespace hip {
 
 const int kWave = 64;
-/*! \brief compute units of the chip, where a dispatch of the headers weighs work against them */
+/*! \brief compute units of the chip, where a dispatch of the headers weighs work against them. A
+ *  constant: these headers have no cheap way to ask (the library asks the device once). On a
+ *  partition with fewer units the choices stay right and are only not the fastest. */
 const uint32_t kChipCus = 256;
 
 __device__ __forceinline__ int LaneId() { return threadIdx.x & (kWave - 1); }
@@ -261,7 +263,12 @@ struct SaverReadsDst<sv::saveto> {
 /*! \brief which piece of the work a workgroup takes. Workgroups are dealt to the 8 XCDs
  *  round-robin, and each XCD has its own L2: handing XCD k the k-th contiguous eighth of
  *  the pieces (the first nblocks % 8 eighths have one more) keeps neighbouring pieces - which
- *  share cache lines, halos or, for windowed expressions, whole operands - behind one L2. */
+ *  share cache lines, halos or, for windowed expressions, whole operands - behind one L2.
+ *  Against eighths only of numbers that 8 divides and linear order otherwise, 100 calls with odd
+ *  numbers of workgroups: (4100,4100) transposed 45 -> 38 us, (33,65,33,36) to (n,w,h,c) 22 -> 10 us,
+ *  a sum over 5 channels of (31,63,55,57) 20 -> 17.5 us, sum_rows of an expression on 500 x 20000
+ *  half_t 16 -> 9 us, most others level; where neighbours share little it loses up to 5 % (rows of 64 permuted
+ *  9.8 -> 10.3 us, a new axis of three 37 -> 38.6 us, sum_rows of 40000 x 1000 half_t 162 -> 168 us). */
 __device__ __forceinline__ uint32_t StripOfBlock(uint32_t block, uint32_t nblocks) {
   const uint32_t kXcd = 8;
   const uint32_t xcd = block % kXcd, longer = nblocks % kXcd;

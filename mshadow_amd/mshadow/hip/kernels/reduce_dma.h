@@ -165,7 +165,8 @@ __global__ void __launch_bounds__(kDmaThreads)
  * as possible more than one round of them (LowestColumnsPerStrip). Measured, sums of floats,
  * before (16 columns per workgroup, 128 KB ring) and now: 8192 x 32000 299 -> 174 us (6.0 TB/s),
  * 2048 x 50257 215 -> 77 us (5.3 TB/s), 512 x 50000 78 -> 20 us, 128 x 128000 106 -> 13 us,
- * 16384 x 8192 149 -> 87 us, 1500 x 1000 12.5 -> 10 us, 128 x 10 3.8 -> 2.8 us; binary16
+ * 16384 x 8192 149 -> 87 us, 1500 x 1000 12.5 -> 10 us, 128 x 10 3.8 -> 2.8 us (the kernel alone: calls that short wait for
+ * their launches); binary16
  * (register-staged kernel of reduce.h before) 8192 x 32000 260 -> 81 us, 4096 x 9000 52 -> 25 us.
  * Sixteen bytes a lane instead of four fetch no faster (8192 x 32000: 174 us both). */
 
@@ -203,8 +204,9 @@ struct LowestStrip {
   static_assert(!SHIFTED || (sizeof(DType) == 2 && PER_LANE == 1 && LOADERS % 2 == 0), "shifted rows");
 };
 typedef LowestStrip<float, 16, 64, 4, 4, 1, false> LowestStrip16;
-/*! \brief 2048 to 8191 rows: longer stages, whose first LDS reads are waited for less often
- *  (4096 x 2000: 20.4 us, with 64 rows a stage 22.9 us, the kernel above 22.1 us) */
+/*! \brief 2048 rows to where the kernel above is the faster one: longer stages, whose first LDS reads
+ *  are waited for less often (4096 x 2000: 20.4 us, with 64 rows a stage 22.9 us, the kernel above
+ *  22.1 us) */
 typedef LowestStrip<float, 16, 256, 4, 8, 1, false> LowestStrip16Long;
 typedef LowestStrip<float, 32, 64, 4, 4, 1, false> LowestStrip32;
 typedef LowestStrip<float, 64, 64, 4, 8, 1, false> LowestStrip64;

@@ -1235,8 +1235,8 @@ struct ReduceRoute<Saver, Reducer, Tensor<gpu, 1, float>, Tensor<gpu, dim, float
 #if defined(__HIPCC__)
 /*! \brief reductions of a half_t tensor in memory: the LDS-ring kernels of the float path
  *  (kernels/reduce_dma.h) instantiated for 16-bit elements, a load bringing two neighbouring
- *  elements of a row. HighDim() returns false when the shape does not allow that (odd row length or
- *  pitch, unaligned base, little work per kept index), Lowest() where the generic kernel is the
+ *  elements of a row. HighDim() returns false when the shape does not allow that (rows of odd length
+ *  or pitch that cannot be walked as one, unaligned base, little work per kept index), Lowest() where the generic kernel is the
  *  faster one; the generic kernel then has to do it. */
 template <typename Saver, typename Reducer, typename R, typename E>
 struct HalfRingRoute {
