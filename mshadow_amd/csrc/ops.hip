@@ -1023,12 +1023,14 @@ static SlideGeom MakeSlideGeom(int planes, int rows, int w, int k) {
   const uint32_t least = static_cast<uint32_t>((rows + 15) / 16);
   uint32_t r = (static_cast<uint32_t>(rows) + least - 1) / least;
   const long long want = 16ll * mshadow_abi::ComputeUnits();  // waves
-  if (k == 5) {
+  const bool turns_of_two = k == 5 && (w >= 24 || (w >= 16 && w % 4 == 0));
+  if (turns_of_two) {
     /* Two waves of the kernel for 5 x 5 windows fill a SIMD, so strips are cut no further than it takes
        to deal every SIMD two: a strip costs its rows and about two and a half for the four pooled rows
        above it, times the turns of eight waves a CU. Against strips cut until there are 16 waves a
        CU: 1.8 M pixels, 7x160 14.6 and 23.8 us, 9x50 13 and 21, 40x100 15 and 20; 4 M, 24x64 19 and 27,
-       16x32 20 and 29; 12 M, 40x40 66 and 75; 0.6 M level. */
+       16x32 20 and 29; 12 M, 40x40 66 and 75; 0.6 M level. Narrow rows stay with those: a wave has
+       many strips then, and long ones are far apart (224x7 319 and 252 us, 100x18 117 and 111). */
     long long best = -1;
     for (uint32_t longest = r; longest >= 2; --longest) {
       const uint32_t n = (static_cast<uint32_t>(rows) + longest - 1) / longest;
@@ -1039,7 +1041,7 @@ static SlideGeom MakeSlideGeom(int planes, int rows, int w, int k) {
       if (best < 0 || cost * 10 < best * 9) { best = cost; r = each; }
     }
   }
-  while (k != 5 && r > 2 && static_cast<long long>(planes) * ((rows + r - 1) / r) / sg.strips_per_wave < want) r = (r + 1) / 2;
+  while (!turns_of_two && r > 2 && static_cast<long long>(planes) * ((rows + r - 1) / r) / sg.strips_per_wave < want) r = (r + 1) / 2;
   sg.strip_rows = r;
   sg.strips_per_plane = static_cast<uint32_t>((rows + r - 1) / r);
   sg.total_strips = static_cast<uint32_t>(planes) * sg.strips_per_plane;
@@ -1268,9 +1270,9 @@ int mshadow_hip_unpool_f32(float *dst, int dstride, const float *src, int sstrid
      the kernels below). A lane has four pixels of a row, so narrow planes make its accesses short
      and scattered, which the staged kernels do not mind; what those mind is many windows a pixel.
      12 M pixels: 3 x 3 56x56 54 us against 51, 63x70 58 against 52, 20x200 46 against 56; 2 x 2 28x28 74 against 64,
-     56x56 50 against 65; 5 x 5 13x13 145 against 127, 16x16 76 against 103, 8x40 72 against 123,
-     28x28 83 against 106, and beyond 4 KB a plane - one plane per workgroup there - 100x14 119 against
-     317, 224x7 251 against 472. Low planes whose rows leave a third of the lanes idle are made twice
+     56x56 50 against 65; 5 x 5 13x13 145 against 127, 16x16 73 against 102, 8x40 69 against 121,
+     28x28 78 against 105, and beyond 4 KB a plane - one plane per workgroup there - 100x14 130 against
+     317, 224x7 251 against 470. Low planes whose rows leave a third of the lanes idle are made twice
      over here, most of their windows being cut off: 7x160 80 against 71 us, 8x140 (24 M pixels) 168
      against 153, 5x128 57 against 46 - unless there are waves for one turn only (1.8 M pixels, 7x160
      14.6 against 15.5 us). */
