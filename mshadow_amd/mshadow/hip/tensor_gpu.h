@@ -811,6 +811,12 @@ struct FastPath<sv::saveto, dim, half::half_t,
         (static_cast<uint64_t>(g.ph) - 1) * S + K > g.h || (static_cast<uint64_t>(g.pw) - 1) * S + K > g.w) {
       return false;
     }
+    /* 2 x 2 windows by two on rows of a fraction of a cache line: a wave's lanes lie eight of them apart and
+       come back to every line, out of L2 as long as the tensor fits that; behind it the map kernel is the
+       faster one (64x10 planes, here and there: 8 M pixels 8.3 and 9.4 us, 24 M 32 and 24, 48 M 66 and
+       51; 64x8: 8 M 8 and 18, 15.5 M 15 and 31, 24 M 54 and 49) */
+    const uint64_t bytes = planes * g.h * src.stride_ * sizeof(half::half_t);
+    if (K == 2 && S == 2 && g.pw < 8 && bytes > (g.pw == 4 ? 36u : 24u) << 20) return false;
     g.total = static_cast<uint32_t>(total);
     g.div_groups = FastDivU32(g.groups);
     g.div_strips = FastDivU32(g.strips);

@@ -26,6 +26,16 @@ def O():
 WINDOWS = [(2, 1), (3, 1), (5, 1), (2, 2), (3, 2), (5, 2), (4, 2), (3, 3)]
 
 
+def test_half_pool_of_many_narrow_planes(G, O):
+    """2x2 by two on rows of ten, more of them than fit L2: the map kernel"""
+    img = O.float2half(uniform(95, (22000, 64, 10)))
+    want = np.empty((22000, 32, 5), np.uint16)
+    O.pool(want, img, 2, 2, 2, 2, MAX)
+    dst = G.buffer(want.shape, np.uint16)
+    G.case_pool(dst, G.to_device(img), 2, 2, 2, 2, MAX)
+    assert np.array_equal(dst.download(), want)
+
+
 @pytest.mark.parametrize("k,s", WINDOWS)
 @pytest.mark.parametrize("h,w", [(5, 5), (7, 11), (9, 10), (12, 13), (13, 13), (17, 33), (24, 8), (40, 67)])
 def test_half_pool(G, O, h, w, k, s):
