@@ -53,6 +53,7 @@ def test_stride_one_pooling(G, O, h, w, k):
 # of the 5x5 gradient by the waves there are; more low planes than waves of one turn, and as many
 @pytest.mark.parametrize("planes,h,w,k", [(5200, 61, 17, 2), (5119, 61, 17, 3), (4200, 88, 16, 3), (5200, 34, 33, 2), (3100, 8, 160, 3),
                                           (300, 11, 130, 2), (2048, 7, 160, 5), (2049, 7, 160, 5), (2100, 40, 20, 5),
-                                          (9000, 16, 20, 5), (700, 33, 16, 5), (40, 130, 64, 5), (2049, 9, 141, 5)])
+                                          (9000, 16, 20, 5), (700, 33, 16, 5), (40, 130, 64, 5), (2049, 9, 141, 5),
+                                          (11364, 32, 33, 2)])
 def test_stride_one_pooling_of_many_planes(G, O, planes, h, w, k):
     check(G, O, planes, h, w, k, (MAX,))
