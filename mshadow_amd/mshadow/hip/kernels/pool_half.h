@@ -3,9 +3,9 @@
  * or two, every window whole (mshadow/extension/spatial_pool.h:20-149 of the reference with DType =
  * half_t; other windows take the map kernel, which fetches every element of every window).
  *
- * A thread makes four adjacent outputs of kPoolHalfRows (S = 1) or half as many rows one below the
- * other, with the K input rows of a window in registers: an input element is fetched
- * (rows + K - 1) / rows times and in 16-byte pieces wherever it lies. The last thread of an output row
+ * A thread makes four adjacent outputs of up to kPoolHalfRows (S = 1) or half as many rows one below
+ * the other (fewer where that leaves the chip short of waves), with the K input rows of a window in
+ * registers: an input element is fetched (rows + K - 1) / rows times and in 16-byte pieces wherever it lies. The last thread of an output row
  * is moved back to end with the row (it makes some outputs a second time, with the same result).
  *
  * Two outputs share a register and an instruction. A sum is K * K packed adds in the window's order,
@@ -64,6 +64,7 @@ struct PoolHalfOp<red::minimum> {
 
 struct PoolHalfGeom {
   uint32_t h, w, ph, pw;
+  uint32_t rows;                   //!< rows of outputs to a strip
   uint32_t groups, strips, total;  //!< threads to a row, strips of rows to a plane, threads in all
   FastDivU32 div_groups, div_strips;
 };
@@ -130,7 +131,8 @@ __global__ void __launch_bounds__(kPoolHalfBlock)
   if (idx >= g.total) return;
   const uint32_t strip = g.div_groups.Div(idx);
   const uint32_t plane = g.div_strips.Div(strip);
-  const uint32_t py0 = (strip - plane * g.strips) * ROWS;
+  const uint32_t py0 = (strip - plane * g.strips) * g.rows;
+  const uint32_t nrows = g.rows < g.ph - py0 ? g.rows : g.ph - py0;
   const uint32_t group = idx - strip * g.groups;
   const uint32_t px0 = group * 4 + 4 <= g.pw ? group * 4 : g.pw - 4;
   const uint16_t *in = reinterpret_cast<const uint16_t *>(src) + static_cast<size_t>(plane) * g.h * sstride + px0 * S;
@@ -157,7 +159,7 @@ __global__ void __launch_bounds__(kPoolHalfBlock)
   for (int k = 0; k < K - S; ++k) MSHADOW_POOL_ROW(k, py0 * S + k)
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
-    if (py0 + r >= g.ph) break;
+    if (static_cast<uint32_t>(r) >= nrows) break;
 #pragma unroll
     for (int k = K - S; k < K; ++k) MSHADOW_POOL_ROW((r * S + k) % K, (py0 + r) * S + k)
     uint32_t left = init, right = init;

@@ -802,10 +802,10 @@ struct FastPath<sv::saveto, dim, half::half_t,
     hip::PoolHalfGeom g;
     g.h = e.src_height_, g.w = e.src_width_, g.ph = e.shape_[dim - 2], g.pw = e.shape_[dim - 1];
     const uint64_t planes = src.shape_.ProdShape(0, dim - 2);
-    const uint32_t rows = hip::kPoolHalfRows / S;
+    g.rows = hip::kPoolHalfRows / S;
     g.groups = (g.pw + 3) / 4;
-    g.strips = (g.ph + rows - 1) / rows;
-    const uint64_t total = planes * g.strips * g.groups;
+    g.strips = (g.ph + g.rows - 1) / g.rows;
+    uint64_t total = planes * g.strips * g.groups;
     /* rows of four outputs at least, whole windows only, 31-bit thread numbers */
     if (planes == 0 || g.ph == 0 || g.pw < 4 || total >= (1ull << 31) - hip::kPoolHalfBlock ||
         (static_cast<uint64_t>(g.ph) - 1) * S + K > g.h || (static_cast<uint64_t>(g.pw) - 1) * S + K > g.w) {
@@ -817,6 +817,14 @@ struct FastPath<sv::saveto, dim, half::half_t,
        51; 64x8: 8 M 8 and 18, 15.5 M 15 and 31, 24 M 54 and 49) */
     const uint64_t bytes = planes * g.h * src.stride_ * sizeof(half::half_t);
     if (K == 2 && S == 2 && g.pw < 8 && bytes > (g.pw == 4 ? 36u : 24u) << 20) return false;
+    /* a row of a strip waits for the one above it: short strips as long as all of them run side by side, of windows
+       of five, whose strips fetch four rows more, half as many (3x3 by one on (130,96,13) 4.5 -> 2.5 us, 5x5 by one on
+       (512,19,28) 4.5 -> 2.4; but 1710 planes of 17x153 6.2 with strips of eight, 6.7 with four) */
+    while (g.rows > 1 && total < (K == 5 ? 4ull : 8ull) * hip::kChipCus * hip::kWave) {
+      g.rows /= 2;
+      g.strips = (g.ph + g.rows - 1) / g.rows;
+      total = planes * g.strips * g.groups;
+    }
     g.total = static_cast<uint32_t>(total);
     g.div_groups = FastDivU32(g.groups);
     g.div_strips = FastDivU32(g.strips);

@@ -59,3 +59,22 @@ def test_half_pool(G, O, h, w, k, s):
         nan = np.isnan(O.half2float(want).astype(f32))
         assert np.array_equal(np.isnan(O.half2float(got).astype(f32)), nan)
         assert np.array_equal(got[~nan], want[~nan]), f"{h}x{w} k{k} s{s} reducer {reducer}"
+
+
+# threads enough for strips of eight, four, two rows of outputs and of one (half of that with a step of two)
+@pytest.mark.parametrize("planes", [7400, 4500, 2300, 300])
+@pytest.mark.parametrize("k,s", WINDOWS[:6])
+def test_half_pool_strips(G, O, planes, k, s):
+    h, w = 21, 23
+    img = O.float2half(uniform(96, (planes, h, w)))
+    img[::7, 3:9, 5] = 0x8000
+    img[::11, 17, ::6] = 0x7e01
+    ph, pw = (h - k) // s + 1, (w - k) // s + 1
+    want = np.empty((planes, ph, pw), np.uint16)
+    O.pool(want, img, k, k, s, s, MAX)
+    dst = G.buffer(want.shape, np.uint16)
+    G.case_pool(dst, G.to_device(img), k, k, s, s, MAX)
+    got = dst.download()
+    nan = np.isnan(O.half2float(want).astype(f32))
+    assert np.array_equal(np.isnan(O.half2float(got).astype(f32)), nan)
+    assert np.array_equal(got[~nan], want[~nan])
