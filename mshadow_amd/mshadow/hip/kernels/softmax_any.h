@@ -105,18 +105,21 @@ __device__ __forceinline__ void MoveHalvesDown(AnyWords *w, uint32_t by) {
   }
   *w = v;
 }
-/*! \brief elements [x, x + kAnyTile) of a row (VEC: whole aligned packs only); what lies past the end
- *  of the row is `absent` or any of the row's elements. A row's last pack that is no whole one is taken
- *  element by element, of 16-bit elements as the row's last eight, moved down: one load whichever lane
+/*! \brief how a kernel moves a row: element by element (short code for short rows), as packs at any
+ *  alignment, as whole aligned packs (cols % kAnyTile == 0 and every row starts 16-byte aligned) */
+const int kAnyApart = 0, kAnyLoose = 1, kAnyWhole = 2;
+/*! \brief elements [x, x + kAnyTile) of a row; what lies past the end of the row is `absent` or
+ *  any of the row's elements. A row's last pack that is no whole one is taken element by element, of 16-bit elements as the row's last eight, moved down: one load whichever lane
  *  has it. Of 131072 x 127 half_t the Softmax took 115 us with every pack of such rows taken apart, 4096 x
  *  50257 the gradient 408 us; with whole packs and single elements side by side in a wave the Softmax
  *  takes 95 us there and 6.0 us of 200 x 10, now 90 and 5.85 (5.6 with every pack taken apart). */
-template <typename DType, bool VEC>
+template <typename DType, int HOW>
 __device__ __forceinline__ void LoadAnyPack(AnyPack<DType> *p, const DType *row, uint32_t x,
                                             uint32_t cols, DType absent) {
-  if (VEC) {
+  if (HOW == kAnyWhole) {
     *p = *reinterpret_cast<const AnyPack<DType> *>(row + x);
-  } else if (x + kAnyTile <= cols || (sizeof(DType) == 2 && cols >= static_cast<uint32_t>(kAnyTile))) {
+  } else if (HOW == kAnyLoose &&
+             (x + kAnyTile <= cols || (sizeof(DType) == 2 && cols >= static_cast<uint32_t>(kAnyTile)))) {
     const uint32_t past = sizeof(DType) == 2 && x + kAnyTile > cols ? x + kAnyTile - cols : 0u;
     AnyWords w[sizeof(AnyPack<DType>) / sizeof(AnyWords)];
 #pragma unroll
@@ -130,12 +133,12 @@ __device__ __forceinline__ void LoadAnyPack(AnyPack<DType> *p, const DType *row,
     for (int i = 0; i < kAnyTile; ++i) p->v[i] = (x + i < cols) ? row[x + i] : absent;
   }
 }
-template <typename DType, bool VEC>
+template <typename DType, int HOW>
 __device__ __forceinline__ void StoreAnyPack(DType *row, uint32_t x, uint32_t cols,
                                              const AnyPack<DType> &p) {
-  if (VEC) {
+  if (HOW == kAnyWhole) {
     *reinterpret_cast<AnyPack<DType> *>(row + x) = p;
-  } else if (x + kAnyTile <= cols) {
+  } else if (HOW == kAnyLoose && x + kAnyTile <= cols) {
     AnyWords w[sizeof(AnyPack<DType>) / sizeof(AnyWords)];
     __builtin_memcpy(w, &p, sizeof(w));
 #pragma unroll
@@ -150,8 +153,7 @@ __device__ __forceinline__ void StoreAnyPack(DType *row, uint32_t x, uint32_t co
   }
 }
 
-/*! \brief VEC: cols % kAnyTile == 0 and every row of src and dst starts 16-byte aligned */
-template <typename DType, bool VEC>
+template <typename DType, int HOW>
 __global__ void __launch_bounds__(kAnyBlock)
     SoftmaxAnyKernel(DType *dst, uint32_t dstride, const DType *src, uint32_t sstride,
                      uint32_t rows, uint32_t cols) {
@@ -176,7 +178,7 @@ __global__ void __launch_bounds__(kAnyBlock)
       for (int q = 0; q < kAnyBatch; ++q) {
         const uint32_t x = x0 + (q * kAnyThreadsPerRow + p) * kAnyTile;
         if (x < cols) {
-          LoadAnyPack<DType, VEC>(&in[q], e, x, cols, first);
+          LoadAnyPack<DType, HOW>(&in[q], e, x, cols, first);
         } else {
 #pragma unroll
           for (int i = 0; i < kAnyTile; ++i) in[q].v[i] = first;
@@ -212,7 +214,7 @@ __global__ void __launch_bounds__(kAnyBlock)
 #pragma unroll
   for (int q = 0; q < kAnyBatch; ++q) {
     const uint32_t x = (q * kAnyThreadsPerRow + p) * kAnyTile;
-    if (live && x < cols) LoadAnyPack<DType, VEC>(&in[q], e, x, cols, mmax);
+    if (live && x < cols) LoadAnyPack<DType, HOW>(&in[q], e, x, cols, mmax);
   }
   /* Tile i's terms are added while tile i + 1 is being made: in step i every thread makes its
      packs of tile i (LDS buffer i & 1), then the chain lanes add tile i - 1 from the other
@@ -226,7 +228,7 @@ __global__ void __launch_bounds__(kAnyBlock)
 #pragma unroll
       for (int q = 0; q < kAnyBatch; ++q) {
         const uint32_t x = x0 + kAnyTileCols + (q * kAnyThreadsPerRow + p) * kAnyTile;
-        if (live && x < cols) LoadAnyPack<DType, VEC>(&next[q], e, x, cols, mmax);
+        if (live && x < cols) LoadAnyPack<DType, HOW>(&next[q], e, x, cols, mmax);
       }
 #pragma unroll
       for (int q = 0; q < kAnyBatch; ++q) {
@@ -235,7 +237,7 @@ __global__ void __launch_bounds__(kAnyBlock)
           AnyPack<DType> t;
 #pragma unroll
           for (int i = 0; i < kAnyTile; ++i) t.v[i] = DType(SoftmaxExp(in[q].v[i] - mmax));
-          StoreAnyPack<DType, VEC>(o, x, cols, t);
+          StoreAnyPack<DType, HOW>(o, x, cols, t);
           tile_packs[step & 1u][r][q * kAnyThreadsPerRow + p] = t;
         }
       }
@@ -298,7 +300,7 @@ __global__ void __launch_bounds__(kAnyBlock)
 #pragma unroll
       for (int q = 0; q < kAnyBatch; ++q) {
         const uint32_t x = x0 + (q * kAnyThreadsPerRow + p) * kAnyTile;
-        if (x < cols) LoadAnyPack<DType, VEC>(&t[q], o, x, cols, sum);
+        if (x < cols) LoadAnyPack<DType, HOW>(&t[q], o, x, cols, sum);
       }
 #pragma unroll
       for (int q = 0; q < kAnyBatch; ++q) {
@@ -306,7 +308,7 @@ __global__ void __launch_bounds__(kAnyBlock)
         if (x < cols) {
 #pragma unroll
           for (int i = 0; i < kAnyTile; ++i) t[q].v[i] /= sum;
-          StoreAnyPack<DType, VEC>(o, x, cols, t[q]);
+          StoreAnyPack<DType, HOW>(o, x, cols, t[q]);
         }
       }
     }
@@ -340,7 +342,7 @@ template <typename DType, int FLAGS>
 __device__ __forceinline__ void GradPack(DType *o, const DType *s, uint32_t x, uint32_t cols, int k,
                                          int ignore_k, float alpha, float smooth) {
   AnyPack<DType> v;
-  LoadAnyPack<DType, false>(&v, s, x, cols, DType(0.0f));
+  LoadAnyPack<DType, kAnyLoose>(&v, s, x, cols, DType(0.0f));
   const bool ignored = (FLAGS & kAnyGradIgnore) && k == ignore_k;
   const uint32_t off = static_cast<uint32_t>(k) - x;  // wraps for k < x
   const bool label_here = k >= 0 && off < static_cast<uint32_t>(kAnyTile);
@@ -351,7 +353,7 @@ __device__ __forceinline__ void GradPack(DType *o, const DType *s, uint32_t x, u
                                          ignored, alpha, smooth);
     }
   }
-  StoreAnyPack<DType, false>(o, x, cols, v);
+  StoreAnyPack<DType, kAnyLoose>(o, x, cols, v);
 }
 /*! \brief blockIdx.x = row, blockIdx.y = stretch of columns; a thread moves packs of kAnyTile */
 template <typename DType, int FLAGS>
