@@ -219,6 +219,13 @@ inline bool SoftmaxRowsOnChip(half::half_t *d, uint32_t dstride, const half::hal
      unless it would fetch them element by element (of 101: 112 against 113 us; of 129: 117 against 105 us) */
   const bool packs = AnyPackable(s, sstride, const_cast<const half::half_t *>(d), dstride, cols, hip::kAnyTile);
   if (cols <= (packs ? 256u : 128u)) return false;
+  /* So do somewhat longer ones where there are rows enough to keep those workgroups busy: whole packs, 7895 x 296
+     10.0 us there and 12.0 here, 15195 x 272 16.8 and 18.2, 28350 x 352 31.7 and 32.4 (4153 x 264 8.8 and 8.2,
+     24734 x 360 28.9 and 28.0; 7862 x 376 11.2 and 12.7); others as long as the chip holds all of them at once there,
+     5735 x 139 7.9 and 9.8, 5583 x 219 9.4 and 10.6, 3352 x 165 7.5 and 8.7 (6246 x 251 15 and 11.8, 2556 x
+     219 8.3 and 7.7) */
+  if (packs && ((cols <= 352 && rows > 4352) || (cols <= 400 && rows > 5376 && rows <= 8192))) return false;
+  if (!packs && cols <= 256 && rows > 3240 && rows <= 6144) return false;
   /* what a wave has to hold where rows start at any column of an aligned pack */
   const bool aligned = (reinterpret_cast<uintptr_t>(s) | sstride * sizeof(half::half_t)) % 16 == 0;
   const uint32_t reach = aligned ? cols : cols + hip::kHalfPack - 1;
