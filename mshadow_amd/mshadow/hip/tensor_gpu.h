@@ -323,8 +323,9 @@ inline void AnyGrad2D(const Tensor<gpu, 2, DType> &dst, const Tensor<gpu, 2, DTy
   uint32_t dstride = dst.stride_, sstride = src.stride_;
   float smooth = SmoothShare(alpha, dst.size(1));
   /* several short rows to a workgroup, a long one over a few workgroups (65536 x 300 half_t: 39 us a
-     workgroup per row, 15 us) */
-  const bool several = cols <= hip::kAnyGradShort;
+     workgroup per row, 15 us). Few rows run side by side as they are, and a workgroup per row starts sooner (590 x 127
+     2.5 against 2.8 us, 404 x 624 2.3 and 2.5, 1157 x 79 2.6 and 2.8; of up to 20 columns 2.4 and 2.2 at 45 x 5) */
+  const bool several = cols <= hip::kAnyGradShort && (cols <= 20 || rows > 1536);
   const uint32_t packs = (cols + hip::kAnyTile - 1) / hip::kAnyTile;
   uint32_t rows_per_block = several ? hip::kAnyBlock / packs : 1u;
   FastDivU32 div_packs(packs);

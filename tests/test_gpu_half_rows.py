@@ -158,3 +158,27 @@ def test_half_gradient_rows(G, O, rows, cols):
         got = dst.download()
         assert np.array_equal(got[:, 7 - shift:7 - shift + cols], want)
         assert np.all(got[:, :7 - shift] == 0x1234) and np.all(got[:, 7 - shift + cols:] == 0x1234)
+
+
+# both sides of the numbers of rows and columns at which the dispatch changes kernels
+@pytest.mark.parametrize("rows,cols", [(64, 100), (65, 100), (64, 101), (65, 15), (65, 63), (6144, 11), (6145, 11), (6145, 7), (6144, 12),
+                                       (3240, 129), (3241, 129), (6144, 256), (6145, 256), (6144, 257)])
+def test_half_rows_routes(G, O, rows, cols):
+    for shift, dst_shift in ((0, 0), (5, 2)):
+        check(G, O, logits("normal", rows, cols), shift, dst_shift)
+
+
+@pytest.mark.parametrize("rows,cols", [(3241, 248), (4352, 264), (4353, 264), (4353, 352), (4353, 360), (5376, 400), (5377, 400),
+                                       (5377, 408), (8192, 376), (8193, 376)])
+def test_half_rows_routes_of_whole_packs(G, O, rows, cols):
+    x = O.float2half(logits("normal", rows, cols))
+    want = np.empty_like(x)
+    O.softmax(want, x)
+    src = G.to_device(x)
+    G.case_softmax(src, src)
+    assert np.array_equal(src.download(), want)
+
+
+@pytest.mark.parametrize("rows,cols", [(1536, 21), (1537, 20), (1537, 21), (1537, 96), (1537, 511), (1537, 1024)])
+def test_half_gradient_routes(G, O, rows, cols):
+    test_half_gradient_rows(G, O, rows, cols)
