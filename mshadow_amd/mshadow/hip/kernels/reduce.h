@@ -139,7 +139,11 @@ __global__ void __launch_bounds__(THREADS)
   const int t = threadIdx.x;
   const int col = t % CW;
   const int rsub = t / CW;
-  const uint32_t x = StripOfBlock(blockIdx.x, gridDim.x) * CW + col;
+  /* few strips of long chains wait for their adds and not for their lines, and are sooner in the order they are
+     dealt (binary16, 31924 x 1206: 131 us, in eighths 136; 18142 x 1170 77 and 80; but 5355 x 1698 28.8 and
+     27.3, and level from 128 strips on) */
+  const bool as_dealt = rows >= 16384u && gridDim.x <= 112u && gridDim.x % 8u != 0u;
+  const uint32_t x = (as_dealt ? blockIdx.x : StripOfBlock(blockIdx.x, gridDim.x)) * CW + col;
   const bool col_ok = x < cols;
   const uint32_t nstage = (rows + TR - 1) / TR;
   const bool chain_lane = (t < CW) && col_ok;  // lanes 0..CW-1 of wave 0 own the chains

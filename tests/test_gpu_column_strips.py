@@ -60,3 +60,15 @@ def test_sum_rows_strips(G, O, rows, cols, half):
             else:
                 G.reduce_keep_lowest(dst, offset_view(src, cols, shift), reducer, saver, scale)
             assert_bits_equal(dst.download(), want, f"{rows}x{cols} half={half} pitch+{extra} start+{shift}")
+
+
+# long chains in strips of 16 that the kernel of other sources sums: both sides of the rows and strips from which the
+# strips are dealt in eighths
+@pytest.mark.parametrize("rows,cols", [(16383, 17), (16384, 17), (16384, 128), (16390, 1785), (16384, 1793)])
+def test_half_sum_rows_long_chains(G, O, rows, cols):
+    m = O.float2half(uniform(77, (rows, cols)))
+    want = np.zeros(cols, np.uint16)
+    dst = G.to_device(want)
+    O.reduce_keep_lowest(want, m, SUM, SAVETO, 0.75)
+    G.case_reduce_keep_lowest(dst, G.to_device(m), SUM, SAVETO, int(O.float2half(np.array([0.75], f32))[0]))
+    assert_bits_equal(dst.download(), want, f"{rows}x{cols}")
