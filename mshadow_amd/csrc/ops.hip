@@ -1276,11 +1276,16 @@ int mshadow_hip_unpool_f32(float *dst, int dstride, const float *src, int sstrid
      over here, most of their windows being cut off: 7x160 80 against 71 us, 8x140 (24 M pixels) 168
      against 153, 5x128 57 against 46 - unless there are waves for one turn only (1.8 M pixels, 7x160
      14.6 against 15.5 us). Rows of 33 to 63 columns that are no packs, 2 x 2: as long as the four tensors
-     stay in the memory-side cache (4 M pixels, 56x50 23 against 30; 12 M 78 and 74; 36 M, 56x34 279 and 239). */
+     stay in the memory-side cache (4 M pixels, 56x50 23 against 30; 12 M 78 and 74; 36 M, 56x34 279 and 239).
+     5 x 5 on few low planes: a strip's rows wait for one another, and the staged kernel has a pixel a
+     thread (103 planes of 8x34 5.3 against 7.2 us, 464 of 8x36 6.3 and 7.1, 23 of 14x32 5.8 and 6.4; 301 of
+     14x25 8.5 and 7.2, 573 of 10x56 9.6 and 7.7, and with two rounds of its lanes 10 of 8x77 7.7 and 6.4). */
   const int slide_lanes = w <= 256 ? (w + 3) / 4 * (64 / ((w + 3) / 4)) : 0;  // of 64 with pixels: 40 at 140 columns
   const bool slides = ky == 5 ? (static_cast<long long>(h) * w > 1024 || (h > 5 && (w >= 24 || (w >= 16 && w % 4 == 0)))) &&
                                     !(slide_lanes < 44 && h <= 9 && static_cast<long long>(h) * w <= 1280 &&
-                                      planes > 8 * mshadow_abi::ComputeUnits())
+                                      planes > 8 * mshadow_abi::ComputeUnits()) &&
+                                    !(w >= (h < 8 ? 16 : 20) && w <= 64 && h <= 16 &&
+                                      static_cast<long long>(planes) * h * w < (w < 20 || h > 9 ? 40000 : h == 9 ? 60000 : 150000))
                       : ky == 2 ? w >= 64 || (w >= 32 && (w % 4 == 0 || static_cast<long long>(planes) * h * w <= 12000000))
                                 : w >= 64 && (h >= 64 || (w >= 96 && h >= 16));
   if (ky == kx && (ky == 2 || ky == 3 || ky == 5) && sy == 1 && sx == 1 && w <= 256 && slides && ph >= 1 && pw >= 1 &&
