@@ -1102,14 +1102,18 @@ int mshadow_hip_pool_f32(float *dst, int dstride, const float *src, int sstride,
      three the two are close: where there are planes for full groups and whole rows fill a wave's
      lanes here, the columns kernel is the faster one only on larger planes (12 M pixels, 3x3, here
      and there: 61x17 25 and 32 us, 32x33 24 and 26, 17x63 24 and 30, 8x160 21 and 22, 45x33 26 and 23;
-     31x35, half the lanes idle here, 35 and 28; 3 M pixels, 17x63: 10 and 9). */
+     31x35, half the lanes idle here, 35 and 28; 3 M pixels, 17x63: 10 and 9). Low wide planes whose rows are no
+     packs, or with windows of three, come later still (2x2: 9x155 15 and 18.5 us, 9x187 11.7 and 13.3; 3x3: 9x148
+     19 and 21, 11x161 17 and 19; 12x159 31 and 26;
+     2x2 8x195, 48 of 64 lanes at work here, 35 and 31). */
   const long long plane_bytes = static_cast<long long>(h) * row_bytes;
   const auto columns_pay = [&]() {
     if (ky == 5) return h * w >= 1024;
     if (w < 16) return false;
     const bool full_groups = planes / ((24 * 1024) / plane_bytes) >= 4ll * mshadow_abi::ComputeUnits();
     const int lanes = pw < 64 ? pw * (64 / pw) : pw * 64 / ((pw + 63) / 64 * 64);  // of 64, at work here
-    return h * w >= (w > 100 && h < 13 ? 1300 : !full_groups || lanes < 51 ? 1024 : w % 4 == 0 && w > 16 ? 1100 : 1400);
+    if (w > 100 && h < 14) return h * w >= (ky == 2 && (w % 4 == 0 || (pw > 192 && lanes < 51)) ? 1300 : 1750);
+    return h * w >= (!full_groups || lanes < 51 ? 1024 : w % 4 == 0 && w > 16 ? 1100 : 1400);
   };
   if (plane_bytes * 2 <= 24 * 1024 && planes >= 2 && !(columns && band >= 1 && columns_pay())) {
     long long per_block = (24 * 1024) / plane_bytes;

@@ -57,3 +57,12 @@ def test_stride_one_pooling(G, O, h, w, k):
                                           (11364, 32, 33, 2)])
 def test_stride_one_pooling_of_many_planes(G, O, planes, h, w, k):
     check(G, O, planes, h, w, k, (MAX,))
+
+
+# few low planes of the 5x5 gradient and wide low planes of the forward pass, around the pixels at which the
+# dispatch changes kernels
+@pytest.mark.parametrize("planes,h,w,k", [(200, 6, 16, 5), (416, 6, 16, 5), (417, 6, 16, 5), (585, 8, 32, 5), (586, 8, 32, 5), (208, 9, 32, 5),
+                                          (209, 9, 32, 5), (78, 16, 32, 5), (79, 16, 32, 5), (20, 9, 64, 5), (20, 9, 65, 5), (5, 17, 20, 5),
+                                          (4300, 9, 155, 2), (4300, 11, 161, 3), (4300, 12, 146, 3), (4300, 10, 136, 2), (4300, 8, 195, 2)])
+def test_stride_one_pooling_of_low_planes(G, O, planes, h, w, k):
+    check(G, O, planes, h, w, k, (MAX,))
