@@ -449,7 +449,7 @@ int RowsOfLaunch(unsigned threads) {
   return most < static_cast<unsigned long long>(INT_MAX) ? static_cast<int>(most) : INT_MAX;
 }
 /*! \brief threads a row of the kernels below takes, where there are many rows */
-unsigned SoftmaxThreadsPerRow(int cols) { return cols <= 32 ? 1u : cols <= 256 ? 32u : cols <= 3072 ? 64u : 1024u; }
+unsigned SoftmaxThreadsPerRow(int cols) { return cols <= 32 ? 1u : cols <= 256 ? 32u : cols <= 2560 ? 64u : 1024u; }
 
 /*! \brief rows that a thread, a part of a wave or a wave takes; false: longer ones, which take a
  *  workgroup */
@@ -476,16 +476,17 @@ bool LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, 
   else if (cols <= 64) SHORT_PART(16, 4);
   else if (cols <= 128) SHORT_PART(16, 8);
   else if (cols <= 256) SHORT_PART(32, 8);
-  /* a wave per row for any number of rows of up to 512 columns, and for many of up to 3072 (65536
-     rows of 300 / 1000 columns: 47 / 94 us against 163 / 193 us with a workgroup per row, 16384 of
-     2304 73 against 120 us; at 4096 columns, 64 of them a lane, 151 against 127 us). 100 rows of
-     500: 5.0 against 5.6 us; 1000 rows of 1000 / 2000: 7.8 / 10.9 against 7.3 / 9.3 us, 2000 rows
-     8.4 / 12.5 against 10.1 / 15.3 us. */
+  /* a wave per row for any number of rows of up to 512 columns, and for many of up to 2560 (65536
+     rows of 300 / 1000 columns: 47 / 93 us against 163 / 174 us with a workgroup per row, 16384 of
+     2304 68 against 75 us, 8000 of 2560 37.6 against 40.9; at 3000 columns 8000 rows 44.3 against 42.2,
+     40000 209 against 199). 100 rows of 500: 5.0 against 5.6 us; 1000 rows of 1000: 7.8 against 7.1 us,
+     3000 rows 9.7 against 12.7; 2000 rows of 2000 13.1 against 11.9, 3000 rows 14.6 against 16.1.
+     (The row sums alone are as they were measured before: up to 3072 columns, from 6 rows a CU on.) */
   else if (cols <= 512) WAVE_SLABS(2);
-  else if (cols > 3072 || rows < 6 * cus) return false;
+  else if (cols > (TERMS_GIVEN ? 3072 : 2560) || rows < (cols > 1024 && !TERMS_GIVEN ? 10 : 6) * cus) return false;
   else if (cols <= 1024) WAVE_SLABS(4);
   else if (cols <= 2048) WAVE_SLABS(8);
-  else WAVE_SLABS(12);
+  else WAVE_SLABS(TERMS_GIVEN ? 12 : 10);
 #undef SHORT_THREAD
 #undef SHORT_PART
 #undef WAVE_SLABS
@@ -612,32 +613,47 @@ int mshadow_hip_softmax_f32(float *dst, int dstride, const float *src, int sstri
 #define SOFTMAX_LAUNCH(T, S, V) \
   LaunchKernelIfFits((SoftmaxRowKernel<T, S, V, false>), dim3(rows), dim3(T), 0, s, dst, dstride, \
                      src, sstride, cols)
-  /* many rows of 8193 to 16384 columns: four waves a row with 64 columns a thread, eight rows to a
-     CU instead of four ((4096,10000): 82 against 104 us, (8192,12288): 153 against 196 us; with
-     2048 rows the eight waves a row below finish them sooner, 57 against 70 us) */
-  if (cols > 8192 && cols <= 16384 && rows >= 16 * mshadow_abi::ComputeUnits()) {
-    SOFTMAX_LAUNCH(256, 16, 4);
-    return AfterLaunch("softmax");
+#define SOFTMAX_LAUNCH_LDS(T, S, L) \
+  LaunchKernelIfFits((SoftmaxRowKernel<T, S, 4, false, 4, L>), dim3(rows), dim3(T), 0, s, dst, dstride, \
+                     src, sstride, cols)
+  const int cus = mshadow_abi::ComputeUnits();
+  /* Up to two rows a CU: the CU has the row to itself, or nearly, and what counts is how soon the row is
+     through, so it gets two to four times the waves (100 rows of 3000 / 7000 / 30000: 6.6 / 8.2 / 19.5
+     against 8.3 / 11.0 / 21.6 us, 500 rows 9.8 / 13.2 / 36.4 against 9.9 / 14.7 / 38.3; 1000 rows are
+     slower that way, 15.6 / 20.6 against 11.8 / 18.0). */
+  if (rows <= 2 * cus && cols > 1024 && cols <= 32768) {
+    if (cols <= 2048) SOFTMAX_LAUNCH(512, 1, 4);
+    else if (cols <= 4096) SOFTMAX_LAUNCH(1024, 1, 4);
+    else if (cols <= 8192) SOFTMAX_LAUNCH(1024, 2, 4);
+    else if (cols <= 16384) SOFTMAX_LAUNCH(1024, 4, 4);
+    else SOFTMAX_LAUNCH(1024, 8, 4);
   }
-  if (cols <= 1024) SOFTMAX_LAUNCH(256, 1, 4);
+  else if (cols <= 1024) SOFTMAX_LAUNCH(256, 1, 4);
   else if (cols <= 2048) SOFTMAX_LAUNCH(256, 2, 4);
   else if (cols <= 4096) SOFTMAX_LAUNCH(256, 4, 4);
   else if (cols <= 8192) SOFTMAX_LAUNCH(256, 8, 4);
   else if (cols <= 16384) SOFTMAX_LAUNCH(512, 8, 4);
   else if (cols <= 32768) SOFTMAX_LAUNCH(512, 16, 4);
+  /* longer rows, part of each in LDS: up to 51200 columns two rows share a CU still (2048 x 50257: 206 us,
+     alone in its registers 264), from 65537 on a row that has the CU to itself stays on the chip
+     (44 x 110032: 48 us, in stretches 77; 1000 x 80000: 179 us, 256; 2048 x 100000: 525 us, 636) */
+  else if (cols <= 51200 && rows > cus) SOFTMAX_LAUNCH_LDS(512, 18, 7);
   else if (cols <= 65536) SOFTMAX_LAUNCH(1024, 16, 4);
-  /* longer rows: stretches of 32768 columns on 512 threads, two rows to a CU ((512,128000): 221 us
-     against 271 us with stretches of 65536 on 1024 threads; up to 65536 columns the single pass
-     above is faster than stretches, 265 against 432 us on (2048,50257)) */
+  else if (cols <= 81920) SOFTMAX_LAUNCH_LDS(1024, 16, 4);
+  /* ... but for one to two rows a CU, which stretches take two at a time (512 x 90000: 142 us, 155) */
+  else if (cols <= 110592 && (rows <= cus || rows > 2 * cus)) SOFTMAX_LAUNCH_LDS(1024, 19, 8);
+  /* longer ones yet: stretches of 32768 columns on 512 threads, two rows to a CU ((512,128000): 183 us
+     against 271 us with stretches of 65536 on 1024 threads) */
   else if (cols > INT_MAX - 32768) {
     return Fail(MSHADOW_HIP_ERR_ARGUMENT, "softmax: row too long for 32-bit column counts");
-  } else if (rows > mshadow_abi::ComputeUnits()) {
+  } else if (rows > cus) {
     LaunchKernelIfFits((SoftmaxStretchRowKernel<512, 16, false, 4>), dim3(rows), dim3(512), 0, s, dst,
                        dstride, src, sstride, cols);
   } else {
     LaunchKernelIfFits((SoftmaxStretchRowKernel<512, 16, false, 2>), dim3(rows), dim3(512), 0, s, dst,
                        dstride, src, sstride, cols);
   }
+#undef SOFTMAX_LAUNCH_LDS
 #undef SOFTMAX_LAUNCH
   return AfterLaunch("softmax");
 }
@@ -671,7 +687,7 @@ int mshadow_hip_softmax_rowsum_f32(float *sums, const float *terms, int tstride,
   LaunchKernelIfFits((SoftmaxRowKernel<T, S, V, true>), dim3(rows), dim3(T), 0, s, sums, 0, terms, \
                      tstride, cols)
   if (vec) {
-    if (cols > 8192 && cols <= 16384 && rows >= 16 * mshadow_abi::ComputeUnits()) ROWSUM_LAUNCH(256, 16, 4);  // as above
+    if (cols > 8192 && cols <= 16384 && rows >= 16 * mshadow_abi::ComputeUnits()) ROWSUM_LAUNCH(256, 16, 4);
     else if (cols <= 1024) ROWSUM_LAUNCH(256, 1, 4);
     else if (cols <= 2048) ROWSUM_LAUNCH(256, 2, 4);
     else if (cols <= 4096) ROWSUM_LAUNCH(256, 4, 4);

@@ -90,14 +90,11 @@ __device__ inline float WaveResolve(float s, const float (&t)[N]) {
  *      list in the row's list of addends; the lists are copied there, each by one wave, with
  *      the run of certain chunks in front of each listed chunk as one more addend  (barrier)
  *   E  wave 0: the chain - the row's addends summed serially, every run verified  (barrier)
- * A row whose plan fails a verification, or that has more listed chunks than slots, is summed
+ * A row whose plan fails a verification, or whose lists are longer than their space, is summed
  * by wave scans instead, chunk after chunk. The sum may start from s0 instead of zero (a row
  * longer than the registers hold is summed stretch by stretch): s0 then stands in front of the
  * approximate prefix sums and is where the chain begins.
  * Lane l keeps the chunk-table entries of chunks l * CPL .. l * CPL + CPL - 1. */
-/*! \brief chunks per row that can hand a list of addends to the chain (a row of softmax
- *  terms has about a dozen) */
-const int kPlanSlots = 24;
 const uint32_t kListedBit = 0x80000000u;
 
 /* hook for a profiling build: a translation unit may define this to record a timestamp
@@ -113,18 +110,46 @@ struct Addend {
   float value;
   uint32_t check;
 };
-/*! \brief the addends of one listed chunk, in row order: at most one per term */
-template <int N>
-struct AddendList {
-  Addend entry[kWave * N];
+/*! \brief a workgroup's row of terms: thread t's N terms of the first REGS slabs in its registers,
+ *  of the other INLDS slabs in LDS (`rest` is where its own lie; it alone reads and writes them) */
+template <int THREADS, int REGS, int INLDS, int N>
+struct RowTerms {
+  static const int kSlabs = REGS + INLDS;
+  float v[REGS][N];
+  float *rest;
+  __device__ __forceinline__ float *InLds(int j) const { return rest + (j - REGS) * (THREADS * N); }
+  /*! \brief slab j, known once the caller's loop is unrolled */
+  __device__ __forceinline__ void Get(float (&t)[N], int j) const {
+    if (INLDS == 0 || j < REGS) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) t[i] = v[j < REGS ? j : 0][i];
+    } else {
+      FetchRest(t, j);
+    }
+  }
+  __device__ __forceinline__ void Set(const float (&t)[N], int j) {
+    if (INLDS == 0 || j < REGS) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[j < REGS ? j : 0][i] = t[i];
+    } else {
+      typedef float V __attribute__((ext_vector_type(N)));
+      V q;
+#pragma unroll
+      for (int i = 0; i < N; ++i) q[i] = t[i];
+      *reinterpret_cast<V *>(InLds(j)) = q;
+    }
+  }
+  __device__ __forceinline__ void FetchRest(float (&t)[N], int j) const {
+    typedef float V __attribute__((ext_vector_type(N)));
+    const V q = *reinterpret_cast<const V *>(InLds(j));
+#pragma unroll
+    for (int i = 0; i < N; ++i) t[i] = q[i];
+  }
 };
 
-template <int W, int SLABS, int N>
+template <int W, int SLABS, int N, int ADDENDS = W <= 4 ? 512 : 2048>
 struct RowSumLds {
   static const int kChunks = W * SLABS;
-  /* small workgroups share a CU with several others: fewer slots each */
-  static const int kWanted = W <= 4 ? kPlanSlots * 2 / 3 : kPlanSlots;
-  static const int kSlots = (kChunks < kWanted) ? kChunks : kWanted;
   float approx[kChunks];
   float cmax[kChunks];
   /*! \brief what a listed chunk's wave needs of the plan. Every wave computes the whole
@@ -133,15 +158,15 @@ struct RowSumLds {
   struct ChunkPlan {
     float start;    //!< approximate prefix sum in front of the chunk
     float low;      //!< what the sum is at least in front of the chunk
-    uint32_t slot;  //!< the chunk's slot, if the plan lists it
     uint32_t peak;  //!< the chunk holds a term above `low` (it can raise the bound inside the chunk)
   };
   MSHADOW_ALIGNED(16) ChunkPlan plan[kChunks];
-  /*! \brief certain chunk: its integer total; listed chunk: kListedBit | addends << 8 | slot */
+  /*! \brief certain chunk: its integer total; listed chunk: kListedBit | addends << 16 | where its
+   *  list begins */
   uint32_t q[kChunks];
-  float s;          //!< the row's sum, from the chain to everybody
-  int fail;         //!< the plan did not hold: redo the row the slow way
-  uint32_t nslots;  //!< lists handed out
+  float s;         //!< the row's sum, from the chain to everybody
+  int fail;        //!< the plan did not hold: redo the row the slow way
+  uint32_t taken;  //!< entries of `list` handed out
   float wmax[W];
   /*! \brief the row's addends in row order, as the chain takes them: for each listed chunk
    *  the run of certain chunks in front of it (one addend) and then its own list, and
@@ -150,10 +175,13 @@ struct RowSumLds {
      behind the crossing listed lane by lane (the bounds cannot tell on which side the sum is)
      and takes 900-1100, so workgroups of eight waves and more, two to a CU, have room for 2048:
      the chain over them is a few microseconds, the fall-back 45 */
-  static const int kRowAddends = W <= 4 ? 512 : 2048;
-  Addend row[kRowAddends];
+  static const int kRowAddends = ADDENDS;
+  MSHADOW_ALIGNED(8) Addend row[kRowAddends];
   uint32_t row_count;
-  MSHADOW_ALIGNED(8) AddendList<N> list[kSlots];
+  /*! \brief the lists of the listed chunks, each in row order and in one piece, the pieces as their
+   *  waves came for them: no more in all than the row's list takes. A piece of 256 entries for each of
+   *  24 chunks was 48 KB, which a CU has twice and then holds nothing else. */
+  MSHADOW_ALIGNED(8) Addend list[kRowAddends];
 };
 
 /*! \brief entry k of a table spread over lanes (CPL entries per lane); k is uniform */
@@ -195,9 +223,13 @@ struct SlabPicker<LO, LO + 1, SLABS, N> {
     }
   }
 };
-template <int SLABS, int N>
-__device__ __forceinline__ void SelectSlab(float (&t)[N], const float (&v)[SLABS][N], int j) {
-  SlabPicker<0, SLABS, SLABS, N>::Pick(t, v, j);
+template <int THREADS, int REGS, int INLDS, int N>
+__device__ __forceinline__ void SelectSlab(float (&t)[N], const RowTerms<THREADS, REGS, INLDS, N> &terms, int j) {
+  if (INLDS != 0 && j >= REGS) {
+    terms.FetchRest(t, j);
+  } else {
+    SlabPicker<0, REGS, REGS, N>::Pick(t, terms.v, j);
+  }
 }
 
 /*! \brief value of v in the lane below (lane 0 receives `first`) */
@@ -242,19 +274,19 @@ __device__ __forceinline__ float ChainBlock(float s, float addend, uint32_t chec
   return ReadLaneF32(sum, count - 1);
 }
 
-template <int THREADS, int SLABS, int N, bool CHECK_SIGN, bool UNIT_PEAK>
-__device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
-                                      RowSumLds<THREADS / kWave, SLABS, N> *lds, float s0 = 0.0f) {
+template <bool CHECK_SIGN, bool UNIT_PEAK, int THREADS, int REGS, int INLDS, int N, typename Lds>
+__device__ inline float RowOrderedSum(const RowTerms<THREADS, REGS, INLDS, N> &terms, Lds *lds, float s0 = 0.0f) {
   using namespace ordered_sum;
   using mshadow::hip::ReadLaneU32;
   using mshadow::hip::WaveInclusiveScanU32;
-  typedef RowSumLds<THREADS / kWave, SLABS, N> Lds;
+  const int SLABS = REGS + INLDS;
   const int W = THREADS / kWave;
   const int NCH = W * SLABS;
-  const int CPL = (NCH + kWave - 1) / kWave;
+  const int NEED = (NCH + kWave - 1) / kWave, CPL = NEED <= 2 ? NEED : NEED <= 4 ? 4 : 8;
   static_assert(NCH % CPL == 0, "chunk table does not tile the lanes");
   static_assert(SLABS <= 32, "the per-wave masks have 32 bits");
-  static_assert(kWave * N <= 256, "a list's length must fit the bits it is filed in");
+  static_assert(kWave * N <= 256 && Lds::kRowAddends < 0xffff, "a list's length and place must fit the bits they are filed in");
+  static_assert(Lds::kChunks == NCH, "the tables are for another row");
   const int wave = __builtin_amdgcn_readfirstlane(WaveId());
   const int lane = LaneId();
 
@@ -263,47 +295,56 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
   if (threadIdx.x == 0) {
     lds->s = 0.0f;
     lds->fail = 0;
-    lds->nslots = 0u;
+    lds->taken = 0u;
   }
   if (CHECK_SIGN) __syncthreads();  // the sign check below may set `fail`
   /* the wave-wide reductions take the slabs in groups of at most sixteen (registers) */
-  const int GRP = SLABS < 16 ? SLABS : 16;
+  const int GRP = SLABS < 16 ? SLABS : INLDS != 0 ? 8 : 16;
 #pragma unroll
   for (int g = 0; g < SLABS; g += GRP) {
     float part[GRP];
 #pragma unroll
     for (int j = 0; j < GRP; ++j) {
-      part[j] = v[g + j][0];
+      part[j] = 0.0f;
+      if (g + j >= SLABS) continue;
+      float t[N];
+      terms.Get(t, g + j);
+      part[j] = t[0];
 #pragma unroll
-      for (int i = 1; i < N; ++i) part[j] += v[g + j][i];
+      for (int i = 1; i < N; ++i) part[j] += t[i];
     }
     const float mine = mshadow::hip::WaveSumMany<GRP>(part);  // lane l: slab g + l % GRP
-    if (lane < GRP) lds->approx[(g + lane) * W + wave] = mine;
+    const bool files = lane < GRP && g + lane < SLABS;
+    if (files) lds->approx[(g + lane) * W + wave] = mine;
     if (!UNIT_PEAK) {
       asm volatile("" ::: "memory");  // the two tables one after the other: fewer registers live
 #pragma unroll
       for (int j = 0; j < GRP; ++j) {
+        part[j] = 0.0f;
+        if (g + j >= SLABS) continue;
+        float t[N];
+        terms.Get(t, g + j);
         if (N == 4) {
-          part[j] = MaxNum(MaxNum3(v[g + j][0], v[g + j][1 % N], v[g + j][2 % N]), v[g + j][3 % N]);
+          part[j] = MaxNum(MaxNum3(t[0], t[1 % N], t[2 % N]), t[3 % N]);
         } else {
-          part[j] = v[g + j][0];
+          part[j] = t[0];
 #pragma unroll
-          for (int i = 1; i < N; ++i) part[j] = MaxNum(part[j], v[g + j][i]);
+          for (int i = 1; i < N; ++i) part[j] = MaxNum(part[j], t[i]);
         }
       }
       const float most = mshadow::hip::WaveReduceMany<mshadow::hip::WaveOpMax, float, GRP>(part);
-      if (lane < GRP) lds->cmax[(g + lane) * W + wave] = most;
+      if (files) lds->cmax[(g + lane) * W + wave] = most;
     } else {
       /* The terms of a softmax are at most 1 and one of them is 1. A chunk's largest term
          serves as a lower bound of the sum behind it, and only a term next to a power of
          two - the 1 - tells more than the approximate sums do: the largest term is looked
          for only in chunks whose sum reaches 1, and taken as 0 elsewhere. */
-      if (lane < GRP) lds->cmax[(g + lane) * W + wave] = 0.0f;
-      for (uint32_t todo = static_cast<uint32_t>(__ballot(lane < GRP && mine >= 1.0f)); todo != 0u;
+      if (files) lds->cmax[(g + lane) * W + wave] = 0.0f;
+      for (uint32_t todo = static_cast<uint32_t>(__ballot(files && mine >= 1.0f)); todo != 0u;
            todo &= todo - 1u) {
         const int j = g + __ffs(static_cast<int>(todo)) - 1;
         float t[N];
-        SelectSlab<SLABS, N>(t, v, j);
+        SelectSlab(t, terms, j);
         float m = t[0];
 #pragma unroll
         for (int i = 1; i < N; ++i) m = MaxNum(m, t[i]);
@@ -316,8 +357,10 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
     float least = 0.0f;
 #pragma unroll
     for (int j = 0; j < SLABS; ++j) {
+      float t[N];
+      terms.Get(t, j);
 #pragma unroll
-      for (int i = 0; i < N; ++i) least = (v[j][i] < least) ? v[j][i] : least;
+      for (int i = 0; i < N; ++i) least = (t[i] < least) ? t[i] : least;
     }
     if (__ballot(least < 0.0f) != 0ull && lane == 0) lds->fail = 1;
   }
@@ -326,7 +369,6 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
 
   /* B: plan per chunk, identical in every wave */
   uint32_t code[CPL];     // 1 + binade of a certain chunk, 0: to be listed
-  uint32_t planned;       // how many chunks the plan lists
   {
     float pre[CPL + 1], seen[CPL + 1], own[CPL];
     pre[0] = 0.0f;
@@ -361,29 +403,17 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
        every run of certain chunks then has one scale */
     const int before = static_cast<int>(FromLaneBelowU32(static_cast<uint32_t>(raw[CPL - 1]),
                                                          static_cast<uint32_t>(-1)));
-    /* the chunks to be listed get their slots in row order, known to every wave alike; a
-       chunk that turns out to hold a tie asks for one of the slots behind those */
-    uint32_t in_lane[CPL];
-    uint32_t mine = 0u, below = 0u;
-    planned = 0u;
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
       const int prev = (c == 0) ? before : raw[c - 1];
       const bool clash = raw[c] >= 0 && prev >= 0 && prev != raw[c];
       code[c] = (raw[c] < 0 || clash) ? 0u : static_cast<uint32_t>(raw[c]) + 1u;
-      const bool to_list = code[c] == 0u && lane * CPL + c < NCH;
-      const unsigned long long listing = __ballot(to_list);
-      in_lane[c] = mine;  // listed chunks of this lane in front of chunk c
-      mine += to_list ? 1u : 0u;
-      below += mshadow::hip::LanesBelow(listing);
-      planned += static_cast<uint32_t>(__popcll(listing));
     }
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
       typename Lds::ChunkPlan cp;
       cp.start = st[c];
       cp.low = lo[c];
-      cp.slot = below + in_lane[c];
       cp.peak = own[c] > lo[c] ? 1u : 0u;
       if (lane * CPL + c < NCH) lds->plan[lane * CPL + c] = cp;
     }
@@ -409,16 +439,20 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
       uint32_t part[GRP];
 #pragma unroll
       for (int j = 0; j < GRP; ++j) {
+        part[j] = 0u;
+        if (g + j >= SLABS) continue;
         const uint32_t ck = ReadLaneU32(my_code, ((g + j) * W + wave) / CPL);
         /* straight-line: a chunk to be listed is quantised too (against any binade) and
            its result dropped */
         const bool certain = ck != 0u;
         const uint32_t base = (certain ? ck - 1u : 1u) << 23;
         float lo = __uint_as_float(base), hi = __uint_as_float(base + 1u);
+        float t[N];
+        terms.Get(t, g + j);
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-          lo = lo + v[g + j][i];
-          hi = hi + v[g + j][i];
+          lo = lo + t[i];
+          hi = hi + t[i];
         }
         all_gaps &= certain ? __float_as_uint(hi) - __float_as_uint(lo) : 1u;
         part[j] = __float_as_uint(lo) - base;
@@ -428,14 +462,14 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
       /* lanes 0 .. GRP-1 file the result of "their" chunk (overwritten below if the chunk is
          listed after all); a total that cannot fit a binade is cut so that sums of totals
          stay inside 32 bits (the run it joins fails its check) */
-      if (lane < GRP) lds->q[(g + lane) * W + wave] = total < (1u << 24) ? total : (1u << 24);
+      if (lane < GRP && g + lane < SLABS) lds->q[(g + lane) * W + wave] = total < (1u << 24) ? total : (1u << 24);
     }
     if (__ballot(all_gaps != 1u) != 0ull) {
       for (int j = 0; j < SLABS; ++j) {
         const uint32_t ck = ReadLaneU32(my_code, (j * W + wave) / CPL);
         if (ck == 0u) continue;
         float t[N];
-        SelectSlab<SLABS, N>(t, v, j);
+        SelectSlab(t, terms, j);
         if (__ballot(!LaneDualQuant<N>(t, ck - 1u).ok) != 0ull) listed |= 1u << j;
       }
     }
@@ -446,20 +480,8 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
     const int j = __ffs(static_cast<int>(todo)) - 1;
     const int k = j * W + wave;
     const typename Lds::ChunkPlan cp = lds->plan[k];
-    uint32_t slot;
-    if (ReadLaneU32(my_code, k / CPL) == 0u) {
-      slot = __builtin_amdgcn_readfirstlane(cp.slot);
-    } else {
-      slot = 0u;
-      if (lane == 0) slot = planned + atomicAdd(&lds->nslots, 1u);
-      slot = __builtin_amdgcn_readfirstlane(slot);
-    }
-    if (slot >= static_cast<uint32_t>(Lds::kSlots)) {  // no room: the row is redone by wave scans
-      if (lane == 0) lds->fail = 1;
-      break;
-    }
     float t[N];
-    SelectSlab<SLABS, N>(t, v, j);
+    SelectSlab(t, terms, j);
     const float st = cp.start;
     const float lb = cp.low;
     /* the lane's own bounds: approximate prefix sums inside the chunk, and the largest term
@@ -499,22 +521,29 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
         static_cast<uint32_t>(heads >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(heads), 0u));
     const uint32_t at = terms_below * N + heads_below;
     const uint32_t count = static_cast<uint32_t>(__popcll(terms)) * N + static_cast<uint32_t>(__popcll(heads));
-    AddendList<N> *out = &lds->list[slot];
+    uint32_t place = 0u;
+    if (lane == 0) place = atomicAdd(&lds->taken, count);
+    place = __builtin_amdgcn_readfirstlane(place);
+    if (place + count > static_cast<uint32_t>(Lds::kRowAddends)) {  // no room: the row is redone by wave scans
+      if (lane == 0) lds->fail = 1;
+      break;
+    }
+    Addend *out = lds->list + place;
     if (term_lane) {
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         Addend e;
         e.value = t[i];
         e.check = 0u;
-        out->entry[at + i] = e;
+        out[at + i] = e;
       }
     } else if (head) {
       Addend e;
       e.value = RunAddend(static_cast<uint32_t>(c), q_end - (q_incl - qi));
       e.check = static_cast<uint32_t>(c + 1);
-      out->entry[at] = e;
+      out[at] = e;
     }
-    if (lane == 0) lds->q[k] = kListedBit | (count << 8) | slot;
+    if (lane == 0) lds->q[k] = kListedBit | (count << 16) | place;
   }
   MSHADOW_ROWSUM_STAMP(8)
   __syncthreads();
@@ -536,7 +565,7 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
       if (is_listed) code[c] = 0u;  // planned certain, found to hold a tie
       pre[c + 1] = pre[c] + (is_listed ? 0u : qk[c]);
       cnt[c + 1] = cnt[c] + (is_listed ? 1u : 0u);
-      len[c + 1] = len[c] + (is_listed ? ((qk[c] >> 8) & 0x1ffu) + 1u : 0u);
+      len[c + 1] = len[c] + (is_listed ? ((qk[c] >> 16) & 0x1ffu) + 1u : 0u);
     }
     uint32_t incl = pre[CPL], cincl = cnt[CPL], lincl = len[CPL];
     mshadow::hip::WaveScanSum3U32(&incl, &cincl, &lincl);
@@ -572,9 +601,9 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
           const uint32_t to = ReadLaneU32(at, l);
           const float a0 = ReadLaneF32(front, l);
           const uint32_t c0 = ReadLaneU32(run, l);
-          const AddendList<N> *from = &lds->list[q & 0xffu];
-          const int n = static_cast<int>((q >> 8) & 0x1ffu);
-          for (int g = lane; g < n; g += kWave) lds->row[to + 1u + g] = from->entry[g];
+          const Addend *from = lds->list + (q & 0xffffu);
+          const int n = static_cast<int>((q >> 16) & 0x1ffu);
+          for (int g = lane; g < n; g += kWave) lds->row[to + 1u + g] = from[g];
           if (lane == 0) {
             Addend e;
             e.value = a0;
@@ -636,7 +665,7 @@ __device__ inline float RowOrderedSum(const float (&v)[SLABS][N], int cols,
   __syncthreads();
   for (int j = 0; j < SLABS; ++j) {
     float t[N];
-    SelectSlab<SLABS, N>(t, v, j);
+    SelectSlab(t, terms, j);
     for (int w = 0; w < W; ++w) {
       if (wave == w) {
         const float r = WaveResolve<true, 0, N>(lds->s, t);
@@ -688,18 +717,54 @@ __device__ inline float BlockMax(float v, float *wmax) {
   return m;
 }
 
-/*! \brief THREADS * SLABS * VEC >= cols. VEC == 4 moves 16-byte packs wherever the rows
- *  start and whatever their length (the last, partial pack of a row element by element). Slab j of wave w holds the 64 * VEC columns from (j * W + w) * 64 * VEC,
- *  lane l of that VEC consecutive ones: each load is one contiguous kilobyte per wave, the
- *  W waves together stream one contiguous stretch per slab, and the order of the row is
+/*! \brief this lane's pack of the 256 columns from c0 (uniform) of a row of at least four columns, 16
+ *  bytes wherever it starts: the pack that the row ends in, and those behind it, are the row's last
+ *  four columns instead. No branch: all loads of a row are in flight together. */
+__device__ __forceinline__ void LoadPackOfRow(float (&t)[4], const float *in, int c0, int cols) {
+  const int c = c0 + static_cast<int>(LaneId() * 4);
+  const F4 q = StreamLoadF4Anywhere(in + (c < cols - 4 ? c : cols - 4));
+  t[0] = q.x; t[1] = q.y; t[2] = q.z; t[3] = q.w;
+}
+/*! \brief what it loaded put into its place: moved down where the row ends inside the pack, `absent`
+ *  behind the end */
+__device__ __forceinline__ void PlacePackOfRow(float (&t)[4], int c0, int cols, float absent) {
+  const int d = c0 + static_cast<int>(LaneId() * 4) - (cols - 4);
+  if (d > 0) {
+    t[0] = d == 1 ? t[1] : d == 2 ? t[2] : d == 3 ? t[3] : absent;
+    t[1] = d == 1 ? t[2] : d == 2 ? t[3] : absent;
+    t[2] = d == 1 ? t[3] : absent;
+    t[3] = absent;
+  }
+}
+
+/*! \brief THREADS * (REGS + INLDS) * VEC >= cols, cols >= 4. VEC == 4 moves 16-byte packs wherever the
+ *  rows start and whatever their length. Slab j of wave w holds the 64 * VEC columns from
+ *  (j * W + w) * 64 * VEC, lane l of that VEC consecutive ones: each load is one contiguous kilobyte per
+ *  wave, the W waves together stream one contiguous stretch per slab, and the order of the row is
  *  slab, wave, lane, element.
+ *  What bounds it: the memory time of a row that shares its CU with another, plus what it does between
+ *  its loads and its stores where nothing else is in flight. All loads of a row are issued before the
+ *  first is waited for (with the row's ragged end in branches between them they went one after the
+ *  other: 5000 x 3500 45 us, now 31; 2048 x 8000 34 and 24; 8192 x 32000 378 and 373).
+ *  INLDS: that many slabs live in LDS, which the registers leave idle. Two rows of 50257 columns then fit
+ *  a CU (18 slabs of 512 threads in registers, 7 in LDS; 2048 of them 264 -> 206 us, 4.0 TB/s), and one of
+ *  up to 110592 on 1024 threads (19 and 8), which went through the caches three times before. Three
+ *  rows of 32000 to a CU that way (11 and 5, 80 registers, 22 of them spilled) took 419 us against 373.
  *  TERMS_GIVEN: src already holds the (non-negative) terms and dst[row] receives their
  *  left-to-right sum - the row-sum stage on its own. */
-template <int THREADS, int SLABS, int VEC, bool TERMS_GIVEN, int MIN_WAVES = 4>
+template <int THREADS, int REGS, int VEC, bool TERMS_GIVEN, int MIN_WAVES = 4, int INLDS = 0>
 __global__ void __launch_bounds__(THREADS, MIN_WAVES)  // 4 waves per SIMD: two 512-thread rows per CU
     SoftmaxRowKernel(float *dst, int dstride, const float *src, int sstride, int cols) {
-  __shared__ RowSumLds<THREADS / kWave, SLABS, VEC> lds;
+  const int SLABS = REGS + INLDS;
   const int W = THREADS / kWave;
+  typedef RowTerms<THREADS, REGS, INLDS, VEC> Terms;
+  /* with terms in LDS beside it the row's list is as long as the rows that share a CU leave room for */
+  const int kRowsPerCu = 4 * MIN_WAVES / W;
+  const int kLeft = 160 * 1024 / kRowsPerCu - INLDS * THREADS * VEC * 4 - W * SLABS * 28 - 256;
+  typedef RowSumLds<W, SLABS, VEC, INLDS != 0 ? kLeft / 16 / 64 * 64 : W <= 4 ? 512 : 2048> Lds;
+  __shared__ Lds lds;
+  __shared__ MSHADOW_ALIGNED(16) float rest[INLDS != 0 ? INLDS * THREADS * VEC : 1];
+  static_assert(INLDS == 0 || (VEC == 4 && (sizeof(Lds) + sizeof(rest)) * kRowsPerCu <= 160 * 1024), "LDS of a CU");
   const int kChunk = kWave * VEC;  // columns of one chunk
   const int wave = __builtin_amdgcn_readfirstlane(WaveId());
   const uint32_t lane_col = LaneId() * VEC;
@@ -712,71 +777,79 @@ __global__ void __launch_bounds__(THREADS, MIN_WAVES)  // 4 waves per SIMD: two 
   MSHADOW_ROWSUM_STAMP(10)
   /* chunk k = j * W + wave starts at column k * kChunk; whether it lies wholly inside the
      row is the same for all lanes, so the common case carries no per-lane guards */
-  float v[SLABS][VEC];
+  Terms terms;
+  terms.rest = rest + threadIdx.x * VEC;
+  float mx = kNegInf;
+  if constexpr (VEC == 4) {
+    float beyond[INLDS != 0 ? INLDS : 1][4];
 #pragma unroll
-  for (int j = 0; j < SLABS; ++j) {
-    const int c0 = (j * W + wave) * kChunk;
-    const float *at = in + c0;  // uniform
-    if (c0 + kChunk <= cols) {
-      if (VEC == 4) {
-        const F4 q = StreamLoadF4Anywhere(at + lane_col);
-        v[j][0] = q.x; v[j][1 % VEC] = q.y; v[j][2 % VEC] = q.z; v[j][3 % VEC] = q.w;
-      } else {
+    for (int j = 0; j < SLABS; ++j) {
+      float (&t)[4] = j < REGS ? terms.v[j < REGS ? j : 0] : beyond[j < REGS ? 0 : j - REGS];
+      LoadPackOfRow(t, in, (j * W + wave) * kChunk, cols);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) v[j][i] = at[lane_col + i];
+    for (int j = 0; j < SLABS; ++j) {
+      const int c0 = (j * W + wave) * kChunk;
+      float (&t)[4] = j < REGS ? terms.v[j < REGS ? j : 0] : beyond[j < REGS ? 0 : j - REGS];
+      if (c0 + kChunk > cols) PlacePackOfRow(t, c0, cols, kAbsent);
+      if (j < REGS) continue;
+      terms.Set(t, j);
+      if (!TERMS_GIVEN) mx = MaxNum3(MaxNum3(mx, t[0], t[1]), t[2], t[3]);  // looked at while at hand
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < SLABS; ++j) {
+      const int c0 = (j * W + wave) * kChunk;
+      float t[VEC];
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        t[i] = kAbsent;
+        if (c0 + kChunk <= cols || c0 + static_cast<int>(lane_col) + i < cols) t[i] = in[c0 + lane_col + i];
       }
-    } else {
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) v[j][i] = kAbsent;
-      if (VEC == 4) {  // whole packs as packs, the one the row ends in element by element
-        if (c0 + static_cast<int>(lane_col) + VEC <= cols) {
-          const F4 q = StreamLoadF4Anywhere(at + lane_col);
-          v[j][0] = q.x; v[j][1 % VEC] = q.y; v[j][2 % VEC] = q.z; v[j][3 % VEC] = q.w;
-        } else {
-#pragma unroll
-          for (int i = 0; i < VEC; ++i) {
-            if (c0 + static_cast<int>(lane_col) + i < cols) v[j][i] = at[lane_col + i];
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-          if (c0 + static_cast<int>(lane_col) + i < cols) v[j][i] = at[lane_col + i];
-        }
-      }
+      terms.Set(t, j);
     }
   }
   if (!TERMS_GIVEN) {
-    float mx = kNegInf;
 #pragma unroll
-    for (int j = 0; j < SLABS; ++j) {
+    for (int j = 0; j < REGS; ++j) {
+      const float (&t)[VEC] = terms.v[j];
       if (VEC == 4) {
-        mx = MaxNum3(mx, v[j][0], v[j][1 % VEC]);
-        mx = MaxNum3(mx, v[j][2 % VEC], v[j][3 % VEC]);
+        mx = MaxNum3(mx, t[0], t[1 % VEC]);
+        mx = MaxNum3(mx, t[2 % VEC], t[3 % VEC]);
       } else {
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) mx = MaxNum(mx, v[j][i]);
+        for (int i = 0; i < VEC; ++i) mx = MaxNum(mx, t[i]);
       }
     }
     MSHADOW_ROWSUM_STAMP(11)
     mx = BlockMax<THREADS>(mx, lds.wmax);
     MSHADOW_ROWSUM_STAMP(12)
 #pragma unroll
-    for (int j = 0; j < SLABS; ++j) {
+    for (int j = 0; j < REGS; ++j) {
+      float (&v)[REGS][VEC] = terms.v;
 #pragma unroll
       for (int i = 0; i < VEC; ++i) v[j][i] = ExpNonPositive(v[j][i] - mx);
       /* one slab at a time: scheduled freely, the sixty-four independent chains would all
          be in flight at once and spill. The empty statement consumes this slab's results
          and hands out the next slab's inputs, so neither side can move across it. */
-      if (j + 1 < SLABS) {
+      if (j + 1 < REGS) {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) asm volatile("" : "+v"(v[j + 1][i]) : "v"(v[j][i]));
       }
     }
+#pragma unroll
+    for (int j = REGS; j < SLABS; ++j) {
+      float t[VEC];
+      terms.Get(t, j);
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) t[i] = ExpNonPositive(t[i] - mx);
+      terms.Set(t, j);
+    }
     MSHADOW_ROWSUM_STAMP(13)
   }
 
-  const float s = RowOrderedSum<THREADS, SLABS, VEC, TERMS_GIVEN, !TERMS_GIVEN>(v, cols, &lds);
+  const float s = RowOrderedSum<TERMS_GIVEN, !TERMS_GIVEN>(terms, &lds);
   if (TERMS_GIVEN) {
     if (threadIdx.x == 0) dst[blockIdx.x] = s;
     return;
@@ -784,13 +857,20 @@ __global__ void __launch_bounds__(THREADS, MIN_WAVES)  // 4 waves per SIMD: two 
 
   /* s >= 1 for finite logits (the maximum contributes exp(0)); anything else (NaN or
      infinite logits) takes the plain division so that specials propagate as on the CPU */
+  /* which packs lie inside the row is worked out again: kept from the loads, the answers are a pair of
+     scalar registers per slab, more than there are */
+  int left = cols;
+  asm volatile("" : "+s"(left));
   const bool fast_div = s >= 1.0f && s < 3.0e38f;
   const float rcp = 1.0f / s;
   if (!fast_div) {
 #pragma unroll
     for (int j = 0; j < SLABS; ++j) {
+      float t[VEC];
+      terms.Get(t, j);
 #pragma unroll
-      for (int i = 0; i < VEC; ++i) v[j][i] = v[j][i] / s;
+      for (int i = 0; i < VEC; ++i) t[i] = t[i] / s;
+      terms.Set(t, j);
     }
   }
 #pragma unroll
@@ -798,23 +878,24 @@ __global__ void __launch_bounds__(THREADS, MIN_WAVES)  // 4 waves per SIMD: two 
     const int c0 = (j * W + wave) * kChunk;
     float *at = out + c0;
     float o[VEC];
+    terms.Get(o, j);
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) o[i] = fast_div ? DivideBy(v[j][i], s, rcp) : v[j][i];
+    for (int i = 0; i < VEC; ++i) o[i] = fast_div ? DivideBy(o[i], s, rcp) : o[i];
     if (VEC == 4) {
       F4 q;
       q.x = o[0]; q.y = o[1 % VEC]; q.z = o[2 % VEC]; q.w = o[3 % VEC];
-      if (c0 + kChunk <= cols || c0 + static_cast<int>(lane_col) + VEC <= cols) {
+      if (c0 + kChunk <= left || c0 + static_cast<int>(lane_col) + VEC <= left) {
         StreamStoreF4Anywhere(at + lane_col, q);
       } else {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) {
-          if (c0 + static_cast<int>(lane_col) + i < cols) at[lane_col + i] = o[i];
+          if (c0 + static_cast<int>(lane_col) + i < left) at[lane_col + i] = o[i];
         }
       }
     } else {
 #pragma unroll
       for (int i = 0; i < VEC; ++i) {
-        if (c0 + static_cast<int>(lane_col) + i < cols) at[lane_col + i] = o[i];
+        if (c0 + static_cast<int>(lane_col) + i < left) at[lane_col + i] = o[i];
       }
     }
   }
@@ -823,8 +904,9 @@ __global__ void __launch_bounds__(THREADS, MIN_WAVES)  // 4 waves per SIMD: two 
 
 /*! \brief SLABS packs per thread of the stretch of a row that begins at `in` and has `left`
  *  columns to the end of the row, in the layout of SoftmaxRowKernel (slab j of wave w holds
- *  the 256 columns from (j * W + w) * 256): 16-byte accesses wherever the stretch starts, the
- *  pack the row ends in element by element, `absent` behind the end */
+ *  the 256 columns from (j * W + w) * 256): 16-byte accesses wherever the stretch starts, none of them
+ *  in a branch (all are in flight together), `absent` behind the end. The pack that the row ends in is
+ *  fetched element by element: another thread may have written the columns next to it already. */
 template <int THREADS, int SLABS>
 __device__ __forceinline__ void LoadStretch(float (&v)[SLABS][4], const float *in, int left, float absent) {
   const int W = THREADS / kWave;
@@ -832,15 +914,18 @@ __device__ __forceinline__ void LoadStretch(float (&v)[SLABS][4], const float *i
   const int lane_col = LaneId() * 4;
 #pragma unroll
   for (int j = 0; j < SLABS; ++j) {
-    const int c0 = (j * W + wave) * 256;  // uniform
-    const float *at = in + c0 + lane_col;
-    if (c0 + 256 <= left || c0 + lane_col + 4 <= left) {
-      const F4 q = StreamLoadF4Anywhere(at);
-      v[j][0] = q.x; v[j][1] = q.y; v[j][2] = q.z; v[j][3] = q.w;
-    } else {
+    const int c = (j * W + wave) * 256 + lane_col;
+    /* behind the end: what lies in front of it in the row (there is a stretch or more), not used */
+    const F4 q = StreamLoadF4Anywhere(in + (c < left - 4 ? c : left - 4));
+    v[j][0] = q.x; v[j][1] = q.y; v[j][2] = q.z; v[j][3] = q.w;
+  }
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[j][i] = (c0 + lane_col + i < left) ? at[i] : absent;
-    }
+  for (int j = 0; j < SLABS; ++j) {
+    const int c0 = (j * W + wave) * 256;  // uniform
+    if (c0 + 256 <= left || c0 + lane_col + 4 <= left) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[j][i] = (c0 + lane_col + i < left) ? in[c0 + lane_col + i] : absent;
   }
 }
 
@@ -861,6 +946,7 @@ template <int THREADS, int SLABS, bool TERMS_GIVEN, int MIN_WAVES>
 __global__ void __launch_bounds__(THREADS, MIN_WAVES)
     SoftmaxStretchRowKernel(float *dst, int dstride, const float *src, int sstride, int cols) {
   __shared__ RowSumLds<THREADS / kWave, SLABS, 4> lds;
+  typedef RowTerms<THREADS, SLABS, 0, 4> Terms;
   const int W = THREADS / kWave;
   const int kStretch = THREADS * SLABS * 4;
   const int wave = __builtin_amdgcn_readfirstlane(WaveId());
@@ -868,7 +954,8 @@ __global__ void __launch_bounds__(THREADS, MIN_WAVES)
   const float *in = src + static_cast<size_t>(blockIdx.x) * sstride;
   float *out = dst + static_cast<size_t>(blockIdx.x) * dstride;
   const float kNegInf = -__builtin_huge_valf();
-  float v[SLABS][4];
+  Terms terms;
+  float (&v)[SLABS][4] = terms.v;
   float mx = kNegInf;
   if (!TERMS_GIVEN) {
     for (int t0 = 0; t0 < cols; t0 += kStretch) {
@@ -896,7 +983,7 @@ __global__ void __launch_bounds__(THREADS, MIN_WAVES)
       }
     }
     __syncthreads();  // everybody has read the sum the stretch in front left in LDS
-    s = RowOrderedSum<THREADS, SLABS, 4, TERMS_GIVEN, !TERMS_GIVEN>(v, cols - t0, &lds, s);
+    s = RowOrderedSum<TERMS_GIVEN, !TERMS_GIVEN>(terms, &lds, s);
   }
   if (TERMS_GIVEN) {
     if (threadIdx.x == 0) dst[blockIdx.x] = s;
