@@ -11,6 +11,7 @@
 
 #include <mshadow/hip/kernels/reduce.h>
 #include <mshadow/hip/kernels/reduce_dma.h>
+#include <mshadow/hip/kernels/reduce_segments.h>
 
 #include "patch_kernels.h"
 #include "pool_kernels.h"
@@ -956,6 +957,8 @@ int mshadow_hip_reduce_keep_highdim_f32(float *dst, const float *src, int sstrid
     v_x = v_stride = y * x;
     v_y = 1;
   }
+  const mshadow::hip::SegmentsPlan seg =
+      mshadow::hip::PlanSegments(n, c, static_cast<uint64_t>(y) * x, mshadow_abi::ComputeUnits(), 4);
   uint32_t *split_partial = NULL, *split_counter = NULL;
   /* With a kept index for (nearly) every CU the one-workgroup-per-kept-index kernel fills the
      chip and ends without a merge; with fewer the inner chains are dealt out by segments:
@@ -963,7 +966,7 @@ int mshadow_hip_reduce_keep_highdim_f32(float *dst, const float *src, int sstrid
      32 per workgroup and 256 bytes of each. */
   const bool few_kept = static_cast<long long>(c) * 4 < 3ll * mshadow_abi::ComputeUnits();
   const bool whole_packs = v_x % 4 == 0 && v_stride % 4 == 0 && Aligned16(src);
-  if (few_kept && static_cast<long long>(n) * y * x >= kDmaMinPerKept &&
+  if (few_kept && !(seg.use && sstride == x) && static_cast<long long>(n) * y * x >= kDmaMinPerKept &&
       static_cast<long long>(n) * c < (1ll << 31)) {
     const int sc = mshadow_hip_reduce_scratch(stream, static_cast<size_t>(n) * c, &split_partial,
                                               &split_counter);
@@ -992,6 +995,18 @@ int mshadow_hip_reduce_keep_highdim_f32(float *dst, const float *src, int sstrid
                        static_cast<uint32_t>(c), static_cast<uint32_t>(y),                     \
                        static_cast<uint32_t>(x), div_x, scale);                                \
   else HIGHDIM_LAUNCH_T(mshadow::hip::kRedBlockSmall, SEGS)
+      if (seg.use && sstride == x) {  // dense planes: waves with sixteen of them each
+#define SEGMENTS(L)                                                                                          \
+  LaunchKernelIfFits((mshadow::hip::ReduceSegmentsKernel<S, R, float, L>),                                   \
+                     dim3((static_cast<uint32_t>(c) + seg.kept - 1) / seg.kept), dim3(seg.waves * 64),          \
+                     (mshadow::hip::SegSlice<float, L>::LdsBytes(seg.waves, seg.kept * n)), s, dst, src,       \
+                     static_cast<uint32_t>(y * x), static_cast<uint32_t>(n), static_cast<uint32_t>(c), seg.kept, \
+                     mshadow::FastDivU32(seg.kept), scale)
+        if (seg.lanes == 8) SEGMENTS(8);
+        else SEGMENTS(16);
+#undef SEGMENTS
+        return MSHADOW_HIP_OK;
+      }
       const bool large = static_cast<long long>(n) * y * x >= kDmaMinPerKept;
       if (large && split_partial != NULL) {
 #define HIGHDIM_SPLIT(RING)                                                                    \

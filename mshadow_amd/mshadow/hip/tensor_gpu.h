@@ -27,6 +27,7 @@
 #include "./kernels/pool_half.h"
 #include "./kernels/reduce.h"
 #include "./kernels/reduce_dma.h"
+#include "./kernels/reduce_segments.h"
 #include "./kernels/rows_by_index.h"
 #include "./kernels/softmax_any.h"
 #include "./kernels/softmax_half.h"
@@ -180,10 +181,10 @@ inline bool AnyPackable(const DType *a, uint32_t astride, const DType *b, uint32
 namespace gpu_detail {
 #if defined(__HIPCC__)
 template <typename K>
-inline void Launch(K kernel, uint32_t grid_x, uint32_t block_x, void **args, void *stream) {
+inline void Launch(K kernel, uint32_t grid_x, uint32_t block_x, void **args, void *stream, size_t lds = 0) {
   const uint32_t grid[3] = {grid_x, 1, 1};
   const uint32_t block[3] = {block_x, 1, 1};
-  MSHADOW_HIP_CALL(mshadow_hip_launch(reinterpret_cast<const void *>(kernel), grid, block, args, 0,
+  MSHADOW_HIP_CALL(mshadow_hip_launch(reinterpret_cast<const void *>(kernel), grid, block, args, lds,
                                       stream));
 }
 
@@ -1304,6 +1305,24 @@ struct HalfRingRoute<Saver, Reducer, Tensor<gpu, 1, half::half_t>, Tensor<gpu, d
                       uint32_t n_out, uint32_t n_keep, uint32_t n_y, uint32_t n_x,
                       half::half_t scale) {
     const uint64_t per_kept = static_cast<uint64_t>(n_out) * n_y * n_x;
+    const hip::SegmentsPlan plan = hip::PlanSegments(n_out, n_keep, static_cast<uint64_t>(n_y) * n_x, hip::kChipCus, 8);
+    if (plan.use && src.stride_ == n_x) {  // dense planes: waves with sixteen of them each
+      half::half_t *d = dst.dptr_;
+      const half::half_t *s = src.dptr_;
+      uint32_t len = n_y * n_x, kept = plan.kept;
+      FastDivU32 div_kept(kept);
+      void *args[] = {&d, &s, &len, &n_out, &n_keep, &kept, &div_kept, &scale};
+      void *stream = Stream<gpu>::GetStream(dst.stream_);
+      const uint32_t grid = (n_keep + kept - 1) / kept, threads = plan.waves * 64;
+      if (plan.lanes == 8) {
+        Launch(hip::ReduceSegmentsKernel<Saver, Reducer, half::half_t, 8>, grid, threads, args, stream,
+               hip::SegSlice<half::half_t, 8>::LdsBytes(plan.waves, kept * n_out));
+      } else {
+        Launch(hip::ReduceSegmentsKernel<Saver, Reducer, half::half_t, 16>, grid, threads, args, stream,
+               hip::SegSlice<half::half_t, 16>::LdsBytes(plan.waves, kept * n_out));
+      }
+      return true;
+    }
     if (per_kept < (1u << 16) || static_cast<uint64_t>(n_y) * n_x >= (1ull << 31)) return false;
     half::half_t *d = dst.dptr_;
     const half::half_t *s = src.dptr_;
