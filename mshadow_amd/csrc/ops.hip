@@ -460,9 +460,12 @@ bool LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, 
 #define SHORT_THREAD(CMAX) \
   LaunchKernelIfFits((SoftmaxThreadRowKernel<CMAX, TERMS_GIVEN>), dim3((rows + 255) / 256), dim3(256), 0, s, \
                      dst, dstride, src, sstride, rows, cols)
-#define SHORT_PART(LANES, N) \
-  LaunchKernelIfFits((SoftmaxPartWaveKernel<LANES, N, TERMS_GIVEN>), dim3((rows + 256 / LANES - 1) / (256 / LANES)), \
+  /* rows that neither start nor end with a pack share cache lines with their neighbours */
+  const bool whole = cols % 4 == 0 && dstride % 4 == 0 && sstride % 4 == 0 && Aligned16(dst) && Aligned16(src);
+#define SHORT_PART_AS(LANES, N, WHOLE) \
+  LaunchKernelIfFits((SoftmaxPartWaveKernel<LANES, N, TERMS_GIVEN, WHOLE>), dim3((rows + 256 / LANES - 1) / (256 / LANES)), \
                      dim3(256), 0, s, dst, dstride, src, sstride, rows, cols)
+#define SHORT_PART(LANES, N) do { if (whole) SHORT_PART_AS(LANES, N, true); else SHORT_PART_AS(LANES, N, false); } while (0)
 #define WAVE_SLABS(SLABS) \
   LaunchKernelIfFits((SoftmaxWaveSlabsKernel<SLABS, TERMS_GIVEN>), dim3((rows + 3) / 4), dim3(256), 0, s, dst, \
                      dstride, src, sstride, rows, cols)
@@ -490,6 +493,7 @@ bool LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, 
   else WAVE_SLABS(TERMS_GIVEN ? 12 : 10);
 #undef SHORT_THREAD
 #undef SHORT_PART
+#undef SHORT_PART_AS
 #undef WAVE_SLABS
   return true;
 }

@@ -1111,8 +1111,10 @@ __device__ inline float PartWaveResolve(float s, const float (&t)[N]) {
  *  row's group holds the N consecutive columns from l * N. The wave-wide steps of a row - the
  *  maximum, the scans of the ordered sum - cost the same instructions whether a wave holds one
  *  short row or four, and rows of up to 256 columns by the hundred thousand are bound by
- *  exactly those. 256 / LANES rows per workgroup, nothing shared between them, no barrier. */
-template <int LANES, int N, bool TERMS_GIVEN>
+ *  exactly those. 256 / LANES rows per workgroup, nothing shared between them, no barrier.
+ *  WHOLE: rows are whole aligned packs, which stream; else ordinary accesses, because neighbouring rows'
+ *  accesses meet in the cache lines that they share (131072 x 127: 45 -> 33 us). */
+template <int LANES, int N, bool TERMS_GIVEN, bool WHOLE>
 __global__ void __launch_bounds__(256)
     SoftmaxPartWaveKernel(float *dst, int dstride, const float *src, int sstride, int rows, int cols) {
   const int row = blockIdx.x * (256 / LANES) + static_cast<int>(threadIdx.x) / LANES;
@@ -1127,7 +1129,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int p = 0; p < N; p += 4) {
     if (base + p + 4 <= cols) {
-      const F4 q = StreamLoadF4Anywhere(in + base + p);
+      const F4 q = WHOLE ? StreamLoadF4Anywhere(in + base + p) : *reinterpret_cast<const F4Loose *>(in + base + p);
       v[p] = q.x; v[p + 1] = q.y; v[p + 2] = q.z; v[p + 3] = q.w;
     } else {
 #pragma unroll
@@ -1175,7 +1177,8 @@ __global__ void __launch_bounds__(256)
     if (base + p + 4 <= cols) {
       F4 q;
       q.x = o[0]; q.y = o[1]; q.z = o[2]; q.w = o[3];
-      StreamStoreF4Anywhere(out + base + p, q);
+      if (WHOLE) StreamStoreF4Anywhere(out + base + p, q);
+      else *reinterpret_cast<F4Loose *>(out + base + p) = q;
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
