@@ -1355,14 +1355,25 @@ int mshadow_hip_unpool_f32(float *dst, int dstride, const float *src, int sstrid
     return AfterLaunch("unpool");
   }
   /* 2 x 2 windows, stride 2: a pixel has one window at most; four pixels and two windows per thread */
-  if (ky == 2 && kx == 2 && sy == 2 && sx == 2 && w >= 4) {
+  if (ky == 2 && kx == 2 && sy == 2 && sx == 2 && w >= 4 && ph >= 1 && pw >= 1 &&
+      static_cast<long long>(planes) * ph * pw >= 2) {
     const long long wpk = (w + 3) / 4;
     const long long packs = static_cast<long long>(planes) * h * wpk;
     if (packs + kPoolBlock < (1ll << 31)) {
       const unsigned blocks = static_cast<unsigned>((packs + kPoolBlock - 1) / kPoolBlock);
-      POOL_SWITCH(Unpool2x2s2Kernel, dim3(blocks), dim3(kPoolBlock), 0, s, dst, dstride, src, sstride,
-                  pooled, pstride, grad, gstride, g, mshadow::FastDivU32(static_cast<uint32_t>(wpk)),
-                  mshadow::FastDivU32(static_cast<uint32_t>(h)), static_cast<uint32_t>(packs))
+#define UNPOOL_2X2(R, WHOLE)                                                                                        \
+  LaunchKernelIfFits((Unpool2x2s2Kernel<R, WHOLE>), dim3(blocks), dim3(kPoolBlock), 0, s, dst, dstride, src, sstride, \
+                     pooled, pstride, grad, gstride, g, mshadow::FastDivU32(static_cast<uint32_t>(wpk)),            \
+                     mshadow::FastDivU32(static_cast<uint32_t>(h)), static_cast<uint32_t>(packs),                   \
+                     (static_cast<size_t>(planes) * h - 1) * sstride + w,                                           \
+                     (static_cast<size_t>(planes) * ph - 1) * pstride + pw,                                         \
+                     (static_cast<size_t>(planes) * ph - 1) * gstride + pw)
+#define UNPOOL_2X2_OF(R) do { if (w % 4 == 0) UNPOOL_2X2(R, true); else UNPOOL_2X2(R, false); } while (0)
+      if (reducer == MSHADOW_HIP_SUM) UNPOOL_2X2_OF(MSHADOW_HIP_SUM);
+      else if (reducer == MSHADOW_HIP_MAX) UNPOOL_2X2_OF(MSHADOW_HIP_MAX);
+      else UNPOOL_2X2_OF(MSHADOW_HIP_MIN);
+#undef UNPOOL_2X2_OF
+#undef UNPOOL_2X2
       return AfterLaunch("unpool");
     }
   }

@@ -84,12 +84,15 @@ __device__ __forceinline__ void StageRows(float *lds, int lpitch, const float *g
     const int total = nrows * width;
     const int lead = (4 - LdsPhase(g)) & 3;
     const int head = lead < total ? lead : total;
-    if (static_cast<int>(threadIdx.x) < head) {
-      const float v = g[threadIdx.x];
-      lds[threadIdx.x] = v;
-      if (WATCH) seen |= IsNegZero(v);
-    }
     const int nvec = (total - head) / 4;
+    const int tail = head + 4 * nvec + static_cast<int>(threadIdx.x);
+    /* what lies in front of the first pack and behind the last one is requested with the packs, not waited
+       for in front of them and again behind them */
+    float first = 0.0f, last = 0.0f;
+    if (threadIdx.x < 4u) {
+      if (static_cast<int>(threadIdx.x) < head) first = g[threadIdx.x];
+      if (tail < total) last = g[tail];
+    }
     const float *gv = g + head;
     F4 *lv = reinterpret_cast<F4 *>(lds + head);
     const int kUnroll = 8;
@@ -107,11 +110,10 @@ __device__ __forceinline__ void StageRows(float *lds, int lpitch, const float *g
         if (WATCH) seen |= IsNegZero(q[u].x) | IsNegZero(q[u].y) | IsNegZero(q[u].z) | IsNegZero(q[u].w);
       }
     }
-    const int tail = head + 4 * nvec + threadIdx.x;
-    if (tail < total) {
-      const float v = g[tail];
-      lds[tail] = v;
-      if (WATCH) seen |= IsNegZero(v);
+    if (threadIdx.x < 4u) {
+      if (static_cast<int>(threadIdx.x) < head) lds[threadIdx.x] = first;
+      if (tail < total) lds[tail] = last;
+      if (WATCH) seen |= IsNegZero(first) | IsNegZero(last);
     }
   } else {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -496,6 +498,9 @@ __global__ void __launch_bounds__(kPoolBlock)
   StreamStoreF4Anywhere(dst + static_cast<size_t>(r) * dstride + x0, out);
 }
 
+template <bool STREAM>
+__device__ __forceinline__ F4 LoadPackFree(const float *base, const float *p, const float *end, bool ok);
+
 /*! \brief two floats fetched as one 8-byte access at any 4-byte boundary */
 typedef F2 F2Loose __attribute__((aligned(4)));
 
@@ -503,12 +508,14 @@ typedef F2 F2Loose __attribute__((aligned(4)));
  *  pixel has at most one - with no staging: a thread takes four neighbouring source pixels of
  *  one row (one 16-byte access each way, any alignment), which lie under two neighbouring windows of one pooled row, and fetches the
  *  pooled values and gradients of those two as one 8-byte access each. The single term is
- *  added to zero as the reference's loop does (mshadow/extension/spatial_unpool.h:102-125). */
-template <int REDUCER>
+ *  added to zero as the reference's loop does (mshadow/extension/spatial_unpool.h:102-125).
+ *  WHOLE: rows of whole packs, wherever they begin. */
+template <int REDUCER, bool WHOLE>
 __global__ void __launch_bounds__(kPoolBlock)
     Unpool2x2s2Kernel(float *dst, int dstride, const float *src, int sstride, const float *pooled,
                       int pstride, const float *grad, int gstride, PoolGeom g,
-                      mshadow::FastDivU32 div_wpk, mshadow::FastDivU32 div_h, uint32_t total_packs) {
+                      mshadow::FastDivU32 div_wpk, mshadow::FastDivU32 div_h, uint32_t total_packs,
+                      size_t src_floats, size_t pooled_floats, size_t grad_floats) {
   typedef PoolOp<REDUCER> Op;
   const uint32_t pk = blockIdx.x * kPoolBlock + threadIdx.x;
   if (pk >= total_packs) return;
@@ -516,34 +523,25 @@ __global__ void __launch_bounds__(kPoolBlock)
   int x0 = static_cast<int>(pk - r * div_wpk.div) * 4;
   /* the last pack of a row of even width is moved back to end with the row (it still starts a
      window); of an odd width it is partial */
-  if (x0 + 4 > g.w && (g.w & 1) == 0) x0 = g.w - 4;
+  if (!WHOLE && x0 + 4 > g.w && (g.w & 1) == 0) x0 = g.w - 4;
   const uint32_t plane = div_h.Div(r);
   const int y = static_cast<int>(r - plane * g.h);
   const int py = y >> 1, px = x0 >> 1;
   const float *in = src + static_cast<size_t>(r) * sstride + x0;
   float *out = dst + static_cast<size_t>(r) * dstride + x0;
-  const int live = min(4, g.w - x0);                 // 4, or 3 when the width is odd
-  float vs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (live == 4) {
-    const F4 q = StreamLoadF4Anywhere(in);
-    vs[0] = q.x; vs[1] = q.y; vs[2] = q.z; vs[3] = q.w;
-  } else {
-    for (int e = 0; e < live; ++e) vs[e] = in[e];
-  }
-  float pv[2] = {0.0f, 0.0f}, gv[2] = {0.0f, 0.0f};
+  const int live = WHOLE ? 4 : min(4, g.w - x0);     // 4, or 3 when the width is odd
+  /* all loads outside any branch, none waits for another ((64,96,55,55) 50 -> 39 us, (256,128,27,27) 68 -> 56). A window that
+     does not exist reads one that does and is not counted; the last float of an array has nothing behind
+     it and comes as the second of the pair before it */
   const bool row_ok = py < g.ph;
-  if (row_ok) {
-    const float *prow = pooled + (static_cast<size_t>(plane) * g.ph + py) * pstride + px;
-    const float *grow = grad + (static_cast<size_t>(plane) * g.ph + py) * gstride + px;
-    if (px + 2 <= g.pw) {
-      const F2 a = *reinterpret_cast<const F2Loose *>(prow);
-      const F2 b = *reinterpret_cast<const F2Loose *>(grow);
-      pv[0] = a.x; pv[1] = a.y; gv[0] = b.x; gv[1] = b.y;
-    } else if (px < g.pw) {
-      pv[0] = prow[0];
-      gv[0] = grow[0];
-    }
-  }
+  const int pxc = px < g.pw ? px : 0;
+  const size_t prow = static_cast<size_t>(plane) * g.ph + (row_ok ? py : 0);
+  const size_t poff = prow * pstride + pxc, goff = prow * gstride + pxc;
+  const bool ptail = poff + 2 > pooled_floats, gtail = goff + 2 > grad_floats;
+  const F2 pp = *reinterpret_cast<const F2Loose *>(pooled + poff - (ptail ? 1 : 0));
+  const F2 gg = *reinterpret_cast<const F2Loose *>(grad + goff - (gtail ? 1 : 0));
+  const F4 vs = WHOLE ? StreamLoadF4Anywhere(in) : LoadPackFree<true>(src, in, src + src_floats, true);
+  const float pv[2] = {ptail ? pp.y : pp.x, pp.y}, gv[2] = {gtail ? gg.y : gg.x, gg.y};
   float o[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -752,7 +750,6 @@ struct UnpoolRowsGeom {
   mshadow::FastDivU32 div_groups, div_half_h;
 };
 
-__device__ __forceinline__ F4 LoadPackFree(const float *base, const float *p, const float *end, bool ok);
 
 /*! \brief unpool for a 3 x 3 window with stride 2 on rows of up to 256 pixels, with no staging:
  *  a thread owns two adjacent 2 x 2 blocks of source pixels - four pixels of row 2a and the four
@@ -763,7 +760,9 @@ __device__ __forceinline__ F4 LoadPackFree(const float *base, const float *p, co
  *  outside any branch and is issued before the first value is used, so a thread waits for memory
  *  once ((64,96,55,55): 52 -> 48 us; with loads inside the branches of the two cases the
  *  compiler waits for all loads under way at each). What this form still pays against the other
- *  (33 us on 56 x 56) are 16-byte accesses at 4-byte borders. The windows that can cover them
+ *  (33 us on 56 x 56) are 16-byte accesses at 4-byte borders; they are ordinary, not streaming ones, because
+ *  the cache lines that two rows, or two waves, have a part of each must wait in L2 for one another ((64,96,55,55)
+ *  51 -> 43 us, (256,128,27,27) 108 -> 66, 113 x 113 146 -> 139). The windows that can cover them
  *  are rows a - 1 and a of the pooled grid, columns 2t - 1, 2t, 2t + 1: the thread fetches
  *  columns 2t and 2t + 1 of both rows (pooled value and gradient) and takes column 2t - 1
  *  from the neighbouring lane, which fetched it as its own 2t' + 1 (a wave takes whole rows).
@@ -792,8 +791,8 @@ __global__ void __launch_bounds__(kPoolBlock)
     top = StreamLoadF4(in), bottom = StreamLoadF4(in + sstride);
   } else {
     const float *send = src + rg.src_floats;
-    top = LoadPackFree(src, in, send, true);
-    bottom = LoadPackFree(src, in + sstride, send, has_bottom);
+    top = LoadPackFree<false>(src, in, send, true);
+    bottom = LoadPackFree<false>(src, in + sstride, send, has_bottom);
   }
   /* [jy][c]: pooled row a - jy, column 2t - 1 + c */
   float pv[2][3], gv[2][3];
@@ -893,15 +892,15 @@ __global__ void __launch_bounds__(kPoolBlock)
     StreamStoreF4(out + dstride, q);
   } else if (live_px == 4) {
     q.x = otop[0], q.y = otop[1], q.z = otop[2], q.w = otop[3];
-    StreamStoreF4Anywhere(out, q);
+    *reinterpret_cast<F4Loose *>(out) = q;
     q.x = obot[0], q.y = obot[1], q.z = obot[2], q.w = obot[3];
-    if (has_bottom) StreamStoreF4Anywhere(out + dstride, q);
+    if (has_bottom) *reinterpret_cast<F4Loose *>(out + dstride) = q;
   } else {
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       if (i < live_px) {
-        StreamStore(out + i, otop[i]);
-        if (has_bottom) StreamStore(out + dstride + i, obot[i]);
+        out[i] = otop[i];
+        if (has_bottom) out[dstride + i] = obot[i];
       }
     }
   }
@@ -923,11 +922,12 @@ struct SlideGeom {
  *  reach past the tensor's end (`end`: one past its last float): it is fetched from end - 4 and
  *  its elements are moved into place, zeros behind them. Floats past the end of a ROW are the
  *  next row's and are the caller's to ignore or mask. */
+template <bool STREAM>
 __device__ __forceinline__ F4 LoadPackFree(const float *base, const float *p, const float *end, bool ok) {
   const float *last = end - 4;
   const bool moved = ok && p > last;
   const float *at = ok ? (moved ? last : p) : base;
-  F4 q = StreamLoadF4Anywhere(at);
+  F4 q = STREAM ? StreamLoadF4Anywhere(at) : *reinterpret_cast<const F4Loose *>(at);
   if (__any(moved)) {  // one wave of the grid at most
     const int sh = moved ? static_cast<int>(p - last) : 0;
     F4 b, c;
@@ -1023,8 +1023,8 @@ __global__ void __launch_bounds__(kPoolBlock)
   for (int k = K - 1; k >= 1; --k) {
     const int py = y0 - k;
     const bool ok = live && py >= 0 && py < g.ph;
-    const F4 pq = LoadPackFree(pbase, pbase + static_cast<ptrdiff_t>(py) * pstride + x0, pend, ok);
-    const F4 gq = KeepColumns(LoadPackFree(gbase, gbase + static_cast<ptrdiff_t>(py) * gstride + x0, gend, ok),
+    const F4 pq = LoadPackFree<true>(pbase, pbase + static_cast<ptrdiff_t>(py) * pstride + x0, pend, ok);
+    const F4 gq = KeepColumns(LoadPackFree<true>(gbase, gbase + static_cast<ptrdiff_t>(py) * gstride + x0, gend, ok),
                               x0, g.pw, ok);
     MSHADOW_SLIDE_PUT(K - k, pq, gq)
   }
@@ -1036,9 +1036,9 @@ __global__ void __launch_bounds__(kPoolBlock)
     const int y = y0 + u;
     okq[u] = live && u < rows && y < g.h;
     const bool pok = okq[u] && y < g.ph;
-    sq[u] = LoadPackFree(sbase, sbase + static_cast<size_t>(y) * sstride + x0, send, okq[u]);
-    pq[u] = LoadPackFree(pbase, pbase + static_cast<size_t>(y) * pstride + x0, pend, pok);
-    gq[u] = KeepColumns(LoadPackFree(gbase, gbase + static_cast<size_t>(y) * gstride + x0, gend, pok), x0, g.pw, pok);
+    sq[u] = LoadPackFree<true>(sbase, sbase + static_cast<size_t>(y) * sstride + x0, send, okq[u]);
+    pq[u] = LoadPackFree<true>(pbase, pbase + static_cast<size_t>(y) * pstride + x0, pend, pok);
+    gq[u] = KeepColumns(LoadPackFree<true>(gbase, gbase + static_cast<size_t>(y) * gstride + x0, gend, pok), x0, g.pw, pok);
   }
   for (int r0 = 0; r0 < rows; r0 += DEPTH) {
 #pragma unroll
@@ -1052,9 +1052,9 @@ __global__ void __launch_bounds__(kPoolBlock)
       const int yn = y + DEPTH;
       okq[u] = live && r + DEPTH < rows && yn < g.h;
       const bool pok = okq[u] && yn < g.ph;
-      sq[u] = LoadPackFree(sbase, sbase + static_cast<size_t>(yn) * sstride + x0, send, okq[u]);
-      pq[u] = LoadPackFree(pbase, pbase + static_cast<size_t>(yn) * pstride + x0, pend, pok);
-      gq[u] = KeepColumns(LoadPackFree(gbase, gbase + static_cast<size_t>(yn) * gstride + x0, gend, pok), x0, g.pw, pok);
+      sq[u] = LoadPackFree<true>(sbase, sbase + static_cast<size_t>(yn) * sstride + x0, send, okq[u]);
+      pq[u] = LoadPackFree<true>(pbase, pbase + static_cast<size_t>(yn) * pstride + x0, pend, pok);
+      gq[u] = KeepColumns(LoadPackFree<true>(gbase, gbase + static_cast<size_t>(yn) * gstride + x0, gend, pok), x0, g.pw, pok);
       F4 out;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
