@@ -481,10 +481,10 @@ bool LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, 
   else if (cols <= 128) SHORT_PART(16, 8);
   else if (cols <= 256) SHORT_PART(32, 8);
   /* a wave per row for any number of rows of up to 512 columns, and for many of up to 2560 (65536
-     rows of 300 / 1000 columns: 47 / 93 us against 163 / 174 us with a workgroup per row, 16384 of
-     2304 68 against 75 us, 8000 of 2560 37.6 against 40.9; at 3000 columns 8000 rows 44.3 against 42.2,
-     40000 209 against 199). 100 rows of 500: 5.0 against 5.6 us; 1000 rows of 1000: 7.8 against 7.1 us,
-     3000 rows 9.7 against 12.7; 2000 rows of 2000 13.1 against 11.9, 3000 rows 14.6 against 16.1.
+     rows of 300 / 1000 columns: 43 / 90 us against 163 / 174 us with a workgroup per row, 16384 of
+     2304 56 against 75 us, 8000 of 2560 33.8 against 40.9; at 3000 columns, before its loads were all under
+     way together, 8000 rows 44.3 against 42.2). 100 rows of 500: 5.0 against 5.6 us; 1000 rows of 1000: 7.8
+     against 7.1 us, 3000 rows 9.7 against 12.7; 2000 rows of 2000 13.1 against 11.9, 3000 rows 14.6 against 16.1.
      (The row sums alone are as they were measured before: up to 3072 columns, from 6 rows a CU on.) */
   else if (cols <= 512) WAVE_SLABS(2);
   else if (cols > (TERMS_GIVEN ? 3072 : 2560) || rows < (cols > 1024 && !TERMS_GIVEN ? 10 : 6) * cus) return false;
