@@ -1032,6 +1032,10 @@ __global__ void __launch_bounds__(256)
                            int cols) {
   const int row = blockIdx.x * 256 + threadIdx.x;
   if (row >= rows) return;
+  if (TERMS_GIVEN && cols == 0) {  // the sum of no terms, of which there may be no memory either
+    dst[row] = 0.0f;
+    return;
+  }
   const float *in = src + static_cast<size_t>(row) * sstride;
   const float kNegInf = -__builtin_huge_valf();
   float v[CMAX];

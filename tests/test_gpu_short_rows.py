@@ -55,6 +55,16 @@ def test_row_sums(G, cols, kind):
         assert_bits_equal(got[~nan], want[~nan], f"{kind} {rows}x{cols}")
 
 
+@pytest.mark.parametrize("rows", [1, 255, 257, 5000])
+def test_row_sums_of_no_terms(G, rows):
+    """rows without a column sum to zero, and no term is read: there may be no tensor at all"""
+    x = G.to_device(np.full((rows, 4), 3.0, f32))
+    for terms_ptr, pitch in ((x.ptr, 4), (x.ptr, 0), (None, 0)):
+        sums = G.to_device(np.full(rows, 7.0, f32))
+        G.check(G.dll.mshadow_hip_softmax_rowsum_f32(sums.ptr, terms_ptr, pitch, rows, 0, None))
+        assert_bits_equal(sums.download(), np.zeros(rows, f32), f"{rows} rows, pitch {pitch}")
+
+
 @pytest.mark.parametrize("rows,cols", [(7, 10), (5000, 16), (9, 50), (4096, 64), (4097, 64), (33, 128), (5000, 101), (70, 200),
                                        (16385, 200), (3, 512), (1535, 513), (1536, 700), (2000, 2304), (2000, 3072)])
 def test_softmax_short_rows(G, O, rows, cols):
