@@ -14,11 +14,10 @@
 #include "../../core/fastdiv.h"
 #include "./common.h"
 #include "./reduce.h"
+#include "./segments_plan.h"
 
 namespace mshadow {
 namespace hip {
-
-const uint32_t kSegMostWaves = 16;
 
 template <typename DType, int LANES>
 struct SegSlice {
@@ -131,55 +130,6 @@ __global__ void __launch_bounds__(kSegMostWaves * kWave)
     for (uint32_t n = 0; n < n_out; ++n) Reducer::Reduce(sum, part[n * kept + threadIdx.x]);
     Saver::template Save<DType>(dst[c], sum * scale);
   }
-}
-
-/*! \brief how (n, c) planes of `len` elements are dealt out */
-struct SegmentsPlan {
-  bool use;        //!< false: the kernels of reduce_dma.h and reduce.h are the sooner ones
-  int lanes;       //!< planes of a wave
-  uint32_t kept, waves;  //!< kept indices and waves of a workgroup
-};
-/*! \brief Measured on (n, c, len), us, the other kernels and this one; floats, binary16 gains as much. It wants planes
- *  enough for a wave of sixteen on every SIMD or nearly, and wins by what the others leave idle.
- *  Few kept indices (workgroups that share out the planes otherwise, and merge in the last of them): short planes
- *  (200,100,400) 38 and 17, (213,58,312) 28 and 15, (60,190,1500) 30 and 21, but (160,40,2296) 27 and 45,
- *  (64,64,12544) 52 and 78. A workgroup per kept index that fills a CU: (248,552,280) 70 and 42, (30,600,2500) 74
- *  and 44, (19,304,5760) 93 and 35, (5,1144,8320) 115 and 49, where chain lanes (n up to the next 64, 16 or 4) and
- *  the last round of workgroups are idle for more than three tenths; (64,256,3136) 35.6 and 40, (64,512,1600) 43 and 41.
- *  A workgroup of four waves per kept index, for fewer than 65536 values of each: (17,896,260) 11.7 and 7.2,
- *  (39,957,384) 14.9 and 11.9, but (8,573,240) 5.1 and 6.3, (256,500,100) 19.8 and 22.3. One plane per kept index,
- *  which is one lane there: (1,2048,3136) 46 and 20. */
-inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, uint32_t cus, int least_len) {
-  SegmentsPlan p = {false, 16, 1, 1};
-  const uint64_t planes = static_cast<uint64_t>(n_out) * n_keep;
-  /* 32-bit numbers of planes, fewer than 2^32 threads */
-  if (len < static_cast<uint64_t>(least_len) || n_out < 1 || n_out > 2048 || n_keep > 1u << 21 || len >= 1ull << 31 ||
-      planes >= 1ull << 31) {
-    return p;
-  }
-  const bool few_kept = static_cast<uint64_t>(n_keep) * 4 < 3ull * cus;
-  const bool middling = n_out >= 5 && n_out <= 16;
-  const uint32_t side = n_out > 16 ? 64 : n_out > 4 ? 16 : n_out > 1 ? 4 : 1;
-  const uint64_t lanes = (n_out + side - 1) / side * side, turns = (n_keep + cus - 1) / cus * cus;
-  if (few_kept) {
-    p.use = !middling && ((len <= 1100 && planes >= 2048) || (len <= 2048 && planes >= 8192));
-  } else if (n_out == 1) {
-    p.use = n_keep >= 2 * cus && len <= 4096 && planes * len >= 800000;
-  } else if (n_out * len >= 1u << 16) {
-    p.use = planes >= 2048 && lanes * turns * 100 > planes * 130;
-  } else {
-    p.use = !middling && ((len <= 1100 && planes >= 2048) || planes >= 4096) && (n_out <= 4 || lanes * 100 > n_out * 102ull);
-  }
-  if (!p.use) return p;
-  if (len >= 512 && planes / 16 < 4 * cus) p.lanes = 8;  // more waves: (32,512,784) 12.4, with sixteen 13.3
-  /* workgroups of four waves or so where planes are few per kept index, but one for every CU */
-  while (p.kept * n_out < 4u * p.lanes && n_keep / (p.kept + 1) >= cus) ++p.kept;
-  const uint32_t all = (p.kept * n_out + p.lanes - 1) / p.lanes;
-  /* a CU holds 20 waves of this kernel: where there are more of them, small workgroups that go round again fill it */
-  const uint32_t most = planes / p.lanes >= 20ull * cus ? 4 : kSegMostWaves;
-  const uint32_t rounds = (all + most - 1) / most;
-  p.waves = (all + rounds - 1) / rounds;
-  return p;
 }
 
 }  // namespace hip

@@ -1,0 +1,103 @@
+/*
+ * Which sums over dense planes ReduceSegmentsKernel takes, and how it deals the planes out: plain C++, for the
+ * library, the expression headers and host code alike.
+ */
+#ifndef MSHADOW_HIP_KERNELS_SEGMENTS_PLAN_H_
+#define MSHADOW_HIP_KERNELS_SEGMENTS_PLAN_H_
+
+#include <stdint.h>
+
+namespace mshadow {
+namespace hip {
+
+const uint32_t kSegMostWaves = 16;  //!< waves of a workgroup
+
+/*! \brief how (n, c) planes of `len` elements are dealt out */
+struct SegmentsPlan {
+  bool use;        //!< false: the kernels of reduce_dma.h and reduce.h are the sooner ones
+  int lanes;       //!< planes of a wave
+  uint32_t kept, waves;  //!< kept indices and waves of a workgroup
+};
+/*! \brief few kept indices (fewer than three quarters of the CUs): whether a workgroup that takes all planes of its
+ *  index is done before the other kernels would be, which deal the planes of an index out.
+ *  The split kernel takes, in us, 8 + 0.08 n or 6 + 0.085 n (its last workgroup's chains) and 8 TB/s of what it reads;
+ *  binary16 10 + 0.09 n and 2 TB/s. A workgroup of this kernel takes 3 us and 32 GB/s, 47 where planes begin with their
+ *  cache lines (binary16 30 and 39), and an element of a chain 10 ns (binary16 7). As measured, split and this one: floats
+ *  (256,16,1024) 29 and 24, (1024,8,1024) 91 and 84, (2048,32,784) 215 and 196, (2048,16,1024) 197 and 166, (200,100,400)
+ *  38 and 16, (60,190,1500) 30 and 19; but (512,16,784) 49.4 and 50.7, (512,16,1500) 54 and 93, (1024,16,1500) 105 and
+ *  176, (2048,1,784) 151 and 179, (2048,4,2048) 178 and 400, (160,40,2296) 27 and 45, (64,64,12544) 52 and 78. Binary16
+ *  (512,16,784) 56 and 32, (826,31,1936) 131 and 95, (64,128,2048) 29 and 15, but (2048,4,2048) 184 and 315; odd planes, which
+ *  the generic kernel has otherwise, (512,16,2025) 141 and 96. Short reductions: 32 planes of 196 6.2 and 4.9, 41 of 132
+ *  5.6 and 4.7, 128 of 100 8.8 and 6.5, but 64 of 100 5.4 and 5.7, 35 of 56 4.3 and 5.1, binary16 40 of 255 7.7 and 8.4. */
+inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, int least_len) {
+  if (!((len <= 1100 && planes >= 2048) || (len <= 2048 && planes >= 8192))) return false;
+  const bool half = least_len == 8;
+  if (n_out * len < 1u << 16) {  // the end of a plane is added value by value: half a slice of 128 halves takes longer
+    return n_out > 64 || (len >= 128 && (!half || len % 128 <= 64));
+  }
+  /* more planes than the split kernel has room for, which leaves a workgroup per index either way: (2048,48,196) 121 and
+     77, (1618,41,100) 75 and 48, (1024,128,100) 49 and 32; binary16 86 and 69, 58 and 54, 39 and 34 */
+  if (planes > 65536) return true;
+  if (half && len % 2 != 0) return true;
+  const uint64_t bytes = n_out * len * (16u / least_len), all = planes / n_out * bytes;
+  const bool lines = bytes / n_out % 128 == 0;
+  if (half) {
+    const uint64_t split = 10000 + 90 * n_out + all / 2000;  // ns, as below; rates are bytes a ns
+    return bytes <= split * (lines ? 39 : 30) && len * 7 <= split;
+  }
+  const uint64_t split = (n_out <= 400 ? 8000 + 80 * n_out : 6000 + 85 * n_out) + all / 8000;
+  return 3000 + bytes / (lines ? 47 : 32) <= split && len * 10 <= split;
+}
+/*! \brief Measured on (n, c, len), us, the other kernels and this one; floats, binary16 gains as much. It wants planes
+ *  enough for a wave of sixteen on every SIMD or nearly, and wins by what the others leave idle.
+ *  A workgroup per kept index that fills a CU: (248,552,280) 70 and 42, (30,600,2500) 74
+ *  and 44, (19,304,5760) 93 and 35, (5,1144,8320) 115 and 49, where chain lanes (n up to the next 64, 16 or 4) and
+ *  the last round of workgroups are idle for more than three tenths; (64,256,3136) 35.6 and 40, (64,512,1600) 43 and 41.
+ *  Up to a kept index a CU there is one round of either, and up to 64 planes an index what counts are the lanes:
+ *  (32,192,3136) 28 and 23, (48,192,3136) 29 and 26, but (48,255,3136) 29 and 31, (64,192,3136) 29.5 and 31; binary16
+ *  (32,192,3136) 19.5 and 16.8, but (48,192,3136) 19.6 and 21, (64,192,1640) 14.3 and 16.2.
+ *  A workgroup of four waves per kept index, for fewer than 65536 values of each: (17,896,260) 11.7 and 7.2,
+ *  (39,957,384) 14.9 and 11.9, but (8,573,240) 5.1 and 6.3, (256,500,100) 19.8 and 22.3. One plane per kept index,
+ *  which is one lane there: (1,2048,3136) 46 and 20. */
+inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, uint32_t cus, int least_len) {
+  SegmentsPlan p = {false, 16, 1, 1};
+  const uint64_t planes = static_cast<uint64_t>(n_out) * n_keep;
+  /* 32-bit numbers of planes, fewer than 2^32 threads */
+  if (len < static_cast<uint64_t>(least_len) || n_out < 1 || n_out > 2048 || n_keep > 1u << 21 || len >= 1ull << 31 ||
+      planes >= 1ull << 31) {
+    return p;
+  }
+  const bool few_kept = static_cast<uint64_t>(n_keep) * 4 < 3ull * cus;
+  const bool middling = n_out >= 5 && n_out <= 16;
+  const uint32_t side = n_out > 16 ? 64 : n_out > 4 ? 16 : n_out > 1 ? 4 : 1;
+  const uint64_t lanes = (n_out + side - 1) / side * side, turns = (n_keep + cus - 1) / cus * cus;
+  if (few_kept) {
+    p.use = !middling && SegmentsOfFewKept(n_out, planes, len, least_len);
+  } else if (n_out == 1) {
+    p.use = n_keep >= 2 * cus && len <= 4096 && planes * len >= 800000;
+  } else if (n_out * len >= 1u << 16) {
+    p.use = planes >= 2048 && lanes * turns * 100 > planes * 130;
+    if (n_out > 40 && n_out <= 64 && n_keep <= cus) {
+      p.use = p.use && least_len == 4 && n_out <= 48 && n_keep * 16ull < 15ull * cus;
+    }
+  } else {
+    p.use = !middling && ((len <= 1100 && planes >= 2048) || planes >= 4096) && (n_out <= 4 || lanes * 100 > n_out * 102ull);
+  }
+  if (!p.use) return p;
+  /* more waves: (32,512,784) 12.4, with sixteen 13.3; not more than a workgroup has, whose waves go round again:
+     (256,16,1024) 32 that way, with sixteen 24 */
+  if (len >= 512 && planes / 16 < 4 * cus && n_out <= 8 * kSegMostWaves) p.lanes = 8;
+  /* workgroups of four waves or so where planes are few per kept index, but one for every CU */
+  while (p.kept * n_out < 4u * p.lanes && n_keep / (p.kept + 1) >= cus) ++p.kept;
+  const uint32_t all = (p.kept * n_out + p.lanes - 1) / p.lanes;
+  /* a CU holds 20 waves of this kernel: where there are more of them, small workgroups that go round again fill it,
+     but not where few kept indices are few workgroups ((1024,128,100): 62 of them that way, now 32) */
+  const uint32_t most = !few_kept && planes / p.lanes >= 20ull * cus ? 4 : kSegMostWaves;
+  const uint32_t rounds = (all + most - 1) / most;
+  p.waves = (all + rounds - 1) / rounds;
+  return p;
+}
+
+}  // namespace hip
+}  // namespace mshadow
+#endif  // MSHADOW_HIP_KERNELS_SEGMENTS_PLAN_H_

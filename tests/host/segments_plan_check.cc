@@ -1,0 +1,66 @@
+// Which sums over dense planes go to the kernel that gives a workgroup all planes of a kept index
+// (mshadow/hip/kernels/segments_plan.h): the measured shapes, (n, c, len), of either side, and what the kernel relies on
+// of every plan.
+#include <cstdio>
+#include <random>
+
+#include <mshadow/hip/kernels/segments_plan.h>
+
+using mshadow::hip::PlanSegments;
+using mshadow::hip::SegmentsPlan;
+
+static const uint32_t kCus = 256;
+static int g_wrong = 0;
+
+static void Expect(uint32_t n, uint32_t c, uint64_t len, int least_len, bool use) {
+  if (PlanSegments(n, c, len, kCus, least_len).use == use) return;
+  ++g_wrong;
+  printf("(%u,%u,%llu) %s: expected %d\n", n, c, static_cast<unsigned long long>(len), least_len == 8 ? "half" : "float", use);
+}
+
+int main() {
+  const int kFloat = 4, kHalf = 8;
+  // few kept indices: the split kernel deals their planes out, a workgroup an index would leave the chip idle
+  const uint32_t split[][3] = {{512, 16, 784}, {2048, 1, 784}, {2048, 2, 784}, {2048, 4, 784}, {2048, 8, 784}, {2048, 4, 2048}, {1024, 8, 2048},
+                               {512, 16, 1500}, {512, 24, 2025}, {1024, 16, 1500}, {2048, 16, 1500}, {256, 32, 1500}, {592, 17, 1521},
+                               {950, 13, 1225}, {826, 31, 1936}, {160, 40, 2296}, {64, 64, 12544}};
+  for (const auto &s : split) Expect(s[0], s[1], s[2], kFloat, false);
+  Expect(2048, 4, 2048, kHalf, false);
+  Expect(64, 48, 100, kFloat, false);
+  Expect(40, 60, 255, kHalf, false);
+  // ... but short planes, or few of them, are done sooner
+  const uint32_t own[][3] = {{256, 16, 1024}, {128, 16, 1024}, {256, 32, 1024}, {250, 64, 784}, {1024, 8, 1024}, {2048, 16, 1024}, {2048, 32, 784},
+                             {200, 100, 400}, {213, 58, 312}, {60, 190, 1500}, {1024, 8, 196}, {2048, 4, 100}, {32, 64, 196}, {128, 16, 196},
+                             {1718, 39, 35}, {1618, 41, 100}, {1024, 128, 100}, {40, 60, 255}};
+  for (const auto &s : own) Expect(s[0], s[1], s[2], kFloat, true);
+  const uint32_t own_half[][3] = {{512, 16, 784}, {2048, 1, 784}, {826, 31, 1936}, {64, 128, 2048}, {48, 180, 2016}, {512, 16, 2025}, {512, 16, 1500}};
+  for (const auto &s : own_half) Expect(s[0], s[1], s[2], kHalf, true);
+  // up to a kept index a CU: one round of workgroups with either kernel
+  const uint32_t ring[][3] = {{64, 192, 3136}, {64, 192, 1640}, {64, 224, 3136}, {60, 196, 3136}, {48, 240, 3136}, {48, 255, 1640}, {64, 256, 3136}};
+  for (const auto &s : ring) {
+    Expect(s[0], s[1], s[2], kFloat, false);
+    Expect(s[0], s[1], s[2], kHalf, false);
+  }
+  Expect(48, 192, 3136, kFloat, true);
+  Expect(48, 192, 3136, kHalf, false);
+  Expect(32, 192, 3136, kFloat, true);
+  Expect(32, 192, 3136, kHalf, true);
+
+  std::mt19937 rng(3);
+  for (int i = 0; i < 2000000; ++i) {
+    const uint32_t n = 1 + (rng() >> (21 + rng() % 11)), c = 1 + (rng() >> (16 + rng() % 16));
+    const uint64_t len = 1 + (rng() >> (8 + rng() % 24));
+    const int least = i % 2 ? kFloat : kHalf;
+    const SegmentsPlan p = PlanSegments(n, c, len, kCus, least);
+    if (!p.use) continue;
+    const uint32_t size = 16 / least, per_wave = (16 + p.lanes * (4096 / p.lanes + 16)) / size;
+    const bool fits = (p.lanes == 8 || p.lanes == 16) && p.waves >= 1 && p.waves <= mshadow::hip::kSegMostWaves &&
+                      p.kept >= 1 && p.kept <= p.waves * 64 && n <= 2048 && len >= static_cast<uint64_t>(least) &&
+                      (static_cast<uint64_t>(p.waves) * per_wave + static_cast<uint64_t>(p.kept) * n) * size <= 80 * 1024 &&
+                      static_cast<uint64_t>((c + p.kept - 1) / p.kept) * p.waves * 64 < (1ull << 32);
+    if (!fits && ++g_wrong < 10) printf("plan of (%u,%u,%llu) does not fit the kernel\n", n, c, static_cast<unsigned long long>(len));
+  }
+  if (g_wrong) return 1;
+  printf("OK\n");
+  return 0;
+}

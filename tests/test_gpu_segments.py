@@ -28,7 +28,11 @@ def O():
 SHAPES = [(100, 100, 1, 4), (100, 100, 1, 8), (33, 270, 1, 9), (17, 300, 3, 21), (17, 301, 8, 8), (17, 302, 5, 13), (48, 257, 1, 127),
           (49, 258, 1, 128), (49, 259, 3, 43), (3, 700, 16, 16), (2, 1100, 257, 1), (4, 800, 1, 255), (1, 1100, 29, 31), (1, 2049, 20, 20),
           (250, 300, 9, 9), (300, 60, 7, 7), (257, 90, 10, 11), (2048, 9, 5, 5), (2049, 9, 5, 5), (600, 193, 2, 33), (700, 300, 4, 24),
-          (70, 384, 31, 33), (20, 400, 50, 51), (19, 304, 72, 80), (5, 600, 130, 101), (13, 530, 74, 69), (60, 190, 30, 50), (16, 400, 15, 10)]
+          (70, 384, 31, 33), (20, 400, 50, 51), (19, 304, 72, 80), (5, 600, 130, 101), (13, 530, 74, 69), (60, 190, 30, 50), (16, 400, 15, 10),
+          # few kept indices: eight and sixteen planes a wave, one round of sixteen waves and several, more planes than the split
+          # kernel has room for, and shapes that it takes
+          (128, 17, 28, 28), (129, 17, 28, 28), (256, 16, 32, 32), (300, 9, 24, 25), (2048, 9, 16, 16), (1100, 61, 9, 7), (1101, 60, 11, 12),
+          (2048, 5, 28, 28), (48, 200, 41, 40), (44, 250, 40, 40)]
 
 
 @pytest.mark.parametrize("n,c,h,w", SHAPES)

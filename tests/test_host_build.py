@@ -161,6 +161,13 @@ def test_planned_row_sum_matches_serial_sum_on_host(tmp_path):
     assert out.startswith("OK"), out[-500:]
 
 
+def test_sums_of_dense_planes_go_to_the_kernel_measured_to_be_the_faster(tmp_path):
+    """the rule that gives a workgroup all planes of a kept index, on measured shapes of both sides:
+    where few indices are kept the chip must not be left to a few workgroups"""
+    out = _compile_and_run(tmp_path, "segments_plan_check.cc", [])
+    assert out.startswith("OK"), out[-500:]
+
+
 def test_signed_column_sums_leave_most_of_the_chain(tmp_path):
     """sum_rows adds signed terms, and on N(0, 1) terms a plan of verified runs (what makes the
     softmax row sum parallel) leaves too much of its chain: cut with full knowledge of the true
