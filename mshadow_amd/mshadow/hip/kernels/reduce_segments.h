@@ -1,10 +1,10 @@
 /*
- * sumall_except_dim<1> and its kin over dense planes, a wave to itself with up to 64 of them.
+ * sumall_except_dim<1> and its kin over dense planes, a wave to itself with eight or sixteen of them.
  *
  * The order is that of the other kernels (one chain per (n, c) plane, then one over n of their results:
  * mshadow/tensor_cpu-inl.h:230-268). A workgroup owns a few neighbouring kept indices c with all their
  * planes, a wave LANES planes, a lane the chain of one. The wave fetches 16 bytes a lane, PACKS lanes
- * next to one another in a plane, three slices ahead in registers, and passes each slice through its own
+ * next to one another in a plane, two slices ahead in registers, and passes each slice through its own
  * piece of LDS to the lanes that add; waves meet only once, for the chains over n. No ring that fills a
  * CU, no scratch memory, and every wave adds, where the kernels of reduce_dma.h have one that does.
  */
@@ -35,6 +35,7 @@ __global__ void __launch_bounds__(kSegMostWaves * kWave)
     ReduceSegmentsKernel(DType *dst, const DType *src, uint32_t seg_len, uint32_t n_out, uint32_t n_keep, uint32_t kept,
                          FastDivU32 div_kept, DType scale) {
   typedef SegSlice<DType, LANES> Slice;
+  static_assert(LANES == 8 || LANES == 16, "a slice is 16 or 32 packs of a plane");
   const int EPP = Slice::kPerPack, PACKS = Slice::kPacks, ELEMS = Slice::kElems, AHEAD = 2;
   typedef uint32_t Pack __attribute__((ext_vector_type(4)));
   typedef Pack LoosePack __attribute__((aligned(2)));  // wherever a plane begins
@@ -98,10 +99,10 @@ __global__ void __launch_bounds__(kSegMostWaves * kWave)
         }
         if (s + AHEAD < slices) fetch(v[a], s + AHEAD);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the lanes' stores before one another's loads
-        if (LANES == kWave || lane < static_cast<uint32_t>(LANES)) {
+        if (lane < static_cast<uint32_t>(LANES)) {
           const DType *mine = tile + lane * Slice::kPitch;
           if (whole) {
-            const int GROUP = PACKS < 8 ? PACKS : 8;
+            const int GROUP = 8;
 #pragma unroll
             for (int p = 0; p < PACKS; p += GROUP) {
               Pack e[GROUP];
@@ -119,7 +120,7 @@ __global__ void __launch_bounds__(kSegMostWaves * kWave)
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
     }
-    if ((LANES == kWave || lane < static_cast<uint32_t>(LANES)) && p0 + lane < planes) part[p0 + lane] = res;
+    if (lane < static_cast<uint32_t>(LANES) && p0 + lane < planes) part[p0 + lane] = res;
   }
   __syncthreads();
   const uint32_t c = c0 + threadIdx.x;

@@ -1,5 +1,6 @@
 """Softmax of rows that are kept partly in LDS (32769 to 51200 columns with more rows than compute units, 65537 to 110592
-columns), and of the wider workgroups that up to two rows a compute unit take: bit for bit what the kernel that goes
+columns), of the wider workgroups that up to two rows a compute unit take, and of the other rows of 1025 to 8192 columns, a
+workgroup or a wave each: bit for bit what the kernel that goes
 stretch by stretch gives for the same logits with columns of -inf behind them, whose terms are zeros at the end of the sum
 and which change neither the maximum nor a quotient. That kernel's row sums are tested against the serial sum."""
 import numpy as np
@@ -47,7 +48,13 @@ SHAPES = [(280, 32769, 0), (280, 36864, 0), (270, 36867, 1), (260, 50257, 0), (3
           (9, 65537, 0), (9, 65540, 3), (260, 70001, 0), (9, 81917, 0), (9, 81920, 0), (9, 81921, 1), (9, 94209, 0), (520, 90001, 0),
           (9, 110589, 0), (9, 110592, 0),
           # wider workgroups for few rows
-          (9, 1025, 0), (9, 2047, 1), (9, 2048, 0), (500, 3001, 0), (9, 4096, 0), (9, 8191, 2), (9, 16384, 0), (9, 16385, 0), (9, 32767, 0)]
+          (9, 1025, 0), (9, 2047, 1), (9, 2048, 0), (500, 3001, 0), (9, 4096, 0), (9, 8191, 2), (9, 16384, 0), (9, 16385, 0), (9, 32767, 0),
+          # a workgroup a row beyond those few rows, at its borders with the kernel of a wave a row
+          (1535, 1025, 0), (1200, 2047, 1), (600, 2048, 0), (1023, 2049, 2), (1023, 3072, 0), (1100, 3073, 0), (513, 4096, 1),
+          (600, 4097, 0), (513, 8191, 0), (513, 8192, 3),
+          # a wave a row, up to 4, 8, 10 and 12 packs a lane
+          (1536, 1024, 0), (1536, 1025, 0), (1537, 2047, 1), (1600, 2048, 0), (1024, 2049, 0), (1025, 2303, 2), (1101, 2560, 0),
+          (1024, 2561, 3), (1026, 2815, 0), (1024, 3072, 0)]
 
 
 @pytest.mark.parametrize("rows,cols,pad", SHAPES)
