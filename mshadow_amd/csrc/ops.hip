@@ -450,7 +450,7 @@ int RowsOfLaunch(unsigned threads) {
   return most < static_cast<unsigned long long>(INT_MAX) ? static_cast<int>(most) : INT_MAX;
 }
 /*! \brief threads a row of the kernels below takes, where there are many rows */
-unsigned SoftmaxThreadsPerRow(int cols) { return cols <= 32 ? 1u : cols <= 256 ? 32u : cols <= 2560 ? 64u : 1024u; }
+unsigned SoftmaxThreadsPerRow(int cols) { return cols <= 32 ? 1u : cols <= 256 ? 32u : cols <= 3072 ? 64u : 1024u; }
 
 /*! \brief rows that a thread, a part of a wave or a wave takes; false: longer ones, which take a
  *  workgroup */
@@ -480,17 +480,18 @@ bool LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, 
   else if (cols <= 64) SHORT_PART(16, 4);
   else if (cols <= 128) SHORT_PART(16, 8);
   else if (cols <= 256) SHORT_PART(32, 8);
-  /* a wave per row for any number of rows of up to 512 columns, and for many of up to 2560 (65536
-     rows of 300 / 1000 columns: 43 / 90 us against 163 / 174 us with a workgroup per row, 16384 of
-     2304 56 against 75 us, 8000 of 2560 33.8 against 40.9; at 3000 columns, before its loads were all under
-     way together, 8000 rows 44.3 against 42.2). 100 rows of 500: 5.0 against 5.6 us; 1000 rows of 1000: 7.8
-     against 7.1 us, 3000 rows 9.7 against 12.7; 2000 rows of 2000 13.1 against 11.9, 3000 rows 14.6 against 16.1.
-     (The row sums alone are as they were measured before: up to 3072 columns, from 6 rows a CU on.) */
+  /* A wave per row for any number of rows of up to 512 columns, and for many of up to 3072: from 6 rows a CU on, above
+     2048 columns from 4. In us, a workgroup a row and a wave: 100 rows of 500 columns 5.6 and 5.0; of 1000 columns 1024
+     rows 7.4 and 7.3, 3000 12.7 and 9.7, 65536 174 and 90; 1024 / 1536 / 2304 rows of 1200 8.6 and 9.0, 10.2 and 9.9,
+     13.0 and 11.0, of 2048 9.4 and 9.7, 10.9 and 10.6, 14.1 and 11.9, of 2300 11.7 and 10.9, 13.9 and 12.0, 18.0 and 13.6,
+     of 3072 12.1 and 11.9, 14.4 and 13.2, 18.4 and 15.3; 8000 rows of 3072 43.5 and 39.4; 600 of 2688 10.6 and 10.9.
+     The row sums alone from 6 rows a CU on at all lengths. */
   else if (cols <= 512) WAVE_SLABS(2);
-  else if (cols > (TERMS_GIVEN ? 3072 : 2560) || rows < (cols > 1024 && !TERMS_GIVEN ? 10 : 6) * cus) return false;
+  else if (cols > 3072 || rows < (cols > 2048 && !TERMS_GIVEN ? 4 : 6) * cus) return false;
   else if (cols <= 1024) WAVE_SLABS(4);
   else if (cols <= 2048) WAVE_SLABS(8);
-  else WAVE_SLABS(TERMS_GIVEN ? 12 : 10);
+  else if (cols <= 2560 && !TERMS_GIVEN) WAVE_SLABS(10);
+  else WAVE_SLABS(12);
 #undef SHORT_THREAD
 #undef SHORT_PART
 #undef SHORT_PART_AS
@@ -614,7 +615,7 @@ int mshadow_hip_softmax_f32(float *dst, int dstride, const float *src, int sstri
   hipStream_t s = AsStream(stream);
   if (LaunchShortSoftmax<false>(dst, dstride, src, sstride, rows, cols, s)) return AfterLaunch("softmax");
   /* 16-byte packs wherever the rows start and whatever their length (the accesses need no
-     alignment; a row's last, partial pack goes element by element) */
+     alignment; a row's last, partial pack is loaded as its last four columns and stored element by element) */
 #define SOFTMAX_LAUNCH(T, S, V) \
   LaunchKernelIfFits((SoftmaxRowKernel<T, S, V, false>), dim3(rows), dim3(T), 0, s, dst, dstride, \
                      src, sstride, cols)

@@ -276,9 +276,9 @@ SOFTMAX_SHAPES = [((64, 32000), 0), ((5, 1000), 0), ((5, 1001), 0), ((3, 7), 1),
                   # rows longer than a workgroup's registers hold: stretch by stretch (two, four and five stretches,
                   # a last stretch of one column, of one pack, pitched rows)
                   ((3, 128000), 0), ((2, 200001), 1), ((1, 262149), 0), ((2, 65537), 3), ((2, 65540), 0), ((2, 131072), 2),
-                  # many rows of a few hundred to 2048 columns: a wave per row, slab after slab
+                  # many rows of a few hundred to 3072 columns: a wave per row, slab after slab
                   ((2100, 300), 0), ((2049, 777), 3), ((2050, 1024), 0), ((2048, 2047), 1), ((4100, 513), 0),
-                  # ... up to 3072 columns; many rows of 8193 to 16384 columns: four waves a row
+                  # ... three packs a lane and more; many rows of 8193 to 16384 columns: a workgroup each
                   ((2100, 2304), 0), ((2050, 3072), 1), ((2049, 2999), 0), ((4100, 8200), 0), ((4096, 12001), 0),
                   # short rows: one thread per row up to 32 columns, one wave per row up to 256
                   ((1000, 10), 0), ((300, 32), 0), ((77, 33), 2), ((130, 64), 0), ((50, 65), 1),
