@@ -474,7 +474,14 @@ bool LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, 
      its end sooner: 4000 rows of 64 columns 3.8 us a wave each, 4.9 us in quarters, of 200 5.5 and
      6.8 us, 16000 of 200 11.2 and 12.3 us; 131072 rows of 128 56 and 35 us, of 193 69 and 63 us */
   const bool few = rows <= (cols <= 128 ? 16 : 64) * cus;
-  if (cols <= 16) SHORT_THREAD(16);
+  /* not more than three loads of columns that are not there: each is a pass of its own over 64 cache lines
+     (300 / 50000 rows of 17 columns: with 15 of them 6.1 / 9.1 us, with three 5.0 / 7.9) */
+  if (cols <= 8) SHORT_THREAD(8);
+  else if (cols <= 12) SHORT_THREAD(12);
+  else if (cols <= 16) SHORT_THREAD(16);
+  else if (cols <= 20) SHORT_THREAD(20);
+  else if (cols <= 24) SHORT_THREAD(24);
+  else if (cols <= 28) SHORT_THREAD(28);
   else if (cols <= 32) SHORT_THREAD(32);
   else if (cols <= 256 && few) WAVE_SLABS(1);
   else if (cols <= 64) SHORT_PART(16, 4);

@@ -76,3 +76,30 @@ def test_softmax_short_rows(G, O, rows, cols):
     got = dst.download().astype(np.float64)
     # the exponential within 3 ulp, the sum of such terms and the quotient within one each: 4e-7 together
     assert np.max(np.abs(got - want) / want) < 1e-6
+
+
+@pytest.mark.parametrize("cols", [1, 8, 9, 12, 13, 16, 17, 20, 21, 24, 25, 28, 29, 32])
+def test_rows_of_a_thread(G, O, cols):
+    """at the lengths that a thread's registers are cut to: Softmax, in place and not, and the row sums, pitched and ending
+    where the tensor ends"""
+    rows = 515
+    x = (np.random.default_rng(cols).standard_normal((rows, cols), dtype=f32) * f32(3)).astype(f32)
+    x[::7, -1] = x[::7].max(axis=1) + f32(1)
+    want = np.empty_like(x)
+    O.softmax(want, x)
+    terms = np.exp(x)
+    sums = np.zeros(rows, f32)
+    for i in range(cols):
+        sums = sums + terms[:, i]
+    for pad in (0, 3):
+        src = G.to_device(x, pad)
+        dst = G.buffer(x.shape, f32, pad)
+        G.softmax(dst, src)
+        got = dst.download()
+        assert np.max(np.abs(got.astype(np.float64) - want) / want) < 1e-6   # as above
+        G.softmax(src, src)
+        assert_bits_equal(src.download(), got, f"{cols} columns in place")
+        out = G.buffer((rows,), f32)
+        t = G.to_device(terms, pad)
+        G.check(G.dll.mshadow_hip_softmax_rowsum_f32(out.ptr, t.ptr, cols + pad, rows, cols, None))
+        assert_bits_equal(out.download(), sums, f"{cols} columns")
