@@ -749,7 +749,8 @@ __device__ __forceinline__ void PlacePackOfRow(float (&t)[4], int c0, int cols, 
  *  INLDS: that many slabs live in LDS, which the registers leave idle. Two rows of 50257 columns then fit
  *  a CU (18 slabs of 512 threads in registers, 7 in LDS; 2048 of them 264 -> 206 us, 4.0 TB/s), and one of
  *  up to 110592 on 1024 threads (19 and 8), which went through the caches three times before. Three
- *  rows of 32000 to a CU that way (11 and 5, 80 registers, 22 of them spilled) took 419 us against 373.
+ *  rows of 32000 to a CU that way (11 and 5, 80 registers, 22 of them spilled) took 419 us against 373; 18 and 7 spill 16
+ *  registers, 19 and 8 spill 35, and are faster all the same.
  *  TERMS_GIVEN: src already holds the (non-negative) terms and dst[row] receives their
  *  left-to-right sum - the row-sum stage on its own. */
 template <int THREADS, int REGS, int VEC, bool TERMS_GIVEN, int MIN_WAVES = 4, int INLDS = 0>
