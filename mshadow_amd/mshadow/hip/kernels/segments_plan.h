@@ -33,7 +33,7 @@ inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, int
   if (!((len <= 1100 && planes >= 2048) || (len <= 2048 && planes >= 8192))) return false;
   const bool half = least_len == 8;
   if (n_out * len < 1u << 16) {  // the end of a plane is added value by value: half a slice of 128 halves takes longer
-    return n_out > 64 || (len >= 128 && (!half || len % 128 <= 64));
+    return n_out > 64 || (len >= 128 && (!half || len >= 256 || len % 128 <= 64));
   }
   /* more planes than the split kernel has room for, which leaves a workgroup per index either way: (2048,48,196) 121 and
      77, (1618,41,100) 75 and 48, (1024,128,100) 49 and 32; binary16 86 and 69, 58 and 54, 39 and 34 */
@@ -47,6 +47,21 @@ inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, int
   }
   const uint64_t split = (n_out <= 400 ? 8000 + 80 * n_out : 6000 + 85 * n_out) + all / 8000;
   return 3000 + bytes / (lines ? 47 : 32) <= split && len * 10 <= split;
+}
+/*! \brief short reductions of many kept indices (fewer than 65536 values of each): whether the ends of their planes, which
+ *  are added value by value - what is left of the last slice of 64 floats or 128 halves -, cost this kernel more than it
+ *  wins. In us, the kernel of a workgroup per index and this one: floats (46,409,120) 6.3 and 7.0, (95,745,50) 9.7 and 10.7,
+ *  (4,667,756) 8.0 and 10.0, but (65,208,117) 8.8 and 6.7, (4,1928,637) 14.2 and 12.3; binary16 (38,1675,55) 7.3 and 10.9,
+ *  (20,346,231) 7.2 and 8.0, (2,1439,1005) 10.2 and 15.9, but (112,335,56) 8.7 and 7.0, (22,422,198) 7.3 and 6.7, (4,1800,840)
+ *  level, and planes of two slices and more, (43,835,1275) 38.8 and 27.0. */
+inline bool SegmentEndsWeighMore(uint32_t n_out, uint32_t n_keep, uint64_t planes, uint64_t len, uint32_t cus, int least_len) {
+  const bool one_round = n_out > 64 && n_keep <= 2 * cus;  // few workgroups of several rounds each with the other kernel
+  if (least_len == 8) {
+    if (n_out <= 4) return len % 128 > 72;
+    return (len < 128 && !one_round) || (len >= 128 && len < 256 && len % 128 > 72);
+  }
+  if (n_out <= 4) return len > 600 && planes < 2800;
+  return len < 128 && len % 64 >= 44 && n_out >= 24 && !one_round;
 }
 /*! \brief Measured on (n, c, len), us, the other kernels and this one; floats, binary16 gains as much. It wants planes
  *  enough for a wave of sixteen on every SIMD or nearly, and wins by what the others leave idle.
@@ -81,7 +96,8 @@ inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, 
       p.use = p.use && least_len == 4 && n_out <= 48 && n_keep * 16ull < 15ull * cus;
     }
   } else {
-    p.use = !middling && ((len <= 1100 && planes >= 2048) || planes >= 4096) && (n_out <= 4 || lanes * 100 > n_out * 102ull);
+    p.use = !middling && ((len <= 1100 && planes >= 2048) || planes >= 4096) && (n_out <= 4 || lanes * 100 > n_out * 102ull) &&
+            !SegmentEndsWeighMore(n_out, n_keep, planes, len, cus, least_len);
   }
   if (!p.use) return p;
   /* more waves: (32,512,784) 12.4, with sixteen 13.3; not more than a workgroup has, whose waves go round again:

@@ -28,6 +28,7 @@ int main() {
   Expect(2048, 4, 2048, kHalf, false);
   Expect(64, 48, 100, kFloat, false);
   Expect(40, 60, 255, kHalf, false);
+  Expect(44, 174, 460, kHalf, true);
   // ... but short planes, or few of them, are done sooner
   const uint32_t own[][3] = {{256, 16, 1024}, {128, 16, 1024}, {256, 32, 1024}, {250, 64, 784}, {1024, 8, 1024}, {2048, 16, 1024}, {2048, 32, 784},
                              {200, 100, 400}, {213, 58, 312}, {60, 190, 1500}, {1024, 8, 196}, {2048, 4, 100}, {32, 64, 196}, {128, 16, 196},
@@ -45,6 +46,18 @@ int main() {
   Expect(48, 192, 3136, kHalf, false);
   Expect(32, 192, 3136, kFloat, true);
   Expect(32, 192, 3136, kHalf, true);
+  // short reductions of many kept indices: ends of planes that are added value by value
+  Expect(46, 409, 120, kFloat, false);
+  Expect(95, 745, 50, kFloat, false);
+  Expect(65, 208, 117, kFloat, true);
+  Expect(4, 667, 756, kFloat, false);
+  Expect(4, 1928, 637, kFloat, true);
+  Expect(38, 1675, 55, kHalf, false);
+  Expect(20, 346, 231, kHalf, false);
+  Expect(2, 1439, 1005, kHalf, false);
+  Expect(112, 335, 56, kHalf, true);
+  Expect(22, 422, 198, kHalf, true);
+  Expect(43, 835, 1275, kHalf, true);
 
   std::mt19937 rng(3);
   for (int i = 0; i < 2000000; ++i) {
