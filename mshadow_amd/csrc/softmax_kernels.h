@@ -1123,7 +1123,7 @@ __device__ inline float PartWaveResolve(float s, const float (&t)[N]) {
  *  maximum, the scans of the ordered sum - cost the same instructions whether a wave holds one
  *  short row or four, and rows of up to 256 columns by the hundred thousand are bound by
  *  exactly those. 256 / LANES rows per workgroup, nothing shared between them, no barrier.
- *  WHOLE: rows are whole aligned packs, which stream; else ordinary accesses, because neighbouring rows'
+ *  WHOLE: streaming accesses, as for rows of whole aligned packs; else ordinary ones, because neighbouring rows'
  *  accesses meet in the cache lines that they share (131072 x 127: 45 -> 33 us). */
 template <int LANES, int N, bool TERMS_GIVEN, bool WHOLE>
 __global__ void __launch_bounds__(256)
