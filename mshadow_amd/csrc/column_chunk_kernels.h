@@ -1,0 +1,411 @@
+/*
+ * sum_rows of long float columns by chunks of 128 rows (column_chunks.h has the arithmetic), in three
+ * launches: the chunks' sums in any order, their maps, and a walk down every column. The matrix is read twice, by
+ * all CUs, where a strip of columns a workgroup leaves most of them idle; the sequence of a column is left
+ * to one wave, which takes a chunk in 55 ns, and one that has no map in 500, where 128 dependent adds
+ * take 450. 65536 x 1000: 50, 56 and 58 to 75 us (the last by the column with the fewest maps).
+ */
+#ifndef MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_
+#define MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_
+
+#include <mshadow/hip/kernels/common.h>
+#include <mshadow/hip/kernels/reduce_dma.h>
+
+#include "column_chunks.h"
+
+namespace mshadow_hipk {
+
+using column_chunks::Map;
+using column_chunks::Step;
+using mshadow::hip::kWave;
+
+/*! \brief a workgroup has four chunks of 64 columns, a wave each */
+const int kChunkWaves = 4;
+const uint32_t kColumnsPerTile = 64;
+
+/*! \brief scratch memory of one call: cells are (chunk, column), the columns padded to whole tiles */
+const uint32_t kChunkCells = 1u << 19;
+const uint32_t kChunkCopies = 1u << 14;
+struct ColumnChunkScratch {
+  Map map[kChunkCells];                             // [column][chunk], what the walk reads
+  float copy[kChunkCopies][column_chunks::kRows];   // terms of chunks that are added one by one
+  float before[kChunkCells];                        // [chunk][column]: sum of the workgroup's chunks in front
+  float group[kChunkCells / kChunkWaves + kChunkCells / kChunkWaves / 2];  // [workgroup of chunks][column]
+};
+
+struct ChunkShape {
+  uint32_t rows, cols, stride;
+  uint32_t chunks, groups, tiles;
+  uint32_t copies;  // copies a (chunk, tile) has room for
+};
+inline bool MakeChunkShape(uint32_t rows, uint32_t cols, uint32_t stride, ChunkShape *g) {
+  g->rows = rows;
+  g->cols = cols;
+  g->stride = stride;
+  g->chunks = (rows + column_chunks::kRows - 1) / column_chunks::kRows;
+  g->groups = (g->chunks + kChunkWaves - 1) / kChunkWaves;
+  g->tiles = (cols + kColumnsPerTile - 1) / kColumnsPerTile;
+  const uint64_t cells = static_cast<uint64_t>(g->chunks) * g->tiles;
+  if (cells * kColumnsPerTile > kChunkCells) return false;
+  const uint32_t room = static_cast<uint32_t>(kChunkCopies / cells);
+  g->copies = room < kColumnsPerTile ? room : kColumnsPerTile;
+  /* groups * kChunkWaves may exceed chunks by three, which the array of groups allows for */
+  return static_cast<uint64_t>(g->groups) * g->tiles * kColumnsPerTile <=
+         sizeof(static_cast<ColumnChunkScratch *>(NULL)->group) / sizeof(float);
+}
+
+/*! \brief where the chunks are the sooner way. Measured, us (MI355X; a classifier's gradients), without and with:
+ *  131072 x 10 448 and 109, 131072 x 100 470 and 120, 65536 x 1000 232 and 185, 30000 x 100 114 and 46, 16384 x 1000
+ *  64 and 53, 16384 x 100 65 and 31, 8192 x 100 36 and 24, 8192 x 10 34 and 26; level at 8192 x 1000 and 4096 x 64,
+ *  slower at 16384 x 4096 (72 and 180: its reads alone take as long as its chain). Without, a row takes 3.5 ns; with,
+ *  0.8 ns, 1.6 ps a column for the second read of the matrix and the less than full rate of the first, and
+ *  17 us for the three launches. More than six columns a CU walk in turns. Columns whose sum misses
+ *  its maps throughout (0.1 added 65536 times) take 0.5 us a chunk: 290 us where the chain takes 232. */
+inline bool ColumnChunksAreSooner(uint32_t rows, uint32_t cols, uint32_t cus) {
+  return cols <= 6u * cus && static_cast<double>(rows) * (2700.0 - 1.6 * cols) > 17e6;
+}
+
+/*! \brief a column's terms of N rows: all loads under way together, rows behind the last as -0, which changes no
+ *  sum */
+template <uint32_t N>
+__device__ __forceinline__ void LoadRows(float (&t)[N], const float *src, const ChunkShape &g, uint32_t row0,
+                                         uint32_t x) {
+  /* a row's address is the wave's, the column's offset a lane's (32 bits: the instruction adds them) */
+  const uint32_t at = x * static_cast<uint32_t>(sizeof(float));
+  const size_t pitch = static_cast<size_t>(g.stride) * sizeof(float);
+  if (row0 + N <= g.rows) {
+    const char *p = reinterpret_cast<const char *>(src) + row0 * pitch;
+#pragma unroll
+    for (uint32_t i = 0; i < N; ++i) {
+      t[i] = *reinterpret_cast<const float *>(p + at);
+      p += pitch;
+    }
+  } else {
+    const uint32_t from = row0 < g.rows ? row0 : g.rows - 1u;
+    const uint32_t left = row0 < g.rows ? g.rows - row0 : 0u;
+    const char *p = reinterpret_cast<const char *>(src) + from * pitch;
+#pragma unroll
+    for (uint32_t i = 0; i < N; ++i) {
+      const float v = *reinterpret_cast<const float *>(p + at);
+      t[i] = i < left ? v : -0.0f;
+      if (i + 1u < left) p += pitch;
+    }
+  }
+}
+
+/*! \brief rows whose loads are under way together in the launch that only sums */
+const uint32_t kSumsAtOnce = 32;
+
+/*! \brief the sums of the chunks, in any order of adds: per workgroup of four chunks the sum of those in
+ *  front of each, and of all. Bound by its read of the matrix. */
+__global__ void __launch_bounds__(kChunkWaves *kWave)
+    ColumnChunkSumsKernel(const float *src, ChunkShape g, float *before, float *group) {
+  __shared__ float sums[kChunkWaves][kWave];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
+  const uint32_t piece = mshadow::hip::StripOfBlock(blockIdx.x, gridDim.x);
+  const uint32_t at = piece / g.tiles, tile = piece % g.tiles;
+  const uint32_t chunk = at * kChunkWaves + wave, pitch = g.tiles * kColumnsPerTile;
+  const uint32_t column = tile * kColumnsPerTile + lane;
+  const uint32_t x = column < g.cols ? column : g.cols - 1;
+  float sum = 0.0f;
+  if (chunk < g.chunks) {
+    float part[kSumsAtOnce] = {0.0f};
+    for (uint32_t i = 0; i < static_cast<uint32_t>(column_chunks::kRows); i += kSumsAtOnce) {
+      float t[kSumsAtOnce];
+      LoadRows(t, src, g, chunk * column_chunks::kRows + i, x);
+#pragma unroll
+      for (uint32_t k = 0; k < kSumsAtOnce; ++k) part[k] += t[k];
+    }
+#pragma unroll
+    for (uint32_t step = 1; step < kSumsAtOnce; step *= 2) {
+#pragma unroll
+      for (uint32_t k = 0; k < kSumsAtOnce; k += 2 * step) part[k] += part[k + step];
+    }
+    sum = part[0];
+  }
+  sums[wave][lane] = sum;
+  __syncthreads();
+  float front = 0.0f;
+  for (uint32_t w = 0; w < wave; ++w) front += sums[w][lane];
+  if (chunk < g.chunks) before[static_cast<size_t>(chunk) * pitch + column] = front;
+  if (wave == kChunkWaves - 1) group[static_cast<size_t>(at) * pitch + column] = front + sum;
+}
+
+/*! \brief the maps of the chunks. A wave keeps its chunk of 64 columns in registers, so that terms to be added
+ *  one by one can be copied out; twelve instructions a term, which the reads hide. Workgroups go through
+ *  the matrix from its end: what the launch before read last is still in the memory-side cache. */
+__global__ void __launch_bounds__(kChunkWaves *kWave)
+    ColumnChunkMapsKernel(const float *src, ChunkShape g, const float *before, const float *group, Map *map,
+                          float (*copy)[column_chunks::kRows]) {
+  __shared__ float part[3][kChunkWaves][kWave];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
+  const uint32_t piece = gridDim.x - 1u - mshadow::hip::StripOfBlock(blockIdx.x, gridDim.x);
+  const uint32_t at = piece / g.tiles, tile = piece % g.tiles;
+  const uint32_t chunk = at * kChunkWaves + wave, pitch = g.tiles * kColumnsPerTile;
+  const uint32_t column = tile * kColumnsPerTile + lane;
+  const uint32_t x = column < g.cols ? column : g.cols - 1;
+  const bool live = chunk < g.chunks;
+  /* the sums in front: a quarter of the groups a wave, with the largest and smallest sum on the way */
+  {
+    const uint32_t each = (at + kChunkWaves - 1) / kChunkWaves;
+    const uint32_t first = wave * each, end = first + each < at ? first + each : at;
+    float sum = 0.0f, high = 0.0f, low = 0.0f;
+    const float *p = group + static_cast<size_t>(first) * pitch + column;
+    uint32_t i = first;
+    for (; i + 8 <= end; i += 8) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = p[static_cast<size_t>(k) * pitch];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        sum += v[k];
+        high = fmaxf(high, sum);
+        low = fminf(low, sum);
+      }
+      p += static_cast<size_t>(8) * pitch;
+    }
+    for (; i < end; ++i) {
+      sum += *p;
+      high = fmaxf(high, sum);
+      low = fminf(low, sum);
+      p += pitch;
+    }
+    part[0][wave][lane] = sum;
+    part[1][wave][lane] = high;
+    part[2][wave][lane] = low;
+  }
+  float t[column_chunks::kRows];
+  const float inside = live ? before[static_cast<size_t>(chunk) * pitch + column] : 0.0f;
+  if (live) LoadRows(t, src, g, chunk * column_chunks::kRows, x);
+  __syncthreads();
+  if (!live) return;
+  float a = 0.0f, most = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kChunkWaves; ++w) {
+    most = fmaxf(most, fmaxf(fabsf(a + part[1][w][lane]), fabsf(a + part[2][w][lane])));
+    a += part[0][w][lane];
+  }
+  a += inside;
+  most = fmaxf(most, fabsf(a));
+  const uint32_t j = column_chunks::StartsOnGrid(a)
+                         ? column_chunks::WindowFor(a, most, sqrtf(static_cast<float>(chunk * column_chunks::kRows)))
+                         : column_chunks::kMaxWindow + 1u;
+  const bool tried = j <= column_chunks::kMaxWindow;
+  column_chunks::Chains chains;
+  const float from = tried ? a : 1.0f;
+  chains.Start(from, tried ? j : column_chunks::kMinWindow);
+#pragma unroll
+  for (int i = 0; i < column_chunks::kRows; ++i) {
+    chains.Add(t[i]);
+    if (i % 4 == 3) {
+      /* else the compiler runs one chain after the other, makes trees of the maxima and ors, and keeps
+         every sum until then (256 registers and as many spilled) */
+      asm volatile("" : "+v"(chains.differ), "+v"(chains.far), "+v"(chains.most), "+v"(chains.term));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  Map m;
+  bool wide;
+  const bool known = chains.Finish(from, tried ? j : column_chunks::kMinWindow, &m, &wide) && tried;
+  if (!known) {
+    uint32_t where = column_chunks::kInMatrix;
+    if (chains.term == 0.0f && chains.s[0] == chains.s[0]) {
+      bool plus = false;
+#pragma unroll
+      for (int i = 0; i < column_chunks::kRows; ++i) plus = plus || __float_as_uint(t[i]) == 0u;
+      where = plus ? column_chunks::kPlusZero : column_chunks::kNothing;
+    }
+    m.how = column_chunks::How(true, 0u, where);
+  }
+  /* copies of the terms that will or may be asked for */
+  const bool copied = column < g.cols && !(known && wide) && column_chunks::WhereOf(m.how) == column_chunks::kInMatrix;
+  const uint32_t place = mshadow::hip::LanesBelow(__ballot(copied));
+  if (copied && place < g.copies) {
+    const uint32_t slot = (chunk * g.tiles + tile) * g.copies + place;
+    float4 *to = reinterpret_cast<float4 *>(copy[slot]);
+#pragma unroll
+    for (int i = 0; i < column_chunks::kRows; i += 4) to[i / 4] = make_float4(t[i], t[i + 1], t[i + 2], t[i + 3]);
+    m.how = column_chunks::How(!known, column_chunks::WindowOf(m.how), column_chunks::kKept + slot);
+  }
+  if (column < g.cols) map[static_cast<size_t>(column) * g.chunks + chunk] = m;
+}
+
+__device__ __forceinline__ void WaveLdsFence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+/*! \brief 128 additions, the terms read from LDS a block of 32 ahead */
+__device__ __forceinline__ void AddTerms(float *sum, const float4 *term) {
+  const int kBlock = 8, kBlocks = column_chunks::kRows / 4 / kBlock;
+  float4 v[2][kBlock];
+#pragma unroll
+  for (int k = 0; k < kBlock; ++k) v[0][k] = term[k];
+#pragma unroll
+  for (int b = 0; b < kBlocks; ++b) {
+    if (b + 1 < kBlocks) {
+#pragma unroll
+      for (int k = 0; k < kBlock; ++k) v[(b + 1) & 1][k] = term[(b + 1) * kBlock + k];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < kBlock; ++k) {
+      *sum += v[b & 1][k].x;
+      *sum += v[b & 1][k].y;
+      *sum += v[b & 1][k].z;
+      *sum += v[b & 1][k].w;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+/*! \brief chunks the walk takes between two barriers, and of these how many at a time; blocks on their way or
+ *  in use; waves that bring them in turn */
+const uint32_t kWalkBlock = 16;
+const uint32_t kChunksAtOnce = 8;
+const uint32_t kWalkLoaders = 2;
+const uint32_t kWalkRing = kWalkLoaders + 1;
+/*! \brief in the place of a window: the terms are here; there are none; there are only zeros, a +0 among them */
+const uint32_t kWalkTerms = 0xbf800000u, kWalkNothing = 0xc0000000u, kWalkPlusZero = 0xc0400000u;  // -1, -2, -3
+struct WalkBlock {
+  float4 step[kWalkBlock];  // Step's a, inverse, e0, grid
+  uint2 rest[kWalkBlock];   // Step's shift, window
+  uint32_t here;            // bit c: the terms of chunk c are here
+  float4 term[kWalkBlock][column_chunks::kRows / 4];  // of the chunks that are added term by term
+};
+
+/*! \brief the sums themselves: a wave walks down a column, every lane with the same sum, and reads nothing but
+ *  LDS. Two more bring it the maps, and the terms of the chunks that have none: a block each in turn,
+ *  asked for two blocks ahead. Bound by the walk's sequence: a wave alone issues an instruction every 3.5 ns. */
+template <typename Saver>
+__global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
+    ColumnChunkWalkKernel(float *dst, const float *src, ChunkShape g, const Map *map,
+                          const float (*copy)[column_chunks::kRows], float scale) {
+  __shared__ WalkBlock ring[kWalkRing];
+  __shared__ uint32_t misses;  // chunks whose map did not cover the sum
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
+  const uint32_t x = blockIdx.x;
+  const uint32_t blocks = (g.chunks + kWalkBlock - 1) / kWalkBlock;
+  if (threadIdx.x == 0) misses = 0u;
+  __syncthreads();
+
+  if (wave != 0) {
+    const Map *mine = map + static_cast<size_t>(x) * g.chunks;
+    auto fetch = [&](uint32_t block) {
+      const uint32_t c = block * kWalkBlock + lane % kWalkBlock;
+      return mine[c < g.chunks ? c : g.chunks - 1];
+    };
+    Map now = fetch(wave - 1);
+    for (uint32_t b = 0; b < blocks + kWalkLoaders; ++b) {
+      if (b % kWalkLoaders == wave - 1) {
+        if (b < blocks) {
+          WalkBlock *to = &ring[b % kWalkRing];
+          const uint32_t first = b * kWalkBlock;
+          /* where the maps keep missing the sum, every chunk's terms */
+          const uint32_t missed =
+              __hip_atomic_load(&misses, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          const bool all = __builtin_amdgcn_readfirstlane(missed > 8u && missed * 4u > first ? 1u : 0u) != 0u;
+          const bool live = lane < kWalkBlock && first + lane < g.chunks;
+          const bool mapped = !column_chunks::IsByTerms(now.how);
+          const uint32_t where = column_chunks::WhereOf(now.how);
+          const bool nothing = where == column_chunks::kNothing, plus = where == column_chunks::kPlusZero;
+          unsigned long long wanted =
+              __ballot(live && (where >= column_chunks::kKept ||
+                                (where == column_chunks::kInMatrix && (all || !mapped))));
+          if (lane < kWalkBlock) {
+            const Step st = column_chunks::StepOf(now);
+            const uint32_t window = !live || nothing ? kWalkNothing
+                                    : plus           ? kWalkPlusZero
+                                    : mapped         ? __float_as_uint(st.window)
+                                                     : kWalkTerms;
+            to->step[lane] = make_float4(st.a, st.inverse, st.e0, st.grid);
+            to->rest[lane] = make_uint2(st.shift, window);
+            to->here = static_cast<uint32_t>(wanted);
+          }
+          while (wanted != 0ull) {
+            const uint32_t c = __builtin_ctzll(wanted);
+            wanted &= wanted - 1ull;
+            const uint32_t place = mshadow::hip::ReadLaneU32(where, c);
+            float *term = reinterpret_cast<float *>(to->term[c]);
+            const uint32_t row0 = (first + c) * column_chunks::kRows;
+            if (place >= column_chunks::kKept) {
+              const float *from = copy[place - column_chunks::kKept];
+              mshadow::hip::LoadDwordToLds(from + lane, term);
+              mshadow::hip::LoadDwordToLds(from + kWave + lane, term + kWave);
+            } else if (row0 + column_chunks::kRows <= g.rows) {
+              const float *from = src + static_cast<size_t>(row0 + lane) * g.stride + x;
+              mshadow::hip::LoadDwordToLds(from, term);
+              mshadow::hip::LoadDwordToLds(from + static_cast<size_t>(kWave) * g.stride, term + kWave);
+            } else {
+              for (uint32_t i = lane; i < static_cast<uint32_t>(column_chunks::kRows); i += kWave) {
+                term[i] = row0 + i < g.rows ? src[static_cast<size_t>(row0 + i) * g.stride + x] : -0.0f;
+              }
+            }
+          }
+          now = fetch(b + kWalkLoaders);
+        }
+      }
+      /* the walk comes to a block kWalkLoaders steps behind its turn */
+      if ((b + 1u) % kWalkLoaders == wave - 1) mshadow::hip::WaitAllLanded();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      mshadow::hip::BareBarrier();
+    }
+    mshadow::hip::WaitAllLanded();  // no load is under way when the workgroup's LDS is handed on
+    return;
+  }
+
+  uint32_t missed = 0u;
+  float sum = -0.0f;  // the identity: the reference starts from the first term
+  for (uint32_t b = 0; b < blocks + kWalkLoaders; ++b) {
+    if (b >= kWalkLoaders) {
+      WalkBlock *blk = &ring[(b - kWalkLoaders) % kWalkRing];
+      const uint32_t first = (b - kWalkLoaders) * kWalkBlock;
+      const uint32_t count = g.chunks - first < kWalkBlock ? g.chunks - first : kWalkBlock;
+      for (uint32_t c = 0; c < count; c += kChunksAtOnce) {
+        float4 va[kChunksAtOnce];
+        uint2 vb[kChunksAtOnce];
+#pragma unroll
+        for (uint32_t i = 0; i < kChunksAtOnce; ++i) {
+          va[i] = blk->step[c + i];
+          vb[i] = blk->rest[c + i];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kChunksAtOnce; ++i) {
+          const Step m = {va[i].x, va[i].y, va[i].z, va[i].w, vb[i].x, __uint_as_float(vb[i].y)};
+          float to;
+          if (__ballot(column_chunks::Apply(m, sum, &to)) != 0ull) {
+            sum = to;
+            continue;
+          }
+          const uint32_t window = __builtin_amdgcn_readfirstlane(vb[i].y);
+          if (window == kWalkNothing) continue;
+          if (window == kWalkPlusZero) {
+            sum += 0.0f;
+            continue;
+          }
+          float4 *term = blk->term[c + i];
+          if (window != kWalkTerms) {
+            /* the map does not cover the sum */
+            if ((__builtin_amdgcn_readfirstlane(blk->here) >> (c + i) & 1u) == 0u) {
+              const uint32_t row0 = (first + c + i) * column_chunks::kRows;
+              for (uint32_t k = lane; k < static_cast<uint32_t>(column_chunks::kRows); k += kWave) {
+                reinterpret_cast<float *>(term)[k] =
+                    row0 + k < g.rows ? src[static_cast<size_t>(row0 + k) * g.stride + x] : -0.0f;
+              }
+            }
+            /* enough of these and the other waves bring all terms */
+            __hip_atomic_store(&misses, ++missed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            WaveLdsFence();
+          }
+          AddTerms(&sum, term);
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    mshadow::hip::BareBarrier();
+  }
+  if (lane == 0) Saver::template Save<float>(dst[x], sum * scale);
+}
+
+}  // namespace mshadow_hipk
+
+#endif  // MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_

@@ -8,11 +8,13 @@
 
 #include <climits>
 #include <mutex>
+#include <type_traits>
 
 #include <mshadow/hip/kernels/reduce.h>
 #include <mshadow/hip/kernels/reduce_dma.h>
 #include <mshadow/hip/kernels/reduce_segments.h>
 
+#include "column_chunk_kernels.h"
 #include "patch_kernels.h"
 #include "pool_kernels.h"
 #include "row_kernels.h"
@@ -540,8 +542,104 @@ ReduceScratchTable &ScratchTable() {
 }
 }  // namespace
 
+/* Scratch memory of the column sums by chunks (column_chunk_kernels.h): like the above a part of the
+   image, a slot per stream that has asked for one, which keeps it until it is destroyed. A call is three launches that
+   pass their results on in it, so the lock is held while they are queued: two threads that share a
+   stream must not come between each other's. */
+namespace {
+const int kColumnScratchSlots = 4;
+static __device__ __align__(256) ColumnChunkScratch g_column_scratch[kColumnScratchSlots];
+
+struct ColumnScratchTable {
+  std::mutex mu;
+  ColumnChunkScratch *base[kReduceScratchDevices];
+  bool used[kReduceScratchDevices][kColumnScratchSlots];
+  void *owner[kReduceScratchDevices][kColumnScratchSlots];
+
+  /* the caller's slot on the current device, NULL where there is none to be had; mu is held */
+  ColumnChunkScratch *Slot(void *stream) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kReduceScratchDevices) {
+      (void)hipGetLastError();
+      return NULL;
+    }
+    int slot = -1;
+    for (int i = 0; i < kColumnScratchSlots && slot < 0; ++i) {
+      if (used[dev][i] && owner[dev][i] == stream) slot = i;
+    }
+    for (int i = 0; i < kColumnScratchSlots && slot < 0; ++i) {
+      if (!used[dev][i]) slot = i;
+    }
+    if (slot < 0) return NULL;
+    if (base[dev] == NULL) {
+      void *p = NULL;
+      if (hipGetSymbolAddress(&p, HIP_SYMBOL(g_column_scratch)) != hipSuccess) {
+        (void)hipGetLastError();
+        return NULL;
+      }
+      base[dev] = static_cast<ColumnChunkScratch *>(p);
+    }
+    used[dev][slot] = true;
+    owner[dev][slot] = stream;
+    return base[dev] + slot;
+  }
+};
+ColumnScratchTable &ColumnTable() {
+  static ColumnScratchTable t = {};
+  return t;
+}
+
+/* A recorded launch may be replayed on any stream, beside the one whose slot it would use; and the handle of the
+   stream per thread is every thread's. */
+bool HasNoSlot(hipStream_t s) {
+  if (s == hipStreamPerThread) return true;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
+/* whether the sums of the columns were queued, by chunks of their rows */
+template <typename Saver>
+bool LaunchColumnChunks(float *dst, const float *src, uint32_t stride, uint32_t rows, uint32_t cols, float scale,
+                        hipStream_t s) {
+  ChunkShape g;
+  if (!ColumnChunksAreSooner(rows, cols, mshadow_abi::ComputeUnits()) || !MakeChunkShape(rows, cols, stride, &g) || HasNoSlot(s)) return false;
+  ColumnScratchTable &t = ColumnTable();
+  std::lock_guard<std::mutex> lock(t.mu);
+  ColumnChunkScratch *w = t.Slot(s);
+  if (w == NULL) return false;
+  const dim3 grid(g.groups * g.tiles), block(kChunkWaves * 64);
+  LaunchKernelIfFits(ColumnChunkSumsKernel, grid, block, 0, s, src, g, w->before, w->group);
+  LaunchKernelIfFits(ColumnChunkMapsKernel, grid, block, 0, s, src, g, w->before, w->group, w->map, w->copy);
+  LaunchKernelIfFits((ColumnChunkWalkKernel<Saver>), dim3(cols), dim3((1 + kWalkLoaders) * 64), 0, s, dst, src, g, w->map, w->copy, scale);
+  return true;
+}
+}  // namespace
+
 namespace mshadow_abi {
+bool HasColumnScratch(void *stream) {
+  ColumnScratchTable &t = ColumnTable();
+  std::lock_guard<std::mutex> lock(t.mu);
+  for (int d = 0; d < kReduceScratchDevices; ++d) {
+    for (int i = 0; i < kColumnScratchSlots; ++i) {
+      if (t.used[d][i] && t.owner[d][i] == stream) return true;
+    }
+  }
+  return false;
+}
 void ReleaseReduceScratch(void *stream) {
+  {
+    ColumnScratchTable &c = ColumnTable();
+    std::lock_guard<std::mutex> lock(c.mu);
+    for (int d = 0; d < kReduceScratchDevices; ++d) {
+      for (int i = 0; i < kColumnScratchSlots; ++i) {
+        if (c.used[d][i] && c.owner[d][i] == stream) c.used[d][i] = false;
+      }
+    }
+  }
   ReduceScratchTable &t = ScratchTable();
   std::lock_guard<std::mutex> lock(t.mu);
   for (int d = 0; d < kReduceScratchDevices; ++d) {
@@ -924,6 +1022,11 @@ int mshadow_hip_reduce_keep_lowest_f32(float *dst, const float *src, int sstride
          lines a row has the sooner they arrive and the earlier the step decides (10 columns:
          4000 rows 18.9 against 19.5 us, 6143 27.7 against 28.7, 3500 level; 64: 6000 rows 27.2
          against 27.8, 4500 level; one: 2500 rows 12.8 against 13.5, 2200 12.7 against 12.1) */
+      if (std::is_same<R, mshadow::red::sum>::value &&
+          LaunchColumnChunks<S>(dst, src, static_cast<uint32_t>(sstride), static_cast<uint32_t>(rows),
+                                static_cast<uint32_t>(cols), scale, s)) {
+        return MSHADOW_HIP_OK;
+      }
       const int long_chain = cols == 1 ? 2400 : cols <= 64 ? 4000 : kDmaMinRows;
       if (strip == 16 && rows >= long_chain) {
         LaunchKernelIfFits((mshadow::hip::ReduceKeepLowestDmaKernel<S, R>),

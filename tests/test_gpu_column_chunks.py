@@ -1,0 +1,139 @@
+"""sum_rows of long float columns, which are summed by chunks of 128 rows: maps from the sum in front of a chunk to
+the sum behind it, looked up one after the other, or the chunk's terms where there is no map. Bit-exact against the
+oracle's serial sum on both sides of the dispatch's border and of tiles, chunks, workgroups and blocks of the walk,
+and on columns that take each of the ways a chunk can go."""
+import threading
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from checkers import MINUSTO, PLUSTO, SAVETO, SUM, Checker
+from gpu_util import assert_bits_equal, f32
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def G():
+    import mshadow_amd
+    g = mshadow_amd.load_cases()
+    g.set_device(0)
+    return g
+
+
+@pytest.fixture(scope="module")
+def O():
+    return Checker("orc")
+
+
+def terms(kind, rows, cols, seed):
+    rng = np.random.default_rng(seed)
+    m = rng.standard_normal((rows, cols), dtype=f32)
+    if kind == "gradient":
+        p = np.exp(m * 3)
+        m = (p / np.maximum(p.sum(1, keepdims=True), f32(90 * 8))).astype(f32)
+        m[np.arange(rows), rng.integers(0, max(cols, 8), rows) % cols] -= (rng.random(rows) < 0.3).astype(f32)
+    elif kind == "constant":      # every rounding goes the same way: the sums miss their maps
+        m[:] = f32(0.1) * (1 + np.arange(cols, dtype=f32))
+    elif kind == "alternating":   # no map at all
+        m = np.abs(m) * np.where(np.arange(rows) % 2, f32(-1), f32(1))[:, None]
+    elif kind == "zeros":         # nothing to add, of either sign, with a few terms between
+        m[:] = np.where(rng.random((1, cols)) < 0.5, f32(-0.0), f32(0.0))
+        m[rows // 3] = rng.integers(-1, 2, cols)
+        m[rows // 2, ::3] = f32(0.0)
+    elif kind == "ties":
+        m = np.round(m * 64).astype(f32) / 64 + f32(2.0 ** -18)
+    elif kind == "wide":
+        m = (m * np.exp2(rng.integers(-40, 40, m.shape))).astype(f32)
+    elif kind == "tiny":
+        m = (m * f32(1e-38)).astype(f32)
+    elif kind == "infinite":
+        m[rng.integers(0, rows, cols), np.arange(cols)] = np.where(np.arange(cols) % 3 == 0, -np.inf, np.inf)
+        m[rows - 1, ::4] = np.nan
+    return np.ascontiguousarray(m)
+
+
+# up to 64 columns from 6400 rows on, 100 from 6695, 1000 from 15455 (8 to 1536 columns otherwise); chunks of 128 rows,
+# workgroups of four chunks and 64 columns, blocks of 16 chunks
+SHAPES = [(6300, 10), (6400, 10), (6528, 64), (6529, 65), (6783, 63), (8192, 1), (8193, 3), (8320, 129), (10240, 128),
+          (16384, 1000), (20481, 17), (33000, 300)]
+
+
+@pytest.mark.parametrize("rows,cols", SHAPES)
+def test_long_columns(G, O, rows, cols):
+    for kind, extra, shift in (("normal", 0, 0), ("gradient", 3, 1)):
+        wide = terms(kind, rows, cols + extra, 7)
+        m = np.ascontiguousarray(wide[:, shift:shift + cols])
+        src = G.to_device(wide)
+        view = SimpleNamespace(ptr=src.ptr + shift * 4, stride=src.stride, rows=rows, cols=cols, dtype=src.dtype,
+                               shape=(rows, cols))
+        start = np.random.default_rng(8).standard_normal(cols, dtype=f32)
+        for saver in (SAVETO, PLUSTO, MINUSTO):
+            want, dst = start.copy(), G.to_device(start)
+            O.reduce_keep_lowest(want, m, SUM, saver, 0.75)
+            G.reduce_keep_lowest(dst, view, SUM, saver, 0.75)
+            assert_bits_equal(dst.download(), want, f"{rows}x{cols} {kind} saver {saver}")
+
+
+@pytest.mark.parametrize("kind", ["constant", "alternating", "zeros", "ties", "wide", "tiny", "infinite"])
+def test_columns_whose_chunks_have_no_map(G, O, kind):
+    rows, cols = 12345, 70
+    m = terms(kind, rows, cols, 11)
+    want, dst = np.empty(cols, f32), G.to_device(np.full(cols, 7, f32))
+    with np.errstate(all="ignore"):
+        O.reduce_keep_lowest(want, m)
+    for _ in range(2):   # the scratch memory as the first call left it
+        G.reduce_keep_lowest(dst, G.to_device(m))
+        got = dst.download()
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got), nan)
+        assert_bits_equal(got[~nan], want[~nan], kind)
+
+
+def test_streams_threads_and_recording(G, O):
+    """streams have scratch memory of their own, more of them than there is such memory for among them; threads that
+    share a stream do not come between each other's launches; a recorded call does without"""
+    mats = [terms("normal", 7000 + 300 * i, 40, 20 + i) for i in range(6)]
+    want = []
+    for m in mats:
+        w = np.empty(40, f32)
+        O.reduce_keep_lowest(w, m)
+        want.append(w)
+    src = [G.to_device(m) for m in mats]
+    out = [G.buffer((40,), f32) for _ in mats]
+    streams = [G.stream_create() for _ in mats]
+    for _ in range(3):
+        for i, s in enumerate(streams):
+            G.reduce_keep_lowest(out[i], src[i], stream=s)
+    for i, s in enumerate(streams):
+        G.stream_sync(s)
+        assert_bits_equal(out[i].download(), want[i], f"stream {i}")
+
+    def work(i):
+        G.set_device(0)
+        for _ in range(20):
+            G.reduce_keep_lowest(out[i], src[i], stream=streams[0])
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    G.stream_sync(streams[0])
+    for i in range(4):
+        assert_bits_equal(out[i].download(), want[i], f"thread {i}")
+
+    G.graph_begin(streams[1])
+    G.reduce_keep_lowest(out[2], src[2], stream=streams[1])
+    graph = G.graph_end(streams[1])
+    for _ in range(3):
+        G.fill(out[2], 3.0, streams[1])
+        G.graph_launch(graph, streams[1])
+        G.reduce_keep_lowest(out[3], src[3], stream=streams[1])
+        G.stream_sync(streams[1])
+        assert_bits_equal(out[2].download(), want[2], "replayed")
+        assert_bits_equal(out[3].download(), want[3], "beside a replay")
+    G.graph_destroy(graph)
+    for s in streams:
+        G.stream_destroy(s)

@@ -186,6 +186,14 @@ def test_signed_column_sums_leave_most_of_the_chain(tmp_path):
     assert shares[1] < 0.01 and shares[64] < 0.2 and hold[16] > 0.94 and 0.8 < hold[64] < 0.95, (shares, hold)
 
 
+def test_column_sums_by_chunks_match_the_serial_sum_on_host(tmp_path):
+    """the chunk maps of the long column sums, walked on the host with the device code's own functions:
+    bit-identical to the serial loop on columns of every kind, with the expected sums also well beside
+    the true ones, and on drawn columns and a classifier's gradients nearly every chunk has a map"""
+    out = _compile_and_run(tmp_path, "column_chunks_sim.cc", [])
+    assert out.endswith("OK\n"), out[-500:]
+
+
 def test_half_sum_pruning_rule_is_exhaustively_sound(tmp_path):
     """the binary16 softmax row sum leaves out the terms below half an ulp of a lower bound of
     the running sum: for every pair of a finite non-negative binary16 sum and term the rule
