@@ -6,6 +6,7 @@ loudly when the library has not been built (run `python -c "import __graft_entry
 g.build()"` or `python -m mshadow_amd.build`).
 """
 import ctypes as C
+import math
 import os
 
 import numpy as np
@@ -26,6 +27,11 @@ _d, _ll = C.c_double, C.c_longlong
 
 class HipError(RuntimeError):
     pass
+
+
+def _planes(shape):
+    """what numpy's product gives (2.4 us of a call whose launch takes 2.5), without it"""
+    return math.prod(shape[:-2])
 
 
 class Props(C.Structure):
@@ -413,14 +419,14 @@ class Library:
     def pool(self, dst, src, ky, kx, sy, sx, reducer=MAX, stream=None):
         h, w = src.shape[-2:]
         ph, pw = dst.shape[-2:]
-        planes = int(np.prod(src.shape[:-2]))
+        planes = _planes(src.shape)
         self.check(self.dll.mshadow_hip_pool_f32(dst.ptr, dst.stride, src.ptr, src.stride, planes,
                                                  h, w, ph, pw, ky, kx, sy, sx, reducer, stream))
 
     def unpool(self, dst, src, pooled, grad, ky, kx, sy, sx, reducer=MAX, stream=None):
         h, w = src.shape[-2:]
         ph, pw = pooled.shape[-2:]
-        planes = int(np.prod(src.shape[:-2]))
+        planes = _planes(src.shape)
         self.check(self.dll.mshadow_hip_unpool_f32(
             dst.ptr, dst.stride, src.ptr, src.stride, pooled.ptr, pooled.stride, grad.ptr,
             grad.stride, planes, h, w, ph, pw, ky, kx, sy, sx, reducer, stream))
@@ -581,9 +587,11 @@ class Library:
                            variant, stream))
 
     def case_softmax(self, dst, src, stream=None):
-        fn = {"float32": self.cases.mshadow_case_softmax_f32,
-              "uint16": self.cases.mshadow_case_softmax_f16,
-              "float64": self.cases.mshadow_case_softmax_f64}[src.dtype.name]
+        if src.dtype == np.uint16:
+            fn = self.cases.mshadow_case_softmax_f16
+        else:
+            fn = {"float32": self.cases.mshadow_case_softmax_f32,
+                  "float64": self.cases.mshadow_case_softmax_f64}[src.dtype.name]
         self.check_case(fn(dst.ptr, dst.stride, src.ptr, src.stride, src.rows, src.cols, stream))
 
     def case_softmax_grad(self, dst, src, label, stream=None):
@@ -614,7 +622,7 @@ class Library:
     def case_pool(self, dst, src, ky, kx, sy, sx, reducer=MAX, variant=0, stream=None):
         h, w = src.shape[-2:]
         ph, pw = dst.shape[-2:]
-        planes = int(np.prod(src.shape[:-2]))
+        planes = _planes(src.shape)
         if src.dtype == np.uint16:   # half_t tensors: the expression API
             self.check_case(self.cases.mshadow_case_pool_f16(
                 dst.ptr, dst.stride, src.ptr, src.stride, planes, h, w, ph, pw, ky, kx, sy, sx,
@@ -628,7 +636,7 @@ class Library:
                     stream=None):
         h, w = src.shape[-2:]
         ph, pw = pooled.shape[-2:]
-        planes = int(np.prod(src.shape[:-2]))
+        planes = _planes(src.shape)
         self.check_case(self.cases.mshadow_case_unpool_f32(
             dst.ptr, dst.stride, src.ptr, src.stride, pooled.ptr, pooled.stride, grad.ptr,
             grad.stride, planes, h, w, ph, pw, ky, kx, sy, sx, reducer, variant, stream))
