@@ -28,11 +28,20 @@ struct Addend {
   int check;  // binade the sum must be in before and after this addend; -1: a term, no check
 };
 
+/* terms that the slabs of the kernel for rows of this length hold (few rows), those behind the row's end zeros */
+static size_t SlabTerms(size_t cols) {
+  for (size_t slabs : {1024, 2048, 4096, 8192, 16384, 32768, 51200, 65536, 81920, 110592}) {
+    if (cols <= slabs) return slabs;
+  }
+  return cols;
+}
+
 template <int N>
 static bool PlannedSum(const std::vector<float> &row, size_t capacity, float *result, size_t *addends) {
   const int chunk_terms = 64 * N;
   std::vector<float> t(row);
   while (t.size() % chunk_terms) t.push_back(0.0f);
+  if (N == 4) t.resize(std::max(t.size(), SlabTerms(t.size())), 0.0f);
   const int nch = static_cast<int>(t.size() / chunk_terms);
   // A: approximate sum and largest term of every chunk
   std::vector<float> approx(nch), cmax(nch);
@@ -102,6 +111,7 @@ static bool PlannedSum(const std::vector<float> &row, size_t capacity, float *re
     flush();
     const size_t before_chunk = list.size();
     ++listed;
+    if (approx[k] == 0.0f) continue;  // zeros, which change no sum
     // lane-level plan of a chunk that is not clean as a whole
     float incl = 0.0f, seen = 0.0f;
     int prev = -1;
@@ -127,7 +137,7 @@ static bool PlannedSum(const std::vector<float> &row, size_t capacity, float *re
         lrun = 0;
       }
       if (c < 0) {
-        for (int i = 0; i < N; ++i) list.push_back({lane[l][i], -1});
+        for (int i = 0; i < N && a != 0.0f; ++i) list.push_back({lane[l][i], -1});
       } else {
         lrun += q.q;
       }
@@ -208,7 +218,7 @@ int main() {
     }
   }
   // sums that end just above a power of two: every chunk behind the crossing is listed
-  for (int n : {32000, 50257, 100000}) {
+  for (int n : {5000, 10000, 16808, 32000, 33000, 50257, 51300, 66000, 90000, 100000}) {
     for (double above : {1e-5, 1e-4, 1e-3, 5e-3}) {
       for (int rep = 0; rep < 4; ++rep) {
         std::vector<double> x(n);
