@@ -22,7 +22,8 @@ struct SegmentsPlan {
  *  index is done before the other kernels would be, which deal the planes of an index out.
  *  The split kernel takes, in us, 8 + 0.08 n or 6 + 0.085 n (its last workgroup's chains) and 8 TB/s of what it reads;
  *  binary16 10 + 0.09 n and 2 TB/s. A workgroup of this kernel takes 3 us and 32 GB/s, 47 where planes begin with their
- *  cache lines (binary16 30 and 39), and an element of a chain 10 ns (binary16 7). As measured, split and this one: floats
+ *  cache lines (binary16 30 and 39), and an element of a chain 5 ns (binary16 6) where the chains
+ *  of a CU are few. As measured, split and this one: floats
  *  (256,16,1024) 29 and 24, (1024,8,1024) 91 and 84, (2048,32,784) 215 and 196, (2048,16,1024) 197 and 166, (200,100,400)
  *  38 and 16, (60,190,1500) 30 and 19; but (512,16,784) 49.4 and 50.7, (512,16,1500) 54 and 93, (1024,16,1500) 105 and
  *  176, (2048,1,784) 151 and 179, (2048,4,2048) 178 and 400, (160,40,2296) 27 and 45, (64,64,12544) 52 and 78. Binary16
@@ -30,8 +31,8 @@ struct SegmentsPlan {
  *  the generic kernel has otherwise, (512,16,2025) 141 and 96. Short reductions: 32 planes of 196 6.2 and 4.9, 41 of 132
  *  5.6 and 4.7, 128 of 100 8.8 and 6.5, but 64 of 100 5.4 and 5.7, 35 of 56 4.3 and 5.1, binary16 40 of 255 7.7 and 8.4. */
 inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, int least_len) {
-  if (!((len <= 1100 && planes >= 2048) || (len <= 2048 && planes >= 8192))) return false;
   const bool half = least_len == 8;
+  if (n_out <= 4 && !half) return false;  // a chain lane a plane and nothing to deal out: (2,16,11445) 54 and 58
   if (n_out * len < 1u << 16) {  // the end of a plane is added value by value: half a slice of 128 halves takes longer
     return n_out > 64 || (len >= 128 && (!half || len >= 256 || len % 128 <= 64));
   }
@@ -43,14 +44,14 @@ inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, int
   const bool lines = bytes / n_out % 128 == 0;
   if (half) {
     const uint64_t split = 10000 + 90 * n_out + all / 2000;  // ns, as below; rates are bytes a ns
-    return bytes <= split * (lines ? 39 : 30) && len * 7 <= split;
+    return bytes <= split * (lines ? 39 : 30) && len * 6 <= split;
   }
   const uint64_t split = (n_out <= 400 ? 8000 + 80 * n_out : 6000 + 85 * n_out) + all / 8000;
-  return 3000 + bytes / (lines ? 47 : 32) <= split && len * 10 <= split;
+  return 3000 + bytes / (lines ? 47 : 32) <= split && 3000 + len * 5 <= split;
 }
-/*! \brief short reductions of many kept indices (fewer than 65536 values of each): whether the ends of their planes, which
- *  are added value by value - what is left of the last slice of 64 floats or 128 halves -, cost this kernel more than it
- *  wins. In us, the kernel of a workgroup per index and this one: floats (46,409,120) 6.3 and 7.0, (95,745,50) 9.7 and 10.7,
+/*! \brief short reductions of many kept indices (fewer than 65536 values of each): whether the ends of their planes - what
+ *  is left of the last slice of 64 floats or 128 halves, which passes through LDS value by value - cost this kernel more than
+ *  it wins. In us, the kernel of a workgroup per index and this one: floats (46,409,120) 6.3 and 7.0, (95,745,50) 9.7 and 10.7,
  *  (4,667,756) 8.0 and 10.0, but (65,208,117) 8.8 and 6.7, (4,1928,637) 14.2 and 12.3; binary16 (38,1675,55) 7.3 and 10.9,
  *  (20,346,231) 7.2 and 8.0, (2,1439,1005) 10.2 and 15.9, but (112,335,56) 8.7 and 7.0, (22,422,198) 7.3 and 6.7, (4,1800,840)
  *  level, and planes of two slices and more, (43,835,1275) 38.8 and 27.0. */
@@ -60,20 +61,22 @@ inline bool SegmentEndsWeighMore(uint32_t n_out, uint32_t n_keep, uint64_t plane
     if (n_out <= 4) return len % 128 > 72;
     return (len < 128 && !one_round) || (len >= 128 && len < 256 && len % 128 > 72);
   }
-  if (n_out <= 4) return len > 600 && planes < 2800;
+  if (n_out <= 4) return len > 600 && planes < 2800 && len % 64 >= 44;
   return len < 128 && len % 64 >= 44 && n_out >= 24 && !one_round;
 }
-/*! \brief Measured on (n, c, len), us, the other kernels and this one; floats, binary16 gains as much. It wants planes
- *  enough for a wave of sixteen on every SIMD or nearly, and wins by what the others leave idle.
+/*! \brief Measured on (n, c, len), us, the other kernels and this one; floats, binary16 gains as much.
  *  A workgroup per kept index that fills a CU: (248,552,280) 70 and 42, (30,600,2500) 74
- *  and 44, (19,304,5760) 93 and 35, (5,1144,8320) 115 and 49, where chain lanes (n up to the next 64, 16 or 4) and
- *  the last round of workgroups are idle for more than three tenths; (64,256,3136) 35.6 and 40, (64,512,1600) 43 and 41.
+ *  and 44, (19,304,5760) 93 and 35, (5,1144,8320) 115 and 49, (114,246,896) 22 and 18, (248,416,450) 54 and 42, where chain
+ *  lanes (n up to the next 64, 16 or 4) and the last round of workgroups are idle for more than a tenth; (64,256,3136) 35.6
+ *  and 40, (64,512,1600) 43 and 41, (16,249,5512) 27 and 29.
  *  Up to a kept index a CU there is one round of either, and up to 64 planes an index what counts are the lanes:
  *  (32,192,3136) 28 and 23, (48,192,3136) 29 and 26, but (48,255,3136) 29 and 31, (64,192,3136) 29.5 and 31; binary16
  *  (32,192,3136) 19.5 and 16.8, but (48,192,3136) 19.6 and 21, (64,192,1640) 14.3 and 16.2.
  *  A workgroup of four waves per kept index, for fewer than 65536 values of each: (17,896,260) 11.7 and 7.2,
- *  (39,957,384) 14.9 and 11.9, but (8,573,240) 5.1 and 6.3, (256,500,100) 19.8 and 22.3. One plane per kept index,
- *  which is one lane there: (1,2048,3136) 46 and 20. */
+ *  (39,957,384) 14.9 and 11.9, (5,1519,3920) 63 and 28, (12,1448,592) 15.7 and 9.5, (16,1400,140) 7.1 and 4.9, (2,1912,2048)
+ *  25.6 and 13.3, (7,216,3392) 24 and 20, and with few kept indices (24,24,2208) 35 and 18, (28,184,1536) 25.5 and 11.4; small
+ *  ones are level within 0.4 us, which is less than their launch. One plane per kept index, which is one lane there:
+ *  (1,2048,3136) 46 and 20, (1,536,5184) 36 and 26, but (1,59,3696) 16.5 and 20; binary16 (1,72,1392) 8.8 and 7.3. */
 inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, uint32_t cus, int least_len) {
   SegmentsPlan p = {false, 16, 1, 1};
   const uint64_t planes = static_cast<uint64_t>(n_out) * n_keep;
@@ -83,26 +86,24 @@ inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, 
     return p;
   }
   const bool few_kept = static_cast<uint64_t>(n_keep) * 4 < 3ull * cus;
-  const bool middling = n_out >= 5 && n_out <= 16;
   const uint32_t side = n_out > 16 ? 64 : n_out > 4 ? 16 : n_out > 1 ? 4 : 1;
   const uint64_t lanes = (n_out + side - 1) / side * side, turns = (n_keep + cus - 1) / cus * cus;
   if (few_kept) {
-    p.use = !middling && SegmentsOfFewKept(n_out, planes, len, least_len);
+    p.use = n_out == 1 ? least_len == 8 && n_keep >= 64 && len >= 512 : SegmentsOfFewKept(n_out, planes, len, least_len);
   } else if (n_out == 1) {
-    p.use = n_keep >= 2 * cus && len <= 4096 && planes * len >= 800000;
+    p.use = n_keep >= 2 * cus || (least_len == 8 && len >= 512);
   } else if (n_out * len >= 1u << 16) {
-    p.use = planes >= 2048 && lanes * turns * 100 > planes * 130;
+    p.use = planes >= 2048 && lanes * turns * 100 > planes * 112;
     if (n_out > 40 && n_out <= 64 && n_keep <= cus) {
       p.use = p.use && least_len == 4 && n_out <= 48 && n_keep * 16ull < 15ull * cus;
     }
   } else {
-    p.use = !middling && ((len <= 1100 && planes >= 2048) || planes >= 4096) && (n_out <= 4 || lanes * 100 > n_out * 102ull) &&
-            !SegmentEndsWeighMore(n_out, n_keep, planes, len, cus, least_len);
+    p.use = !SegmentEndsWeighMore(n_out, n_keep, planes, len, cus, least_len);
   }
   if (!p.use) return p;
-  /* more waves: (32,512,784) 12.4, with sixteen 13.3; not more than a workgroup has, whose waves go round again:
-     (256,16,1024) 32 that way, with sixteen 24 */
-  if (len >= 512 && planes / 16 < 4 * cus && n_out <= 8 * kSegMostWaves) p.lanes = 8;
+  /* more waves: (32,512,784) 12.4, with sixteen 13.3; up to two waves a SIMD of a workgroup's CU, which take turns
+     beyond that */
+  if (len >= 512 && planes / 16 < 4 * cus && n_out <= 64) p.lanes = 8;
   /* workgroups of four waves or so where planes are few per kept index, but one for every CU */
   while (p.kept * n_out < 4u * p.lanes && n_keep / (p.kept + 1) >= cus) ++p.kept;
   const uint32_t all = (p.kept * n_out + p.lanes - 1) / p.lanes;
