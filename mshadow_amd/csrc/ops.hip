@@ -207,7 +207,9 @@ int Im2Col(T *col, int cstride, const T *img, int istride, const PatchGeom &g, v
   if (band > g.oh) band = g.oh;
   const long long planes = static_cast<long long>(g.n) * g.c;
   while (band > 8 && planes * ((g.oh + band - 1) / band) < 1024) band = (band + 1) / 2;
-  if (band >= 1) {
+  /* patch rows shorter than a pack would be written element by element there */
+  const bool short_rows = g.ow < EPT && cols < (1ll << 31) && (cols + kPatchBlock * EPT - 1) / (kPatchBlock * EPT) * rows < (1ll << 31);
+  if (band >= 1 && !short_rows) {
     const long long nb = (g.oh + band - 1) / band;
     band = (g.oh + nb - 1) / nb;
     PatchTile t;
@@ -221,13 +223,13 @@ int Im2Col(T *col, int cstride, const T *img, int istride, const PatchGeom &g, v
     LaunchKernelIfFits((Im2ColTiledKernel<T, EPT>), dim3(static_cast<unsigned>(blocks)),
                        dim3(kPatchBlock), lds, AsStream(stream), col, cstride, img, istride, g, t);
   } else {
-    const unsigned chunks =
-        static_cast<unsigned>((cols + kPatchBlock * EPT - 1) / (kPatchBlock * EPT));
+    const long long chunks = (cols + kPatchBlock * EPT - 1) / (kPatchBlock * EPT);
     const long long blocks = rows * chunks;
     if (blocks >= (1ll << 31)) return Fail(MSHADOW_HIP_ERR_ARGUMENT, "im2col: too many workgroups");
     LaunchKernelIfFits((Im2ColKernel<T, EPT>), dim3(static_cast<unsigned>(blocks)),
                        dim3(kPatchBlock), 0, AsStream(stream), col, cstride, img, istride, g,
-                       chunks);
+                       static_cast<unsigned>(chunks), mshadow::FastDivU32(static_cast<uint32_t>(chunks)),
+                       mshadow::FastDivU32(static_cast<uint32_t>(g.ow)), mshadow::FastDivU32(static_cast<uint32_t>(g.oh)));
   }
   return AfterLaunch("im2col");
 }
@@ -317,6 +319,29 @@ int Col2Im(T *img, int istride, const T *col, int cstride, const PatchGeom &g, v
                          img, istride, col, cstride, g, dv, mshadow::FastDivU32(static_cast<uint32_t>(wpk)),
                          mshadow::FastDivU32(static_cast<uint32_t>(g.h)),
                          mshadow::FastDivU32(static_cast<uint32_t>(g.c)), static_cast<uint32_t>(packs));
+      return AfterLaunch("col2im");
+    }
+  }
+  /* image rows shorter than a pack: pixel by pixel (3x3 on (128,256,7,7) binary16 236 us staged) */
+  {
+    const int over_y = (g.ky + g.sy - 1) / g.sy, over_x = (g.kx + g.sx - 1) / g.sx;
+    const int over = over_y > over_x ? over_y : over_x;
+    if (g.w < EPT && g.dy == 1 && g.dx == 1 && over <= 5 && total + kPatchBlock < (1ll << 31) && cols < (1ll << 31)) {
+      const PatchDivs dv = {mshadow::FastDivU32(static_cast<uint32_t>(g.sy)),
+                            mshadow::FastDivU32(static_cast<uint32_t>(g.sx)), mshadow::FastDivU32(1u),
+                            mshadow::FastDivU32(1u)};
+#define COL2IM_PIXEL(TY, TX)                                                                                       \
+  LaunchKernelIfFits((Col2ImPixelKernel<T, TY, TX>),                                                               \
+                     dim3(static_cast<unsigned>((total + kPatchBlock - 1) / kPatchBlock)), dim3(kPatchBlock), 0,   \
+                     AsStream(stream), img, istride, col, cstride, g, dv,                                          \
+                     mshadow::FastDivU32(static_cast<uint32_t>(g.w)), mshadow::FastDivU32(static_cast<uint32_t>(g.h)), \
+                     mshadow::FastDivU32(static_cast<uint32_t>(g.n)), static_cast<uint32_t>(total))
+      if (over <= 1) COL2IM_PIXEL(1, 1);
+      else if (over == 2) COL2IM_PIXEL(2, 2);
+      else if (over == 3) COL2IM_PIXEL(3, 3);
+      else if (over == 4) COL2IM_PIXEL(4, 4);
+      else COL2IM_PIXEL(5, 5);
+#undef COL2IM_PIXEL
       return AfterLaunch("col2im");
     }
   }

@@ -749,54 +749,52 @@ __global__ void __launch_bounds__(kPatchBlock)
   }
 }
 
-/*! \brief EPT consecutive column-matrix elements per thread; grid.x = rows of the column
- *  matrix (c, a, b) times `chunks` pieces of kPatchBlock * EPT columns each. */
+/*! \brief EPT consecutive column-matrix elements per thread, wherever patch rows end; grid.x = rows of the column
+ *  matrix (c, a, b) times `chunks` pieces of kPatchBlock * EPT columns each. For patch rows shorter than a pack, which
+ *  the other kernels would write element by element: 3x3 stride 2 on (96,112,48,13) binary16, patch rows of 7, 52 us staged.
+ *  An element is a load of its own, all of a thread's under way together (one that is outside the image reads its
+ *  channel's first and is dropped); neighbouring lanes find them in the same cache lines. */
 template <typename T, int EPT>
 __global__ void __launch_bounds__(kPatchBlock)
-    Im2ColKernel(T *col, int cstride, const T *img, int istride, PatchGeom g, unsigned chunks) {
-  const int i = blockIdx.x / chunks;
-  const int piece = blockIdx.x - i * chunks;
-  const int b = (i % g.kx) * g.dx;
-  const int irest = i / g.kx;
-  const int a = (irest % g.ky) * g.dy;
-  const int ch = irest / g.ky;
-  const int ncols = g.n * g.oh * g.ow;
-  const int j0 = (piece * kPatchBlock + threadIdx.x) * EPT;
+    Im2ColKernel(T *col, int cstride, const T *img, int istride, PatchGeom g, unsigned chunks, mshadow::FastDivU32 div_chunks,
+                 mshadow::FastDivU32 div_ow, mshadow::FastDivU32 div_oh) {
+  typedef T Pack __attribute__((ext_vector_type(EPT)));
+  typedef Pack LoosePack __attribute__((aligned(sizeof(T))));
+  const uint32_t i = div_chunks.Div(blockIdx.x), piece = blockIdx.x - i * chunks;
+  const uint32_t irest = i / g.kx;
+  const int b = static_cast<int>(i - irest * g.kx) * g.dx;
+  const uint32_t ch = irest / g.ky;
+  const int a = static_cast<int>(irest - ch * g.ky) * g.dy;
+  const uint32_t ncols = static_cast<uint32_t>(g.n) * g.oh * g.ow;
+  const uint32_t j0 = (piece * kPatchBlock + threadIdx.x) * EPT;
   if (j0 >= ncols) return;
-  int ox = j0 % g.ow;
-  int jrest = j0 / g.ow;
-  int oy = jrest % g.oh;
-  int n = jrest / g.oh;
-  T vals[EPT];
+  const uint32_t jrest = div_ow.Div(j0);
+  int ox = static_cast<int>(j0 - jrest * g.ow);
+  int n = static_cast<int>(div_oh.Div(jrest));
+  int oy = static_cast<int>(jrest) - n * g.oh;
+  const T *plane = img + (static_cast<size_t>(n) * g.c + ch) * g.h * istride;
+  const size_t image = static_cast<size_t>(g.c) * g.h * istride;
+  Pack vals;
+  bool in[EPT];
 #pragma unroll
   for (int e = 0; e < EPT; ++e) {
-    T v = 0;
-    if (j0 + e < ncols) {
-      /* coordinates in the padded image; outside the stored image reads as zero */
-      const int y = oy * g.sy + a - g.pad_y;
-      const int x = ox * g.sx + b - g.pad_x;
-      if (y >= 0 && y < g.h && x >= 0 && x < g.w) {
-        v = img[(static_cast<size_t>(n * g.c + ch) * g.h + y) * istride + x];
-      }
-    }
-    vals[e] = v;
+    /* coordinates in the image; outside it the matrix has zeros */
+    const int y = oy * g.sy + a - g.pad_y, x = ox * g.sx + b - g.pad_x;
+    in[e] = y >= 0 && y < g.h && x >= 0 && x < g.w && j0 + e < ncols;
+    vals[e] = *(in[e] ? plane + static_cast<size_t>(y) * istride + x : img);
     if (++ox == g.ow) {
       ox = 0;
       if (++oy == g.oh) {
         oy = 0;
-        ++n;
+        plane += image;
       }
     }
   }
-  T *out = col + static_cast<size_t>(i) * cstride + j0;
-  const bool vec_ok = (j0 + EPT <= ncols) &&
-                      (reinterpret_cast<uintptr_t>(out) % (sizeof(T) * EPT) == 0);
-  if (vec_ok) {
-    typedef T Vec __attribute__((ext_vector_type(EPT)));
-    Vec pack;
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) pack[e] = vals[e];
-    *reinterpret_cast<Vec *>(out) = pack;
+  for (int e = 0; e < EPT; ++e) vals[e] = in[e] ? vals[e] : static_cast<T>(0);
+  T *out = col + static_cast<size_t>(i) * cstride + j0;
+  if (j0 + EPT <= ncols) {
+    *reinterpret_cast<LoosePack *>(out) = vals;
   } else {
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
@@ -912,6 +910,46 @@ __global__ void __launch_bounds__(kPatchBlock)
     SetPackElement(&acc, e, res);
   }
   StorePackAnywhere(img + static_cast<size_t>(rowi) * istride + x0, acc);
+}
+
+/*! \brief Col2ImGatherFlatKernel for image rows shorter than a pack: a thread sums one pixel. The pixels are numbered
+ *  (channel, n, y, x), so that neighbouring threads read on in the same rows of the column matrix, of which there are ky * kx
+ *  times as many bytes as of the image: planes of 7 x 7 binary16 went to the staged kernel, a workgroup and a barrier for
+ *  49 pixels (3x3 on (128,256,7,7): 236 us). */
+template <typename T, int TY, int TX>
+__global__ void __launch_bounds__(kPatchBlock)
+    Col2ImPixelKernel(T *img, int istride, const T *col, int cstride, PatchGeom g, PatchDivs dv, mshadow::FastDivU32 div_w,
+                      mshadow::FastDivU32 div_h, mshadow::FastDivU32 div_n, uint32_t total) {
+  const uint32_t pixel = blockIdx.x * kPatchBlock + threadIdx.x;
+  if (pixel >= total) return;
+  const uint32_t row = div_w.Div(pixel), plane = div_h.Div(row), ch = div_n.Div(plane);
+  const int cx = static_cast<int>(pixel - row * g.w), cy = static_cast<int>(row - plane * g.h);
+  const uint32_t n = plane - ch * g.n;
+  const int y = cy + g.pad_y, x = cx + g.pad_x;      // position in the padded image
+  const int py_min = y < g.ky ? 0 : static_cast<int>(dv.sy.Div(y - g.ky + g.sy));
+  const int py_max = min(static_cast<int>(dv.sy.Div(y + g.sy)), g.oh);
+  const int px_min = x < g.kx ? 0 : static_cast<int>(dv.sx.Div(x - g.kx + g.sx));
+  const int px_max = min(static_cast<int>(dv.sx.Div(x + g.sx)), g.ow);
+  const T *base = col + static_cast<size_t>(ch) * g.ky * g.kx * cstride + static_cast<size_t>(n) * g.oh * g.ow;
+  T term[TY][TX];
+#pragma unroll
+  for (int i = 0; i < TY; ++i) {
+    const int py = py_min + i, a = y - py * g.sy;
+#pragma unroll
+    for (int j = 0; j < TX; ++j) {
+      const int px = px_min + j, b = x - px * g.sx;
+      const bool there = py < py_max && px < px_max;
+      const T v = base[there ? static_cast<size_t>(a * g.kx + b) * cstride + py * g.ow + px : 0];
+      term[i][j] = there ? v : Acc<T>::Zero();
+    }
+  }
+  T res = Acc<T>::Zero();
+#pragma unroll
+  for (int i = 0; i < TY; ++i) {
+#pragma unroll
+    for (int j = 0; j < TX; ++j) res = Acc<T>::Add(res, term[i][j]);
+  }
+  img[((static_cast<size_t>(n) * g.c + ch) * g.h + cy) * istride + cx] = res;
 }
 
 /*! \brief eight bytes of the column matrix at any element border */
