@@ -3,7 +3,7 @@
  * launches: the chunks' sums in any order, their maps, and a walk down every column. The matrix is read twice, by
  * all CUs, where a strip of columns a workgroup leaves most of them idle; the sequence of a column is left
  * to one wave, which takes a chunk in 60 ns, and one that has no map in 500, where 128 dependent adds
- * take 450. 65536 x 1000: 50, 56 and 58 to 75 us (the last by the column with the fewest maps).
+ * take 450. 65536 x 1000: 50, 56 and 60 to 63 us (the last by the column with the fewest maps).
  */
 #ifndef MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_
 #define MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_
@@ -55,8 +55,8 @@ inline bool MakeChunkShape(uint32_t rows, uint32_t cols, uint32_t stride, ChunkS
 }
 
 /*! \brief where the chunks are the sooner way. Measured, us (MI355X; a classifier's gradients), without and with:
- *  131072 x 10 448 and 109, 131072 x 100 470 and 120, 65536 x 1000 232 and 185, 30000 x 100 114 and 46, 16384 x 1000
- *  64 and 53, 16384 x 100 65 and 31, 8192 x 100 36 and 24, 8192 x 10 34 and 26; level at 8192 x 1000 and 4096 x 64,
+ *  131072 x 10 448 and 99, 131072 x 100 470 and 109, 65536 x 1000 232 and 169, 30000 x 100 114 and 44, 16384 x 1000
+ *  64 and 53, 16384 x 100 65 and 30, 8192 x 100 36 and 23, 8192 x 10 34 and 26; level at 8192 x 1000 and 4096 x 64,
  *  slower at 16384 x 4096 (72 and 180: its reads alone take as long as its chain). Without, a row takes 3.5 ns; with,
  *  0.8 ns, 1.6 ps a column for the second read of the matrix and the less than full rate of the first, and
  *  17 us for the three launches. More than six columns a CU walk in turns. Columns whose sum misses
@@ -235,6 +235,9 @@ __device__ __forceinline__ void WaveLdsFence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
+/*! \brief columns up to which the walk takes its maps sixteen at once */
+inline uint32_t ColumnsOfWideWalk(uint32_t cus) { return 2u * cus; }
+
 /*! \brief 128 additions, the terms read from LDS a block of 32 ahead */
 __device__ __forceinline__ void AddTerms(float *sum, const float4 *term) {
   const int kBlock = 8, kBlocks = column_chunks::kRows / 4 / kBlock;
@@ -259,10 +262,8 @@ __device__ __forceinline__ void AddTerms(float *sum, const float4 *term) {
   }
 }
 
-/*! \brief chunks the walk takes between two barriers, and of these how many at a time; blocks on their way or
- *  in use; waves that bring them in turn */
+/*! \brief chunks the walk takes between two barriers; blocks on their way or in use; waves that bring them in turn */
 const uint32_t kWalkBlock = 16;
-const uint32_t kChunksAtOnce = 8;
 const uint32_t kWalkLoaders = 2;
 const uint32_t kWalkRing = kWalkLoaders + 1;
 /*! \brief in the place of a window: the terms are here; there are none; there are only zeros, a +0 among them */
@@ -276,8 +277,12 @@ struct WalkBlock {
 
 /*! \brief the sums themselves: a wave walks down a column, every lane with the same sum, and reads nothing but
  *  LDS. Two more bring it the maps, and the terms of the chunks that have none: a block each in turn,
- *  asked for two blocks ahead. Bound by the walk's sequence: a wave alone issues an instruction every 3.5 ns. */
-template <typename Saver>
+ *  asked for two blocks ahead. Bound by the walk's sequence: a wave alone issues an instruction every 3.5 ns.
+ *  AT_ONCE: maps in registers together. All of a block where two columns a CU at most leave the registers for it
+ *  (65536 x 64 of columns with a map for every chunk 28.9 us, 35.0 with eight; 30000 x 100 gradients 25.2 and 27.8), four
+ *  where five have to share a CU (65536 x 1000 gradients 60 to 63 us, with eight 58 to 76, with sixteen 80: columns then wait
+ *  for others to end). */
+template <typename Saver, uint32_t AT_ONCE>
 __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
     ColumnChunkWalkKernel(float *dst, const float *src, ChunkShape g, const Map *map,
                           const float (*copy)[column_chunks::kRows], float scale) {
@@ -361,16 +366,16 @@ __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
       WalkBlock *blk = &ring[(b - kWalkLoaders) % kWalkRing];
       const uint32_t first = (b - kWalkLoaders) * kWalkBlock;
       const uint32_t count = g.chunks - first < kWalkBlock ? g.chunks - first : kWalkBlock;
-      for (uint32_t c = 0; c < count; c += kChunksAtOnce) {
-        float4 va[kChunksAtOnce];
-        uint2 vb[kChunksAtOnce];
+      for (uint32_t c = 0; c < count; c += AT_ONCE) {
+        float4 va[AT_ONCE];
+        uint2 vb[AT_ONCE];
 #pragma unroll
-        for (uint32_t i = 0; i < kChunksAtOnce; ++i) {
+        for (uint32_t i = 0; i < AT_ONCE; ++i) {
           va[i] = blk->step[c + i];
           vb[i] = blk->rest[c + i];
         }
 #pragma unroll
-        for (uint32_t i = 0; i < kChunksAtOnce; ++i) {
+        for (uint32_t i = 0; i < AT_ONCE; ++i) {
           const Step m = {va[i].x, va[i].y, va[i].z, va[i].w, vb[i].x, __uint_as_float(vb[i].y)};
           float to;
           if (__ballot(column_chunks::Apply(m, sum, &to)) != 0ull) {

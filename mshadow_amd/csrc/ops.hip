@@ -639,7 +639,12 @@ bool LaunchColumnChunks(float *dst, const float *src, uint32_t stride, uint32_t 
   const dim3 grid(g.groups * g.tiles), block(kChunkWaves * 64);
   LaunchKernelIfFits(ColumnChunkSumsKernel, grid, block, 0, s, src, g, w->before, w->group);
   LaunchKernelIfFits(ColumnChunkMapsKernel, grid, block, 0, s, src, g, w->before, w->group, w->map, w->copy);
-  LaunchKernelIfFits((ColumnChunkWalkKernel<Saver>), dim3(cols), dim3((1 + kWalkLoaders) * 64), 0, s, dst, src, g, w->map, w->copy, scale);
+  const dim3 walk((1 + kWalkLoaders) * 64);
+  if (cols <= ColumnsOfWideWalk(mshadow_abi::ComputeUnits())) {
+    LaunchKernelIfFits((ColumnChunkWalkKernel<Saver, 16>), dim3(cols), walk, 0, s, dst, src, g, w->map, w->copy, scale);
+  } else {
+    LaunchKernelIfFits((ColumnChunkWalkKernel<Saver, 4>), dim3(cols), walk, 0, s, dst, src, g, w->map, w->copy, scale);
+  }
   return true;
 }
 }  // namespace

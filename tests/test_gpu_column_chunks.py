@@ -55,9 +55,10 @@ def terms(kind, rows, cols, seed):
 
 
 # up to 64 columns from 6400 rows on, 100 from 6695, 1000 from 15455 (8 to 1536 columns otherwise); chunks of 128 rows,
-# workgroups of four chunks and 64 columns, blocks of 16 chunks
+# workgroups of four chunks and 64 columns, blocks of 16 chunks; up to two columns a compute unit (512) the walk takes a block's
+# maps at once, beyond that four
 SHAPES = [(6300, 10), (6400, 10), (6528, 64), (6529, 65), (6783, 63), (8192, 1), (8193, 3), (8320, 129), (10240, 128),
-          (16384, 1000), (20481, 17), (33000, 300)]
+          (9200, 512), (9200, 513), (16384, 1000), (20481, 17), (33000, 300)]
 
 
 @pytest.mark.parametrize("rows,cols", SHAPES)
