@@ -208,7 +208,7 @@ int Im2Col(T *col, int cstride, const T *img, int istride, const PatchGeom &g, v
   const long long planes = static_cast<long long>(g.n) * g.c;
   while (band > 8 && planes * ((g.oh + band - 1) / band) < 1024) band = (band + 1) / 2;
   /* patch rows shorter than a pack would be written element by element there */
-  const bool short_rows = g.ow < EPT && cols < (1ll << 31) && (cols + kPatchBlock * EPT - 1) / (kPatchBlock * EPT) * rows < (1ll << 31);
+  const bool short_rows = g.ow < EPT && Im2ColPacksFit(rows, cols, EPT);
   if (band >= 1 && !short_rows) {
     const long long nb = (g.oh + band - 1) / band;
     band = (g.oh + nb - 1) / nb;
@@ -224,7 +224,7 @@ int Im2Col(T *col, int cstride, const T *img, int istride, const PatchGeom &g, v
                        dim3(kPatchBlock), lds, AsStream(stream), col, cstride, img, istride, g, t);
   } else {
     const long long chunks = (cols + kPatchBlock * EPT - 1) / (kPatchBlock * EPT);
-    const long long blocks = rows * chunks;
+    const long long blocks = Im2ColPackBlocks(rows, cols, EPT);
     if (blocks >= (1ll << 31)) return Fail(MSHADOW_HIP_ERR_ARGUMENT, "im2col: too many workgroups");
     LaunchKernelIfFits((Im2ColKernel<T, EPT>), dim3(static_cast<unsigned>(blocks)),
                        dim3(kPatchBlock), 0, AsStream(stream), col, cstride, img, istride, g,

@@ -21,11 +21,10 @@
 
 #include <mshadow/core/fastdiv.h>
 
+#include "patch_plan.h"
 #include "stream_access.h"
 
 namespace mshadow_hipk {
-
-const int kPatchBlock = 256;
 
 struct PatchGeom {
   int n, c, h, w;          // unpadded image

@@ -168,6 +168,13 @@ def test_sums_of_dense_planes_go_to_the_kernel_measured_to_be_the_faster(tmp_pat
     assert out.startswith("OK"), out[-500:]
 
 
+def test_short_patch_rows_go_to_a_kernel_that_can_be_launched(tmp_path):
+    """im2col of patch rows shorter than a pack: the kernel of packs wants a workgroup for every row of the column
+    matrix, which one launch does not have for very many channels"""
+    out = _compile_and_run(tmp_path, "patch_plan_check.cc", [])
+    assert out.startswith("OK"), out[-500:]
+
+
 def test_signed_column_sums_leave_most_of_the_chain(tmp_path):
     """sum_rows adds signed terms, and on N(0, 1) terms a plan of verified runs (what makes the
     softmax row sum parallel) leaves too much of its chain: cut with full knowledge of the true
