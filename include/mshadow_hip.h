@@ -78,7 +78,10 @@ int mshadow_hip_get_props(int device, mshadow_hip_props *out);
 int mshadow_hip_device_sync(void);
 
 /* Stream<gpu>: mshadow/stream_gpu-inl.h:61-74 (Wait, CheckIdle), :181-211
-   (NewStream / DeleteStream -> cudaStreamCreate / cudaStreamDestroy) */
+   (NewStream / DeleteStream -> cudaStreamCreate / cudaStreamDestroy). A stream that has scratch
+   memory of the library (mshadow_hip_reduce_scratch, and long column sums of
+   mshadow_hip_reduce_keep_lowest_f32) is waited for before it is destroyed: another stream may
+   get that memory. */
 int mshadow_hip_stream_create(void **stream);
 int mshadow_hip_stream_destroy(void *stream);
 int mshadow_hip_stream_sync(void *stream);

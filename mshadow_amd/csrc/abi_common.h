@@ -61,10 +61,10 @@ int ComputeUnits();
 bool CopyRowsOnDevice(void *dst, size_t dpitch_bytes, const void *src, size_t spitch_bytes,
                       size_t width_bytes, size_t rows, hipStream_t s);
 
-/* a stream is going away: whatever scratch memory of the library it was given is free again */
-void ReleaseReduceScratch(void *stream);
-/* whether launches on the stream may be using scratch memory of the sums by chunks */
-bool HasColumnScratch(void *stream);
+/* whether launches on the stream may be using scratch memory of the split reductions or of the sums by chunks */
+bool HasReduceScratch(void *stream);
+/* a stream is going away: that memory is free again if its work is done, else nobody gets it */
+void ReleaseReduceScratch(void *stream, bool done);
 /* looks up, once per device, where the scratch slots of the split reductions live on the current
    device (csrc/ops.hip) */
 void ResolveReduceScratch();

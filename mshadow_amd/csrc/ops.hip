@@ -18,6 +18,7 @@
 #include "patch_kernels.h"
 #include "pool_kernels.h"
 #include "row_kernels.h"
+#include "scratch_slots.h"
 #include "softmax_kernels.h"
 
 using namespace mshadow_abi;
@@ -548,7 +549,6 @@ bool LaunchShortSoftmax(float *dst, int dstride, const float *src, int sstride, 
 namespace {
 const int kReduceScratchSlots = 8;
 const size_t kReduceScratchWords = 1u << 16;
-const int kReduceScratchDevices = 16;
 struct ReduceScratchSlot {
   uint32_t partial[kReduceScratchWords];
   uint32_t counter[mshadow::hip::kSplitCounterWords];  // zero between launches
@@ -557,9 +557,8 @@ static __device__ __align__(256) ReduceScratchSlot g_reduce_scratch[kReduceScrat
 
 struct ReduceScratchTable {
   std::mutex mu;
-  ReduceScratchSlot *base[kReduceScratchDevices];
-  bool used[kReduceScratchDevices][kReduceScratchSlots];
-  void *owner[kReduceScratchDevices][kReduceScratchSlots];
+  ReduceScratchSlot *base[mshadow_abi::kScratchDevices];
+  mshadow_abi::ScratchSlots<kReduceScratchSlots> slots;
 };
 ReduceScratchTable &ScratchTable() {
   static ReduceScratchTable t = {};
@@ -577,25 +576,16 @@ static __device__ __align__(256) ColumnChunkScratch g_column_scratch[kColumnScra
 
 struct ColumnScratchTable {
   std::mutex mu;
-  ColumnChunkScratch *base[kReduceScratchDevices];
-  bool used[kReduceScratchDevices][kColumnScratchSlots];
-  void *owner[kReduceScratchDevices][kColumnScratchSlots];
+  ColumnChunkScratch *base[mshadow_abi::kScratchDevices];
+  mshadow_abi::ScratchSlots<kColumnScratchSlots> slots;
 
   /* the caller's slot on the current device, NULL where there is none to be had; mu is held */
   ColumnChunkScratch *Slot(void *stream) {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kReduceScratchDevices) {
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= mshadow_abi::kScratchDevices) {
       (void)hipGetLastError();
       return NULL;
     }
-    int slot = -1;
-    for (int i = 0; i < kColumnScratchSlots && slot < 0; ++i) {
-      if (used[dev][i] && owner[dev][i] == stream) slot = i;
-    }
-    for (int i = 0; i < kColumnScratchSlots && slot < 0; ++i) {
-      if (!used[dev][i]) slot = i;
-    }
-    if (slot < 0) return NULL;
     if (base[dev] == NULL) {
       void *p = NULL;
       if (hipGetSymbolAddress(&p, HIP_SYMBOL(g_column_scratch)) != hipSuccess) {
@@ -604,9 +594,8 @@ struct ColumnScratchTable {
       }
       base[dev] = static_cast<ColumnChunkScratch *>(p);
     }
-    used[dev][slot] = true;
-    owner[dev][slot] = stream;
-    return base[dev] + slot;
+    const int slot = slots.Take(dev, stream);
+    return slot < 0 ? NULL : base[dev] + slot;
   }
 };
 ColumnScratchTable &ColumnTable() {
@@ -650,39 +639,31 @@ bool LaunchColumnChunks(float *dst, const float *src, uint32_t stride, uint32_t 
 }  // namespace
 
 namespace mshadow_abi {
-bool HasColumnScratch(void *stream) {
-  ColumnScratchTable &t = ColumnTable();
-  std::lock_guard<std::mutex> lock(t.mu);
-  for (int d = 0; d < kReduceScratchDevices; ++d) {
-    for (int i = 0; i < kColumnScratchSlots; ++i) {
-      if (t.used[d][i] && t.owner[d][i] == stream) return true;
-    }
-  }
-  return false;
-}
-void ReleaseReduceScratch(void *stream) {
+bool HasReduceScratch(void *stream) {
   {
     ColumnScratchTable &c = ColumnTable();
     std::lock_guard<std::mutex> lock(c.mu);
-    for (int d = 0; d < kReduceScratchDevices; ++d) {
-      for (int i = 0; i < kColumnScratchSlots; ++i) {
-        if (c.used[d][i] && c.owner[d][i] == stream) c.used[d][i] = false;
-      }
-    }
+    if (c.slots.Has(stream)) return true;
   }
   ReduceScratchTable &t = ScratchTable();
   std::lock_guard<std::mutex> lock(t.mu);
-  for (int d = 0; d < kReduceScratchDevices; ++d) {
-    for (int i = 0; i < kReduceScratchSlots; ++i) {
-      if (t.used[d][i] && t.owner[d][i] == stream) t.used[d][i] = false;
-    }
+  return t.slots.Has(stream);
+}
+void ReleaseReduceScratch(void *stream, bool done) {
+  {
+    ColumnScratchTable &c = ColumnTable();
+    std::lock_guard<std::mutex> lock(c.mu);
+    c.slots.Release(stream, done);
   }
+  ReduceScratchTable &t = ScratchTable();
+  std::lock_guard<std::mutex> lock(t.mu);
+  t.slots.Release(stream, done);
 }
 /* called when a device is selected: where the scratch array lives on that device is looked up
    then, not inside the first reduction that wants a slot (which may be being recorded) */
 void ResolveReduceScratch() {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kReduceScratchDevices) {
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kScratchDevices) {
     (void)hipGetLastError();
     return;
   }
@@ -707,7 +688,7 @@ extern "C" int mshadow_hip_reduce_scratch(void *stream, size_t words, uint32_t *
   if (words > kReduceScratchWords) return MSHADOW_HIP_OK;
   int dev = 0;
   ABI_HIP(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kReduceScratchDevices) return MSHADOW_HIP_OK;
+  if (dev < 0 || dev >= kScratchDevices) return MSHADOW_HIP_OK;
   ReduceScratchTable &t = ScratchTable();
   std::lock_guard<std::mutex> lock(t.mu);
   if (t.base[dev] == NULL) {
@@ -716,17 +697,7 @@ extern "C" int mshadow_hip_reduce_scratch(void *stream, size_t words, uint32_t *
     ABI_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(g_reduce_scratch)));
     t.base[dev] = static_cast<ReduceScratchSlot *>(p);
   }
-  int slot = -1;
-  for (int i = 0; i < kReduceScratchSlots && slot < 0; ++i) {
-    if (t.used[dev][i] && t.owner[dev][i] == stream) slot = i;
-  }
-  for (int i = 0; i < kReduceScratchSlots && slot < 0; ++i) {
-    if (!t.used[dev][i]) {
-      t.used[dev][i] = true;
-      t.owner[dev][i] = stream;
-      slot = i;
-    }
-  }
+  const int slot = t.slots.Take(dev, stream);
   if (slot < 0) return MSHADOW_HIP_OK;
   *partial = t.base[dev][slot].partial;
   *counter = t.base[dev][slot].counter;

@@ -98,8 +98,12 @@ int mshadow_hip_stream_create(void **stream) {
 int mshadow_hip_stream_destroy(void *stream) {
   if (stream == NULL) return MSHADOW_HIP_OK;
   /* another stream may get the scratch memory: nothing queued here may still be using it */
-  if (HasColumnScratch(stream) && hipStreamSynchronize(AsStream(stream)) != hipSuccess) (void)hipGetLastError();
-  ReleaseReduceScratch(stream);
+  bool done = true;
+  if (HasReduceScratch(stream) && hipStreamSynchronize(AsStream(stream)) != hipSuccess) {
+    (void)hipGetLastError();
+    done = false;
+  }
+  ReleaseReduceScratch(stream, done);
   ABI_HIP(hipStreamDestroy(AsStream(stream)));
   return MSHADOW_HIP_OK;
 }

@@ -175,6 +175,13 @@ def test_short_patch_rows_go_to_a_kernel_that_can_be_launched(tmp_path):
     assert out.startswith("OK"), out[-500:]
 
 
+def test_scratch_slots_of_streams(tmp_path):
+    """a stream that goes away gives its scratch slot back only when its work is known to be done: not where the wait
+    for it failed"""
+    out = _compile_and_run(tmp_path, "scratch_slots_check.cc", [])
+    assert out.startswith("OK"), out[-500:]
+
+
 def test_signed_column_sums_leave_most_of_the_chain(tmp_path):
     """sum_rows adds signed terms, and on N(0, 1) terms a plan of verified runs (what makes the
     softmax row sum parallel) leaves too much of its chain: cut with full knowledge of the true
