@@ -3,10 +3,12 @@
  * launches: the chunks' sums in any order, their maps, and a walk down every column. The matrix is read twice, by
  * all CUs, where a strip of columns a workgroup leaves most of them idle; the sequence of a column is left
  * to one wave, which takes a chunk in 60 ns, and one that has no map in 500, where 128 dependent adds
- * take 450. 65536 x 1000: 50, 56 and 60 to 63 us (the last by the column with the fewest maps).
+ * take 450. 65536 x 1000: 38, 58 and 64 us (the last by the column with the fewest maps).
  */
 #ifndef MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_
 #define MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_
+
+#include <float.h>
 
 #include <mshadow/hip/kernels/common.h>
 #include <mshadow/hip/kernels/reduce_dma.h>
@@ -17,11 +19,14 @@ namespace mshadow_hipk {
 
 using column_chunks::Map;
 using column_chunks::Step;
+using column_chunks::Windows;
 using mshadow::hip::kWave;
 
 /*! \brief a workgroup has four chunks of 64 columns, a wave each */
 const int kChunkWaves = 4;
 const uint32_t kColumnsPerTile = 64;
+
+const uint32_t kMostChunkColumns = 1536;
 
 /*! \brief scratch memory of one call: cells are (chunk, column), the columns padded to whole tiles */
 const uint32_t kChunkCells = 1u << 19;
@@ -31,14 +36,17 @@ struct ColumnChunkScratch {
   float copy[kChunkCopies][column_chunks::kRows];   // terms of chunks that are added one by one
   float before[kChunkCells];                        // [chunk][column]: sum of the workgroup's chunks in front
   float group[kChunkCells / kChunkWaves + kChunkCells / kChunkWaves / 2];  // [workgroup of chunks][column]
+  uint32_t bare[kMostChunkColumns];                 // of a column: chunks that have neither a map nor a copy
 };
 
 struct ChunkShape {
   uint32_t rows, cols, stride;
   uint32_t chunks, groups, tiles;
   uint32_t copies;  // copies a (chunk, tile) has room for
+  uint32_t strips;  // strips of 16 columns that may be chained, 0: none
+  uint32_t most_bare;  // bare chunks of a column that is walked
 };
-inline bool MakeChunkShape(uint32_t rows, uint32_t cols, uint32_t stride, ChunkShape *g) {
+inline bool MakeChunkShape(uint32_t rows, uint32_t cols, uint32_t stride, uint32_t cus, ChunkShape *g) {
   g->rows = rows;
   g->cols = cols;
   g->stride = stride;
@@ -46,9 +54,14 @@ inline bool MakeChunkShape(uint32_t rows, uint32_t cols, uint32_t stride, ChunkS
   g->groups = (g->chunks + kChunkWaves - 1) / kChunkWaves;
   g->tiles = (cols + kColumnsPerTile - 1) / kColumnsPerTile;
   const uint64_t cells = static_cast<uint64_t>(g->chunks) * g->tiles;
-  if (cells * kColumnsPerTile > kChunkCells) return false;
+  if (cells * kColumnsPerTile > kChunkCells || cols > kMostChunkColumns) return false;
   const uint32_t room = static_cast<uint32_t>(kChunkCopies / cells);
   g->copies = room < kColumnsPerTile ? room : kColumnsPerTile;
+  /* A bare chunk's terms, read from the matrix 4 bytes of a cache line at a time, take 0.5 us where a column has a CU to itself,
+     1.2 us where all of 512 columns have such chunks, 2.3 us of 1000 (65536 x 1000: 1180 us in all). In a strip of 16 columns
+     128 terms of each take 0.53 us. */
+  g->strips = cols <= cus ? 0u : (cols + mshadow::hip::kLowestCols - 1) / mshadow::hip::kLowestCols;
+  g->most_bare = static_cast<uint32_t>(static_cast<uint64_t>(g->chunks) * cus / cols) + 8u;
   /* groups * kChunkWaves may exceed chunks by three, which the array of groups allows for */
   return static_cast<uint64_t>(g->groups) * g->tiles * kColumnsPerTile <=
          sizeof(static_cast<ColumnChunkScratch *>(NULL)->group) / sizeof(float);
@@ -59,48 +72,44 @@ inline bool MakeChunkShape(uint32_t rows, uint32_t cols, uint32_t stride, ChunkS
  *  64 and 53, 16384 x 100 65 and 30, 8192 x 100 36 and 23, 8192 x 10 34 and 26; level at 8192 x 1000 and 4096 x 64,
  *  slower at 16384 x 4096 (72 and 180: its reads alone take as long as its chain). Without, a row takes 3.5 ns; with,
  *  0.8 ns, 1.6 ps a column for the second read of the matrix and the less than full rate of the first, and
- *  17 us for the three launches. More than six columns a CU walk in turns. Columns whose sum misses
- *  its maps throughout (0.1 added 65536 times) take 0.5 us a chunk: 290 us where the chain takes 232. */
+ *  17 us for the three launches. More than six columns a CU walk in turns.
+ *  What the terms are can take the gain away. Columns with roundings that all go one way (equal terms, 1 / 0.9 nine times of
+ *  ten), or with an infinity or a NaN: 16384 x 1000 63 and 48 to 57, 65536 x 1000 230 and 140 to 199, 131072 x 10 450 and 90 to
+ *  190. Columns that have no map throughout, their sums back at nothing after every other term, pay for the first two launches in
+ *  vain: 6800 x 10 29 and 42, 16384 x 100 64 and 79, 16384 x 1000 62 and 110, 40000 x 1200 142 and 265, 65536 x 1000 231 and 406,
+ *  131072 x 100 464 and 504; with one such column in a hundred nearly as much. */
 inline bool ColumnChunksAreSooner(uint32_t rows, uint32_t cols, uint32_t cus) {
   return cols <= 6u * cus && static_cast<double>(rows) * (2700.0 - 1.6 * cols) > 17e6;
 }
 
-/*! \brief a column's terms of N rows: all loads under way together, rows behind the last as -0, which changes no
- *  sum */
+/*! \brief a column's terms of N rows: all loads under way together */
 template <uint32_t N>
 __device__ __forceinline__ void LoadRows(float (&t)[N], const float *src, const ChunkShape &g, uint32_t row0,
                                          uint32_t x) {
   /* a row's address is the wave's, the column's offset a lane's (32 bits: the instruction adds them) */
   const uint32_t at = x * static_cast<uint32_t>(sizeof(float));
   const size_t pitch = static_cast<size_t>(g.stride) * sizeof(float);
-  if (row0 + N <= g.rows) {
-    const char *p = reinterpret_cast<const char *>(src) + row0 * pitch;
+  const char *p = reinterpret_cast<const char *>(src) + row0 * pitch;
 #pragma unroll
-    for (uint32_t i = 0; i < N; ++i) {
-      t[i] = *reinterpret_cast<const float *>(p + at);
-      p += pitch;
-    }
-  } else {
-    const uint32_t from = row0 < g.rows ? row0 : g.rows - 1u;
-    const uint32_t left = row0 < g.rows ? g.rows - row0 : 0u;
-    const char *p = reinterpret_cast<const char *>(src) + from * pitch;
-#pragma unroll
-    for (uint32_t i = 0; i < N; ++i) {
-      const float v = *reinterpret_cast<const float *>(p + at);
-      t[i] = i < left ? v : -0.0f;
-      if (i + 1u < left) p += pitch;
-    }
+  for (uint32_t i = 0; i < N; ++i) {
+    t[i] = *reinterpret_cast<const float *>(p + at);
+    p += pitch;
   }
+}
+/*! \brief whether all rows of a chunk are there: a last one of fewer is added term by term, and nothing waits for its
+ *  sum */
+__device__ __forceinline__ bool IsWhole(const ChunkShape &g, uint32_t chunk) {
+  return (chunk + 1u) * column_chunks::kRows <= g.rows;
 }
 
 /*! \brief rows whose loads are under way together in the launch that only sums */
 const uint32_t kSumsAtOnce = 32;
 
 /*! \brief the sums of the chunks, in any order of adds: per workgroup of four chunks the sum of those in
- *  front of each, and of all. Bound by its read of the matrix: 65536 x 1000 50 us, 5.2 TB/s; four columns a lane, which
- *  leaves a quarter of the waves, 57. */
+ *  front of each, and of all. Bound by its read of the matrix: 65536 x 1000 38 us, 6.9 TB/s; four columns a lane, which
+ *  leaves a quarter of the waves, was a seventh slower. */
 __global__ void __launch_bounds__(kChunkWaves *kWave)
-    ColumnChunkSumsKernel(const float *src, ChunkShape g, float *before, float *group) {
+    ColumnChunkSumsKernel(const float *src, ChunkShape g, float *before, float *group, uint32_t *bare) {
   __shared__ float sums[kChunkWaves][kWave];
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
   const uint32_t piece = mshadow::hip::StripOfBlock(blockIdx.x, gridDim.x);
@@ -109,7 +118,7 @@ __global__ void __launch_bounds__(kChunkWaves *kWave)
   const uint32_t column = tile * kColumnsPerTile + lane;
   const uint32_t x = column < g.cols ? column : g.cols - 1;
   float sum = 0.0f;
-  if (chunk < g.chunks) {
+  if (IsWhole(g, chunk)) {
     float part[kSumsAtOnce] = {0.0f};
     for (uint32_t i = 0; i < static_cast<uint32_t>(column_chunks::kRows); i += kSumsAtOnce) {
       float t[kSumsAtOnce];
@@ -124,6 +133,7 @@ __global__ void __launch_bounds__(kChunkWaves *kWave)
     }
     sum = part[0];
   }
+  if (at == 0 && wave == 0 && column < g.cols) bare[column] = 0u;
   sums[wave][lane] = sum;
   __syncthreads();
   float front = 0.0f;
@@ -133,11 +143,12 @@ __global__ void __launch_bounds__(kChunkWaves *kWave)
 }
 
 /*! \brief the maps of the chunks. A wave keeps its chunk of 64 columns in registers, so that terms to be added
- *  one by one can be copied out; fourteen instructions a term, which the reads hide (56 us on 65536 x 1000, 4.7 TB/s). Workgroups go through
+ *  one by one can be copied out; sixteen instructions a term, which the reads hide (58 us on 65536 x 1000, 4.5 TB/s; with
+ *  fourteen, without the third window, 55). Workgroups go through
  *  the matrix from its end: what the launch before read last is still in the memory-side cache. */
-__global__ void __launch_bounds__(kChunkWaves *kWave)
+__global__ void __launch_bounds__(kChunkWaves *kWave, 3)
     ColumnChunkMapsKernel(const float *src, ChunkShape g, const float *before, const float *group, Map *map,
-                          float (*copy)[column_chunks::kRows]) {
+                          float (*copy)[column_chunks::kRows], uint32_t *bare) {
   __shared__ float part[3][kChunkWaves][kWave];
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
   const uint32_t piece = gridDim.x - 1u - mshadow::hip::StripOfBlock(blockIdx.x, gridDim.x);
@@ -177,7 +188,8 @@ __global__ void __launch_bounds__(kChunkWaves *kWave)
   }
   float t[column_chunks::kRows];
   const float inside = live ? before[static_cast<size_t>(chunk) * pitch + column] : 0.0f;
-  if (live) LoadRows(t, src, g, chunk * column_chunks::kRows, x);
+  const bool whole = IsWhole(g, chunk);
+  if (whole) LoadRows(t, src, g, chunk * column_chunks::kRows, x);
   __syncthreads();
   if (!live) return;
   float a = 0.0f, most = 0.0f;
@@ -187,36 +199,52 @@ __global__ void __launch_bounds__(kChunkWaves *kWave)
     a += part[0][w][lane];
   }
   a += inside;
+  if (!whole) {
+    const Map m = {a, 0.0f, 0u, column_chunks::How(true, 0u, column_chunks::kInMatrix)};
+    if (column < g.cols) map[static_cast<size_t>(column) * g.chunks + chunk] = m;
+    return;
+  }
   most = fmaxf(most, fabsf(a));
-  const uint32_t j = column_chunks::StartsOnGrid(a)
-                         ? column_chunks::WindowFor(a, most, sqrtf(static_cast<float>(chunk * column_chunks::kRows)))
-                         : column_chunks::kMaxWindow + 1u;
-  const bool tried = j <= column_chunks::kMaxWindow;
+  const float rows_before = static_cast<float>(chunk * column_chunks::kRows);
+  Windows j = {column_chunks::kMaxWindow + 1u, 0u};
+  if (column_chunks::StartsOnGrid(a)) j = column_chunks::WindowsFor(a, most, rows_before, sqrtf(rows_before));
+  const bool tried = j.second <= column_chunks::kMaxWindow;
+  if (!tried) j.second = j.third = column_chunks::kMinWindow;
   column_chunks::Chains chains;
-  const float from = tried ? a : 1.0f;
-  chains.Start(from, tried ? j : column_chunks::kMinWindow);
+  chains.Start(tried ? a : 1.0f, j);
+  /* all that is needed of these behind the chains, in one register: there are 168 for three waves a SIMD */
+  uint32_t windows = j.second | j.third << 8 | (tried ? 1u << 16 : 0u);
+  asm volatile("" : "+v"(windows), "+v"(a));
 #pragma unroll
   for (int i = 0; i < column_chunks::kRows; ++i) {
     chains.Add(t[i]);
     if (i % 4 == 3) {
       /* else the compiler runs one chain after the other, makes trees of the maxima and ors, and keeps
          every sum until then (256 registers and as many spilled) */
-      asm volatile("" : "+v"(chains.differ), "+v"(chains.far), "+v"(chains.most), "+v"(chains.term));
+      asm volatile("" : "+v"(chains.differ), "+v"(chains.far), "+v"(chains.farthest), "+v"(chains.most));
       __builtin_amdgcn_sched_barrier(0);
     }
   }
   Map m;
   bool wide;
-  const bool known = chains.Finish(from, tried ? j : column_chunks::kMinWindow, &m, &wide) && tried;
+  j.second = windows & 255u;
+  j.third = windows >> 8 & 255u;
+  const bool known = chains.Finish(windows >> 16 != 0u ? a : 1.0f, j, &m, &wide) && windows >> 16 != 0u;
   if (!known) {
     uint32_t where = column_chunks::kInMatrix;
-    if (chains.term == 0.0f && chains.s[0] == chains.s[0]) {
+    float term = 0.0f;
+#pragma unroll
+    for (int i = 0; i < column_chunks::kRows; ++i) term = fmaxf(term, fabsf(t[i]));
+    const bool nan = chains.s[0] != chains.s[0];
+    if (term == 0.0f && !nan) {
       bool plus = false;
 #pragma unroll
       for (int i = 0; i < column_chunks::kRows; ++i) plus = plus || __float_as_uint(t[i]) == 0u;
       where = plus ? column_chunks::kPlusZero : column_chunks::kNothing;
     }
     m.how = column_chunks::How(true, 0u, where);
+    m.a = a;
+    m.shift = term <= FLT_MAX && !nan ? 1u : 0u;
   }
   /* copies of the terms that will or may be asked for */
   const bool copied = column < g.cols && !(known && wide) && column_chunks::WhereOf(m.how) == column_chunks::kInMatrix;
@@ -227,6 +255,8 @@ __global__ void __launch_bounds__(kChunkWaves *kWave)
 #pragma unroll
     for (int i = 0; i < column_chunks::kRows; i += 4) to[i / 4] = make_float4(t[i], t[i + 1], t[i + 2], t[i + 3]);
     m.how = column_chunks::How(!known, column_chunks::WindowOf(m.how), column_chunks::kKept + slot);
+  } else if (copied && !known && column_chunks::Exponent(a) != 255u) {
+    __hip_atomic_fetch_add(bare + column, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (column < g.cols) map[static_cast<size_t>(column) * g.chunks + chunk] = m;
 }
@@ -237,6 +267,11 @@ __device__ __forceinline__ void WaveLdsFence() {
 }
 /*! \brief columns up to which the walk takes its maps sixteen at once */
 inline uint32_t ColumnsOfWideWalk(uint32_t cus) { return 2u * cus; }
+/*! \brief stages of a strip's chain, in the LDS that a CU has for each of two or six columns: the longer they are the less
+ *  often their first reads are waited for (65536 x 1000 in stages of 64, 96 and 128 rows: 5.1, 4.5 and 4.0 ns a row; but with
+ *  128 a CU holds four workgroups, and 30000 x 1000 columns that have maps take 86 us instead of 76) */
+typedef mshadow::hip::DmaRing<5, 2048, 2> StripRingOfTwo;
+typedef mshadow::hip::DmaRing<4, 1536, 2> StripRingOfSix;
 
 /*! \brief 128 additions, the terms read from LDS a block of 32 ahead */
 __device__ __forceinline__ void AddTerms(float *sum, const float4 *term) {
@@ -266,8 +301,9 @@ __device__ __forceinline__ void AddTerms(float *sum, const float4 *term) {
 const uint32_t kWalkBlock = 16;
 const uint32_t kWalkLoaders = 2;
 const uint32_t kWalkRing = kWalkLoaders + 1;
-/*! \brief in the place of a window: the terms are here; there are none; there are only zeros, a +0 among them */
-const uint32_t kWalkTerms = 0xbf800000u, kWalkNothing = 0xc0000000u, kWalkPlusZero = 0xc0400000u;  // -1, -2, -3
+/*! \brief in the place of a window: the terms are here; there are none; there are only zeros, a +0 among them; the sum in
+ *  front is expected to be infinite or NaN, which mostly asks for no terms */
+const uint32_t kWalkTerms = 0xbf800000u, kWalkNothing = 0xc0000000u, kWalkPlusZero = 0xc0400000u, kWalkNoSum = 0xc0800000u;
 struct WalkBlock {
   float4 step[kWalkBlock];  // Step's a, inverse, e0, grid
   uint2 rest[kWalkBlock];   // Step's shift, window
@@ -275,32 +311,51 @@ struct WalkBlock {
   float4 term[kWalkBlock][column_chunks::kRows / 4];  // of the chunks that are added term by term
 };
 
+/*! \brief whether a column has so many chunks that ask for the matrix that it is left to the chain */
+__device__ __forceinline__ bool TakesChain(uint32_t bare, const ChunkShape &g) { return g.strips != 0u && bare > g.most_bare; }
+
 /*! \brief the sums themselves: a wave walks down a column, every lane with the same sum, and reads nothing but
  *  LDS. Two more bring it the maps, and the terms of the chunks that have none: a block each in turn,
- *  asked for two blocks ahead. Bound by the walk's sequence: a wave alone issues an instruction every 3.5 ns.
+ *  asked for two blocks ahead. Bound by the walk's sequence: a wave alone issues an instruction every 3.5 ns. The
+ *  first workgroups have a strip of 16 columns each, of which they add those that TakesChain from top to bottom.
  *  AT_ONCE: maps in registers together. All of a block where two columns a CU at most leave the registers for it
  *  (65536 x 64 of columns with a map for every chunk 28.9 us, 35.0 with eight; 30000 x 100 gradients 25.2 and 27.8), four
- *  where five have to share a CU (65536 x 1000 gradients 60 to 63 us, with eight 58 to 76, with sixteen 80: columns then wait
+ *  where four have to share a CU (65536 x 1000 gradients 60 to 63 us, with eight 58 to 76, with sixteen 80: columns then wait
  *  for others to end). */
-template <typename Saver, uint32_t AT_ONCE>
+template <typename Saver, uint32_t AT_ONCE, typename StripRing>
 __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
     ColumnChunkWalkKernel(float *dst, const float *src, ChunkShape g, const Map *map,
-                          const float (*copy)[column_chunks::kRows], float scale) {
-  __shared__ WalkBlock ring[kWalkRing];
+                          const float (*copy)[column_chunks::kRows], const uint32_t *bare, float scale) {
+  __shared__ union {
+    WalkBlock ring[kWalkRing];
+    __attribute__((aligned(16))) float strip[StripRing::kSlots][StripRing::kElems];
+  } lds;
   __shared__ uint32_t misses;  // chunks whose map did not cover the sum
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
-  const uint32_t x = blockIdx.x;
+  if (blockIdx.x < g.strips) {
+    const uint32_t x0 = mshadow::hip::StripOfBlock(blockIdx.x, g.strips) * mshadow::hip::kLowestCols;
+    const bool chain = lane < static_cast<uint32_t>(mshadow::hip::kLowestCols) && x0 + lane < g.cols && TakesChain(bare[x0 + lane], g);
+    if (__ballot(chain) != 0ull) {
+      mshadow::hip::ReduceKeepLowestDma<Saver, mshadow::red::sum, StripRing>(lds.strip, dst, src, g.stride, g.rows, g.cols, x0,
+                                                                                 chain, scale);
+    }
+    return;
+  }
+  WalkBlock *ring = lds.ring;
+  const uint32_t x = blockIdx.x - g.strips;
   const uint32_t blocks = (g.chunks + kWalkBlock - 1) / kWalkBlock;
+  const Map *mine = map + static_cast<size_t>(x) * g.chunks;
+  auto fetch = [&](uint32_t block) {
+    const uint32_t c = block * kWalkBlock + lane % kWalkBlock;
+    return mine[c < g.chunks ? c : g.chunks - 1];
+  };
+  Map now = {};
+  if (wave != 0) now = fetch(wave - 1);
+  if (TakesChain(bare[x], g)) return;
   if (threadIdx.x == 0) misses = 0u;
   __syncthreads();
 
   if (wave != 0) {
-    const Map *mine = map + static_cast<size_t>(x) * g.chunks;
-    auto fetch = [&](uint32_t block) {
-      const uint32_t c = block * kWalkBlock + lane % kWalkBlock;
-      return mine[c < g.chunks ? c : g.chunks - 1];
-    };
-    Map now = fetch(wave - 1);
     for (uint32_t b = 0; b < blocks + kWalkLoaders; ++b) {
       if (b % kWalkLoaders == wave - 1) {
         if (b < blocks) {
@@ -314,13 +369,15 @@ __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
           const bool mapped = !column_chunks::IsByTerms(now.how);
           const uint32_t where = column_chunks::WhereOf(now.how);
           const bool nothing = where == column_chunks::kNothing, plus = where == column_chunks::kPlusZero;
+          const bool no_sum = !mapped && column_chunks::Exponent(now.a) == 255u;
           unsigned long long wanted =
-              __ballot(live && (where >= column_chunks::kKept ||
-                                (where == column_chunks::kInMatrix && (all || !mapped))));
+              __ballot(live && !no_sum && (where >= column_chunks::kKept ||
+                                           (where == column_chunks::kInMatrix && (all || !mapped))));
           if (lane < kWalkBlock) {
             const Step st = column_chunks::StepOf(now);
             const uint32_t window = !live || nothing ? kWalkNothing
                                     : plus           ? kWalkPlusZero
+                                    : no_sum         ? kWalkNoSum
                                     : mapped         ? __float_as_uint(st.window)
                                                      : kWalkTerms;
             to->step[lane] = make_float4(st.a, st.inverse, st.e0, st.grid);
@@ -390,7 +447,12 @@ __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
           }
           float4 *term = blk->term[c + i];
           if (window != kWalkTerms) {
-            /* the map does not cover the sum */
+            /* The map does not cover the sum, or there is none. A sum that is infinite or NaN stays what it is, but for an
+               infinity that meets another or a NaN. */
+            if (column_chunks::Exponent(sum) == 255u &&
+                (sum != sum || window != kWalkNoSum || __builtin_amdgcn_readfirstlane(vb[i].x) != 0u)) {
+              continue;
+            }
             if ((__builtin_amdgcn_readfirstlane(blk->here) >> (c + i) & 1u) == 0u) {
               const uint32_t row0 = (first + c + i) * column_chunks::kRows;
               for (uint32_t k = lane; k < static_cast<uint32_t>(column_chunks::kRows); k += kWave) {

@@ -620,20 +620,23 @@ template <typename Saver>
 bool LaunchColumnChunks(float *dst, const float *src, uint32_t stride, uint32_t rows, uint32_t cols, float scale,
                         hipStream_t s) {
   ChunkShape g;
-  if (!ColumnChunksAreSooner(rows, cols, mshadow_abi::ComputeUnits()) || !MakeChunkShape(rows, cols, stride, &g) || HasNoSlot(s)) return false;
+  const uint32_t cus = mshadow_abi::ComputeUnits();
+  if (!ColumnChunksAreSooner(rows, cols, cus) || !MakeChunkShape(rows, cols, stride, cus, &g) || HasNoSlot(s)) return false;
   ColumnScratchTable &t = ColumnTable();
   std::lock_guard<std::mutex> lock(t.mu);
   ColumnChunkScratch *w = t.Slot(s);
   if (w == NULL) return false;
   const dim3 grid(g.groups * g.tiles), block(kChunkWaves * 64);
-  LaunchKernelIfFits(ColumnChunkSumsKernel, grid, block, 0, s, src, g, w->before, w->group);
-  LaunchKernelIfFits(ColumnChunkMapsKernel, grid, block, 0, s, src, g, w->before, w->group, w->map, w->copy);
-  const dim3 walk((1 + kWalkLoaders) * 64);
-  if (cols <= ColumnsOfWideWalk(mshadow_abi::ComputeUnits())) {
-    LaunchKernelIfFits((ColumnChunkWalkKernel<Saver, 16>), dim3(cols), walk, 0, s, dst, src, g, w->map, w->copy, scale);
-  } else {
-    LaunchKernelIfFits((ColumnChunkWalkKernel<Saver, 4>), dim3(cols), walk, 0, s, dst, src, g, w->map, w->copy, scale);
-  }
+  LaunchKernelIfFits(ColumnChunkSumsKernel, grid, block, 0, s, src, g, w->before, w->group, w->bare);
+  LaunchKernelIfFits(ColumnChunkMapsKernel, grid, block, 0, s, src, g, w->before, w->group, w->map, w->copy,
+                     w->bare);
+  const dim3 columns(g.strips + cols), walk((1 + kWalkLoaders) * 64);
+#define WALK(AT_ONCE, RING)                                                                                              \
+  LaunchKernelIfFits((ColumnChunkWalkKernel<Saver, AT_ONCE, RING>), columns, walk, 0, s, dst, src, g, w->map, w->copy,   \
+                     w->bare, scale)
+  if (cols <= ColumnsOfWideWalk(cus)) WALK(16, StripRingOfTwo);
+  else WALK(4, StripRingOfSix);
+#undef WALK
   return true;
 }
 }  // namespace

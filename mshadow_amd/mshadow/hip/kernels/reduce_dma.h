@@ -42,13 +42,14 @@ const int kDmaThreads = (kDmaLoaders + 1) * kWave;
  *  are in flight. KeepHighDim is bound by HBM and takes many small stages (deep queue);
  *  KeepLowest is bound by its chain of dependent adds and takes few large ones, so that
  *  the LDS latency at the start of a stage is paid less often. */
-template <int SLOTS_, int ELEMS_>
+template <int SLOTS_, int ELEMS_, int LOADERS_ = kDmaLoaders>
 struct DmaRing {
+  static const int kLoaders = LOADERS_;
   static const int kSlots = SLOTS_;
   static const int kElems = ELEMS_;
   static const int kAhead = SLOTS_ - 2;
   /*! \brief load instructions per loader wave per stage (64 dwords each) */
-  static const int kPerWave = ELEMS_ / kWave / kDmaLoaders;
+  static const int kPerWave = ELEMS_ / kWave / LOADERS_;
   static_assert(kAhead * kPerWave < 64, "the wait-by-count immediate has 6 bits");
 };
 typedef DmaRing<4, 8192> LowestRing;
@@ -92,19 +93,16 @@ __device__ __forceinline__ void BareBarrier() { asm volatile("s_barrier" ::: "me
  * four rows: lane l fetches row 4 g + (l & 3), column l >> 2, so the slot holds
  * [group][column][row & 3] and a chain lane reads rows 4g..4g+3 of its column as one
  * 128-bit word, 64 floats from the next group. */
-template <typename Saver, typename Reducer>
-__global__ void __launch_bounds__(kDmaThreads)
-    ReduceKeepLowestDmaKernel(float *dst, const float *src, uint32_t stride, uint32_t rows,
-                              uint32_t cols, float scale) {
-  typedef LowestRing Ring;
+/*! \brief a workgroup of 1 + Ring::kLoaders waves; lane l of wave 0 folds column x0 + l if that is `wanted` */
+template <typename Saver, typename Reducer, typename Ring>
+__device__ __forceinline__ void ReduceKeepLowestDma(float (*ring)[Ring::kElems], float *dst, const float *src, uint32_t stride,
+                                                    uint32_t rows, uint32_t cols, uint32_t x0, bool wanted, float scale) {
   const int kDmaSlots = Ring::kSlots, kDmaAhead = Ring::kAhead, kDmaPerWave = Ring::kPerWave;
   const int CW = kLowestCols;
   const int TR = Ring::kElems / CW;
-  __shared__ MSHADOW_ALIGNED(16) float ring[Ring::kSlots][Ring::kElems];
 
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  const uint32_t x0 = StripOfBlock(blockIdx.x, gridDim.x) * CW;
   const uint32_t nstage = (rows + TR - 1) / TR;
   const uint32_t nstep = nstage == 0 ? 0 : nstage + kDmaAhead;
 
@@ -119,7 +117,7 @@ __global__ void __launch_bounds__(kDmaThreads)
         float *slot = ring[i % kDmaSlots];
 #pragma unroll
         for (int q = 0; q < kDmaPerWave; ++q) {
-          const uint32_t g = q * kDmaLoaders + lw;
+          const uint32_t g = q * Ring::kLoaders + lw;
           uint32_t row = i * TR + g * 4 + r;
           row = row < rows ? row : rows - 1;
           LoadDwordToLds(colp + static_cast<size_t>(row) * stride, slot + g * kWave);
@@ -131,7 +129,7 @@ __global__ void __launch_bounds__(kDmaThreads)
       BareBarrier();
     }
   } else {
-    const bool chain_lane = lane < static_cast<uint32_t>(CW) && x0 + lane < cols;
+    const bool chain_lane = lane < static_cast<uint32_t>(CW) && x0 + lane < cols && wanted;
     float res = 0.0f;
     for (uint32_t i = 0; i < nstep; ++i) {
       BareBarrier();
@@ -150,6 +148,14 @@ __global__ void __launch_bounds__(kDmaThreads)
     }
     if (chain_lane) Saver::template Save<float>(dst[x0 + lane], res * scale);
   }
+}
+template <typename Saver, typename Reducer>
+__global__ void __launch_bounds__(kDmaThreads)
+    ReduceKeepLowestDmaKernel(float *dst, const float *src, uint32_t stride, uint32_t rows,
+                              uint32_t cols, float scale) {
+  __shared__ MSHADOW_ALIGNED(16) float ring[LowestRing::kSlots][LowestRing::kElems];
+  ReduceKeepLowestDma<Saver, Reducer, LowestRing>(ring, dst, src, stride, rows, cols,
+                                                  StripOfBlock(blockIdx.x, gridDim.x) * kLowestCols, true, scale);
 }
 
 /* ------------------------------------------------------------------ KeepLowest in strips

@@ -1,5 +1,5 @@
 // The column sums by chunks (csrc/column_chunks.h) on the host: the functions of the device code, walked down
-// columns as the kernels walk them - approximate sums in front of every chunk, ten chains a chunk, one
+// columns as the kernels walk them - approximate sums in front of every chunk, twelve chains a chunk, one
 // look-up a chunk or 128 additions - against the reference's serial loop, bit for bit. Prints, per kind of
 // column, the share of the chunks that were added term by term.
 #include <cmath>
@@ -33,9 +33,10 @@ static float Walk(const std::vector<float> &t, double beside, long *chunks, long
     bool known = false, wide;
     Map m;
     if (StartsOnGrid(a)) {
-      const uint32_t j = WindowFor(a, most, std::sqrt(static_cast<float>(c * kRows)));
-      if (j <= kMaxWindow) {
-        if (beside != 0) a += static_cast<float>(beside) * Window(a, j);
+      const float rows = static_cast<float>(c * kRows);
+      const Windows j = WindowsFor(a, most, rows, std::sqrt(rows));
+      if (j.second <= kMaxWindow) {
+        if (beside != 0) a += static_cast<float>(beside) * Window(a, j.second);
         if (StartsOnGrid(a)) {
           Chains chains;
           chains.Start(a, j);
@@ -75,7 +76,8 @@ int main() {
   };
   const Kind kinds[] = {{"normal", 16384, 0.06}, {"normal", 65537, 0.06}, {"gradient", 65536, 0.05},
                         {"gradient100", 30000, 0.08}, {"positive", 30001, 0.05}, {"small", 16384, 0.06},
-                        {"halves", 20000, 1}, {"integers", 20000, 1}, {"constant", 20000, 1}, {"alternating", 9000, 1},
+                        {"halves", 20000, 1}, {"integers", 20000, 1}, {"constant", 20000, 0.1}, {"constant", 65536, 0.06}, {"mean", 65536, 0.06},
+                        {"kept", 65536, 0.06}, {"then constant", 65536, 0.06}, {"constant first", 65536, 0.06}, {"alternating", 9000, 1},
                         {"subnormal", 9000, 1}, {"wide", 9000, 1}, {"huge", 9000, 1}, {"infinity", 9000, 1},
                         {"nan", 9000, 1}, {"zeros", 9000, 1}, {"minus zeros", 9000, 1}, {"cancelling", 9000, 1},
                         {"one", 1, 1}, {"short", 127, 1}, {"chunk", 128, 1}, {"odd", 129, 1}};
@@ -97,6 +99,10 @@ int main() {
         if (name == "halves") v = std::round(v * 64) / 64;
         if (name == "integers") v = std::round(v * 1000) * 4099;
         if (name == "constant") v = 0.1f * (column + 1);
+        if (name == "mean") v = 1.0f / (65536.0f * (97 + column));
+        if (name == "kept") v = unit(gen) < 0.1f + 0.03f * column ? 1.0f / (0.1f + 0.03f * column) : 0.0f;
+        if (name == "then constant" && i > 30000) v = 0.03f * (column + 1);
+        if (name == "constant first" && i < 30000) v = 0.03f * (column + 1);
         if (name == "alternating") v = (i & 1 ? -1.0f : 1.0f) * (1 + column);
         if (name == "subnormal") v *= 1e-42f;
         if (name == "wide") v *= std::exp2(std::floor(unit(gen) * 60) - 30);
