@@ -33,7 +33,7 @@ struct SegmentsPlan {
 inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, int least_len) {
   const bool half = least_len == 8;
   if (n_out <= 4 && !half) return false;  // a chain lane a plane and nothing to deal out: (2,16,11445) 54 and 58
-  if (n_out * len < 1u << 16) {  // the end of a plane is added value by value: half a slice of 128 halves takes longer
+  if (n_out * len < 1u << 16) {  // the end of a plane costs more: half a slice of 128 halves takes longer
     return n_out > 64 || (len >= 128 && (!half || len >= 256 || len % 128 <= 64));
   }
   /* more planes than the split kernel has room for, which leaves a workgroup per index either way: (2048,48,196) 121 and
@@ -50,8 +50,8 @@ inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, int
   return 3000 + bytes / (lines ? 47 : 32) <= split && 3000 + len * 5 <= split;
 }
 /*! \brief short reductions of many kept indices (fewer than 65536 values of each): whether the ends of their planes - what
- *  is left of the last slice of 64 floats or 128 halves, which passes through LDS value by value - cost this kernel more than
- *  it wins. In us, the kernel of a workgroup per index and this one: floats (46,409,120) 6.3 and 7.0, (95,745,50) 9.7 and 10.7,
+ *  is left of the last slice of 64 floats or 128 halves: floats come from LDS by packs and are selected by the plane's length,
+ *  halves by whole packs and then one by one - cost this kernel more than it wins. In us, the kernel of a workgroup per index and this one: floats (46,409,120) 6.3 and 7.0, (95,745,50) 9.7 and 10.7,
  *  (4,667,756) 8.0 and 10.0, but (65,208,117) 8.8 and 6.7, (4,1928,637) 14.2 and 12.3; binary16 (38,1675,55) 7.3 and 10.9,
  *  (20,346,231) 7.2 and 8.0, (2,1439,1005) 10.2 and 15.9, but (112,335,56) 8.7 and 7.0, (22,422,198) 7.3 and 6.7, (4,1800,840)
  *  level, and planes of two slices and more, (43,835,1275) 38.8 and 27.0. */
@@ -76,7 +76,9 @@ inline bool SegmentEndsWeighMore(uint32_t n_out, uint32_t n_keep, uint64_t plane
  *  (39,957,384) 14.9 and 11.9, (5,1519,3920) 63 and 28, (12,1448,592) 15.7 and 9.5, (16,1400,140) 7.1 and 4.9, (2,1912,2048)
  *  25.6 and 13.3, (7,216,3392) 24 and 20, and with few kept indices (24,24,2208) 35 and 18, (28,184,1536) 25.5 and 11.4; small
  *  ones are level within 0.4 us, which is less than their launch. One plane per kept index, which is one lane there:
- *  (1,2048,3136) 46 and 20, (1,536,5184) 36 and 26, but (1,59,3696) 16.5 and 20; binary16 (1,72,1392) 8.8 and 7.3. */
+ *  (1,2048,3136) 46 and 20, (1,536,5184) 36 and 26, (1,512,32768) 144 and 142, (1,1100,50000) 347 and 229, (1,512,400000)
+ *  2740 and 1735, but (1,59,3696) 16.5 and 20, (1,512,50000) 203 and 217, (1,1000,40000) 173 and 184, (1,1000,65500) 263 and
+ *  298; binary16 (1,72,1392) 8.8 and 7.3, (1,64,200000) 773 and 691, (1,512,50176) 205 and 154. */
 inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, uint32_t cus, int least_len) {
   SegmentsPlan p = {false, 16, 1, 1};
   const uint64_t planes = static_cast<uint64_t>(n_out) * n_keep;
@@ -91,7 +93,9 @@ inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, 
   if (few_kept) {
     p.use = n_out == 1 ? least_len == 8 && n_keep >= 64 && len >= 512 : SegmentsOfFewKept(n_out, planes, len, least_len);
   } else if (n_out == 1) {
-    p.use = n_keep >= 2 * cus || (least_len == 8 && len >= 512);
+    /* up to a workgroup of the other kernel for every SIMD, and long planes below its own limit */
+    const bool other = least_len == 4 && n_keep <= 4 * cus && len > 36000 && len < 1u << 16;
+    p.use = (n_keep >= 2 * cus && !other) || (least_len == 8 && len >= 512);
   } else if (n_out * len >= 1u << 16) {
     p.use = planes >= 2048 && lanes * turns * 100 > planes * 112;
     if (n_out > 40 && n_out <= 64 && n_keep <= cus) {

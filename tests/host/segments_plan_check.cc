@@ -46,7 +46,14 @@ int main() {
   Expect(48, 192, 3136, kHalf, false);
   Expect(32, 192, 3136, kFloat, true);
   Expect(32, 192, 3136, kHalf, true);
-  // short reductions of many kept indices: ends of planes that are added value by value
+  // a plane a kept index: the other kernel's waves hide more of a long plane's reads, up to four workgroups a CU
+  const uint32_t single[][3] = {{512, 50000, 0}, {512, 40000, 0}, {640, 50000, 0}, {1000, 40000, 0}, {1000, 65500, 0}, {1024, 65535, 0},
+                                {512, 32768, 1}, {1000, 32768, 1}, {1024, 24000, 1}, {1100, 50000, 1}, {2048, 50000, 1}, {512, 65536, 1},
+                                {700, 400000, 1}, {768, 300, 1}};
+  for (const auto &s : single) Expect(1, s[0], s[1], kFloat, s[2] != 0);
+  for (const auto &s : single) Expect(1, s[0], s[1], kHalf, true);
+  for (const uint32_t c : {64u, 150u, 191u}) Expect(1, c, 200000, kHalf, true);
+  // short reductions of many kept indices: ends of planes
   Expect(46, 409, 120, kFloat, false);
   Expect(95, 745, 50, kFloat, false);
   Expect(65, 208, 117, kFloat, true);
