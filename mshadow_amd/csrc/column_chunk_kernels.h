@@ -3,7 +3,8 @@
  * launches: the chunks' sums in any order, their maps, and a walk down every column. The matrix is read twice, by
  * all CUs, where a strip of columns a workgroup leaves most of them idle; the sequence of a column is left
  * to one wave, which takes a chunk in 60 ns, and one that has no map in 500, where 128 dependent adds
- * take 450. 65536 x 1000: 38, 58 and 64 us (the last by the column with the fewest maps).
+ * take 450. 65536 x 1000: 38, 58 and 64 us (the last by the column with the fewest maps). Where the scratch memory does not
+ * hold the cells of all rows, they go band by band, the three launches each, from the sums that the walk of the band before left.
  */
 #ifndef MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_
 #define MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_
@@ -13,7 +14,7 @@
 #include <mshadow/hip/kernels/common.h>
 #include <mshadow/hip/kernels/reduce_dma.h>
 
-#include "column_chunks.h"
+#include "column_chunk_plan.h"
 
 namespace mshadow_hipk {
 
@@ -22,65 +23,15 @@ using column_chunks::Step;
 using column_chunks::Windows;
 using mshadow::hip::kWave;
 
-/*! \brief a workgroup has four chunks of 64 columns, a wave each */
-const int kChunkWaves = 4;
-const uint32_t kColumnsPerTile = 64;
-
-const uint32_t kMostChunkColumns = 1536;
-
-/*! \brief scratch memory of one call: cells are (chunk, column), the columns padded to whole tiles */
-const uint32_t kChunkCells = 1u << 19;
-const uint32_t kChunkCopies = 1u << 14;
 struct ColumnChunkScratch {
   Map map[kChunkCells];                             // [column][chunk], what the walk reads
   float copy[kChunkCopies][column_chunks::kRows];   // terms of chunks that are added one by one
   float before[kChunkCells];                        // [chunk][column]: sum of the workgroup's chunks in front
-  float group[kChunkCells / kChunkWaves + kChunkCells / kChunkWaves / 2];  // [workgroup of chunks][column]
+  float group[kChunkGroupCells];                    // [workgroup of chunks][column]
   uint32_t bare[kMostChunkColumns];                 // of a column: chunks that have neither a map nor a copy
+  float carry[kMostChunkColumns];                   // a column's sum behind the bands so far
 };
-
-struct ChunkShape {
-  uint32_t rows, cols, stride;
-  uint32_t chunks, groups, tiles;
-  uint32_t copies;  // copies a (chunk, tile) has room for
-  uint32_t strips;  // strips of 16 columns that may be chained, 0: none
-  uint32_t most_bare;  // bare chunks of a column that is walked
-};
-inline bool MakeChunkShape(uint32_t rows, uint32_t cols, uint32_t stride, uint32_t cus, ChunkShape *g) {
-  g->rows = rows;
-  g->cols = cols;
-  g->stride = stride;
-  g->chunks = (rows + column_chunks::kRows - 1) / column_chunks::kRows;
-  g->groups = (g->chunks + kChunkWaves - 1) / kChunkWaves;
-  g->tiles = (cols + kColumnsPerTile - 1) / kColumnsPerTile;
-  const uint64_t cells = static_cast<uint64_t>(g->chunks) * g->tiles;
-  if (cells * kColumnsPerTile > kChunkCells || cols > kMostChunkColumns) return false;
-  const uint32_t room = static_cast<uint32_t>(kChunkCopies / cells);
-  g->copies = room < kColumnsPerTile ? room : kColumnsPerTile;
-  /* A bare chunk's terms, read from the matrix 4 bytes of a cache line at a time, take 0.5 us where a column has a CU to itself,
-     1.2 us where all of 512 columns have such chunks, 2.3 us of 1000 (65536 x 1000: 1180 us in all). In a strip of 16 columns
-     128 terms of each take 0.53 us. */
-  g->strips = cols <= cus ? 0u : (cols + mshadow::hip::kLowestCols - 1) / mshadow::hip::kLowestCols;
-  g->most_bare = static_cast<uint32_t>(static_cast<uint64_t>(g->chunks) * cus / cols) + 8u;
-  /* groups * kChunkWaves may exceed chunks by three, which the array of groups allows for */
-  return static_cast<uint64_t>(g->groups) * g->tiles * kColumnsPerTile <=
-         sizeof(static_cast<ColumnChunkScratch *>(NULL)->group) / sizeof(float);
-}
-
-/*! \brief where the chunks are the sooner way. Measured, us (MI355X; a classifier's gradients), without and with:
- *  131072 x 10 448 and 99, 131072 x 100 470 and 109, 65536 x 1000 232 and 169, 30000 x 100 114 and 44, 16384 x 1000
- *  64 and 53, 16384 x 100 65 and 30, 8192 x 100 36 and 23, 8192 x 10 34 and 26; level at 8192 x 1000 and 4096 x 64,
- *  slower at 16384 x 4096 (72 and 180: its reads alone take as long as its chain). Without, a row takes 3.5 ns; with,
- *  0.8 ns, 1.6 ps a column for the second read of the matrix and the less than full rate of the first, and
- *  17 us for the three launches. More than six columns a CU walk in turns.
- *  What the terms are can take the gain away. Columns with roundings that all go one way (equal terms, 1 / 0.9 nine times of
- *  ten), or with an infinity or a NaN: 16384 x 1000 63 and 48 to 57, 65536 x 1000 230 and 140 to 199, 131072 x 10 450 and 90 to
- *  190. Columns that have no map throughout, their sums back at nothing after every other term, pay for the first two launches in
- *  vain: 6800 x 10 29 and 42, 16384 x 100 64 and 79, 16384 x 1000 62 and 110, 40000 x 1200 142 and 265, 65536 x 1000 231 and 406,
- *  131072 x 100 464 and 504; with one such column in a hundred nearly as much. */
-inline bool ColumnChunksAreSooner(uint32_t rows, uint32_t cols, uint32_t cus) {
-  return cols <= 6u * cus && static_cast<double>(rows) * (2700.0 - 1.6 * cols) > 17e6;
-}
+static_assert(kChunkStrip == mshadow::hip::kLowestCols, "a strip of the walk is one of the chain kernel's");
 
 /*! \brief a column's terms of N rows: all loads under way together */
 template <uint32_t N>
@@ -148,7 +99,7 @@ __global__ void __launch_bounds__(kChunkWaves *kWave)
  *  the matrix from its end: what the launch before read last is still in the memory-side cache. */
 __global__ void __launch_bounds__(kChunkWaves *kWave, 3)
     ColumnChunkMapsKernel(const float *src, ChunkShape g, const float *before, const float *group, Map *map,
-                          float (*copy)[column_chunks::kRows], uint32_t *bare) {
+                          float (*copy)[column_chunks::kRows], uint32_t *bare, const float *carry) {
   __shared__ float part[3][kChunkWaves][kWave];
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
   const uint32_t piece = gridDim.x - 1u - mshadow::hip::StripOfBlock(blockIdx.x, gridDim.x);
@@ -192,7 +143,7 @@ __global__ void __launch_bounds__(kChunkWaves *kWave, 3)
   if (whole) LoadRows(t, src, g, chunk * column_chunks::kRows, x);
   __syncthreads();
   if (!live) return;
-  float a = 0.0f, most = 0.0f;
+  float a = g.begun != 0u ? carry[x] : 0.0f, most = 0.0f;
 #pragma unroll
   for (int w = 0; w < kChunkWaves; ++w) {
     most = fmaxf(most, fmaxf(fabsf(a + part[1][w][lane]), fabsf(a + part[2][w][lane])));
@@ -325,7 +276,7 @@ __device__ __forceinline__ bool TakesChain(uint32_t bare, const ChunkShape &g) {
 template <typename Saver, uint32_t AT_ONCE, typename StripRing>
 __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
     ColumnChunkWalkKernel(float *dst, const float *src, ChunkShape g, const Map *map,
-                          const float (*copy)[column_chunks::kRows], const uint32_t *bare, float scale) {
+                          const float (*copy)[column_chunks::kRows], const uint32_t *bare, float *carry, float scale) {
   __shared__ union {
     WalkBlock ring[kWalkRing];
     __attribute__((aligned(16))) float strip[StripRing::kSlots][StripRing::kElems];
@@ -333,11 +284,15 @@ __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
   __shared__ uint32_t misses;  // chunks whose map did not cover the sum
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
   if (blockIdx.x < g.strips) {
-    const uint32_t x0 = mshadow::hip::StripOfBlock(blockIdx.x, g.strips) * mshadow::hip::kLowestCols;
-    const bool chain = lane < static_cast<uint32_t>(mshadow::hip::kLowestCols) && x0 + lane < g.cols && TakesChain(bare[x0 + lane], g);
-    if (__ballot(chain) != 0ull) {
-      mshadow::hip::ReduceKeepLowestDma<Saver, mshadow::red::sum, StripRing>(lds.strip, dst, src, g.stride, g.rows, g.cols, x0,
-                                                                                 chain, scale);
+    const uint32_t x0 = mshadow::hip::StripOfBlock(blockIdx.x, g.strips) * kChunkStrip;
+    const bool chain = lane < kChunkStrip && x0 + lane < g.cols && TakesChain(bare[x0 + lane], g);
+    if (__ballot(chain) == 0ull) return;
+    const float from = chain && g.begun != 0u ? carry[x0 + lane] : -0.0f;
+    const float sum = mshadow::hip::LowestDmaFold<mshadow::red::sum, StripRing, true>(lds.strip, src, g.stride, g.rows, g.cols, x0,
+                                                                                      chain, from);
+    if (wave == 0 && chain) {
+      if (g.more != 0u) carry[x0 + lane] = sum;
+      else Saver::template Save<float>(dst[x0 + lane], sum * scale);
     }
     return;
   }
@@ -417,7 +372,7 @@ __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
   }
 
   uint32_t missed = 0u;
-  float sum = -0.0f;  // the identity: the reference starts from the first term
+  float sum = g.begun != 0u ? carry[x] : -0.0f;  // the identity: the reference starts from the first term
   for (uint32_t b = 0; b < blocks + kWalkLoaders; ++b) {
     if (b >= kWalkLoaders) {
       WalkBlock *blk = &ring[(b - kWalkLoaders) % kWalkRing];
@@ -471,7 +426,10 @@ __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     mshadow::hip::BareBarrier();
   }
-  if (lane == 0) Saver::template Save<float>(dst[x], sum * scale);
+  if (lane == 0) {
+    if (g.more != 0u) carry[x] = sum;
+    else Saver::template Save<float>(dst[x], sum * scale);
+  }
 }
 
 }  // namespace mshadow_hipk

@@ -619,24 +619,29 @@ bool HasNoSlot(hipStream_t s) {
 template <typename Saver>
 bool LaunchColumnChunks(float *dst, const float *src, uint32_t stride, uint32_t rows, uint32_t cols, float scale,
                         hipStream_t s) {
-  ChunkShape g;
   const uint32_t cus = mshadow_abi::ComputeUnits();
-  if (!ColumnChunksAreSooner(rows, cols, cus) || !MakeChunkShape(rows, cols, stride, cus, &g) || HasNoSlot(s)) return false;
+  if (!ColumnChunksAreSooner(rows, cols, cus) || HasNoSlot(s)) return false;
   ColumnScratchTable &t = ColumnTable();
   std::lock_guard<std::mutex> lock(t.mu);
   ColumnChunkScratch *w = t.Slot(s);
   if (w == NULL) return false;
-  const dim3 grid(g.groups * g.tiles), block(kChunkWaves * 64);
-  LaunchKernelIfFits(ColumnChunkSumsKernel, grid, block, 0, s, src, g, w->before, w->group, w->bare);
-  LaunchKernelIfFits(ColumnChunkMapsKernel, grid, block, 0, s, src, g, w->before, w->group, w->map, w->copy,
-                     w->bare);
-  const dim3 columns(g.strips + cols), walk((1 + kWalkLoaders) * 64);
-#define WALK(AT_ONCE, RING)                                                                                              \
-  LaunchKernelIfFits((ColumnChunkWalkKernel<Saver, AT_ONCE, RING>), columns, walk, 0, s, dst, src, g, w->map, w->copy,   \
-                     w->bare, scale)
-  if (cols <= ColumnsOfWideWalk(cus)) WALK(16, StripRingOfTwo);
-  else WALK(4, StripRingOfSix);
+  const uint32_t band = ChunkBandRows(rows, cols);
+  for (uint32_t row0 = 0; row0 < rows; row0 += band) {
+    ChunkShape g = MakeChunkShape(rows - row0 < band ? rows - row0 : band, cols, stride, cus);
+    g.begun = row0 != 0;
+    g.more = g.rows < rows - row0;
+    const float *from = src + static_cast<size_t>(row0) * stride;
+    const dim3 grid(g.groups * g.tiles), block(kChunkWaves * 64), columns(g.strips + cols), walk((1 + kWalkLoaders) * 64);
+    LaunchKernelIfFits(ColumnChunkSumsKernel, grid, block, 0, s, from, g, w->before, w->group, w->bare);
+    LaunchKernelIfFits(ColumnChunkMapsKernel, grid, block, 0, s, from, g, w->before, w->group, w->map, w->copy, w->bare,
+                       w->carry);
+#define WALK(AT_ONCE, RING)                                                                                             \
+  LaunchKernelIfFits((ColumnChunkWalkKernel<Saver, AT_ONCE, RING>), columns, walk, 0, s, dst, from, g, w->map, w->copy, \
+                     w->bare, w->carry, scale)
+    if (cols <= ColumnsOfWideWalk(cus)) WALK(16, StripRingOfTwo);
+    else WALK(4, StripRingOfSix);
 #undef WALK
+  }
   return true;
 }
 }  // namespace

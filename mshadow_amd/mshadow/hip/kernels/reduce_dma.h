@@ -93,10 +93,11 @@ __device__ __forceinline__ void BareBarrier() { asm volatile("s_barrier" ::: "me
  * four rows: lane l fetches row 4 g + (l & 3), column l >> 2, so the slot holds
  * [group][column][row & 3] and a chain lane reads rows 4g..4g+3 of its column as one
  * 128-bit word, 64 floats from the next group. */
-/*! \brief a workgroup of 1 + Ring::kLoaders waves; lane l of wave 0 folds column x0 + l if that is `wanted` */
-template <typename Saver, typename Reducer, typename Ring>
-__device__ __forceinline__ void ReduceKeepLowestDma(float (*ring)[Ring::kElems], float *dst, const float *src, uint32_t stride,
-                                                    uint32_t rows, uint32_t cols, uint32_t x0, bool wanted, float scale) {
+/*! \brief a workgroup of 1 + Ring::kLoaders waves; lane l of wave 0 folds column x0 + l if that is `wanted`. BEGUN: on from
+ *  `res`; else from the first row. */
+template <typename Reducer, typename Ring, bool BEGUN>
+__device__ __forceinline__ float LowestDmaFold(float (*ring)[Ring::kElems], const float *src, uint32_t stride, uint32_t rows,
+                                               uint32_t cols, uint32_t x0, bool wanted, float res) {
   const int kDmaSlots = Ring::kSlots, kDmaAhead = Ring::kAhead, kDmaPerWave = Ring::kPerWave;
   const int CW = kLowestCols;
   const int TR = Ring::kElems / CW;
@@ -130,7 +131,6 @@ __device__ __forceinline__ void ReduceKeepLowestDma(float (*ring)[Ring::kElems],
     }
   } else {
     const bool chain_lane = lane < static_cast<uint32_t>(CW) && x0 + lane < cols && wanted;
-    float res = 0.0f;
     for (uint32_t i = 0; i < nstep; ++i) {
       BareBarrier();
       if (i >= static_cast<uint32_t>(kDmaAhead) && chain_lane) {
@@ -139,23 +139,26 @@ __device__ __forceinline__ void ReduceKeepLowestDma(float (*ring)[Ring::kElems],
         const float *mine = ring[st % kDmaSlots] + lane * 4;
         const int count = (rows - row0 < (uint32_t)TR) ? static_cast<int>(rows - row0) : TR;
         int begin = 0;
-        if (st == 0) {  // the reference starts from src(0, x), not from an initial value
+        if (!BEGUN && st == 0) {  // the reference starts from src(0, x), not from an initial value
           res = mine[0];
           begin = 1;
         }
         ChainFold<Reducer, kWave>(res, mine, begin, count);
       }
     }
-    if (chain_lane) Saver::template Save<float>(dst[x0 + lane], res * scale);
   }
+  return res;
 }
 template <typename Saver, typename Reducer>
 __global__ void __launch_bounds__(kDmaThreads)
     ReduceKeepLowestDmaKernel(float *dst, const float *src, uint32_t stride, uint32_t rows,
                               uint32_t cols, float scale) {
   __shared__ MSHADOW_ALIGNED(16) float ring[LowestRing::kSlots][LowestRing::kElems];
-  ReduceKeepLowestDma<Saver, Reducer, LowestRing>(ring, dst, src, stride, rows, cols,
-                                                  StripOfBlock(blockIdx.x, gridDim.x) * kLowestCols, true, scale);
+  const uint32_t x0 = StripOfBlock(blockIdx.x, gridDim.x) * kLowestCols;
+  const float res = LowestDmaFold<Reducer, LowestRing, false>(ring, src, stride, rows, cols, x0, true, 0.0f);
+  if (threadIdx.x < static_cast<uint32_t>(kLowestCols) && x0 + threadIdx.x < cols) {
+    Saver::template Save<float>(dst[x0 + threadIdx.x], res * scale);
+  }
 }
 
 /* ------------------------------------------------------------------ KeepLowest in strips

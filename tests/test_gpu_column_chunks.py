@@ -65,11 +65,12 @@ def terms(kind, rows, cols, seed):
     return np.ascontiguousarray(m)
 
 
-# up to 64 columns from 6400 rows on, 100 from 6695, 1000 from 15455 (8 to 1536 columns otherwise); chunks of 128 rows,
-# workgroups of four chunks and 64 columns, blocks of 16 chunks; up to two columns a compute unit (512) the walk takes a block's
-# maps at once, beyond that four
-SHAPES = [(6300, 10), (6400, 10), (6528, 64), (6529, 65), (6783, 63), (8192, 1), (8193, 3), (8320, 129), (10240, 128),
-          (9200, 512), (9200, 513), (16384, 1000), (20481, 17), (33000, 300)]
+# with 10 columns from 6335 rows on, with 64 from 6545, with 1000 from 15455 (tests/host/column_chunk_plan_check.cc looks these up);
+# chunks of 128 rows, workgroups of four chunks and 64 columns, blocks of 16 chunks; up to two columns a compute unit (512) the walk
+# takes a block's maps at once, beyond that four; bands of 8192 chunks of up to 64 columns, 512 of up to 1024
+SHAPES = [(6300, 10), (6400, 10), (6528, 64), (6656, 64), (6657, 65), (6783, 63), (8192, 1), (8193, 3), (8320, 129), (10240, 128),
+          (9200, 512), (9200, 513), (16384, 1000), (20481, 17), (33000, 300), (65536, 1000), (65537, 1000), (1048576, 3),
+          (1048577, 3), (2097281, 5)]
 
 
 @pytest.mark.parametrize("rows,cols", SHAPES)
@@ -81,7 +82,7 @@ def test_long_columns(G, O, rows, cols):
         view = SimpleNamespace(ptr=src.ptr + shift * 4, stride=src.stride, rows=rows, cols=cols, dtype=src.dtype,
                                shape=(rows, cols))
         start = np.random.default_rng(8).standard_normal(cols, dtype=f32)
-        for saver in (SAVETO, PLUSTO, MINUSTO):
+        for saver in (SAVETO, PLUSTO, MINUSTO) if rows * cols < 1 << 24 else (PLUSTO,):
             want, dst = start.copy(), G.to_device(start)
             O.reduce_keep_lowest(want, m, SUM, saver, 0.75)
             G.reduce_keep_lowest(dst, view, SUM, saver, 0.75)
@@ -125,6 +126,22 @@ def test_time_without_usable_maps(G, kind):
         return min(times)
 
     assert least(terms(kind, rows, cols, 3)) < 2 * least(terms("normal", rows, cols, 3))
+
+
+@pytest.mark.parametrize("kind", ["constant", "cancelling", "late", "few", "infinite"])
+def test_bands_of_columns_without_maps(G, O, kind):
+    """a column that is chained in one band and walked in the next, or was left infinite or NaN by the one before"""
+    rows, cols = 66001, 1000   # two bands of 260 chunks and less
+    m = terms("normal", rows, cols, 5)
+    m[rows // 4:3 * rows // 4] = terms(kind, 3 * rows // 4 - rows // 4, cols, 6)
+    want, dst = np.full(cols, 7, f32), G.to_device(np.full(cols, 7, f32))
+    with np.errstate(all="ignore"):
+        O.reduce_keep_lowest(want, m, SUM, PLUSTO, 0.75)
+    G.reduce_keep_lowest(dst, G.to_device(m), SUM, PLUSTO, 0.75)
+    got = dst.download()
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert_bits_equal(got[~nan], want[~nan], kind)
 
 
 def test_streams_threads_and_recording(G, O):

@@ -208,6 +208,13 @@ def test_column_sums_by_chunks_match_the_serial_sum_on_host(tmp_path):
     assert out.endswith("OK\n"), out[-500:]
 
 
+def test_long_column_sums_go_by_chunks_in_bands_that_fit(tmp_path):
+    """which column sums go by chunks, the shapes of the GPU tests among them, and in which bands of rows: none is
+    left to the chain because the scratch memory holds no more, and every band fits it"""
+    out = _compile_and_run(tmp_path, "column_chunk_plan_check.cc", [])
+    assert out.startswith("OK"), out[-500:]
+
+
 def test_half_sum_pruning_rule_is_exhaustively_sound(tmp_path):
     """the binary16 softmax row sum leaves out the terms below half an ulp of a lower bound of
     the running sum: for every pair of a finite non-negative binary16 sum and term the rule
