@@ -579,6 +579,16 @@ struct ColumnScratchTable {
   ColumnChunkScratch *base[mshadow_abi::kScratchDevices];
   mshadow_abi::ScratchSlots<kColumnScratchSlots> slots;
 
+  /* where the slots of the current device are, looked up once; mu is held */
+  void Resolve(int dev) {
+    if (base[dev] != NULL) return;
+    void *p = NULL;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(g_column_scratch)) == hipSuccess) {
+      base[dev] = static_cast<ColumnChunkScratch *>(p);
+    } else {
+      (void)hipGetLastError();
+    }
+  }
   /* the caller's slot on the current device, NULL where there is none to be had; mu is held */
   ColumnChunkScratch *Slot(void *stream) {
     int dev = 0;
@@ -586,14 +596,8 @@ struct ColumnScratchTable {
       (void)hipGetLastError();
       return NULL;
     }
-    if (base[dev] == NULL) {
-      void *p = NULL;
-      if (hipGetSymbolAddress(&p, HIP_SYMBOL(g_column_scratch)) != hipSuccess) {
-        (void)hipGetLastError();
-        return NULL;
-      }
-      base[dev] = static_cast<ColumnChunkScratch *>(p);
-    }
+    Resolve(dev);
+    if (base[dev] == NULL) return NULL;
     const int slot = slots.Take(dev, stream);
     return slot < 0 ? NULL : base[dev] + slot;
   }
@@ -667,8 +671,9 @@ void ReleaseReduceScratch(void *stream, bool done) {
   std::lock_guard<std::mutex> lock(t.mu);
   t.slots.Release(stream, done);
 }
-/* called when a device is selected: where the scratch array lives on that device is looked up
-   then, not inside the first reduction that wants a slot (which may be being recorded) */
+/* called when a device is selected: where the scratch arrays live on that device is looked up
+   then, not inside the first reduction that wants a slot (which may be being recorded, or queued while
+   the same thread records another stream) */
 void ResolveReduceScratch() {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kScratchDevices) {
@@ -685,6 +690,9 @@ void ResolveReduceScratch() {
       (void)hipGetLastError();
     }
   }
+  ColumnScratchTable &c = ColumnTable();
+  std::lock_guard<std::mutex> column_lock(c.mu);
+  c.Resolve(dev);
 }
 }  // namespace mshadow_abi
 

@@ -177,14 +177,20 @@ def test_streams_threads_and_recording(G, O):
     for i in range(4):
         assert_bits_equal(out[i].download(), want[i], f"thread {i}")
 
+    # a slot of its own in the recording stream, which sums others' columns while its recording is replayed beside it
     G.graph_begin(streams[1])
     G.reduce_keep_lowest(out[2], src[2], stream=streams[1])
+    G.reduce_keep_lowest(out[4], src[4], stream=streams[0])   # not recorded, while the same thread records
     graph = G.graph_end(streams[1])
-    for _ in range(3):
-        G.fill(out[2], 3.0, streams[1])
-        G.graph_launch(graph, streams[1])
-        G.reduce_keep_lowest(out[3], src[3], stream=streams[1])
+    G.stream_sync(streams[0])
+    assert_bits_equal(out[4].download(), want[4], "beside a recording")
+    for _ in range(5):
+        G.fill(out[2], 3.0, streams[2])
+        for i in range(6):
+            G.graph_launch(graph, streams[2])
+            G.reduce_keep_lowest(out[3], src[3], stream=streams[1])
         G.stream_sync(streams[1])
+        G.stream_sync(streams[2])
         assert_bits_equal(out[2].download(), want[2], "replayed")
         assert_bits_equal(out[3].download(), want[3], "beside a replay")
     G.graph_destroy(graph)
