@@ -196,3 +196,29 @@ def test_streams_threads_and_recording(G, O):
     G.graph_destroy(graph)
     for s in streams:
         G.stream_destroy(s)
+
+
+def test_slots_of_streams_that_go_away(G, O):
+    """a stream destroyed with sums queued gives its scratch memory to the next one only when they are done"""
+    rows, cols = 20000, 200
+    mats = [terms(k, rows, cols, 30 + i) for i, k in enumerate(("normal", "gradient"))]
+    want = []
+    for m in mats:
+        w = np.empty(cols, f32)
+        O.reduce_keep_lowest(w, m)
+        want.append(w)
+    src = [G.to_device(m) for m in mats]
+    out = [G.buffer((cols,), f32) for _ in mats]
+    for _ in range(6):   # more of them than slots
+        a, b = G.stream_create(), G.stream_create()
+        for _ in range(8):
+            G.reduce_keep_lowest(out[0], src[0], stream=a)
+        G.stream_destroy(a)
+        c = G.stream_create()
+        G.reduce_keep_lowest(out[1], src[1], stream=c)
+        G.reduce_keep_lowest(out[0], src[0], stream=b)
+        G.device_sync()
+        for i in range(2):
+            assert_bits_equal(out[i].download(), want[i], f"stream {i}")
+        G.stream_destroy(b)
+        G.stream_destroy(c)
