@@ -27,8 +27,23 @@ def test_row_sums_that_end_above_a_power_of_two(cols):
     sums = G.buffer((len(terms),), f32)
     G.softmax_rowsum(sums, G.to_device(terms))
     assert_bits_equal(sums.download(), want, f"{cols} columns")
-    x = np.log(np.maximum(terms, 1e-30)).astype(f32)   # the softmax of the same rows sums to 1
+    # Softmax of rows whose largest term is a power of two, so that its terms, divided by that, end there too. The probability of
+    # that term is 1 / sum. Against the same serial sum of numpy's exponentials, which differ from the device's by few ulps: two sums
+    # with roundings of their own, uniform in half an ulp (2^-24 of the sum) to either side, so 2^-24 sqrt(cols / 3) off the exact one
+    # each; six times what both are off together, and 8 ulps for the exponentials and the quotient.
+    rest = terms[:, 1:].astype(np.float64)
+    total = terms.astype(np.float64).sum(1)
+    largest = 2.0 ** np.ceil(np.log2(rest.max(1)))
+    rest *= ((total - largest) / rest.sum(1))[:, None]
+    largest = np.where(rest.max(1) > largest, 2 * largest, largest)
+    x = np.log(np.maximum(np.column_stack([largest, rest]) / largest[:, None], 1e-30)).astype(f32)
+    assert np.all(x.max(1) == 0) and np.all(x[:, 0] == 0)
+    want = np.array([np.add.accumulate(np.exp(r), dtype=f32)[-1] for r in x]).astype(np.float64)
     p = G.buffer(x.shape, f32)
     G.softmax(p, G.to_device(x))
-    got = p.download().astype(np.float64).sum(1)
-    assert np.all(np.abs(got - 1) < cols * 2.0 ** -24)   # a sum's cols roundings of at most half an ulp
+    got = p.download().astype(np.float64)
+    bound = 6 * np.sqrt(2 * cols / 3) * 2.0 ** -24 + 8 * 2.0 ** -24
+    assert np.all(np.abs(got[:, 0] * want - 1) < bound), np.abs(got[:, 0] * want - 1).max() / bound
+    ratio = got * want[:, None] / np.exp(x.astype(np.float64))
+    normal = got > 2.0 ** -120   # not where quotients round to subnormals
+    assert np.all(np.abs(ratio[normal] - 1) < bound)
