@@ -30,7 +30,7 @@ struct SegmentsPlan {
  *  (512,16,784) 56 and 32, (826,31,1936) 131 and 95, (64,128,2048) 29 and 15, but (2048,4,2048) 184 and 315; odd planes, which
  *  the generic kernel has otherwise, (512,16,2025) 141 and 96. Short reductions: 32 planes of 196 6.2 and 4.9, 41 of 132
  *  5.6 and 4.7, 128 of 100 8.8 and 6.5, but 64 of 100 5.4 and 5.7, 35 of 56 4.3 and 5.1, binary16 40 of 255 7.7 and 8.4. */
-inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, int least_len) {
+inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, uint32_t cus, int least_len) {
   const bool half = least_len == 8;
   if (n_out <= 4 && !half) return false;  // a chain lane a plane and nothing to deal out: (2,16,11445) 54 and 58
   if (n_out * len < 1u << 16) {  // the end of a plane costs more: half a slice of 128 halves takes longer
@@ -39,12 +39,25 @@ inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, int
   /* more planes than the split kernel has room for, which leaves a workgroup per index either way: (2048,48,196) 121 and
      77, (1618,41,100) 75 and 48, (1024,128,100) 49 and 32; binary16 86 and 69, 58 and 54, 39 and 34 */
   if (planes > 65536) return true;
-  if (half && len % 2 != 0) return true;
+  /* what the generic kernel has otherwise, whose large workgroups (from 2^18 values an index on) are the sooner ones where
+     its 16 chain lanes are in use and this kernel has two waves: (10,46,40001) 176 and 199, (16,64,31251) 130 and 139, but
+     (8,46,40001) 251 and 143, (16,46,10001) 68 and 52, (16,180,20001) 82 and 71 */
+  if (half && len % 2 != 0) return n_out < 9 || n_out > 16 || n_out * len < 1u << 18 || planes >= 100 * n_out;
   const uint64_t bytes = n_out * len * (16u / least_len), all = planes / n_out * bytes;
   const bool lines = bytes / n_out % 128 == 0;
   if (half) {
     const uint64_t split = 10000 + 90 * n_out + all / 2000;  // ns, as below; rates are bytes a ns
-    return bytes <= split * (lines ? 39 : 30) && len * 6 <= split;
+    if (bytes > split * (lines ? 39 : 30) || len * 6 > split) return false;
+    /* One round of workgroups of the split kernel, 16 planes of whole packs each or 32: it takes, in us, 5 + 0.085 n and 3.5 ns
+       an element (5.3 + 0.056 n and 4.4). Of this kernel's chains an element takes 5.5 ns, where there are eight to a wave 6 to
+       4, the fewer the more indices are kept and while every wave has a SIMD to itself: (64,46,5000) 28 and 33, (40,46,3000) 20 and 24, (64,64,8000) 38 and 45, (81,50,6384) 34.5 and
+       39, but (64,46,1400) 15.4 and 12.9, (72,46,3000) 22 and 19.5, (32,100,2048) 15.2 and 13.5, and in two rounds (64,80,5000) 45
+       and 30, (81,64,8000) 65 and 46 */
+    const bool packs = len % 8 == 0;
+    if (planes > (packs ? 16u : 32u) * cus) return true;
+    const uint64_t kept = planes / n_out;
+    const uint64_t ps = n_out > 64 ? 5500 : kept < 64 ? 6000 : kept < 96 ? 5000 : n_out > 32 ? 4600 : 4000;  // an element
+    return 4500 + len * ps / 1000 <= (packs ? 5000 + 85 * n_out + len * 7 / 2 : 5300 + 56 * n_out + len * 22 / 5);
   }
   const uint64_t split = (n_out <= 400 ? 8000 + 80 * n_out : 6000 + 85 * n_out) + all / 8000;
   return 3000 + bytes / (lines ? 47 : 32) <= split && 3000 + len * 5 <= split;
@@ -91,7 +104,7 @@ inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, 
   const uint32_t side = n_out > 16 ? 64 : n_out > 4 ? 16 : n_out > 1 ? 4 : 1;
   const uint64_t lanes = (n_out + side - 1) / side * side, turns = (n_keep + cus - 1) / cus * cus;
   if (few_kept) {
-    p.use = n_out == 1 ? least_len == 8 && n_keep >= 64 && len >= 512 : SegmentsOfFewKept(n_out, planes, len, least_len);
+    p.use = n_out == 1 ? least_len == 8 && n_keep >= 64 && len >= 512 : SegmentsOfFewKept(n_out, planes, len, cus, least_len);
   } else if (n_out == 1) {
     /* up to a workgroup of the other kernel for every SIMD, and long planes below its own limit */
     const bool other = least_len == 4 && n_keep <= 4 * cus && len > 36000 && len < 1u << 16;

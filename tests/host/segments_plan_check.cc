@@ -53,6 +53,14 @@ int main() {
   for (const auto &s : single) Expect(1, s[0], s[1], kFloat, s[2] != 0);
   for (const auto &s : single) Expect(1, s[0], s[1], kHalf, true);
   for (const uint32_t c : {64u, 150u, 191u}) Expect(1, c, 200000, kHalf, true);
+  // half_t, few kept indices: one round of the split kernel's workgroups is sooner done than long chains ...
+  const uint32_t half_split[][3] = {{64, 46, 5000}, {64, 64, 8000}, {40, 46, 3000}, {40, 8, 2048}, {48, 80, 6384}, {81, 50, 6384}, {81, 46, 5000},
+                                    {10, 46, 40001}, {16, 64, 31251}, {16, 8, 20001}, {10, 8, 26215}};
+  for (const auto &s : half_split) Expect(s[0], s[1], s[2], kHalf, false);
+  // ... short ones and two rounds are not
+  const uint32_t half_own[][3] = {{64, 46, 1400}, {64, 80, 5000}, {72, 46, 3000}, {81, 64, 8000}, {32, 100, 2048}, {32, 180, 6384}, {128, 46, 8000},
+                                  {8, 46, 40001}, {16, 46, 10001}, {16, 180, 20001}, {17, 46, 40001}};
+  for (const auto &s : half_own) Expect(s[0], s[1], s[2], kHalf, true);
   // short reductions of many kept indices: ends of planes
   Expect(46, 409, 120, kFloat, false);
   Expect(95, 745, 50, kFloat, false);
