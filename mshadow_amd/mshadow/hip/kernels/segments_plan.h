@@ -62,19 +62,26 @@ inline bool SegmentsOfFewKept(uint64_t n_out, uint64_t planes, uint64_t len, uin
   const uint64_t split = (n_out <= 400 ? 8000 + 80 * n_out : 6000 + 85 * n_out) + all / 8000;
   return 3000 + bytes / (lines ? 47 : 32) <= split && 3000 + len * 5 <= split;
 }
-/*! \brief short reductions of many kept indices (fewer than 65536 values of each): whether the ends of their planes - what
- *  is left of the last slice of 64 floats or 128 halves: floats come from LDS by packs and are selected by the plane's length,
- *  halves by whole packs and then one by one - cost this kernel more than it wins. In us, the kernel of a workgroup per index and this one: floats (46,409,120) 6.3 and 7.0, (95,745,50) 9.7 and 10.7,
+/*! \brief short reductions of many kept indices (fewer than 65536 values of each) that are not this kernel's: mostly where the
+ *  ends of their planes - what is left of the last slice of 64 floats or 128 halves: floats come from LDS by packs and are
+ *  selected by the plane's length, halves by whole packs and then one by one - cost more than it wins. In us, the kernel of a
+ *  workgroup per index and this one: floats (46,409,120) 6.3 and 7.0, (95,745,50) 9.7 and 10.7,
  *  (4,667,756) 8.0 and 10.0, but (65,208,117) 8.8 and 6.7, (4,1928,637) 14.2 and 12.3; binary16 (38,1675,55) 7.3 and 10.9,
  *  (20,346,231) 7.2 and 8.0, (2,1439,1005) 10.2 and 15.9, but (112,335,56) 8.7 and 7.0, (22,422,198) 7.3 and 6.7, (4,1800,840)
  *  level, and planes of two slices and more, (43,835,1275) 38.8 and 27.0. */
-inline bool SegmentEndsWeighMore(uint32_t n_out, uint32_t n_keep, uint64_t planes, uint64_t len, uint32_t cus, int least_len) {
+inline bool ShortSumsGoElsewhere(uint32_t n_out, uint32_t n_keep, uint64_t planes, uint64_t len, uint32_t cus, int least_len) {
   const bool one_round = n_out > 64 && n_keep <= 2 * cus;  // few workgroups of several rounds each with the other kernel
   if (least_len == 8) {
     if (n_out <= 4) return len % 128 > 72;
+    if (n_out <= 16 && len < 256) return true;  // (15,1400,133) 5.1 and 7.1, (9,1400,161) 5.2 and 5.4
     return (len < 128 && !one_round) || (len >= 128 && len < 256 && len % 128 > 72);
   }
-  if (n_out <= 4) return len > 600 && planes < 2800 && len % 64 >= 44;
+  if (n_out <= 4) return n_keep <= cus || (len > 600 && planes < 2800 && len % 64 >= 44);  // (3,220,1000) 6.8 and 7.8
+  if (n_out <= 16) {
+    /* short planes, (14,600,161) 3.8 and 4.2, (11,686,234) 4.3 and 4.6, and more than the memory-side cache has, (15,8000,2385) 195 and 226, (13,4000,4000)
+       151 and 170, but (14,2947,1500) 47 and 37 */
+    return (len < (n_out < 9 ? 200u : 256u) && n_keep <= 4 * cus) || (n_out >= 12 && planes * len > 80000000);
+  }
   return len < 128 && len % 64 >= 44 && n_out >= 24 && !one_round;
 }
 /*! \brief Measured on (n, c, len), us, the other kernels and this one; floats, binary16 gains as much.
@@ -115,7 +122,7 @@ inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, 
       p.use = p.use && least_len == 4 && n_out <= 48 && n_keep * 16ull < 15ull * cus;
     }
   } else {
-    p.use = !SegmentEndsWeighMore(n_out, n_keep, planes, len, cus, least_len);
+    p.use = !ShortSumsGoElsewhere(n_out, n_keep, planes, len, cus, least_len);
   }
   if (!p.use) return p;
   /* more waves: (32,512,784) 12.4, with sixteen 13.3; up to two waves a SIMD of a workgroup's CU, which take turns

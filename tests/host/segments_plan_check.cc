@@ -61,6 +61,12 @@ int main() {
   const uint32_t half_own[][3] = {{64, 46, 1400}, {64, 80, 5000}, {72, 46, 3000}, {81, 64, 8000}, {32, 100, 2048}, {32, 180, 6384}, {128, 46, 8000},
                                   {8, 46, 40001}, {16, 46, 10001}, {16, 180, 20001}, {17, 46, 40001}};
   for (const auto &s : half_own) Expect(s[0], s[1], s[2], kHalf, true);
+  // up to sixteen planes of many kept indices
+  const uint32_t middling[][4] = {{3, 220, 1000, 0}, {4, 256, 6119, 0}, {3, 280, 1000, 1}, {14, 600, 161, 0}, {9, 600, 161, 0}, {14, 600, 250, 0}, {14, 600, 257, 1}, {8, 600, 250, 1},
+                                  {14, 1400, 161, 1}, {15, 8000, 2385, 0}, {13, 4000, 4000, 0}, {14, 2947, 1500, 1}, {10, 12000, 4000, 1}, {15, 906, 881, 1}};
+  for (const auto &s : middling) Expect(s[0], s[1], s[2], kFloat, s[3] != 0);
+  const uint32_t middling_half[][4] = {{15, 1400, 133, 0}, {9, 1400, 161, 0}, {16, 2947, 250, 0}, {15, 1400, 257, 1}, {5, 600, 400, 1}};
+  for (const auto &s : middling_half) Expect(s[0], s[1], s[2], kHalf, s[3] != 0);
   // short reductions of many kept indices: ends of planes
   Expect(46, 409, 120, kFloat, false);
   Expect(95, 745, 50, kFloat, false);
