@@ -84,6 +84,26 @@ inline bool ShortSumsGoElsewhere(uint32_t n_out, uint32_t n_keep, uint64_t plane
   }
   return len < 128 && len % 64 >= 44 && n_out >= 24 && !one_round;
 }
+/*! \brief kept indices of a workgroup where an index has five to sixteen planes: what two to eight waves hold. What counts are the
+ *  waves of the CU that has the most: (14,906,881) two indices and four waves a workgroup, two of those a CU, 10.2 us, three
+ *  indices and six waves 12.4; (9,1024,2385) four indices, five waves, one workgroup a CU 16.8, three indices, four waves, two 18.8.
+ *  Within an eighth the fewer workgroups: (11,1079,2385) three indices, ten waves a CU 22.7, two, nine waves 24.1. */
+inline uint32_t KeptOfMiddling(uint32_t n_out, uint32_t n_keep, uint32_t lanes, uint32_t cus) {
+  const uint32_t kMost = 8;
+  uint32_t kept[kMost + 1], load[kMost + 1], least = ~0u, best = 1;
+  for (uint32_t waves = 2; waves <= kMost; ++waves) {
+    kept[waves] = waves * lanes / n_out;
+    if (kept[waves] > n_keep / cus) kept[waves] = n_keep / cus;
+    if (kept[waves] < 1) kept[waves] = 1;
+    const uint32_t groups = (n_keep + kept[waves] - 1) / kept[waves];
+    load[waves] = (groups + cus - 1) / cus * ((kept[waves] * n_out + lanes - 1) / lanes);
+    if (load[waves] < least) least = load[waves];
+  }
+  for (uint32_t waves = 2; waves <= kMost; ++waves) {
+    if (static_cast<uint64_t>(load[waves]) * 8 <= static_cast<uint64_t>(least) * 9) best = kept[waves];
+  }
+  return best;
+}
 /*! \brief Measured on (n, c, len), us, the other kernels and this one; floats, binary16 gains as much.
  *  A workgroup per kept index that fills a CU: (248,552,280) 70 and 42, (30,600,2500) 74
  *  and 44, (19,304,5760) 93 and 35, (5,1144,8320) 115 and 49, (114,246,896) 22 and 18, (248,416,450) 54 and 42, where chain
@@ -129,7 +149,11 @@ inline SegmentsPlan PlanSegments(uint32_t n_out, uint32_t n_keep, uint64_t len, 
      beyond that */
   if (len >= 512 && planes / 16 < 4 * cus && n_out <= 64) p.lanes = 8;
   /* workgroups of four waves or so where planes are few per kept index, but one for every CU */
-  while (p.kept * n_out < 4u * p.lanes && n_keep / (p.kept + 1) >= cus) ++p.kept;
+  if (n_out >= 5 && n_out <= 16) {
+    p.kept = KeptOfMiddling(n_out, n_keep, p.lanes, cus);
+  } else {
+    while (p.kept * n_out < 4u * p.lanes && n_keep / (p.kept + 1) >= cus) ++p.kept;
+  }
   const uint32_t all = (p.kept * n_out + p.lanes - 1) / p.lanes;
   /* a CU holds 20 waves of this kernel: where there are more of them, small workgroups that go round again fill it,
      but not where few kept indices are few workgroups ((1024,128,100): 62 of them that way, now 32) */

@@ -67,6 +67,8 @@ int main() {
   for (const auto &s : middling) Expect(s[0], s[1], s[2], kFloat, s[3] != 0);
   const uint32_t middling_half[][4] = {{15, 1400, 133, 0}, {9, 1400, 161, 0}, {16, 2947, 250, 0}, {15, 1400, 257, 1}, {5, 600, 400, 1}};
   for (const auto &s : middling_half) Expect(s[0], s[1], s[2], kHalf, s[3] != 0);
+  // ... and how they are dealt out: no CU has more waves than need be
+  if (PlanSegments(14, 906, 881, kCus, kFloat).kept != 2 || PlanSegments(9, 1024, 2385, kCus, kFloat).kept != 4) ++g_wrong, printf("kept\n");
   // short reductions of many kept indices: ends of planes
   Expect(46, 409, 120, kFloat, false);
   Expect(95, 745, 50, kFloat, false);
