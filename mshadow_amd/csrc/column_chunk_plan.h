@@ -75,9 +75,9 @@ inline ChunkShape MakeChunkShape(uint32_t rows, uint32_t cols, uint32_t stride, 
  *  vain: 6800 x 10 29 and 42, 16384 x 100 64 and 79, 16384 x 1000 62 and 110, 40000 x 1200 142 and 265, 65536 x 1000 231 and 406,
  *  131072 x 100 464 and 504; with one such column in a hundred nearly as much. */
 inline bool ColumnChunksAreSooner(uint32_t rows, uint32_t cols, uint32_t cus) {
-  if (cols > 6u * cus || cols > kMostChunkColumns) return false;
+  if (cols > 6u * cus || cols > kMostChunkColumns || static_cast<double>(rows) * (2700.0 - 1.6 * cols) <= 17e6) return false;
   const uint32_t band = ChunkBandRows(rows, cols), bands = (rows + band - 1) / band;
-  return static_cast<double>(rows) * ((bands == 1 ? 2700.0 : 2350.0) - 1.6 * cols) > 17e6 * bands;
+  return bands == 1 || static_cast<double>(rows) * (2350.0 - 1.6 * cols) > 17e6 * bands;
 }
 
 }  // namespace mshadow_hipk
