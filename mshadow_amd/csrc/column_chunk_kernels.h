@@ -3,7 +3,7 @@
  * launches: the chunks' sums in any order, their maps, and a walk down every column. The matrix is read twice, by
  * all CUs, where a strip of columns a workgroup leaves most of them idle; the sequence of a column is left
  * to one wave, which takes a chunk in 60 ns, and one that has no map in 500, where 128 dependent adds
- * take 450. 65536 x 1000: 38, 58 and 64 us (the last by the column with the fewest maps). Where the scratch memory does not
+ * take 450. 65536 x 1000: 48, 58 and 63 us (the last by the column with the fewest maps). Where the scratch memory does not
  * hold the cells of all rows, they go band by band, the three launches each, from the sums that the walk of the band before left.
  */
 #ifndef MSHADOW_AMD_CSRC_COLUMN_CHUNK_KERNELS_H_
@@ -57,8 +57,8 @@ __device__ __forceinline__ bool IsWhole(const ChunkShape &g, uint32_t chunk) {
 const uint32_t kSumsAtOnce = 32;
 
 /*! \brief the sums of the chunks, in any order of adds: per workgroup of four chunks the sum of those in
- *  front of each, and of all. Bound by its read of the matrix: 65536 x 1000 38 us, 6.9 TB/s; four columns a lane, which
- *  leaves a quarter of the waves, was a seventh slower. */
+ *  front of each, and of all. Bound by its read of the matrix: 65536 x 1000 48 us, 5.5 TB/s; four columns a lane, which
+ *  leaves a quarter of the waves, 57. */
 __global__ void __launch_bounds__(kChunkWaves *kWave)
     ColumnChunkSumsKernel(const float *src, ChunkShape g, float *before, float *group, uint32_t *bare) {
   __shared__ float sums[kChunkWaves][kWave];
@@ -271,7 +271,7 @@ __device__ __forceinline__ bool TakesChain(uint32_t bare, const ChunkShape &g) {
  *  first workgroups have a strip of 16 columns each, of which they add those that TakesChain from top to bottom.
  *  AT_ONCE: maps in registers together. All of a block where two columns a CU at most leave the registers for it
  *  (65536 x 64 of columns with a map for every chunk 28.9 us, 35.0 with eight; 30000 x 100 gradients 25.2 and 27.8), four
- *  where four have to share a CU (65536 x 1000 gradients 60 to 63 us, with eight 58 to 76, with sixteen 80: columns then wait
+ *  where four have to share a CU (65536 x 1000 gradients 61 to 64 us, with eight 58 to 76, with sixteen 80: columns then wait
  *  for others to end). */
 template <typename Saver, uint32_t AT_ONCE, typename StripRing>
 __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
@@ -288,12 +288,11 @@ __global__ void __launch_bounds__((1 + kWalkLoaders) * kWave)
     const bool chain = lane < kChunkStrip && x0 + lane < g.cols && TakesChain(bare[x0 + lane], g);
     if (__ballot(chain) == 0ull) return;
     const float from = chain && g.begun != 0u ? carry[x0 + lane] : -0.0f;
-    const float sum = mshadow::hip::LowestDmaFold<mshadow::red::sum, StripRing, true>(lds.strip, src, g.stride, g.rows, g.cols, x0,
-                                                                                      chain, from);
-    if (wave == 0 && chain) {
-      if (g.more != 0u) carry[x0 + lane] = sum;
-      else Saver::template Save<float>(dst[x0 + lane], sum * scale);
-    }
+    mshadow::hip::LowestDmaFold<mshadow::red::sum, StripRing, true>(
+        lds.strip, src, g.stride, g.rows, g.cols, x0, chain, from, [=](float sum, uint32_t l) {
+          if (g.more != 0u) carry[x0 + l] = sum;
+          else Saver::template Save<float>(dst[x0 + l], sum * scale);
+        });
     return;
   }
   WalkBlock *ring = lds.ring;

@@ -93,11 +93,11 @@ __device__ __forceinline__ void BareBarrier() { asm volatile("s_barrier" ::: "me
  * four rows: lane l fetches row 4 g + (l & 3), column l >> 2, so the slot holds
  * [group][column][row & 3] and a chain lane reads rows 4g..4g+3 of its column as one
  * 128-bit word, 64 floats from the next group. */
-/*! \brief a workgroup of 1 + Ring::kLoaders waves; lane l of wave 0 folds column x0 + l if that is `wanted`. BEGUN: on from
- *  `res`; else from the first row. */
-template <typename Reducer, typename Ring, bool BEGUN>
-__device__ __forceinline__ float LowestDmaFold(float (*ring)[Ring::kElems], const float *src, uint32_t stride, uint32_t rows,
-                                               uint32_t cols, uint32_t x0, bool wanted, float res) {
+/*! \brief a workgroup of 1 + Ring::kLoaders waves; lane l of wave 0 folds column x0 + l if that is `wanted`, and calls
+ *  done(result, l). BEGUN: on from `res`; else from the first row. */
+template <typename Reducer, typename Ring, bool BEGUN, typename Done>
+__device__ __forceinline__ void LowestDmaFold(float (*ring)[Ring::kElems], const float *src, uint32_t stride, uint32_t rows,
+                                              uint32_t cols, uint32_t x0, bool wanted, float res, Done done) {
   const int kDmaSlots = Ring::kSlots, kDmaAhead = Ring::kAhead, kDmaPerWave = Ring::kPerWave;
   const int CW = kLowestCols;
   const int TR = Ring::kElems / CW;
@@ -146,8 +146,8 @@ __device__ __forceinline__ float LowestDmaFold(float (*ring)[Ring::kElems], cons
         ChainFold<Reducer, kWave>(res, mine, begin, count);
       }
     }
+    if (chain_lane) done(res, lane);
   }
-  return res;
 }
 template <typename Saver, typename Reducer>
 __global__ void __launch_bounds__(kDmaThreads)
@@ -155,10 +155,9 @@ __global__ void __launch_bounds__(kDmaThreads)
                               uint32_t cols, float scale) {
   __shared__ MSHADOW_ALIGNED(16) float ring[LowestRing::kSlots][LowestRing::kElems];
   const uint32_t x0 = StripOfBlock(blockIdx.x, gridDim.x) * kLowestCols;
-  const float res = LowestDmaFold<Reducer, LowestRing, false>(ring, src, stride, rows, cols, x0, true, 0.0f);
-  if (threadIdx.x < static_cast<uint32_t>(kLowestCols) && x0 + threadIdx.x < cols) {
-    Saver::template Save<float>(dst[x0 + threadIdx.x], res * scale);
-  }
+  LowestDmaFold<Reducer, LowestRing, false>(
+      ring, src, stride, rows, cols, x0, true, 0.0f,
+      [=](float res, uint32_t lane) { Saver::template Save<float>(dst[x0 + lane], res * scale); });
 }
 
 /* ------------------------------------------------------------------ KeepLowest in strips
