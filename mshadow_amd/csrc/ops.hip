@@ -1033,17 +1033,17 @@ int mshadow_hip_reduce_keep_lowest_f32(float *dst, const float *src, int sstride
                      dim3(mshadow::hip::STRIP::kThreads), 0, s, dst, src,                       \
                      static_cast<uint32_t>(sstride), static_cast<uint32_t>(rows),               \
                      static_cast<uint32_t>(cols), scale)
+      if (std::is_same<R, mshadow::red::sum>::value &&
+          LaunchColumnChunks<S>(dst, src, static_cast<uint32_t>(sstride), static_cast<uint32_t>(rows),
+                                static_cast<uint32_t>(cols), scale, s)) {
+        return MSHADOW_HIP_OK;
+      }
       /* a strip for each CU at most and a long chain: four rows to an LDS read and stages of
          512 rows make its step 3.5 instead of 4.2 ns (65536 x 1000: 231 against 276 us;
          8191 x 1000: 36.7 against 38.2 us; level at 6000; 4096 x 2000: 22 against 20 us). The fewer
          lines a row has the sooner they arrive and the earlier the step decides (10 columns:
          4000 rows 18.9 against 19.5 us, 6143 27.7 against 28.7, 3500 level; 64: 6000 rows 27.2
          against 27.8, 4500 level; one: 2500 rows 12.8 against 13.5, 2200 12.7 against 12.1) */
-      if (std::is_same<R, mshadow::red::sum>::value &&
-          LaunchColumnChunks<S>(dst, src, static_cast<uint32_t>(sstride), static_cast<uint32_t>(rows),
-                                static_cast<uint32_t>(cols), scale, s)) {
-        return MSHADOW_HIP_OK;
-      }
       const int long_chain = cols == 1 ? 2400 : cols <= 64 ? 4000 : kDmaMinRows;
       if (strip == 16 && rows >= long_chain) {
         LaunchKernelIfFits((mshadow::hip::ReduceKeepLowestDmaKernel<S, R>),

@@ -751,8 +751,8 @@ __global__ void __launch_bounds__(kPatchBlock)
 /*! \brief EPT consecutive column-matrix elements per thread, wherever patch rows end; grid.x = rows of the column
  *  matrix (c, a, b) times `chunks` pieces of kPatchBlock * EPT columns each. For patch rows shorter than a pack, which
  *  the other kernels would write element by element: 3x3 stride 2 on (96,112,48,13) binary16, patch rows of 7, 52 us staged.
- *  An element is a load of its own, all of a thread's under way together (one that is outside the image reads its
- *  channel's first and is dropped); neighbouring lanes find them in the same cache lines. */
+ *  An element is a load of its own, all of a thread's under way together (one that is outside the image reads the
+ *  tensor's first and is dropped); neighbouring lanes find them in the same cache lines. */
 template <typename T, int EPT>
 __global__ void __launch_bounds__(kPatchBlock)
     Im2ColKernel(T *col, int cstride, const T *img, int istride, PatchGeom g, unsigned chunks, mshadow::FastDivU32 div_chunks,
